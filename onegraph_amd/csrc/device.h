@@ -22,14 +22,14 @@ namespace og {
 
 constexpr int kWave = 64;
 constexpr int kBlock = 256;             // threads per block of the frontier kernels
-// Frontier compaction windows: each thread of a count / write workgroup
-// takes FV uint4 loads of flags (16 * FV vertices), so a workgroup covers
-// kBlock * 16 * FV vertices.  Graphs up to kSmallFrontierV vertices use
-// FV = 1 (more, shorter-lived workgroups: their rounds are latency bound);
-// larger ones FV = 2 (half the blocks for the single-workgroup scan).
+// Frontier compaction: a workgroup of kCompactBlock threads takes NW windows
+// of four vertices per thread.  Graphs up to kSmallFrontierV vertices use one
+// (their rounds are latency bound); larger ones four (a quarter of the
+// workgroups that reserve list places one after another).
+constexpr int kCompactBlock = 1024;
 constexpr uint64_t kSmallFrontierV = 1ull << 22;
-constexpr int frontier_fv(uint64_t V) { return V <= kSmallFrontierV ? 1 : 2; }
-constexpr uint64_t verts_per_block(int fv) { return (uint64_t)kBlock * 16 * fv; }
+constexpr int compact_nw(uint64_t V) { return V <= kSmallFrontierV ? 1 : 4; }
+constexpr uint64_t verts_per_block(int nw) { return 4ull * kCompactBlock * nw; }
 constexpr int kDynEdgesPerThread = 8;   // dynamic relax: edges per lane
 constexpr int kDynEdgesPerBlock = kBlock * kDynEdgesPerThread;
 constexpr int kMaxSlots = 16;           // staging slots of the dynamic-region pipeline
@@ -114,12 +114,12 @@ struct FrontierInfo {
     uint32_t nfar;          // active vertices held back (value >= threshold)
     uint32_t min_far;       // smallest value among them
     uint32_t live;          // 1 while active or held-back vertices remain
-    uint32_t dyn_held;      // 1: the dynamic list was held back this round (n[3] = 0)
-    uint32_t pull;          // 1: BFS round runs bottom-up (the lists are not built)
+    uint32_t dyn_held;      // 1: dynamic vertices were held back this round
+    uint32_t pull;          // 1: BFS round runs bottom-up (the lists are not read)
     uint32_t heavy;         // 1: light/heavy split, this round relaxes heavy edges
 };
 
-// Device-resident driver state of one traversal.  The scan of each
+// Device-resident driver state of one traversal.  The end of each
 // compaction advances it, so rounds can be enqueued without a host round
 // trip: the near-far threshold moves on the device and the statistics the
 // host used to add up per round accumulate here.
@@ -148,47 +148,58 @@ struct RoundCtl {
     uint64_t static_work_edges;  // ... over the static bins
     uint64_t dyn_rounds;         // rounds with a dynamic list
     uint32_t halt;               // 1 (device-driven runs): once a compaction finds nothing live, the
-                                 // count passes of rounds enqueued past the end skip their sweep
-    uint32_t pad_;
+                                 // compactions of rounds enqueued past the end skip their sweep
+    uint32_t hold;               // defer 1: the next compaction holds the dynamic vertices back
 };
 
-constexpr int kBcntRows = 5;            // per-block rows: bins 0-3, any flag
-constexpr uint32_t kSbBlocks = 64;      // compaction blocks per super-block (one lane each in the write pass)
-constexpr int kSbVals = 9;              // super-block totals: bins 0|1, bins 2|3, dynamic degrees, zero, hub,
-                                        // far, static degrees, lagging, min far
-constexpr uint8_t kCode0 = 2;           // count pass: flag byte = kCode0 + bin of the vertex
+constexpr uint32_t kDeferOnce = 3;      // RoundCtl::defer: hold the dynamic vertices back until the static region
+                                        // has settled once
 
-// Per-block and per-super-block counts of the compaction passes.
-struct BlockCounts {
-    uint32_t *bcnt;
-    uint64_t *bdeg;
-    uint64_t *sbt;
-    uint64_t *sbp;
-    uint32_t nblk, nsb;
+// Totals of one compaction, in 128-byte lines so that the device-scope
+// atomics of different totals do not queue behind each other: list
+// reservations (bins 0|1, hub tiles|hub vertices, the dynamic list's
+// vertices|edges, their wide form), arrivals, and kTotSlots slots of the
+// sums that nothing is reserved with (vertices without edges | held back,
+// static degrees, lagging | held dynamic vertices, smallest held-back value),
+// block b adding to slot b % kTotSlots.
+constexpr uint32_t kTotLine = 16;                  // u64 per line
+constexpr uint32_t kTotBins = 0 * kTotLine;
+constexpr uint32_t kTotTiles = 1 * kTotLine;
+constexpr uint32_t kTotDyn = 2 * kTotLine;
+constexpr uint32_t kTotWide = 3 * kTotLine;        // lock, vertices, edges
+constexpr uint32_t kTotRoot = 4 * kTotLine;        // arrived groups
+constexpr uint32_t kTotSlot = 8 * kTotLine;
+constexpr uint32_t kTotSlots = 32;
+constexpr uint32_t kTotArrive = kTotSlot + kTotSlots * kTotLine;  // arrivals per group of kTotGroup blocks
+constexpr uint32_t kTotGroup = 32;
+constexpr uint64_t totals_words(uint64_t nblk) {
+    return kTotArrive + (nblk + kTotGroup - 1) / kTotGroup * kTotLine;
+}
+struct CompactTotals {
+    unsigned long long *t;
+    uint32_t nblk;
+    uint32_t dsh;  // dynamic list: vertices in the low dsh bits of one word, edges above; 0: the wide form
 };
+constexpr uint32_t bits_of(uint64_t x) { return x ? 64u - (uint32_t)__builtin_clzll(x) : 0u; }
 
 // Buffers of one frontier traversal: next-frontier flags, the compacted bin
-// lists, the dynamic degree prefix and the per-block scan scratch.  A graph's
+// lists, the dynamic degree prefix and the compaction's totals.  A graph's
 // single-source runs use DeviceState::fr; each serving engine owns its own so
 // that engines can iterate concurrently on different streams.
 struct Frontier {
     uint8_t *flag = nullptr;         // Vpad next-frontier flags
     uint8_t *hflag = nullptr;        // Vpad light/heavy split: heavy-pending flags
-    uint32_t *list = nullptr;        // V: bin0 | bin1 | dynamic lists
+    uint32_t *list = nullptr;        // V: bin 0 up from 0, bin 1 down from vsplit - 1, dynamic list up from vsplit
     uint64_t *hub = nullptr;         // hub tiles (tile << 32 | vertex)
     uint64_t hub_cap = 0;
     uint64_t *doff = nullptr;        // V + 1 degree prefix of the dynamic list
     uint32_t *dchunk = nullptr;      // list entry holding edge c * kDynEdgesPerBlock of the dynamic edge space
     uint64_t dchunk_cap = 0;
-    uint32_t *bcnt = nullptr;        // kBcntRows * nblk per-block counts
-    uint64_t *bdeg = nullptr;        // nblk per-block dynamic degree sums
-    uint64_t *sbt = nullptr;         // kSbVals * nsb super-block totals (added by the count pass; zero, the
-                                     // min row all ones, between compactions)
-    uint64_t *sbp = nullptr;         // 3 * nsb super-block exclusive prefixes (bins 0|1, 2|3, dynamic degrees)
+    unsigned long long *tot = nullptr;  // compaction totals (cleared between compactions)
     uint32_t nblk = 0;
-    uint32_t nsb = 0;
-    BlockCounts counts() const { return BlockCounts{bcnt, bdeg, sbt, sbp, nblk, nsb}; }
-    uint32_t fv = 2;                 // flag vectors per thread of the compaction (frontier_fv)
+    uint32_t dsh = 0;
+    CompactTotals totals() const { return CompactTotals{tot, nblk, dsh}; }
+    uint32_t nw = 4;                 // windows per workgroup of the compaction (compact_nw)
     uint64_t V = 0;
     FrontierInfo *info = nullptr;
     FrontierInfo *h_info = nullptr;  // pinned
@@ -312,7 +323,7 @@ struct DeviceState {
     void *m_edges = nullptr;
 
     // per-vertex state
-    uint32_t *d_val = nullptr;       // V
+    uint32_t *d_val = nullptr;       // Vpad
     Frontier fr;                     // frontier buffers of single-source / batch runs
 
     // pinned host mirrors of the dynamic list
@@ -376,6 +387,42 @@ __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t x, int m) {
     uint32_t lo = (uint32_t)x, hi = (uint32_t)(x >> 32);
     lo = __shfl_xor(lo, m, kWave);
     hi = __shfl_xor(hi, m, kWave);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// Inclusive scan over the wave with DPP moves (rows of 16 lanes, then the
+// rows' last lanes broadcast): no LDS round trips.
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t x) {
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, false);  // row_shr:1
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, false);  // row_shr:2
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, false);  // row_shr:4
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, false);  // row_shr:8
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false);  // row_bcast:15 to rows 1, 3
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false);  // row_bcast:31 to rows 2, 3
+    return x;
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint64_t dpp_add_u64(uint64_t x) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, ROWS, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), CTRL, ROWS, 0xF, false);
+    return x + (((uint64_t)hi << 32) | lo);
+}
+
+__device__ __forceinline__ uint64_t wave_scan_u64(uint64_t x) {
+    x = dpp_add_u64<0x111, 0xF>(x);
+    x = dpp_add_u64<0x112, 0xF>(x);
+    x = dpp_add_u64<0x114, 0xF>(x);
+    x = dpp_add_u64<0x118, 0xF>(x);
+    x = dpp_add_u64<0x142, 0xA>(x);
+    x = dpp_add_u64<0x143, 0xC>(x);
+    return x;
+}
+
+// Lane l's value (l the same for the whole wave).
+__device__ __forceinline__ uint64_t wave_read_u64(uint64_t x, int l) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), l);
     return ((uint64_t)hi << 32) | lo;
 }
 
@@ -548,7 +595,7 @@ void lane_run_sssp(og_graph *g, DeviceState *lane, uint32_t src, uint32_t *out, 
 void frontier_begin(Frontier &f, hipStream_t s, uint32_t delta, uint32_t defer = 0, uint64_t dir_opt_edges = 0,
                     bool split = false);
 
-// One compaction: flags -> bin lists / hub tiles / sorted dynamic list with
+// One compaction: flags -> bin lists / hub tiles / dynamic list with
 // its degree prefix, flags cleared; f.info and f.ctl updated on the device.
 // With `val` non-null, vertices whose value is >= f.ctl->thresh stay flagged
 // and are only counted (near-far order).  With to_host, the summary is also

@@ -4,10 +4,9 @@
 // memory through a double-buffered staging area on a copy stream.
 //
 // One iteration (reference loop: BFS/oneGraph_BFS/CalculateOpt.h:75-188):
-//   1. k_frontier_count / k_frontier_scan (one workgroup) / k_frontier_write:
-//      two passes over the next-frontier flags build the
-//      static bin lists (ordered), the hub tile list, the sorted dynamic list
-//      and its degree prefix, and clear the flags.  Replaces K1-K6
+//   1. k_frontier_compact: one pass over the next-frontier flags builds the
+//      static bin lists, the hub tile list, the dynamic list (in vertex order
+//      within windows) and its degree prefix, and clears the flags.  Replaces K1-K6
 //      (gpu_kernels.h:243-379), the host prefix H4 (CalculateOpt.h:110-123)
 //      and every per-iteration .wait(): counts stay on the device, and rounds
 //      without a host-side loader are replayed from captured hipGraphs.
@@ -52,527 +51,459 @@ __global__ void k_set_source(uint32_t *val, uint8_t *flag, uint32_t src) {
     flag[src] = 1;
 }
 
-// Per-thread flag window: 16 * FV consecutive vertices.
-template <int FV>
-__device__ __forceinline__ void load_flags(const uint8_t *flag, uint64_t base, uint64_t Vpad, uint4 (&w)[FV]) {
-#pragma unroll
-    for (int k = 0; k < FV; ++k) {
-        uint64_t at = base + 16ull * k;
-        w[k] = at < Vpad ? *(const uint4 *)(flag + at) : make_uint4(0, 0, 0, 0);
-    }
-}
-
-template <int FV>
-__device__ __forceinline__ void store_flags(uint8_t *flag, uint64_t base, uint64_t Vpad,
-                                            const uint32_t (&word)[4 * FV]) {
-#pragma unroll
-    for (int k = 0; k < FV; ++k) {
-        const uint64_t at = base + 16ull * k;
-        if (at < Vpad)
-            *(uint4 *)(flag + at) = make_uint4(word[4 * k], word[4 * k + 1], word[4 * k + 2], word[4 * k + 3]);
-    }
-}
-
 // Bin of an active vertex: 0..2 static bins, 3 dynamic, 4 no out-edges,
 // 5 held back for a later round (near-far order: value >= threshold, checked
-// first so that held-back vertices need no degree).
-__device__ __forceinline__ int bin_of(bool far, uint64_t v, uint64_t vsplit, uint64_t deg, const Tuning &tn) {
+// first so that held-back vertices need no degree), 6 a dynamic vertex held
+// back by the deferred order.
+__device__ __forceinline__ int bin_of(bool far, bool hold, uint64_t v, uint64_t vsplit, uint64_t deg,
+                                      const Tuning &tn) {
     if (far) return 5;
     if (deg == 0) return 4;
-    if (v >= vsplit) return 3;
+    if (v >= vsplit) return hold ? 6 : 3;
     if (deg <= tn.t1) return 0;
     if (deg <= tn.t2) return 1;
     return 2;
 }
 
-__device__ __forceinline__ uint32_t block_min_u32(uint32_t x, uint64_t *lds) {
-#pragma unroll
-    for (int m = 1; m < kWave; m <<= 1) x = min(x, (uint32_t)__shfl_xor(x, m, kWave));
-    __syncthreads();
-    if ((threadIdx.x & (kWave - 1)) == 0) lds[threadIdx.x / kWave] = x;
-    __syncthreads();
-    uint32_t r = 0xFFFFFFFFu;
-    for (int w = 0; w < (int)(blockDim.x / kWave); ++w) r = min(r, (uint32_t)lds[w]);
-    __syncthreads();
-    return r;
-}
+// Waits until the wave's memory operations, atomics among them, are done.
+// With device-scope atomics on both sides (performed at one place for the
+// whole device) this orders a workgroup's reservations before its arrival
+// without a release fence, which on gfx950 writes the whole L2 of the XCD
+// back.
+__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-constexpr int kLoadBatch = 8;  // flagged vertices whose row bounds are read together
-
-// Bit j set when byte j of the thread's flag window is >= lo.  The passes
-// then walk the set bits only (lowest first, i.e. in vertex order), which
-// keeps their code small: a per-slot unrolled switch over 32 slots does not
-// fit the instruction cache.
-template <int FV>
-__device__ __forceinline__ uint32_t window_mask(const uint4 (&w)[FV], uint32_t lo) {
-    uint32_t m = 0;
-#pragma unroll
-    for (int k = 0; k < FV; ++k) {
-        const uint32_t q[4] = {w[k].x, w[k].y, w[k].z, w[k].w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-                m |= (((q[i] >> (8 * b)) & 0xFFu) >= lo ? 1u : 0u) << (16 * k + 4 * i + b);
+// Reserves n entries with dd edges at the end of the dynamic list; the two
+// counts move together, so the list's degree prefix rises with the list.
+// One word holds both when they fit (count in the low dsh bits); else a lock
+// guards two words: its holder waits for nothing, so every waiter gets it.
+__device__ __forceinline__ void reserve_dyn(const CompactTotals &ct, uint64_t n, uint64_t dd, uint64_t &p, uint64_t &pd) {
+    unsigned long long *t = ct.t;
+    if (ct.dsh) {
+        const uint64_t old = atomicAdd(t + kTotDyn, (unsigned long long)(n | (dd << ct.dsh)));
+        p = old & ((1ull << ct.dsh) - 1);
+        pd = old >> ct.dsh;
+        return;
     }
-    return m;
+    while (atomicCAS(t + kTotWide, 0ull, 1ull) != 0) __builtin_amdgcn_s_sleep(2);
+    p = atomicAdd(t + kTotWide + 1, (unsigned long long)n);
+    pd = atomicAdd(t + kTotWide + 2, (unsigned long long)dd);
+    wait_vmem();
+    atomicExch(t + kTotWide, 0ull);
 }
 
-__device__ void scan_counts(const BlockCounts &bc, FrontierInfo *__restrict__ info, uint64_t *__restrict__ doff,
-                            RoundCtl *__restrict__ ctl, uint64_t *__restrict__ m_doff, uint64_t *lds);
-
-// Most lanes of the one-workgroup scan, one per super-block
-constexpr uint32_t kScanThreads = 1024;
-
-// Super-block totals between compactions: sums zero, the min row all ones.
-__global__ void k_sb_init(uint64_t *sbt, uint32_t nsb) {
-    const uint64_t n = (uint64_t)kSbVals * nsb;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        sbt[i] = i / nsb == kSbVals - 1 ? ~0ull : 0ull;
+// True in the workgroup that arrives last (called by one thread of each).
+// Arrivals are counted in two levels, kTotGroup workgroups per first-level
+// counter: same-address atomics take about 12 ns each.
+__device__ __forceinline__ bool arrive_last(const CompactTotals &ct) {
+    const uint32_t g = blockIdx.x / kTotGroup, ng = (ct.nblk + kTotGroup - 1) / kTotGroup;
+    unsigned long long *at = ct.t + kTotArrive + (uint64_t)g * kTotLine;
+    if (atomicAdd(at, 1ull) + 1 != min(kTotGroup, ct.nblk - g * kTotGroup)) return false;
+    atomicExch(at, 0ull);
+    if (ng > 1) {
+        if (atomicAdd(ct.t + kTotRoot, 1ull) + 1 != ng) return false;
+        atomicExch(ct.t + kTotRoot, 0ull);
+    }
+    return true;
 }
 
-// Compaction pass 1: classifies every flagged vertex of the block's window,
-// stores kCode0 + bin in its flag byte and publishes the per-block counts.
-// The window's flags are loaded 16 bytes per lane and transposed through
-// LDS, so that slot j of thread t is vertex j * kBlock + t of the window:
-// consecutive lanes then read consecutive row bounds and values and store
-// consecutive flag bytes (only the block totals depend on the mapping).  Row
-// bounds (and values, for near-far) of kLoadBatch flagged vertices are read
-// before any is used, so their latencies overlap.
-template <int FV>
-__global__ __launch_bounds__(kBlock) void k_frontier_count(uint8_t *__restrict__ flag_a, uint8_t *__restrict__ hflag,
-                                                           uint64_t Vpad, uint64_t vsplit,
-                                                           const uint64_t *__restrict__ ptr,
-                                                           const uint64_t *__restrict__ pmid,
-                                                           const uint32_t *__restrict__ deg,
-                                                           const uint32_t *__restrict__ hdeg, Tuning tn,
-                                                           const uint32_t *__restrict__ val_a,
-                                                           const RoundCtl *__restrict__ ctl, BlockCounts bc) {
-    const uint32_t nblk = bc.nblk;
-    __shared__ uint64_t lds[6 * kBlock / kWave];
-    __shared__ uint4 s_win[(kBlock * 16 * FV) / 16];  // the window's flag bytes
-    // a round enqueued after the traversal ended: no vertex is flagged and
-    // the block counts of the last pass (all zero) stand
+// Totals between compactions: zero, each slot's smallest held-back value all
+// ones.
+__global__ void k_totals_init(unsigned long long *t, uint64_t n) {
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+        const bool far = i >= kTotSlot && i < kTotArrive && i % kTotLine == 3;
+        t[i] = far ? ~0ull : 0ull;
+    }
+}
+
+// End of a compaction, run by the first wave of the workgroup that arrived
+// last: takes the totals (leaving them cleared for the next compaction),
+// publishes the round's summary and advances the traversal state: statistics,
+// liveness, the BFS direction and, when the near set is empty but vertices
+// are held back, the near-far threshold (min held-back value + delta) for
+// the next compaction.
+__device__ __forceinline__ void compact_finish(const CompactTotals &ct, FrontierInfo *__restrict__ info,
+                                               uint64_t *__restrict__ doff, RoundCtl *__restrict__ ctl) {
+    const uint32_t lane = threadIdx.x;
+    RoundCtl c = *ctl;
+    uint64_t zf = 0, sd = 0, lh = 0, mf = ~0ull, a01 = 0, ath = 0, dyn = 0, wn = 0, wd = 0;
+    if (lane < kTotSlots && lane < ct.nblk) {
+        unsigned long long *sl = ct.t + kTotSlot + lane * kTotLine;
+        zf = atomicExch(sl + 0, 0ull);
+        sd = atomicExch(sl + 1, 0ull);
+        lh = atomicExch(sl + 2, 0ull);
+        mf = atomicExch(sl + 3, ~0ull);
+    }
+    if (lane == 0) {
+        a01 = atomicExch(ct.t + kTotBins, 0ull);
+        ath = atomicExch(ct.t + kTotTiles, 0ull);
+        if (ct.dsh) {
+            dyn = atomicExch(ct.t + kTotDyn, 0ull);
+            wn = dyn & ((1ull << ct.dsh) - 1);
+            wd = dyn >> ct.dsh;
+        } else {
+            wn = atomicExch(ct.t + kTotWide + 1, 0ull);
+            wd = atomicExch(ct.t + kTotWide + 2, 0ull);
+        }
+    }
+#pragma unroll
+    for (int m = 1; m < (int)kTotSlots; m <<= 1) {
+        zf += shfl_xor_u64(zf, m);
+        sd += shfl_xor_u64(sd, m);
+        lh += shfl_xor_u64(lh, m);
+        mf = min(mf, shfl_xor_u64(mf, m));
+    }
+    if (lane != 0) return;
+    FrontierInfo fi;
+    fi.n[0] = (uint32_t)a01;
+    fi.n[1] = (uint32_t)(a01 >> 32);
+    fi.n[2] = (uint32_t)ath;
+    fi.n[3] = (uint32_t)wn;
+    fi.nzero = (uint32_t)zf;
+    fi.nhub = (uint32_t)(ath >> 32);
+    fi.static_deg = sd;
+    fi.dyn_deg = wd;
+    fi.nfar = (uint32_t)(zf >> 32);
+    fi.min_far = (uint32_t)min(mf, (uint64_t)0xFFFFFFFFull);
+    const uint32_t lagging = (uint32_t)lh, hd = (uint32_t)(lh >> 32);
+    fi.dyn_held = hd ? 1u : 0u;
+    const uint64_t snodes = (uint64_t)fi.n[0] + fi.n[1] + fi.nhub;
+    const bool was_heavy = c.mode != 0;
+    const uint64_t active = snodes + fi.n[3] + fi.nzero;
+    // light/heavy split: light rounds count the vertices they relax (they
+    // turn heavy-pending); once a bucket's light rounds find nothing near,
+    // the next compaction collects the heavy-pending vertices (their
+    // distances are final within the bucket) before the threshold moves
+    bool heavy_next = false;
+    if (c.split) {
+        if (was_heavy) {
+            c.hpend = 0;
+        } else if (active) {
+            c.hpend += active;
+        } else if (c.hpend && !hd) {
+            heavy_next = true;
+        }
+    }
+    // (after a heavy round a light compaction always follows: the held-back
+    // vertices sit in the other flag array)
+    fi.live = (active || fi.nfar || hd || heavy_next || was_heavy) ? 1u : 0u;
+    // BFS direction (Beamer et al., SC'12): bottom-up once the frontier's
+    // edges exceed 1/14 of the unexplored ones, back to top-down when
+    // the frontier falls below V / 24.
+    fi.pull = 0;
+    fi.heavy = c.mode;
+    if (c.dir_opt && active) {
+        const uint64_t mf2 = fi.static_deg + fi.dyn_deg;
+        if (!c.pull && mf2 > c.unexplored / 14) c.pull = 1;
+        else if (c.pull && active < c.nverts / 24) c.pull = 0;
+        c.unexplored -= min(mf2, c.unexplored);
+        fi.pull = c.pull;
+        c.pull_rounds += c.pull;
+    }
+    *info = fi;
+    doff[fi.n[3]] = fi.dyn_deg;
+    c.compactions++;
+    c.live = fi.live;
+    if (active) {
+        c.rounds++;
+        c.node_sum += active;
+        c.static_node_sum += snodes;
+        c.dyn_node_sum += fi.n[3];
+        c.work_edges += fi.static_deg + fi.dyn_deg;
+        c.static_work_edges += fi.static_deg;
+        c.dyn_rounds += fi.n[3] ? 1 : 0;
+    } else if (heavy_next || hd) {
+        // the threshold stays: a heavy round's offers are all >= it, and held
+        // dynamic vertices are below it
+    } else if (fi.nfar && c.delta) {
+        // Near set empty.  Lagged order: every vertex below the threshold
+        // has relaxed except the waiting dynamic ones, which go next (a
+        // static vertex they improve is below the threshold and joins
+        // them).  Otherwise every held-back value is >= the threshold and
+        // it moves to the smallest of them + delta.
+        if (lagging) c.fbound = c.thresh;
+        else c.thresh = (uint32_t)min((uint64_t)0xFFFFFFFFull, (uint64_t)fi.min_far + c.delta);
+    }
+    // deferred order: the dynamic list is held back (its vertices stay
+    // flagged) until a compaction finds nothing else to relax; kDeferOnce
+    // holds it back no more after that
+    if (c.defer == kDeferOnce) c.hold = c.hold && active ? 1u : 0u;
+    else c.hold = c.defer == 1 && !was_heavy && active ? 1u : 0u;
+    c.mode = heavy_next ? 1u : 0u;
+    *ctl = c;
+}
+
+// Frontier compaction, one launch: flags -> bin lists, hub tiles, the dynamic
+// list with its degree prefix and chunk table (dchunk[c]: the list entry
+// holding edge c * kDynEdgesPerBlock of the dynamic edge space); the window's
+// flags become 1 for held-back vertices, 0 elsewhere.
+//
+// A workgroup takes NW windows of kCompactBlock * 4 vertices, thread t the
+// four consecutive ones from 4t of each, whose flags, values and degrees are
+// one 4- or 16-byte load each (consecutive lanes on consecutive addresses)
+// and whose bins stay in registers.  The block's counts reserve their place in
+// each list with one atomic per list: blocks land in the lists in the order
+// of these atomics (within a block in vertex order, so that neighbouring
+// dynamic rows share link lines), and no pass over the other blocks' counts is
+// needed.  Bin 0 grows up from list[0], bin 1 down from list[vsplit - 1], the
+// dynamic list up from list[vsplit].  The workgroup that arrives last finishes
+// the round (compact_finish).
+//
+// What bounds it: on graphs up to a few million vertices, latency: launch,
+// the flag -> value -> degree chain, and three round trips of device-scope
+// atomics (reservation, arrival, totals).  A dense round of a larger graph is
+// bound by the flag, value and degree sweeps and the list stores.  Against the
+// count pass, one-workgroup scan and write pass it replaces: 1 M vertices,
+// dense round 41 -> 12 us, nearly empty 16 -> 7 us; 16.7 M vertices, the 33
+// compactions of an out-of-memory SSSP 1.67 -> 1.13 ms.
+template <int NW>
+__global__ __launch_bounds__(kCompactBlock) void k_frontier_compact(
+    uint8_t *__restrict__ flag_a, uint8_t *__restrict__ hflag, uint64_t Vpad, uint64_t vsplit,
+    const uint64_t *__restrict__ ptr, const uint64_t *__restrict__ pmid, const uint32_t *__restrict__ deg,
+    const uint32_t *__restrict__ hdeg, Tuning tn, const uint32_t *__restrict__ val_a, RoundCtl *ctl, CompactTotals ct,
+    FrontierInfo *__restrict__ info, uint32_t *__restrict__ list, uint64_t *__restrict__ hub, uint64_t hub_cap,
+    uint64_t *__restrict__ doff, uint32_t *__restrict__ dchunk, uint64_t dchunk_cap) {
+    constexpr int kWaves = kCompactBlock / kWave;
+    static_assert(NW * kWaves <= kWave, "one lane per (window, wave)");
+    __shared__ uint64_t s_cnt[NW * kWaves], s_deg[NW * kWaves];  // per window and wave: packed counts, degrees
+    __shared__ uint32_t s_tile[NW * kWaves];
+    __shared__ unsigned long long s_stat[2];  // static degrees, packed statistics
+    __shared__ uint32_t s_more[3];            // lagging, held, smallest held-back value
+    __shared__ uint64_t s_base[4];            // reserved places: bins 0 | 1, tiles, dynamic list, its edges
+    // a round enqueued after the traversal ended: no vertex is flagged, and
+    // the summary and the traversal state stand
     if (ctl->halt && !ctl->live) return;
     // light/heavy split: a heavy compaction collects the heavy-pending
     // vertices (no near-far test) and sizes them by their heavy edges
     const bool heavy = pmid && ctl->mode;
+    const bool mark = pmid && !heavy;  // light round: relaxed vertices turn heavy-pending
     uint8_t *flag = heavy ? hflag : flag_a;
     const uint32_t *val = heavy ? nullptr : val_a;
-    const uint64_t wbase = (uint64_t)blockIdx.x * (kBlock * 16 * FV);
-    uint4 w[FV];
-    load_flags(flag, wbase + (uint64_t)threadIdx.x * (16 * FV), Vpad, w);
-    uint32_t nz = 0;
+    const uint64_t v0 = ((uint64_t)blockIdx.x * NW * kCompactBlock + threadIdx.x) * 4;  // window q: v0 + q * kWin
+    constexpr uint64_t kWin = (uint64_t)kCompactBlock * 4;
+    uint32_t fw[NW], any = 0;
 #pragma unroll
-    for (int k = 0; k < FV; ++k) nz |= w[k].x | w[k].y | w[k].z | w[k].w;
-    // a window without flags (most of them in a small round) publishes zero
-    // counts without the transpose and the block scans; the write pass
-    // skips it by row 7
-    if (!__syncthreads_or(nz != 0)) {
-        if (threadIdx.x == 0) {
+    for (int q = 0; q < NW; ++q) fw[q] = v0 + q * kWin < Vpad ? *(const uint32_t *)(flag + v0 + q * kWin) : 0u;
 #pragma unroll
-            for (int r = 0; r < kBcntRows; ++r) bc.bcnt[r * nblk + blockIdx.x] = 0;
-            bc.bdeg[blockIdx.x] = 0;
+    for (int q = 0; q < NW; ++q) any |= fw[q];
+    if (threadIdx.x < 2) s_stat[threadIdx.x] = 0;
+    if (threadIdx.x < 3) s_more[threadIdx.x] = threadIdx.x == 2 ? 0xFFFFFFFFu : 0u;
+    if (!__syncthreads_or(any != 0)) {  // no flags here (most blocks in a small round)
+        if (threadIdx.x < kWave) {
+            const bool last = threadIdx.x == 0 && arrive_last(ct);
+            if (__ballot(last)) compact_finish(ct, info, doff, ctl);
         }
         return;
     }
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    uint32_t bins[NW];  // byte j: bin of vertex j of the window, 7 when not flagged
+    uint64_t dg[NW][4];
+    uint32_t c01[NW], c3[NW], tiles[NW];  // c01: bin 0 | bin 1 << 16
+    uint64_t ddeg[NW];
+    uint64_t stat = 0, sdeg = 0;          // stat: zero | hub << 16 | far << 32 | lagging << 48
+    uint32_t held = 0, mf = 0xFFFFFFFFu;
+    const uint32_t thresh = val ? ctl->thresh : 0xFFFFFFFFu;
+    const bool hold = !heavy && ctl->hold;
+    // lagged order: a dynamic vertex below the threshold but not below fbound
+    // waits until the static part of its bucket has settled
+    const bool lagged = val && ctl->defer == 2;
+    const uint32_t fbound = lagged ? ctl->fbound : 0u;
+    uint4 vv[NW];
+    if (val) {
 #pragma unroll
-    for (int k = 0; k < FV; ++k) s_win[threadIdx.x * FV + k] = w[k];
+        for (int q = 0; q < NW; ++q)  // (the value array is padded to Vpad entries)
+            if (fw[q]) vv[q] = *(const uint4 *)(val + v0 + q * kWin);
+    }
+    uint32_t farm = 0;  // bit 4q + j: held back by its value
+    if (val) {
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            if (!fw[q]) continue;
+            const uint32_t x[4] = {vv[q].x, vv[q].y, vv[q].z, vv[q].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (!((fw[q] >> (8 * j)) & 0xFFu)) continue;
+                const bool lag = lagged && x[j] < thresh && x[j] >= fbound && v0 + q * kWin + j >= vsplit;
+                const bool far = x[j] >= thresh || lag;
+                stat += lag ? 1ull << 48 : 0ull;
+                if (far) {
+                    mf = min(mf, x[j]);
+                    farm |= 1u << (4 * q + j);
+                }
+            }
+        }
+    }
+    auto near_any = [&](int q) {  // a vertex of window q is flagged and not held back by its value
+        uint32_t f = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) f |= ((fw[q] >> (8 * j)) & 0xFFu) && !((farm >> (4 * q + j)) & 1u) ? 1u : 0u;
+        return f != 0;
+    };
+    const uint32_t *dt = pmid && heavy ? hdeg : deg;
+    const bool whole = !pmid && hdeg;  // whole rows of a split graph
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dg[q][j] = 0;
+        if (!fw[q] || !near_any(q)) continue;
+        const uint64_t v = v0 + q * kWin;
+        if (deg) {
+            const uint4 x = *(const uint4 *)(dt + v);
+            dg[q][0] = x.x;
+            dg[q][1] = x.y;
+            dg[q][2] = x.z;
+            dg[q][3] = x.w;
+            if (whole) {
+                const uint4 y = *(const uint4 *)(hdeg + v);
+                dg[q][0] += y.x;
+                dg[q][1] += y.y;
+                dg[q][2] += y.z;
+                dg[q][3] += y.w;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if ((fw[q] >> (8 * j)) & 0xFFu) dg[q][j] = round_deg(deg, hdeg, ptr, pmid, heavy, v + j);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {
+        bins[q] = 0x07070707u;
+        c01[q] = c3[q] = tiles[q] = 0;
+        ddeg[q] = 0;
+        if (!fw[q]) continue;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (!((fw[q] >> (8 * j)) & 0xFFu)) continue;
+            const uint64_t d = dg[q][j];
+            const int b = bin_of((farm >> (4 * q + j)) & 1u, hold, v0 + q * kWin + j, vsplit, d, tn);
+            bins[q] ^= (uint32_t)(7 ^ b) << (8 * j);
+            switch (b) {
+                case 0: c01[q] += 1; sdeg += d; break;
+                case 1: c01[q] += 1u << 16; sdeg += d; break;
+                case 2: tiles[q] += (uint32_t)((d + tn.tile - 1) / tn.tile); stat += 1ull << 16; sdeg += d; break;
+                case 3: ++c3[q]; ddeg[q] += d; break;
+                case 5: stat += 1ull << 32; break;
+                case 6: ++held; break;
+                default: ++stat; break;
+            }
+        }
+    }
+    // inclusive scans over the wave (a block's packed counts stay below 2^16)
+    uint32_t i01[NW], i3[NW], it[NW];
+    uint64_t id[NW];
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {
+        i01[q] = i3[q] = it[q] = 0;
+        id[q] = 0;
+        if (__ballot(fw[q] != 0)) {
+            i01[q] = wave_scan_u32(c01[q]);
+            if (__ballot(c3[q] != 0)) {
+                i3[q] = wave_scan_u32(c3[q]);
+                id[q] = wave_scan_u64(ddeg[q]);
+            }
+            if (__ballot(tiles[q] != 0)) it[q] = wave_scan_u32(tiles[q]);
+        }
+        if (lane == kWave - 1) {
+            s_cnt[q * kWaves + wid] = (uint64_t)i01[q] | ((uint64_t)i3[q] << 32);
+            s_deg[q * kWaves + wid] = id[q];
+            s_tile[q * kWaves + wid] = it[q];
+        }
+    }
+    if (__ballot(any != 0)) {  // statistics of the wave: one LDS atomic each
+        const uint64_t ws = wave_scan_u64(sdeg), wp = wave_scan_u64(stat);
+        if (lane == kWave - 1) {
+            if (ws) atomicAdd(&s_stat[0], (unsigned long long)ws);
+            if (wp) atomicAdd(&s_stat[1], (unsigned long long)wp);
+        }
+        if (held) atomicAdd(&s_more[1], held);
+        if (mf != 0xFFFFFFFFu) atomicMin(&s_more[2], mf);
+    }
     __syncthreads();
-    const uint8_t *sb = (const uint8_t *)s_win;
-    uint32_t m = 0;
-#pragma unroll
-    for (int j = 0; j < (16 * FV); ++j) m |= (sb[j * kBlock + threadIdx.x] != 0 ? 1u : 0u) << j;
-    const uint64_t base = wbase + threadIdx.x;  // slot j: vertex base + j * kBlock
-    uint32_t c0 = 0, c1 = 0, c2 = 0, c3 = 0, cz = 0, ch = 0, cf = 0, cl = 0, mf = 0xFFFFFFFFu;
-    uint64_t sdeg = 0, ddeg = 0;
-    if (m) {
-        const uint32_t thresh = val ? ctl->thresh : 0xFFFFFFFFu;
-        // lagged order: a dynamic vertex below the threshold but not below
-        // fbound waits until the static part of its bucket has settled
-        const bool lagged = val && ctl->defer == 2;
-        const uint32_t fbound = lagged ? ctl->fbound : 0u;
-        while (m) {
-            uint32_t jj[kLoadBatch];
-            uint64_t dg[kLoadBatch];
-            uint32_t vv[kLoadBatch];
-            bool far[kLoadBatch];
-#pragma unroll
-            for (int k = 0; k < kLoadBatch; ++k) {
-                jj[k] = (16 * FV);  // empty slot
-                dg[k] = 0;
-                vv[k] = 0;
-                if (m) {
-                    const uint32_t j = (uint32_t)__builtin_ctz(m);
-                    m &= m - 1;
-                    jj[k] = j;
-                    if (val) vv[k] = val[base + (uint64_t)j * kBlock];
-                    else dg[k] = round_deg(deg, hdeg, ptr, pmid, heavy, base + (uint64_t)j * kBlock);
-                }
-            }
-            // near-far: a held-back vertex needs only its value, so the
-            // degrees are read for the near ones alone
-#pragma unroll
-            for (int k = 0; k < kLoadBatch; ++k) {
-                far[k] = false;
-                if (jj[k] == (16 * FV) || !val) continue;
-                const bool lag = lagged && vv[k] < thresh && vv[k] >= fbound && base + (uint64_t)jj[k] * kBlock >= vsplit;
-                far[k] = vv[k] >= thresh || lag;
-                if (!far[k]) dg[k] = round_deg(deg, hdeg, ptr, pmid, heavy, base + (uint64_t)jj[k] * kBlock);
-            }
-#pragma unroll
-            for (int k = 0; k < kLoadBatch; ++k) {
-                if (jj[k] == (16 * FV)) continue;
-                const uint64_t d = dg[k];
-                const bool lag = lagged && vv[k] < thresh && vv[k] >= fbound && base + (uint64_t)jj[k] * kBlock >= vsplit;
-                cl += lag ? 1u : 0u;
-                const int b = bin_of(far[k], base + (uint64_t)jj[k] * kBlock, vsplit, d, tn);
-                switch (b) {
-                    case 0: ++c0; sdeg += d; break;
-                    case 1: ++c1; sdeg += d; break;
-                    case 2: c2 += (uint32_t)((d + tn.tile - 1) / tn.tile); ++ch; sdeg += d; break;
-                    case 3: ++c3; ddeg += d; break;
-                    case 5: ++cf; mf = min(mf, vv[k]); break;
-                    default: ++cz; break;
-                }
-                flag[base + (uint64_t)jj[k] * kBlock] = (uint8_t)(kCode0 + b);
-            }
-        }
-    }
-    const uint64_t x[6] = {(uint64_t)c0 | ((uint64_t)c1 << 32), (uint64_t)c2 | ((uint64_t)c3 << 32),
-                           (uint64_t)cz | ((uint64_t)ch << 32), sdeg, ddeg, (uint64_t)cf | ((uint64_t)cl << 16)};
-    uint64_t ex[6], t[6];
-    block_scan_n<6>(x, ex, t, lds);
-    const uint32_t bm = block_min_u32(mf, lds);
-    if (threadIdx.x == 0) {
-        bc.bcnt[0 * nblk + blockIdx.x] = (uint32_t)t[0];
-        bc.bcnt[1 * nblk + blockIdx.x] = (uint32_t)(t[0] >> 32);
-        bc.bcnt[2 * nblk + blockIdx.x] = (uint32_t)t[1];
-        bc.bcnt[3 * nblk + blockIdx.x] = (uint32_t)(t[1] >> 32);
-        bc.bcnt[4 * nblk + blockIdx.x] = 1;
-        bc.bdeg[blockIdx.x] = t[4];
-    }
-    // the block's totals into its super-block's, one lane per value (packed
-    // pairs add without carries: each half stays below 2^32)
-    if (threadIdx.x < (unsigned)kSbVals) {
-        const uint32_t sb = blockIdx.x / kSbBlocks;
-        const uint64_t v[kSbVals] = {t[0], t[1], t[4], (uint32_t)t[2], t[2] >> 32, t[5] & 0xFFFFu, t[3],
-                                     t[5] >> 16, bm};
-        uint64_t x = 0;
-#pragma unroll
-        for (int i = 0; i < kSbVals; ++i)
-            if ((int)threadIdx.x == i) x = v[i];
-        unsigned long long *at = (unsigned long long *)bc.sbt + threadIdx.x * (uint64_t)bc.nsb + sb;
-        if (threadIdx.x == kSbVals - 1) {
-            if (x != 0xFFFFFFFFull) atomicMin(at, (unsigned long long)x);
-        } else if (x) {
-            atomicAdd(at, (unsigned long long)x);
-        }
-    }
-}
-
-// Compaction pass 2: one workgroup scans the counts (scan_counts).  A
-// separate launch rather than a last-workgroup-arrives tail in pass 1: on
-// gfx950 the device-scope release/acquire fences such a tail needs write
-// back and invalidate the whole L2 of each XCD, once per workgroup.
-__global__ __launch_bounds__(kScanThreads) void k_frontier_scan(BlockCounts bc, FrontierInfo *__restrict__ info,
-                                                                uint64_t *__restrict__ doff,
-                                                                RoundCtl *__restrict__ ctl,
-                                                                uint64_t *__restrict__ m_doff) {
-    __shared__ uint64_t lds[8 * kScanThreads / kWave];
-    scan_counts(bc, info, doff, ctl, m_doff, lds);
-}
-
-// Compaction pass 2 body: one workgroup turns the per-block counts into
-// exclusive offsets (in place), publishes
-// the round's summary and advances the traversal state: statistics,
-// liveness, the BFS direction and, when the near set is empty but vertices
-// are held back, the near-far threshold (min held-back value + delta) for
-// the next compaction.  Each thread scans a run of consecutive blocks, so the
-// whole pass is one multi-value block scan.  `lds` holds 8 * blockDim / 64.
-__device__ void scan_counts(const BlockCounts &bc, FrontierInfo *__restrict__ info, uint64_t *__restrict__ doff,
-                            RoundCtl *__restrict__ ctl, uint64_t *__restrict__ m_doff, uint64_t *lds) {
-    // a round enqueued after the traversal ended (its count pass returned at
-    // once): the summary and the traversal state stand
-    if (ctl->halt && !ctl->live) return;
-    const uint32_t nsb = bc.nsb;
-    const uint64_t *sbt = bc.sbt;
-    const uint32_t per = (nsb + blockDim.x - 1) / blockDim.x;
-    const uint32_t b0 = min(nsb, threadIdx.x * per), b1 = min(nsb, b0 + per);
-    uint64_t s01 = 0, s23 = 0, sdd = 0, zs = 0, hs = 0, fs = 0, ss = 0, ls = 0;
-    uint32_t fm = 0xFFFFFFFFu;
-    for (uint32_t b = b0; b < b1; ++b) {
-        s01 += sbt[0 * nsb + b];
-        s23 += sbt[1 * nsb + b];
-        sdd += sbt[2 * nsb + b];
-        zs += sbt[3 * nsb + b];
-        hs += sbt[4 * nsb + b];
-        fs += sbt[5 * nsb + b];
-        ss += sbt[6 * nsb + b];
-        ls += sbt[7 * nsb + b];
-        fm = (uint32_t)min((uint64_t)fm, sbt[8 * nsb + b]);
-    }
-    const uint64_t x[8] = {s01, s23, sdd, zs, hs, fs, ss, ls};
-    uint64_t ex[8], t[8];
-    block_scan_n<8>(x, ex, t, lds);
-    const uint32_t fmin = block_min_u32(fm, lds);
-    // super-block prefixes for the write pass, and the totals cleared for
-    // the next compaction
-    uint64_t r01 = ex[0], r23 = ex[1], rdd = ex[2];
-    for (uint32_t b = b0; b < b1; ++b) {
-        bc.sbp[0 * nsb + b] = r01;
-        bc.sbp[1 * nsb + b] = r23;
-        bc.sbp[2 * nsb + b] = rdd;
-        r01 += sbt[0 * nsb + b];
-        r23 += sbt[1 * nsb + b];
-        rdd += sbt[2 * nsb + b];
-#pragma unroll
-        for (int i = 0; i < kSbVals - 1; ++i) bc.sbt[i * nsb + b] = 0;
-        bc.sbt[(kSbVals - 1) * nsb + b] = ~0ull;
-    }
-    if (threadIdx.x == 0) {
-        FrontierInfo fi;
-        fi.n[0] = (uint32_t)t[0];
-        fi.n[1] = (uint32_t)(t[0] >> 32);
-        fi.n[2] = (uint32_t)t[1];
-        fi.n[3] = (uint32_t)(t[1] >> 32);
-        fi.nzero = (uint32_t)t[3];
-        fi.nhub = (uint32_t)t[4];
-        fi.static_deg = t[6];
-        fi.dyn_deg = t[2];
-        fi.nfar = (uint32_t)t[5];
-        fi.min_far = fmin;
-        RoundCtl c = *ctl;
-        const uint64_t snodes = (uint64_t)fi.n[0] + fi.n[1] + fi.nhub;
-        // deferred order: while static vertices are active, the dynamic list
-        // stays flagged for a later round (the write pass keeps its flags)
-        const bool was_heavy = c.mode != 0;
-        fi.dyn_held = (c.defer == 1 && !was_heavy && snodes && fi.n[3]) ? 1u : 0u;
-        const uint32_t held = fi.dyn_held ? fi.n[3] : 0u;
-        if (held) {
-            fi.n[3] = 0;
-            fi.dyn_deg = 0;
-        }
-        const uint64_t active = snodes + fi.n[3] + fi.nzero;
-        // light/heavy split: light rounds count the vertices they relax (they
-        // turn heavy-pending); once a bucket's light rounds find nothing near,
-        // the next compaction collects the heavy-pending vertices (their
-        // distances are final within the bucket) before the threshold moves
-        bool heavy_next = false;
-        if (c.split) {
-            if (was_heavy) {
-                c.hpend = 0;
-            } else if (active) {
-                c.hpend += active;
-            } else if (c.hpend) {
-                heavy_next = true;
-            }
-        }
-        // (after a heavy round a light compaction always follows: the held-back
-        // vertices sit in the other flag array)
-        fi.live = (active || fi.nfar || held || heavy_next || was_heavy) ? 1u : 0u;
-        // BFS direction (Beamer et al., SC'12): bottom-up once the frontier's
-        // edges exceed 1/14 of the unexplored ones, back to top-down when
-        // the frontier falls below V / 24.
-        fi.pull = 0;
-        fi.heavy = c.mode;
-        if (c.dir_opt && active) {
-            const uint64_t mf = fi.static_deg + fi.dyn_deg;
-            if (!c.pull && mf > c.unexplored / 14) c.pull = 1;
-            else if (c.pull && active < c.nverts / 24) c.pull = 0;
-            c.unexplored -= min(mf, c.unexplored);
-            fi.pull = c.pull;
-            c.pull_rounds += c.pull;
-        }
-        *info = fi;
-        doff[fi.n[3]] = fi.dyn_deg;
-        if (m_doff) m_doff[fi.n[3]] = fi.dyn_deg;
-        c.compactions++;
-        c.live = fi.live;
-        if (active) {
-            c.rounds++;
-            c.node_sum += active;
-            c.static_node_sum += snodes;
-            c.dyn_node_sum += fi.n[3];
-            c.work_edges += fi.static_deg + fi.dyn_deg;
-            c.static_work_edges += fi.static_deg;
-            c.dyn_rounds += fi.n[3] ? 1 : 0;
-        } else if (heavy_next) {
-            // the threshold stays: the heavy round's offers are all >= it
-        } else if (fi.nfar && c.delta) {
-            // Near set empty.  Lagged order: every vertex below the threshold
-            // has relaxed except the waiting dynamic ones, which go next (a
-            // static vertex they improve is below the threshold and joins
-            // them).  Otherwise every held-back value is >= the threshold and
-            // it moves to the smallest of them + delta.
-            if (t[7]) c.fbound = c.thresh;
-            else c.thresh = (uint32_t)min((uint64_t)0xFFFFFFFFull, (uint64_t)fi.min_far + c.delta);
-        }
-        c.mode = heavy_next ? 1u : 0u;
-        *ctl = c;
-    }
-}
-
-// Compaction pass 3: emits the lists in vertex order from the codes of pass
-// 1 (bins 0/1 need no reads; hub tiles and the dynamic degree prefix read
-// the row bounds again, kLoadBatch at a time) with the chunk table of the
-// dynamic relax (dchunk[c]: the list entry holding edge c *
-// kDynEdgesPerBlock of the dynamic edge space), and rewrites the window:
-// 1 for held-back vertices, 0 elsewhere.  m_dlist / m_doff, when not null,
-// receive a copy of the dynamic list and its degree prefix: pinned host
-// memory the staged loader gathers from without a copy back.
-template <int FV>
-__global__ __launch_bounds__(kBlock) void k_frontier_write(uint8_t *__restrict__ flag_a, uint8_t *__restrict__ hflag,
-                                                           uint64_t Vpad, const uint64_t *__restrict__ ptr,
-                                                           const uint64_t *__restrict__ pmid,
-                                                           const uint32_t *__restrict__ deg,
-                                                           const uint32_t *__restrict__ hdeg, Tuning tn,
-                                                           BlockCounts bc, const FrontierInfo *__restrict__ info,
-                                                           uint32_t *__restrict__ list, uint64_t *__restrict__ hub,
-                                                           uint64_t hub_cap, uint64_t *__restrict__ doff,
-                                                           uint32_t *__restrict__ m_dlist,
-                                                           uint64_t *__restrict__ m_doff,
-                                                           uint32_t *__restrict__ dchunk, uint64_t dchunk_cap) {
-    __shared__ uint64_t lds[3 * kBlock / kWave];
-    __shared__ uint32_t s_win[4 * FV * kBlock];  // word i of thread t at [i * kBlock + t]
-    __shared__ uint64_t s_pre[3];                // the block's exclusive prefixes (bins 0|1, 2|3, degrees)
-    const uint32_t nblk = bc.nblk;
-    if (!info->live) return;  // nothing is flagged: no list, and the window is already clear
-    if (!bc.bcnt[4 * nblk + blockIdx.x]) return;  // the count pass found no flag in this window
-    // prefix = the super-block's + the counts of the blocks before this one
-    // in its super-block (one lane each; read before the block scan below,
-    // whose barriers publish s_pre)
-    if (threadIdx.x < kWave) {
-        static_assert(kSbBlocks <= kWave, "one lane per block of a super-block");
-        const uint32_t sb = blockIdx.x / kSbBlocks, q = sb * kSbBlocks + threadIdx.x;
-        uint64_t a01 = 0, a23 = 0, add = 0;
-        if (q < blockIdx.x) {
-            a01 = (uint64_t)bc.bcnt[0 * nblk + q] | ((uint64_t)bc.bcnt[1 * nblk + q] << 32);
-            a23 = (uint64_t)bc.bcnt[2 * nblk + q] | ((uint64_t)bc.bcnt[3 * nblk + q] << 32);
-            add = bc.bdeg[q];
-        }
-#pragma unroll
-        for (int m = kWave / 2; m >= 1; m >>= 1) {
-            a01 += shfl_xor_u64(a01, m);
-            a23 += shfl_xor_u64(a23, m);
-            add += shfl_xor_u64(add, m);
-        }
-        if (threadIdx.x == 0) {
-            s_pre[0] = bc.sbp[0 * bc.nsb + sb] + a01;
-            s_pre[1] = bc.sbp[1 * bc.nsb + sb] + a23;
-            s_pre[2] = bc.sbp[2 * bc.nsb + sb] + add;
-        }
-    }
-    // the array and row ranges the count pass used (light/heavy split)
-    const bool heavy = pmid && info->heavy;
-    uint8_t *flag = heavy ? hflag : flag_a;
-    const bool mark = pmid && !heavy;  // light round: relaxed vertices turn heavy-pending
-    const uint64_t base = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * (16 * FV);
-    uint4 w[FV];
-    load_flags(flag, base, Vpad, w);
-#pragma unroll
-    for (int k = 0; k < FV; ++k) {
-        s_win[(4 * k + 0) * kBlock + threadIdx.x] = w[k].x;
-        s_win[(4 * k + 1) * kBlock + threadIdx.x] = w[k].y;
-        s_win[(4 * k + 2) * kBlock + threadIdx.x] = w[k].z;
-        s_win[(4 * k + 3) * kBlock + threadIdx.x] = w[k].w;
-    }
-    // bin of slot j (codes of pass 1; each thread reads its own words)
-    auto bin_at = [&](uint32_t j) -> int {
-        return (int)((s_win[(j >> 2) * kBlock + threadIdx.x] >> (8 * (j & 3))) & 0xFFu) - kCode0;
-    };
-    const uint32_t all = window_mask(w, kCode0);
-    uint32_t c0 = 0, c1 = 0, c2 = 0, c3 = 0;
-    uint64_t ddeg = 0;
-    // walks the set bits kLoadBatch at a time; degrees read for bins 2 / 3
-    auto walk = [&](auto &&use) {
-        for (uint32_t m = all; m;) {
-            uint32_t jj[kLoadBatch];
-            int bb[kLoadBatch];
-            uint64_t dg[kLoadBatch];
-#pragma unroll
-            for (int k = 0; k < kLoadBatch; ++k) {
-                jj[k] = (16 * FV);
-                bb[k] = -1;
-                dg[k] = 0;
-                if (m) {
-                    const uint32_t j = (uint32_t)__builtin_ctz(m);
-                    m &= m - 1;
-                    jj[k] = j;
-                    bb[k] = bin_at(j);
-                    if (bb[k] == 2 || bb[k] == 3) dg[k] = round_deg(deg, hdeg, ptr, pmid, heavy, base + j);
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < kLoadBatch; ++k)
-                if (jj[k] != (16 * FV)) use(jj[k], bb[k], dg[k]);
-        }
-    };
-    walk([&](uint32_t, int b, uint64_t deg) {
-        switch (b) {
-            case 0: ++c0; break;
-            case 1: ++c1; break;
-            case 2: c2 += (uint32_t)((deg + tn.tile - 1) / tn.tile); break;
-            case 3: ++c3; ddeg += deg; break;
+    // prefixes of the (window, wave) pairs and the block's totals, per wave
+    const bool own = lane < NW * kWaves;
+    const uint64_t xc = own ? s_cnt[lane] : 0, xd = own ? s_deg[lane] : 0;
+    const uint32_t xt = own ? s_tile[lane] : 0;
+    const uint64_t wc = wave_scan_u64(xc), wd = wave_scan_u64(xd);
+    const uint32_t wt = wave_scan_u32(xt);
+    const uint64_t tc = wave_read_u64(wc, kWave - 1), td = wave_read_u64(wd, kWave - 1);
+    const uint32_t tt = (uint32_t)__builtin_amdgcn_readlane((int)wt, kWave - 1);
+    bool last = false;
+    if (wid == 0) {
+        // one lane per total, so that their round trips overlap
+        const uint64_t st = s_stat[1];
+        const uint32_t n0 = (uint32_t)(tc & 0xFFFFu), n1 = (uint32_t)((tc >> 16) & 0xFFFFu), n3 = (uint32_t)(tc >> 32);
+        unsigned long long *sl = ct.t + kTotSlot + (blockIdx.x % kTotSlots) * kTotLine;
+        unsigned long long *to = nullptr;
+        uint64_t add = 0;
+        switch (lane) {
+            case 0: to = ct.t + kTotBins; add = n0 | (uint64_t)n1 << 32; break;
+            case 1: to = ct.t + kTotTiles; add = tt | ((st >> 16) & 0xFFFFu) << 32; break;
+            case 2: to = sl + 0; add = (st & 0xFFFFu) | ((st >> 32) & 0xFFFFu) << 32; break;
+            case 3: to = sl + 1; add = s_stat[0]; break;
+            case 4: to = sl + 2; add = (st >> 48) | (uint64_t)s_more[1] << 32; break;
             default: break;
         }
-    });
-    const uint64_t x[3] = {(uint64_t)c0 | ((uint64_t)c1 << 32), (uint64_t)c2 | ((uint64_t)c3 << 32), ddeg};
-    uint64_t ex[3], t[3];
-    block_scan_n<3>(x, ex, t, lds);
-    if (!all) return;
-    uint32_t keep = 0;  // slots that stay flagged: held back (bin 5) or a held dynamic list
-    if (!info->pull) {  // bottom-up round: no lists, the frontier is its level
-        const uint32_t n0 = info->n[0], n1 = info->n[1];
-        uint64_t p0 = (uint64_t)(uint32_t)s_pre[0] + (uint32_t)ex[0];
-        uint64_t p1 = (uint64_t)n0 + (uint32_t)(s_pre[0] >> 32) + (uint32_t)(ex[0] >> 32);
-        uint64_t p2 = (uint64_t)(uint32_t)s_pre[1] + (uint32_t)ex[1];
-        uint64_t p3 = (uint64_t)(uint32_t)(s_pre[1] >> 32) + (uint32_t)(ex[1] >> 32);
-        uint64_t pd = s_pre[2] + ex[2];
-        const uint64_t dyn_base = (uint64_t)n0 + n1;
-        const bool held = info->dyn_held != 0;
-        walk([&](uint32_t j, int b, uint64_t deg) {
-            const uint64_t v = base + j;
-            if (mark && b <= 4 && !(b == 3 && held)) hflag[v] = 1;
-            switch (b) {
-                case 0: list[p0++] = (uint32_t)v; break;
-                case 1: list[p1++] = (uint32_t)v; break;
-                case 2: {
-                    const uint32_t nt = (uint32_t)((deg + tn.tile - 1) / tn.tile);
-                    for (uint32_t q = 0; q < nt; ++q, ++p2)
-                        if (p2 < hub_cap) hub[p2] = ((uint64_t)q << 32) | v;
-                    break;
-                }
-                case 3:
-                    if (held) {
-                        keep |= 1u << j;
-                        break;
-                    }
-                    list[dyn_base + p3] = (uint32_t)v;
-                    doff[p3] = pd;
-                    // the dynamic relax's chunks of kDynEdgesPerBlock edges
-                    // whose first edge is one of v's: they start at entry p3
-                    for (uint64_t c = (pd + kDynEdgesPerBlock - 1) / kDynEdgesPerBlock;
-                         c * kDynEdgesPerBlock < pd + deg && c < dchunk_cap; ++c)
-                        dchunk[c] = (uint32_t)p3;
-                    if (m_dlist) {  // pinned host mirrors for the host-side gather
-                        m_dlist[p3] = (uint32_t)v;
-                        m_doff[p3] = pd;
-                    }
-                    ++p3;
-                    pd += deg;
-                    break;
-                case 5: keep |= 1u << j; break;
-                default: break;
-            }
-        });
+        if (add) {
+            const uint64_t old = atomicAdd(to, (unsigned long long)add);
+            if (lane < 2) s_base[lane] = old;
+        }
+        if (lane == 5 && s_more[2] != 0xFFFFFFFFu) atomicMin(sl + 3, (unsigned long long)s_more[2]);
+        if (lane == 6 && n3) {
+            uint64_t p, pd;
+            reserve_dyn(ct, n3, td, p, pd);
+            s_base[2] = p;
+            s_base[3] = pd;
+        }
+        wait_vmem();
+        last = lane == 0 && arrive_last(ct);
     }
-    uint32_t word[4 * FV];
+    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 4 * FV; ++k) word[k] = 0;
+    for (int q = 0; q < NW; ++q) {
+        // exclusive prefix of this wave in window q
+        const uint64_t pc = wave_read_u64(wc - xc, q * kWaves + wid), pw = wave_read_u64(wd - xd, q * kWaves + wid);
+        const uint32_t ptile = (uint32_t)__builtin_amdgcn_readlane((int)(wt - xt), q * kWaves + wid);
+        if (!fw[q]) continue;
+        const uint32_t e01 = i01[q] - c01[q];
+        uint64_t p0 = (uint64_t)(uint32_t)s_base[0] + (uint32_t)(pc & 0xFFFFu) + (e01 & 0xFFFFu);
+        uint64_t p1 = (uint64_t)(uint32_t)(s_base[0] >> 32) + (uint32_t)((pc >> 16) & 0xFFFFu) + (e01 >> 16);
+        uint64_t p2 = (uint64_t)(uint32_t)s_base[1] + ptile + (it[q] - tiles[q]);
+        uint64_t p3 = s_base[2] + (uint32_t)(pc >> 32) + (i3[q] - c3[q]);
+        uint64_t pd = s_base[3] + pw + (id[q] - ddeg[q]);
+        uint32_t left = 0, hw = 0;  // flags left (bins 5 and 6), heavy-pending flags to set
 #pragma unroll
-    for (int j = 0; j < (16 * FV); ++j) word[j >> 2] |= ((keep >> j) & 1u) << (8 * (j & 3));
-    store_flags<FV>(flag, base, Vpad, word);
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t v = (uint32_t)(v0 + q * kWin + j);
+            const uint32_t b = (bins[q] >> (8 * j)) & 0xFFu;
+            if (b <= 4) hw |= 1u << (8 * j);
+            if (b == 0) {
+                list[p0++] = v;
+            } else if (b == 1) {
+                list[vsplit - 1 - p1++] = v;
+            } else if (b == 2) {
+                const uint32_t nt = (uint32_t)((dg[q][j] + tn.tile - 1) / tn.tile);
+                for (uint32_t i = 0; i < nt; ++i, ++p2)
+                    if (p2 < hub_cap) hub[p2] = ((uint64_t)i << 32) | v;
+            } else if (b == 3) {
+                const uint64_t d = dg[q][j];
+                list[vsplit + p3] = v;
+                doff[p3] = pd;
+                // the dynamic relax's chunks of kDynEdgesPerBlock edges whose
+                // first edge is one of v's: they start at entry p3
+                for (uint64_t c = (pd + kDynEdgesPerBlock - 1) / kDynEdgesPerBlock;
+                     c * kDynEdgesPerBlock < pd + d && c < dchunk_cap; ++c)
+                    dchunk[c] = (uint32_t)p3;
+                ++p3;
+                pd += d;
+            } else if (b == 5 || b == 6) {
+                left |= 1u << (8 * j);
+            }
+        }
+        if (left != fw[q]) *(uint32_t *)(flag + v0 + q * kWin) = left;
+        // (the word belongs to this thread alone)
+        if (mark && hw) *(uint32_t *)(hflag + v0 + q * kWin) |= hw;
+    }
+    if (wid == 0 && __ballot(last)) compact_finish(ct, info, doff, ctl);
 }
 
 __global__ void k_ctl_reset(RoundCtl *ctl, uint32_t delta, uint32_t defer, uint64_t dir_opt_edges, uint64_t V,
@@ -586,6 +517,7 @@ __global__ void k_ctl_reset(RoundCtl *ctl, uint32_t delta, uint32_t defer, uint6
     c.nverts = V;
     c.thresh = delta ? (uint32_t)min((uint64_t)0xFFFFFFFFull, 1ull + delta) : 0xFFFFFFFFu;
     c.fbound = 0;
+    c.hold = defer == 1 || defer == kDeferOnce ? 1u : 0u;
     c.live = 1;
     c.halt = 1;
     *ctl = c;
@@ -664,24 +596,24 @@ __device__ __forceinline__ uint32_t commit(const RelaxArgs &a, typename SrcOf<AL
 // the device and stride over them, so a launch needs no host-side count: a
 // round can be enqueued (or captured in a graph) before its compaction ran.
 
-// Bins 0 and 1: LPV lanes per frontier vertex (LPV = 64: one wave).  BIN
-// selects the list segment: bin 0 at list[0, n0), bin 1 at list[n0, n0 + n1).
+// Bins 0 and 1: LPV lanes per frontier vertex (LPV = 64: one wave).  `bin`
+// selects the list segment: item i of bin 0 at list[i], of bin 1 at
+// list[vsplit - 1 - i].
 // The bodies take the workgroup's index and the number of workgroups of its
 // kind (bid, nb), so that one launch can run several kinds side by side.
 template <int ALGO, bool W, bool PK, int LPV>
-__device__ __forceinline__ uint32_t relax_group_body(const uint32_t *__restrict__ list, int bin,
+__device__ __forceinline__ uint32_t relax_group_body(const uint32_t *__restrict__ list, uint64_t vsplit, int bin,
                                                      const FrontierInfo *__restrict__ info,
                                                      const uint64_t *__restrict__ ptr, const void *__restrict__ edges,
                                                      const RelaxArgs &a, uint32_t bid, uint32_t nb) {
     if (info->pull) return 0;
     const bool heavy = info->heavy != 0;
     const uint32_t n = info->n[bin];
-    const uint32_t *lst = list + (bin ? info->n[0] : 0u);
     const uint32_t sub = threadIdx.x % LPV;
     const uint64_t stride = (uint64_t)nb * (kBlock / LPV);
     uint32_t cnt = 0;
     for (uint64_t item = ((uint64_t)bid * kBlock + threadIdx.x) / LPV; item < n; item += stride) {
-        const uint32_t u = lst[item];
+        const uint32_t u = list[bin ? vsplit - 1 - item : item];
         uint64_t b, e;
         row_range(ptr, a.pmid, heavy, u, b, e);
         const auto s = load_src<ALGO>(a, u);
@@ -707,12 +639,12 @@ __device__ __forceinline__ uint32_t relax_group_body(const uint32_t *__restrict_
 }
 
 template <int ALGO, bool W, bool PK, int LPV>
-__global__ __launch_bounds__(kBlock) void k_relax_group(const uint32_t *__restrict__ list, int bin,
+__global__ __launch_bounds__(kBlock) void k_relax_group(const uint32_t *__restrict__ list, uint64_t vsplit, int bin,
                                                         const FrontierInfo *__restrict__ info,
                                                         const uint64_t *__restrict__ ptr,
                                                         const void *__restrict__ edges, RelaxArgs a,
                                                         unsigned long long *upd) {
-    wave_add(upd, relax_group_body<ALGO, W, PK, LPV>(list, bin, info, ptr, edges, a, blockIdx.x, gridDim.x));
+    wave_add(upd, relax_group_body<ALGO, W, PK, LPV>(list, vsplit, bin, info, ptr, edges, a, blockIdx.x, gridDim.x));
 }
 
 template <int ALGO, bool W, bool PK>
@@ -777,7 +709,7 @@ __global__ __launch_bounds__(kBlock) void k_relax_hub(const uint64_t *__restrict
 
 // Dynamic region, edges [c0, min(c1, D)) of the concatenated active dynamic
 // edge space (D = sum of the dynamic list's degrees; the list sits at
-// list[n0 + n1, n0 + n1 + n3)).  STAGED (DIRECT = false): they sit in a
+// list[vsplit, vsplit + n3)).  STAGED (DIRECT = false): they sit in a
 // staging slot, edge q at q - c0.  DIRECT: edge q of vertex u is CSR edge
 // x = ptr[u] + (q - doff[i]); when u's chunk of kResChunk vertices is
 // resident in HBM (rdelta[u >> kResChunkShift] != kNotResident) it is read
@@ -813,7 +745,7 @@ __device__ __forceinline__ uint32_t relax_dyn_body(const uint32_t *__restrict__ 
     uint64_t *s_off = L.off;
     uint32_t *s_i = L.i;
     const uint32_t ndyn = info->n[3];
-    const uint32_t *dlist = list + info->n[0] + info->n[1];
+    const uint32_t *dlist = list + vsplit;
     const uint64_t c1 = min(c1max, info->dyn_deg);
     const bool heavy = info->heavy != 0;
     uint32_t c = 0, h = 0;
@@ -961,10 +893,10 @@ __global__ __launch_bounds__(kBlock) void k_relax_round(RoundRelax r, RelaxArgs 
     const uint32_t k = blockIdx.x / P, j = blockIdx.x - k * P;
     if (j < 2) {
         wave_add(r.counters + 0,
-                 relax_group_body<ALGO, W, PK, LPV>(r.list, 0, r.info, r.ptr, r.sedges, a, 2 * k + j, 2 * K));
+                 relax_group_body<ALGO, W, PK, LPV>(r.list, r.vsplit, 0, r.info, r.ptr, r.sedges, a, 2 * k + j, 2 * K));
     } else if (j < 4) {
         wave_add(r.counters + 0,
-                 relax_group_body<ALGO, W, PK, 64>(r.list, 1, r.info, r.ptr, r.sedges, a, 2 * k + j - 2, 2 * K));
+                 relax_group_body<ALGO, W, PK, 64>(r.list, r.vsplit, 1, r.info, r.ptr, r.sedges, a, 2 * k + j - 2, 2 * K));
     } else if (j == 4) {
         wave_add(r.counters + 0, relax_hub_body<ALGO, W, PK>(r.hub, r.hub_cap, r.info, r.tile, r.ptr, r.sedges, a,
                                                               (uint32_t *)s_fuse, k, K));
@@ -1019,10 +951,10 @@ __global__ __launch_bounds__(kBlock) void k_srv_round(RoundRelax r, RelaxArgs a,
     const uint32_t K = gridDim.x / P;
     const uint32_t k = blockIdx.x / P, j = blockIdx.x - k * P;
     if (j < 2) {
-        wave_add(r.counters + 0, relax_group_body<ALGO_MSBFS, W, PK, LPV>(r.list, 0, r.info, r.ptr, r.sedges, a,
+        wave_add(r.counters + 0, relax_group_body<ALGO_MSBFS, W, PK, LPV>(r.list, r.vsplit, 0, r.info, r.ptr, r.sedges, a,
                                                                          2 * k + j, 2 * K));
     } else if (j < 4) {
-        wave_add(r.counters + 0, relax_group_body<ALGO_MSBFS, W, PK, 64>(r.list, 1, r.info, r.ptr, r.sedges, a,
+        wave_add(r.counters + 0, relax_group_body<ALGO_MSBFS, W, PK, 64>(r.list, r.vsplit, 1, r.info, r.ptr, r.sedges, a,
                                                                         2 * k + j - 2, 2 * K));
     } else if (j == 4) {
         wave_add(r.counters + 0, relax_hub_body<ALGO_MSBFS, W, PK>(r.hub, r.hub_cap, r.info, r.tile, r.ptr, r.sedges,
@@ -1293,16 +1225,17 @@ void frontier_alloc(DeviceState *d, const og_graph *g, Frontier &f, MemPool &m) 
     const uint64_t dyn_edges = d->plan.vsplit < V ? g->E - g->ptr[d->plan.vsplit] : 0;
     f.dchunk_cap = dyn_edges / kDynEdgesPerBlock + 2;
     f.dchunk = (uint32_t *)m.dalloc(f.dchunk_cap * sizeof(uint32_t));
-    f.fv = (uint32_t)frontier_fv(V);
-    f.nblk = (uint32_t)((d->Vpad + verts_per_block(f.fv) - 1) / verts_per_block(f.fv));
+    f.nw = (uint32_t)compact_nw(V);
+    f.nblk = (uint32_t)((d->Vpad + verts_per_block(f.nw) - 1) / verts_per_block(f.nw));
     f.V = V;
-    f.bcnt = (uint32_t *)m.dalloc((uint64_t)kBcntRows * f.nblk * sizeof(uint32_t));
-    f.bdeg = (uint64_t *)m.dalloc((uint64_t)f.nblk * sizeof(uint64_t));
-    f.nsb = (f.nblk + kSbBlocks - 1) / kSbBlocks;
-    f.sbt = (uint64_t *)m.dalloc((uint64_t)kSbVals * f.nsb * sizeof(uint64_t));
-    f.sbp = (uint64_t *)m.dalloc(3ull * f.nsb * sizeof(uint64_t));
-    OG_HIP(hipMemset(f.sbt, 0, (uint64_t)(kSbVals - 1) * f.nsb * sizeof(uint64_t)));
-    OG_HIP(hipMemset(f.sbt + (uint64_t)(kSbVals - 1) * f.nsb, 0xFF, (uint64_t)f.nsb * sizeof(uint64_t)));
+    f.tot = (unsigned long long *)m.dalloc(totals_words(f.nblk) * 8);
+    // dynamic list: its count and its edges in one word when they fit
+    const uint32_t nb = bits_of(V - d->plan.vsplit), eb = bits_of(dyn_edges);
+    f.dsh = nb + eb <= 64 && nb < 64 ? std::max(nb, 1u) : 0;
+    hipLaunchKernelGGL(k_totals_init, dim3(fill_grid(totals_words(f.nblk))), dim3(256), 0, d->s_compute, f.tot,
+                       totals_words(f.nblk));
+    OG_HIP(hipGetLastError());
+    OG_HIP(hipStreamSynchronize(d->s_compute));
     f.info = (FrontierInfo *)m.dalloc(sizeof(FrontierInfo));
     f.ctl = (RoundCtl *)m.dalloc(sizeof(RoundCtl));
     f.counters = (unsigned long long *)m.dalloc(16 * sizeof(unsigned long long));
@@ -1327,32 +1260,17 @@ void frontier_begin(Frontier &f, hipStream_t s, uint32_t delta, uint32_t defer, 
 
 void frontier_compact(DeviceState *d, Frontier &f, hipStream_t s, const uint32_t *val, bool to_host,
                       const uint64_t *pmid) {
-    // (pinned mirrors of the dynamic list written by pass 3 cost one small
-    // PCIe write per vertex: slower than one bulk copy back, so unused)
-    uint32_t *m_dlist = nullptr;
-    uint64_t *m_doff = nullptr;
     // the degree table (a split round needs its light and heavy parts)
     const uint32_t *deg = d->d_deg && (!pmid || d->deg_split) ? d->d_deg : nullptr;
     const uint32_t *hdeg = deg ? d->deg_heavy() : nullptr;
-    if (f.fv == 1)
-        hipLaunchKernelGGL(k_frontier_count<1>, dim3(f.nblk), dim3(kBlock), 0, s, f.flag, f.hflag, d->Vpad,
-                           d->plan.vsplit, d->d_ptr, pmid, deg, hdeg, d->tune, val, f.ctl, f.counts());
+    if (f.nw == 1)
+        hipLaunchKernelGGL(k_frontier_compact<1>, dim3(f.nblk), dim3(kCompactBlock), 0, s, f.flag, f.hflag, d->Vpad,
+                           d->plan.vsplit, d->d_ptr, pmid, deg, hdeg, d->tune, val, f.ctl, f.totals(), f.info, f.list,
+                           f.hub, f.hub_cap, f.doff, f.dchunk, f.dchunk_cap);
     else
-        hipLaunchKernelGGL(k_frontier_count<2>, dim3(f.nblk), dim3(kBlock), 0, s, f.flag, f.hflag, d->Vpad,
-                           d->plan.vsplit, d->d_ptr, pmid, deg, hdeg, d->tune, val, f.ctl, f.counts());
-    // one lane per super-block up to kScanThreads lanes (one wave up to
-    // 2^25 vertices)
-    const unsigned scan_threads =
-        (unsigned)std::min<uint64_t>(kScanThreads, (std::max<uint64_t>(f.nsb, 1) + kWave - 1) / kWave * kWave);
-    hipLaunchKernelGGL(k_frontier_scan, dim3(1), dim3(scan_threads), 0, s, f.counts(), f.info, f.doff, f.ctl, m_doff);
-    if (f.fv == 1)
-        hipLaunchKernelGGL(k_frontier_write<1>, dim3(f.nblk), dim3(kBlock), 0, s, f.flag, f.hflag, d->Vpad, d->d_ptr,
-                           pmid, deg, hdeg, d->tune, f.counts(), f.info, f.list, f.hub, f.hub_cap, f.doff, m_dlist,
-                           m_doff, f.dchunk, f.dchunk_cap);
-    else
-        hipLaunchKernelGGL(k_frontier_write<2>, dim3(f.nblk), dim3(kBlock), 0, s, f.flag, f.hflag, d->Vpad, d->d_ptr,
-                           pmid, deg, hdeg, d->tune, f.counts(), f.info, f.list, f.hub, f.hub_cap, f.doff, m_dlist,
-                           m_doff, f.dchunk, f.dchunk_cap);
+        hipLaunchKernelGGL(k_frontier_compact<4>, dim3(f.nblk), dim3(kCompactBlock), 0, s, f.flag, f.hflag, d->Vpad,
+                           d->plan.vsplit, d->d_ptr, pmid, deg, hdeg, d->tune, val, f.ctl, f.totals(), f.info, f.list,
+                           f.hub, f.hub_cap, f.doff, f.dchunk, f.dchunk_cap);
     OG_HIP(hipGetLastError());
     if (to_host) OG_HIP(hipMemcpyAsync(f.h_info, f.info, sizeof(FrontierInfo), hipMemcpyDeviceToHost, s));
 }
@@ -1810,7 +1728,7 @@ static void prepare_impl(og_graph *g, og_approach approach, const og_plan_params
     }
 
     // ---- vertex state
-    d->d_val = (uint32_t *)d->dalloc(V * sizeof(uint32_t));
+    d->d_val = (uint32_t *)d->dalloc(d->Vpad * sizeof(uint32_t));
     OG_HIP(hipStreamSynchronize(d->s_compute));
     frontier_alloc(d.get(), g, d->fr, d->mem);
     pl.device_bytes = d->device_bytes();
@@ -1981,7 +1899,7 @@ static void launch_static_relax_fmt(DeviceState *d, Frontier &f, const FrontierI
         switch (lpv0) {
 #define OG_LPV(L)                                                                                                 \
     case L:                                                                                                       \
-        hipLaunchKernelGGL((k_relax_group<ALGO, W, PK, L>), gr, dim3(kBlock), 0, s, f.list, 0, f.info, d->d_ptr, \
+        hipLaunchKernelGGL((k_relax_group<ALGO, W, PK, L>), gr, dim3(kBlock), 0, s, f.list, d->plan.vsplit, 0, f.info, d->d_ptr, \
                            edges, a, upd);                                                                        \
         break;
             OG_LPV(1) OG_LPV(2) OG_LPV(4) OG_LPV(8) OG_LPV(16) OG_LPV(32)
@@ -1993,7 +1911,7 @@ static void launch_static_relax_fmt(DeviceState *d, Frontier &f, const FrontierI
         hipLaunchKernelGGL((k_relax_group<ALGO, W, PK, 64>),
                            dim3(hfi ? capped(((uint64_t)hfi->n[1] * 64 + kBlock - 1) / kBlock, kGroupGridCap)
                                     : kGroupGridCap),
-                           dim3(kBlock), 0, s, f.list, 1, f.info, d->d_ptr, edges, a, upd);
+                           dim3(kBlock), 0, s, f.list, d->plan.vsplit, 1, f.info, d->d_ptr, edges, a, upd);
     if (!hfi || hfi->n[2])
         hipLaunchKernelGGL((k_relax_hub<ALGO, W, PK>), dim3(hfi ? capped(hfi->n[2], kHubGridCap) : kHubGridCap),
                            dim3(kBlock), d->tune.tile * d->eb, s, f.hub, f.hub_cap, f.info, d->tune.tile, d->d_ptr,
@@ -2105,6 +2023,7 @@ static void launch_srv_round_fmt(DeviceState *d, Frontier &f, const RelaxArgs &a
     r.hub = f.hub;
     r.hub_cap = f.hub_cap;
     r.tile = d->tune.tile;
+    r.vsplit = d->plan.vsplit;
     r.counters = f.counters;
     SrvPull p{};
     if (pull) p = *pull;
@@ -2155,7 +2074,7 @@ static void run_dynamic(DeviceState *d, const og_graph *g, const FrontierInfo &f
     const uint32_t ndyn = fi.n[3];
     const uint64_t D = fi.dyn_deg;
     if (!ndyn || !D) return;
-    const uint32_t *d_dlist = d->fr.list + fi.n[0] + fi.n[1];
+    const uint32_t *d_dlist = d->fr.list + d->plan.vsplit;
     const uint64_t eb = d->deb;
     OG_HIP(hipMemcpyAsync(d->h_dlist, d_dlist, (size_t)ndyn * 4, hipMemcpyDeviceToHost, d->s_copy));
     OG_HIP(hipMemcpyAsync(d->h_doff, d->fr.doff, ((size_t)ndyn + 1) * 8, hipMemcpyDeviceToHost, d->s_copy));
@@ -2226,8 +2145,14 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
     const bool has_dyn = d->plan.vsplit < d->V;
     const bool staged = has_dyn && !zero_copy;
     // deferring dynamic vertices reorders relaxations across levels, which
-    // only the atomicMin relaxes (SSSP, CC) tolerate
-    const uint32_t defer = (ALGO == ALGO_SSSP || ALGO == ALGO_CC) && has_dyn ? d->tune.defer : 0;
+    // only the atomicMin relaxes (SSSP, CC) tolerate.  CC starts with every
+    // vertex active: unless a tuning says otherwise its dynamic vertices wait
+    // until the static region has settled once, so that most of them carry
+    // their final label when their rows cross the link (ER 3 M x 32, a
+    // quarter of the edges on the device: the rows are read once instead of
+    // about twice, 10.5 -> 7.9 ms).
+    uint32_t defer = (ALGO == ALGO_SSSP || ALGO == ALGO_CC) && has_dyn ? d->tune.defer : 0;
+    if (ALGO == ALGO_CC && has_dyn && d->plan.vsplit && !defer) defer = kDeferOnce;
     const bool dir_opt = ALGO == ALGO_BFS && d->d_in_ptr != nullptr;
     // light/heavy split: near-far SSSP on a graph prepared with it
     const bool split = ALGO == ALGO_SSSP && delta && d->d_pmid;
@@ -2552,7 +2477,7 @@ DeviceState *lane_state_create(og_graph *g, uint32_t delta) {
     l->s_copy = l->s_static = l->s_compute;
     OG_HIP(hipEventCreateWithFlags(&l->ev_static, hipEventDisableTiming));
     OG_HIP(hipEventCreateWithFlags(&l->ev_fork, hipEventDisableTiming));
-    l->d_val = (uint32_t *)l->dalloc(l->V * sizeof(uint32_t));
+    l->d_val = (uint32_t *)l->dalloc(l->Vpad * sizeof(uint32_t));
     frontier_alloc(l.get(), g, l->fr, l->mem);
     OG_HIP(hipDeviceSynchronize());
     return l.release();
@@ -2561,15 +2486,14 @@ DeviceState *lane_state_create(og_graph *g, uint32_t delta) {
 uint64_t lane_state_bytes(const og_graph *g) {
     const DeviceState *d = g->dev;
     const uint64_t V = d->V, Vpad = d->Vpad;
-    const uint64_t nblk = (Vpad + verts_per_block(frontier_fv(V)) - 1) / verts_per_block(frontier_fv(V));
-    const uint64_t nsb = (nblk + kSbBlocks - 1) / kSbBlocks;
+    const uint64_t nblk = (Vpad + verts_per_block(compact_nw(V)) - 1) / verts_per_block(compact_nw(V));
     const uint64_t hub = std::max<uint64_t>(hub_capacity(g, d->plan.vsplit, d->tune), 1);
     // what lane_state_create and frontier_alloc request: values, flags (and
     // the heavy-round flags with the split), bin lists, degree prefix, the
-    // (empty) dynamic chunk table, block counts, super-block sums and
-    // prefixes, round summary, control block, counters and hub tiles
-    return 4 * V + Vpad * (d->d_pmid ? 2 : 1) + 4 * V + 8 * (V + 1) + 4 * 2 + 4ull * kBcntRows * nblk + 8 * nblk +
-           8ull * kSbVals * nsb + 24 * nsb + sizeof(FrontierInfo) + sizeof(RoundCtl) + 16 * 8 + 8 * hub;
+    // (empty) dynamic chunk table, compaction totals, round summary, control
+    // block, counters and hub tiles
+    return 4 * Vpad + Vpad * (d->d_pmid ? 2 : 1) + 4 * V + 8 * (V + 1) + 4 * 2 + 8 * totals_words(nblk) +
+           sizeof(FrontierInfo) + sizeof(RoundCtl) + 16 * 8 + 8 * hub;
 }
 
 void lane_run_sssp(og_graph *g, DeviceState *lane, uint32_t src, uint32_t *out, og_run_stats *st) {
@@ -3027,18 +2951,14 @@ constexpr uint64_t na_up(uint64_t x) { return (x + kNoAlign - 1) / kNoAlign * kN
 // of degree d > t2 takes ceil(d / tile) <= d / tile + 1 tiles, and at most
 // E / (t2 + 1) vertices exceed t2.
 constexpr uint64_t kNoAllocHubCap = kNoAllocMaxE / 2048 + kNoAllocMaxE / 4097 + 1;
-static_assert(frontier_fv(kNoAllocMaxV) == 1, "the allocation-free BFS runs the one-vector compaction");
+static_assert(compact_nw(kNoAllocMaxV) == 1, "the allocation-free BFS runs the one-window compaction");
 constexpr uint64_t kNoAllocMaxBlk = (kNoAllocMaxV + verts_per_block(1) - 1) / verts_per_block(1);
 constexpr uint64_t kNaFlag = 0;
 constexpr uint64_t kNaList = kNaFlag + na_up(kNoAllocMaxV);
 constexpr uint64_t kNaHub = kNaList + na_up(4 * kNoAllocMaxV);
 constexpr uint64_t kNaDoff = kNaHub + na_up(8 * kNoAllocHubCap);
-constexpr uint64_t kNoAllocMaxSb = (kNoAllocMaxBlk + kSbBlocks - 1) / kSbBlocks;
-constexpr uint64_t kNaBcnt = kNaDoff + na_up(8 * 16);
-constexpr uint64_t kNaBdeg = kNaBcnt + na_up(4 * kBcntRows * kNoAllocMaxBlk);
-constexpr uint64_t kNaSbt = kNaBdeg + na_up(8 * kNoAllocMaxBlk);
-constexpr uint64_t kNaSbp = kNaSbt + na_up(8 * kSbVals * kNoAllocMaxSb);
-constexpr uint64_t kNaInfo = kNaSbp + na_up(8 * 3 * kNoAllocMaxSb);
+constexpr uint64_t kNaTot = kNaDoff + na_up(8 * 16);
+constexpr uint64_t kNaInfo = kNaTot + na_up(8 * totals_words(kNoAllocMaxBlk));
 constexpr uint64_t kNaCtl = kNaInfo + na_up(sizeof(FrontierInfo));
 constexpr uint64_t kNaCounters = kNaCtl + na_up(sizeof(RoundCtl));
 constexpr uint64_t kNoAllocScratchBytes = kNaCounters + na_up(16 * 8);
@@ -3087,9 +3007,7 @@ static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t 
     uint32_t *list = (uint32_t *)(base + kNaList);
     uint64_t *hub = (uint64_t *)(base + kNaHub);
     uint64_t *doff = (uint64_t *)(base + kNaDoff);
-    const uint32_t nsb = (nblk + kSbBlocks - 1) / kSbBlocks;
-    const BlockCounts bc{(uint32_t *)(base + kNaBcnt), (uint64_t *)(base + kNaBdeg), (uint64_t *)(base + kNaSbt),
-                         (uint64_t *)(base + kNaSbp), nblk, nsb};
+    const CompactTotals ct{(unsigned long long *)(base + kNaTot), nblk, 1};  // (no dynamic list)
     FrontierInfo *info = (FrontierInfo *)(base + kNaInfo);
     RoundCtl *ctl = (RoundCtl *)(base + kNaCtl);
     unsigned long long *ctr = (unsigned long long *)(base + kNaCounters);
@@ -3102,17 +3020,12 @@ static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t 
     hipLaunchKernelGGL(k_fill_u32, dim3(fill_grid(V)), dim3(256), 0, s, d_levels, V, OG_UNREACHED);
     hipLaunchKernelGGL(k_set_source, dim3(1), dim3(1), 0, s, d_levels, flag, src);
     hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(1), 0, s, ctl, 0u, 0u, (uint64_t)0, V, 0u);
-    hipLaunchKernelGGL(k_sb_init, dim3(1), dim3(64), 0, s, bc.sbt, nsb);
+    hipLaunchKernelGGL(k_totals_init, dim3(fill_grid(totals_words(nblk))), dim3(256), 0, s, ct.t, totals_words(nblk));
     auto compact = [&] {
-        hipLaunchKernelGGL(k_frontier_count<1>, dim3(nblk), dim3(kBlock), 0, s, flag, (uint8_t *)nullptr, Vpad, V,
+        hipLaunchKernelGGL(k_frontier_compact<1>, dim3(nblk), dim3(kCompactBlock), 0, s, flag, (uint8_t *)nullptr, Vpad, V,
                            d_ptr, (const uint64_t *)nullptr, (const uint32_t *)nullptr, (const uint32_t *)nullptr, tn,
-                           (const uint32_t *)nullptr, ctl, bc);
-        hipLaunchKernelGGL(k_frontier_scan, dim3(1), dim3(kWave), 0, s, bc, info, doff, ctl, (uint64_t *)nullptr);
-        hipLaunchKernelGGL(k_frontier_write<1>, dim3(nblk), dim3(kBlock), 0, s, flag, (uint8_t *)nullptr, Vpad, d_ptr,
-                           (const uint64_t *)nullptr, (const uint32_t *)nullptr, (const uint32_t *)nullptr, tn, bc,
-                           info, list, hub,
-                           kNoAllocHubCap, doff, (uint32_t *)nullptr, (uint64_t *)nullptr, (uint32_t *)nullptr,
-                           (uint64_t)0);
+                           (const uint32_t *)nullptr, ctl, ct, info, list, hub, kNoAllocHubCap, doff,
+                           (uint32_t *)nullptr, (uint64_t)0);
     };
     RoundRelax r{};
     r.list = list;
@@ -3123,6 +3036,7 @@ static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t 
     r.hub_cap = kNoAllocHubCap;
     r.tile = tn.tile;
     r.cd = 0;  // the whole graph is static: three bins in one launch
+    r.vsplit = V;
     r.counters = ctr;
     const RelaxArgs a{d_levels, flag, nullptr, nullptr, nullptr, 0, nullptr, nullptr};
     static_assert(Tuning{}.lpv0 == 8, "the relax below is instantiated for 8 lanes per bin-0 vertex");

@@ -225,13 +225,13 @@ __global__ void k_srv_direction(uint64_t used, uint64_t V, uint64_t E, int dir_o
 
 // After the relax: the masks of the round's listed vertices (bins 0/1 and
 // hub tiles) are cleared; the next commit sets the new ones.
-__global__ __launch_bounds__(kBlock) void k_srv_clear_front(const uint32_t *__restrict__ list,
+__global__ __launch_bounds__(kBlock) void k_srv_clear_front(const uint32_t *__restrict__ list, uint64_t vsplit,
                                                             const uint64_t *__restrict__ hub, uint64_t hub_cap,
                                                             const FrontierInfo *__restrict__ info, uint64_t *front) {
-    const uint64_t n01 = (uint64_t)info->n[0] + info->n[1];
+    const uint64_t n0 = info->n[0], n01 = n0 + info->n[1];
     const uint64_t nh = min((uint64_t)info->n[2], hub_cap);
     for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n01 + nh; i += (uint64_t)gridDim.x * kBlock)
-        front[i < n01 ? list[i] : (uint32_t)hub[i - n01]] = 0;
+        front[i < n0 ? list[i] : i < n01 ? list[vsplit - 1 - (i - n0)] : (uint32_t)hub[i - n01]] = 0;
 }
 
 // Clears the visit bits of finished slots (before the slots are reused).
@@ -1059,7 +1059,8 @@ void BfsEngine::step() {
     RelaxArgs a{nullptr, f.flag, visit, front, next, d->wbits, dir_opt ? (const uint64_t *)d_pull : nullptr};
     const SrvPull pl{d->d_in_ptr, d->d_in_cols, V, visit, front, next, f.flag, d_pull};
     launch_srv_round(d, f, a, s, dir_opt ? &pl : nullptr, g->kind == OG_KIND_WEIGHTED);
-    hipLaunchKernelGGL(k_srv_clear_front, dim3(1024), dim3(kBlock), 0, s, f.list, f.hub, f.hub_cap, f.info, front);
+    hipLaunchKernelGGL(k_srv_clear_front, dim3(1024), dim3(kBlock), 0, s, f.list, d->plan.vsplit, f.hub,
+                       f.hub_cap, f.info, front);
     OG_HIP(hipGetLastError());
     // The host needs only the commit's summary: while it finishes slots and
     // admits queries, the round's compaction and relax go on, and the next

@@ -152,6 +152,24 @@ struct RoundCtl {
     uint32_t hold;               // defer 1: the next compaction holds the dynamic vertices back
 };
 
+// Time of a device-driven run by kind of work, from the device's constant
+// 100 MHz clock.  A kernel that begins work of one kind after another kind
+// adds its start time to the old kind and subtracts it from its own, two
+// atomics that nothing waits for, so that each kind sums up to end - begin.
+// (Event nodes in the stream or the captured graph stalled each kernel for
+// about 10 us: two of them per round.)
+enum ClockKind { kClkRelax = 0, kClkFront = 1, kClkOther = 2 };
+struct RoundClock {
+    unsigned long long acc[3];
+};
+
+// What a run leaves on the device beside its values; one copy brings it over.
+struct RunBlock {
+    RoundCtl ctl;
+    RoundClock clk;
+    unsigned long long counters[16];  // [0] updates static, [1] updates dynamic, [2..] scratch
+};
+
 constexpr uint32_t kDeferOnce = 3;      // RoundCtl::defer: hold the dynamic vertices back until the static region
                                         // has settled once
 
@@ -203,10 +221,11 @@ struct Frontier {
     uint64_t V = 0;
     FrontierInfo *info = nullptr;
     FrontierInfo *h_info = nullptr;  // pinned
-    RoundCtl *ctl = nullptr;
-    RoundCtl *h_ctl = nullptr;       // pinned
-    unsigned long long *counters = nullptr;    // [0] updates static, [1] updates dynamic, [2..] scratch
-    unsigned long long *h_counters = nullptr;  // pinned
+    RunBlock *blk = nullptr;
+    RunBlock *h_blk = nullptr;       // pinned
+    RoundCtl *ctl = nullptr;         // parts of blk
+    unsigned long long *counters = nullptr;
+    RoundClock *clk = nullptr;
 };
 
 // Timing of one class of launches: pairs of events on the launching stream.
@@ -277,6 +296,7 @@ struct MemPool {
 struct DeviceState {
     og_approach approach = OG_ASCETIC;
     int device = 0;
+    int clock_khz = 100000;          // rate of the device's constant clock
     uint64_t V = 0, E = 0, Vpad = 0;
     uint32_t eb = 4;                 // bytes per edge on the device (static region, staging) and the link
     og_plan_info plan{};
@@ -585,25 +605,16 @@ uint64_t lane_state_bytes(const og_graph *g);
 // og_sssp from src on a lane; out (V values) may be null.
 void lane_run_sssp(og_graph *g, DeviceState *lane, uint32_t src, uint32_t *out, og_run_stats *st);
 
-// Resets f.ctl for a new traversal on stream s (a kernel, so it may sit in a
-// captured graph): statistics zeroed, near-far width `delta` with the first
-// threshold 1 + delta (the source's value is 1), or none for delta = 0;
-// `defer` 1 holds the dynamic list back in rounds with static work, 2 lets
-// dynamic vertices relax only once the static part of their bucket settled;
-// dir_opt_edges > 0 turns on the BFS direction choice over that many edges.
-// split: light/heavy split rounds (the graph's pmid rows; SSSP near-far).
-void frontier_begin(Frontier &f, hipStream_t s, uint32_t delta, uint32_t defer = 0, uint64_t dir_opt_edges = 0,
-                    bool split = false);
-
 // One compaction: flags -> bin lists / hub tiles / dynamic list with
 // its degree prefix, flags cleared; f.info and f.ctl updated on the device.
 // With `val` non-null, vertices whose value is >= f.ctl->thresh stay flagged
 // and are only counted (near-far order).  With to_host, the summary is also
 // copied to f.h_info (stream-ordered, not synchronised).
-// pmid (light/heavy split, with frontier_begin's split): rows are ranged by
-// the round's mode.
+// pmid (light/heavy split, a run with RoundCtl::split): rows are ranged by
+// the round's mode.  clk (optional): the run's clock, which leaves `prev`.
 void frontier_compact(DeviceState *d, Frontier &f, hipStream_t s, const uint32_t *val = nullptr,
-                      bool to_host = true, const uint64_t *pmid = nullptr);
+                      bool to_host = true, const uint64_t *pmid = nullptr, RoundClock *clk = nullptr,
+                      int prev = kClkOther);
 
 
 // Launches the static-region relax of the bins for op ALGO.  The kernels

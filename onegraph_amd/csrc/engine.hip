@@ -51,6 +51,41 @@ __global__ void k_set_source(uint32_t *val, uint8_t *flag, uint32_t src) {
     flag[src] = 1;
 }
 
+__device__ __forceinline__ void clock_stamp(RoundClock *clk, int prev, int kind) {
+    if (clk && blockIdx.x == 0 && threadIdx.x == 0) {
+        const unsigned long long t = wall_clock64();
+        atomicAdd(&clk->acc[prev], t);
+        atomicAdd(&clk->acc[kind], 0ull - t);
+    }
+}
+
+// Start of a single-source run, one launch: values (unreached, or with IOTA
+// each vertex its own label), next-frontier flags (the source, or every
+// vertex), counters, clock and traversal state.  Four vertices per lane.
+template <bool IOTA>
+__global__ __launch_bounds__(kBlock) void k_run_init(uint32_t *__restrict__ val, uint8_t *__restrict__ flag, uint64_t V,
+                                                     uint64_t Vpad, uint32_t src, RunBlock *__restrict__ blk,
+                                                     RoundCtl c) {
+    const uint64_t tid = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < 16) blk->counters[threadIdx.x] = 0;
+        if (threadIdx.x < 3) blk->clk.acc[threadIdx.x] = 0;
+        if (threadIdx.x == 0) blk->ctl = c;
+    }
+    for (uint64_t i = tid; i < Vpad / 4; i += (uint64_t)gridDim.x * kBlock) {
+        const uint64_t v = 4 * i;
+        uint32_t x[4], f = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const bool on = IOTA ? v + j < V : v + j == src;
+            x[j] = IOTA ? (uint32_t)(v + j) : on ? 1u : OG_UNREACHED;
+            f |= (on ? 1u : 0u) << (8 * j);
+        }
+        ((uint4 *)val)[i] = make_uint4(x[0], x[1], x[2], x[3]);
+        ((uint32_t *)flag)[i] = f;
+    }
+}
+
 // Bin of an active vertex: 0..2 static bins, 3 dynamic, 4 no out-edges,
 // 5 held back for a later round (near-far order: value >= threshold, checked
 // first so that held-back vertices need no degree), 6 a dynamic vertex held
@@ -261,7 +296,7 @@ __global__ __launch_bounds__(kCompactBlock) void k_frontier_compact(
     const uint64_t *__restrict__ ptr, const uint64_t *__restrict__ pmid, const uint32_t *__restrict__ deg,
     const uint32_t *__restrict__ hdeg, Tuning tn, const uint32_t *__restrict__ val_a, RoundCtl *ctl, CompactTotals ct,
     FrontierInfo *__restrict__ info, uint32_t *__restrict__ list, uint64_t *__restrict__ hub, uint64_t hub_cap,
-    uint64_t *__restrict__ doff, uint32_t *__restrict__ dchunk, uint64_t dchunk_cap) {
+    uint64_t *__restrict__ doff, uint32_t *__restrict__ dchunk, uint64_t dchunk_cap, RoundClock *clk, int clk_prev) {
     constexpr int kWaves = kCompactBlock / kWave;
     static_assert(NW * kWaves <= kWave, "one lane per (window, wave)");
     __shared__ uint64_t s_cnt[NW * kWaves], s_deg[NW * kWaves];  // per window and wave: packed counts, degrees
@@ -269,6 +304,7 @@ __global__ __launch_bounds__(kCompactBlock) void k_frontier_compact(
     __shared__ unsigned long long s_stat[2];  // static degrees, packed statistics
     __shared__ uint32_t s_more[3];            // lagging, held, smallest held-back value
     __shared__ uint64_t s_base[4];            // reserved places: bins 0 | 1, tiles, dynamic list, its edges
+    clock_stamp(clk, clk_prev, kClkFront);
     // a round enqueued after the traversal ended: no vertex is flagged, and
     // the summary and the traversal state stand
     if (ctl->halt && !ctl->live) return;
@@ -506,22 +542,30 @@ __global__ __launch_bounds__(kCompactBlock) void k_frontier_compact(
     if (wid == 0 && __ballot(last)) compact_finish(ct, info, doff, ctl);
 }
 
-__global__ void k_ctl_reset(RoundCtl *ctl, uint32_t delta, uint32_t defer, uint64_t dir_opt_edges, uint64_t V,
-                            uint32_t split) {
+// Traversal state at the start: near-far width `delta` with the first
+// threshold 1 + delta (the source's value is 1), or none for delta = 0;
+// `defer` 1 holds the dynamic list back in rounds with static work, 2 lets
+// dynamic vertices relax only once the static part of their bucket settled,
+// kDeferOnce holds them back until the static region has settled once;
+// dir_opt_edges > 0 turns on the BFS direction choice over that many edges;
+// split: light/heavy split rounds (the graph's pmid rows; SSSP near-far).
+static RoundCtl ctl_begin(uint64_t V, uint32_t delta, uint32_t defer, uint64_t dir_opt_edges, bool split) {
     RoundCtl c{};
-    c.split = split;
+    c.split = split ? 1u : 0u;
     c.delta = delta;
     c.defer = defer;
     c.dir_opt = dir_opt_edges ? 1u : 0u;
     c.unexplored = dir_opt_edges;
     c.nverts = V;
-    c.thresh = delta ? (uint32_t)min((uint64_t)0xFFFFFFFFull, 1ull + delta) : 0xFFFFFFFFu;
+    c.thresh = delta ? (uint32_t)std::min<uint64_t>(0xFFFFFFFFull, 1ull + delta) : 0xFFFFFFFFu;
     c.fbound = 0;
     c.hold = defer == 1 || defer == kDeferOnce ? 1u : 0u;
     c.live = 1;
     c.halt = 1;
-    *ctl = c;
+    return c;
 }
+
+__global__ void k_ctl_set(RoundCtl *ctl, RoundCtl c) { *ctl = c; }
 
 // ---------------------------------------------------------------- relax
 
@@ -882,12 +926,14 @@ struct RoundRelax {
     const uint32_t *dchunk;     // chunk table of the dynamic edge space
     uint64_t nl, vsplit;
     unsigned long long *counters;  // [0] static updates, [1] dynamic updates, [5] HBM-served dynamic edges
+    RoundClock *clk;            // null: not timed
 };
 constexpr uint32_t kFuseStatic = 5;
 
 template <int ALGO, bool W, bool PK, int LPV>
 __global__ __launch_bounds__(kBlock) void k_relax_round(RoundRelax r, RelaxArgs a) {
     extern __shared__ uint64_t s_fuse[];
+    clock_stamp(r.clk, kClkFront, kClkRelax);
     const uint32_t P = kFuseStatic + r.cd;
     const uint32_t K = gridDim.x / P;
     const uint32_t k = blockIdx.x / P, j = blockIdx.x - k * P;
@@ -1010,15 +1056,22 @@ __device__ __forceinline__ uint64_t d_mix64(uint64_t z) {
 // checksum = digest of val.
 // deg / hdeg: the degree table (hdeg: heavy degrees with the split, else
 // null), or null for the row bounds.  With the table, each lane reads four
-// values and four degrees per 16-byte load.
-__global__ __launch_bounds__(kBlock) void k_reach_stats(const uint32_t *__restrict__ val,
+// values and four degrees per 16-byte load.  Few, large workgroups
+// (stats_grid): each ends with three device-scope atomics on one line, which
+// queue at about 12 ns each (1024 workgroups of 256: 41 us at 1 M vertices).
+constexpr int kStatsBlock = 1024;
+__global__ __launch_bounds__(kStatsBlock) void k_reach_stats(const uint32_t *__restrict__ val,
                                                         const uint64_t *__restrict__ ptr,
                                                         const uint32_t *__restrict__ deg,
                                                         const uint32_t *__restrict__ hdeg, uint64_t V,
-                                                        unsigned long long *out) {
-    __shared__ uint64_t lds[kBlock / kWave];
+                                                        unsigned long long *out, RoundClock *clk) {
+    __shared__ unsigned long long s_sum[3];
+    if (threadIdx.x < 3) s_sum[threadIdx.x] = 0;
+    clock_stamp(clk, kClkFront, kClkOther);
+    __syncthreads();
     uint64_t r = 0, t = 0, h = 0;
-    const uint64_t tid = (uint64_t)blockIdx.x * kBlock + threadIdx.x, nth = (uint64_t)gridDim.x * kBlock;
+    const uint64_t tid = (uint64_t)blockIdx.x * kStatsBlock + threadIdx.x,
+                   nth = (uint64_t)gridDim.x * kStatsBlock;
     auto add = [&](uint64_t v, uint32_t x, uint64_t dv) {
         if (x != OG_UNREACHED) {
             ++r;
@@ -1057,14 +1110,12 @@ __global__ __launch_bounds__(kBlock) void k_reach_stats(const uint32_t *__restri
         const uint32_t x = val[v];
         add(v, x, deg ? (uint64_t)deg[v] + (hdeg ? hdeg[v] : 0u) : (x != OG_UNREACHED ? ptr[v + 1] - ptr[v] : 0));
     }
-    r = block_sum(r, lds);
-    t = block_sum(t, lds);
-    h = block_sum(h, lds);
-    if (threadIdx.x == 0) {
-        atomicAdd(out + 0, (unsigned long long)r);
-        atomicAdd(out + 1, (unsigned long long)t);
-        atomicAdd(out + 2, (unsigned long long)h);
-    }
+    const uint64_t w[3] = {wave_scan_u64(r), wave_scan_u64(t), wave_scan_u64(h)};
+    if ((threadIdx.x & (kWave - 1)) == kWave - 1)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) atomicAdd(&s_sum[i], (unsigned long long)w[i]);
+    __syncthreads();
+    if (threadIdx.x < 3 && s_sum[threadIdx.x]) atomicAdd(out + threadIdx.x, s_sum[threadIdx.x]);
 }
 
 // ------------------------------------------------------- multi-source BFS
@@ -1087,7 +1138,9 @@ __global__ void k_ms_init(const uint32_t *__restrict__ src, uint32_t n, uint64_t
 // active vertices so far + 1, read from the device state; a level past 255
 // sets ctl->overflow); vertices with nothing new leave the frontier.
 __global__ __launch_bounds__(kBlock) void k_ms_commit(uint8_t *__restrict__ flag, uint64_t V, uint64_t *visit,
-                                                      uint64_t *front, uint64_t *next, uint8_t *lvl, RoundCtl *ctl) {
+                                                      uint64_t *front, uint64_t *next, uint8_t *lvl, RoundCtl *ctl,
+                                                      RoundClock *clk) {
+    clock_stamp(clk, kClkRelax, kClkOther);
     const uint32_t lv32 = ctl->rounds + 1;
     const uint8_t level = (uint8_t)min(lv32, 255u);
     for (uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x; v < V; v += (uint64_t)gridDim.x * kBlock) {
@@ -1116,7 +1169,8 @@ __global__ __launch_bounds__(kBlock) void k_ms_commit(uint8_t *__restrict__ flag
 // vertex), partial sums leave with one atomic per lane per block.
 __global__ __launch_bounds__(kBlock) void k_ms_digest(const uint8_t *__restrict__ lvl,
                                                       const uint64_t *__restrict__ ptr, uint64_t V,
-                                                      unsigned long long *out /* 3 x 64 */) {
+                                                      unsigned long long *out /* 3 x 64 */, RoundClock *clk) {
+    clock_stamp(clk, kClkFront, kClkOther);
     const int lane = threadIdx.x & (kWave - 1);
     const uint64_t wave = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
     const uint64_t nwaves = (uint64_t)gridDim.x * kBlock / kWave;
@@ -1145,6 +1199,10 @@ __global__ void k_ms_extract(const uint8_t *__restrict__ lvl, uint64_t V, uint32
 // ============================================================ host driver
 
 static unsigned fill_grid(uint64_t n) { return (unsigned)std::min<uint64_t>(8192, std::max<uint64_t>(1, (n + 255) / 256)); }
+
+static unsigned stats_grid(uint64_t V) {
+    return (unsigned)std::min<uint64_t>(256, std::max<uint64_t>(1, (V + 8 * kStatsBlock - 1) / (8 * kStatsBlock)));
+}
 
 void device_state_free(DeviceState *d) {
     if (!d) return;
@@ -1237,11 +1295,12 @@ void frontier_alloc(DeviceState *d, const og_graph *g, Frontier &f, MemPool &m) 
     OG_HIP(hipGetLastError());
     OG_HIP(hipStreamSynchronize(d->s_compute));
     f.info = (FrontierInfo *)m.dalloc(sizeof(FrontierInfo));
-    f.ctl = (RoundCtl *)m.dalloc(sizeof(RoundCtl));
-    f.counters = (unsigned long long *)m.dalloc(16 * sizeof(unsigned long long));
+    f.blk = (RunBlock *)m.dalloc(sizeof(RunBlock));
+    f.ctl = &f.blk->ctl;
+    f.clk = &f.blk->clk;
+    f.counters = f.blk->counters;
     f.h_info = (FrontierInfo *)m.palloc(sizeof(FrontierInfo));
-    f.h_ctl = (RoundCtl *)m.palloc(sizeof(RoundCtl));
-    f.h_counters = (unsigned long long *)m.palloc(16 * sizeof(unsigned long long));
+    f.h_blk = (RunBlock *)m.palloc(sizeof(RunBlock));
     const uint64_t cap = std::max<uint64_t>(hub_capacity(g, d->plan.vsplit, d->tune), 1);
     f.hub = (uint64_t *)m.dalloc(cap * sizeof(uint64_t));
     f.hub_cap = cap;
@@ -1251,26 +1310,19 @@ void frontier_alloc(DeviceState *d, const og_graph *g, Frontier &f, MemPool &m) 
     OG_HIP(hipMemcpy(f.ctl, &c, sizeof c, hipMemcpyHostToDevice));
 }
 
-void frontier_begin(Frontier &f, hipStream_t s, uint32_t delta, uint32_t defer, uint64_t dir_opt_edges,
-                    bool split) {
-    hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(1), 0, s, f.ctl, delta, defer, dir_opt_edges, f.V,
-                       split ? 1u : 0u);
-    OG_HIP(hipGetLastError());
-}
-
 void frontier_compact(DeviceState *d, Frontier &f, hipStream_t s, const uint32_t *val, bool to_host,
-                      const uint64_t *pmid) {
+                      const uint64_t *pmid, RoundClock *clk, int prev) {
     // the degree table (a split round needs its light and heavy parts)
     const uint32_t *deg = d->d_deg && (!pmid || d->deg_split) ? d->d_deg : nullptr;
     const uint32_t *hdeg = deg ? d->deg_heavy() : nullptr;
     if (f.nw == 1)
         hipLaunchKernelGGL(k_frontier_compact<1>, dim3(f.nblk), dim3(kCompactBlock), 0, s, f.flag, f.hflag, d->Vpad,
                            d->plan.vsplit, d->d_ptr, pmid, deg, hdeg, d->tune, val, f.ctl, f.totals(), f.info, f.list,
-                           f.hub, f.hub_cap, f.doff, f.dchunk, f.dchunk_cap);
+                           f.hub, f.hub_cap, f.doff, f.dchunk, f.dchunk_cap, clk, prev);
     else
         hipLaunchKernelGGL(k_frontier_compact<4>, dim3(f.nblk), dim3(kCompactBlock), 0, s, f.flag, f.hflag, d->Vpad,
                            d->plan.vsplit, d->d_ptr, pmid, deg, hdeg, d->tune, val, f.ctl, f.totals(), f.info, f.list,
-                           f.hub, f.hub_cap, f.doff, f.dchunk, f.dchunk_cap);
+                           f.hub, f.hub_cap, f.doff, f.dchunk, f.dchunk_cap, clk, prev);
     OG_HIP(hipGetLastError());
     if (to_host) OG_HIP(hipMemcpyAsync(f.h_info, f.info, sizeof(FrontierInfo), hipMemcpyDeviceToHost, s));
 }
@@ -1511,6 +1563,7 @@ static void prepare_impl(og_graph *g, og_approach approach, const og_plan_params
     }
     std::unique_ptr<DeviceState, void (*)(DeviceState *)> d(new DeviceState, device_state_free);
     OG_HIP(hipGetDevice(&d->device));
+    OG_HIP(hipDeviceGetAttribute(&d->clock_khz, hipDeviceAttributeWallClockRate, d->device));
     d->approach = approach;
     d->V = g->V;
     d->E = g->E;
@@ -1742,6 +1795,7 @@ enum { kClsFront = 0, kClsStat = 1, kClsDyn = 2, kClsCopy = 3 };
 
 struct RunTimers {
     TimedClass front, stat, dyn, copy;
+    int clocked = -1;  // the relax class that the device's clock timed (with front), -1: none
     TimedClass &at(int c) { return c == kClsFront ? front : c == kClsStat ? stat : c == kClsDyn ? dyn : copy; }
 };
 
@@ -1764,9 +1818,7 @@ struct RoundGraph {
 
 // Timing marks of enqueued work.  EagerSpan: an EventSpan of the run per
 // launch sequence.  GraphSpan: a pair of event-record nodes in the graph
-// being captured; with `chain`, a span that follows another on the same
-// stream with nothing enqueued between them starts at that span's end event
-// (each event node costs the replay about ten microseconds).
+// being captured.  NoSpan: none (work that the device's clock times).
 struct EagerSpan {
     DeviceState *d;
     RunTimers &tm;
@@ -1779,26 +1831,24 @@ struct EagerSpan {
 
 struct GraphSpan {
     RoundGraph *rg;
-    bool chain = false;
-    mutable hipEvent_t last = nullptr;
-    mutable hipStream_t last_s = nullptr;
     template <class F>
     void operator()(int cls, hipStream_t s, F &&fn) const {
         hipEvent_t a = nullptr, b = nullptr;
-        if (chain && last && last_s == s) {
-            a = last;
-        } else {
-            OG_HIP(hipEventCreate(&a));
-            rg->events.push_back(a);
-            OG_HIP(hipEventRecordWithFlags(a, s, hipEventRecordExternal));
-        }
+        OG_HIP(hipEventCreate(&a));
+        rg->events.push_back(a);
+        OG_HIP(hipEventRecordWithFlags(a, s, hipEventRecordExternal));
         OG_HIP(hipEventCreate(&b));
         rg->events.push_back(b);
         fn();
         OG_HIP(hipEventRecordWithFlags(b, s, hipEventRecordExternal));
         rg->marks.push_back({cls, a, b});
-        last = b;
-        last_s = s;
+    }
+};
+
+struct NoSpan {
+    template <class F>
+    void operator()(int, hipStream_t, F &&fn) const {
+        fn();
     }
 };
 
@@ -1993,6 +2043,7 @@ static void launch_round_fmt(DeviceState *d, bool with_dyn) {
     r.nl = d->split_nl;
     r.vsplit = d->plan.vsplit;
     r.counters = d->fr.counters;
+    r.clk = d->fr.clk;
     const unsigned grid = (kFuseStatic + r.cd) * kHubGridCap;
     const size_t lds = std::max<size_t>(with_dyn ? sizeof(DynLds) : 0, (size_t)d->tune.tile * d->eb);
     switch (d->tune.lpv0) {
@@ -2132,11 +2183,13 @@ constexpr int kRoundBatchMax = 64;  // largest first batch (sized from the previ
 // trip: each costs about 50 us); later batches kRoundBatch.  The staged loader needs
 // the host in every round (gather, copies), so it synchronises on each
 // round's summary.
-// quiet_after: after() enqueues nothing (its rounds' timing spans may chain).
-template <int ALGO, bool W, class After>
+// quiet_after: after() enqueues nothing (the compaction follows the relax).
+// begin(ctl): enqueues the start of the run with that traversal state.
+template <int ALGO, bool W, class Begin, class After>
 static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTimers &tm, double &gather_ms,
-                          double &overload_wall, After after, bool quiet_after) {
+                          double &overload_wall, Begin begin, After after, bool quiet_after) {
     hipStream_t s = d->s_compute;
+    const uint64_t V = d->V;
     // SSSP near-far order: only vertices below the threshold relax in a
     // round; when none is left it moves to (smallest held-back value + delta).
     const uint32_t delta = ALGO == ALGO_SSSP ? d->tune.delta : 0;
@@ -2158,10 +2211,9 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
     const bool split = ALGO == ALGO_SSSP && delta && d->d_pmid;
     d->run_pmid = split ? d->d_pmid : nullptr;
     const uint64_t *pm = d->run_pmid;
-    frontier_begin(d->fr, s, delta, defer, dir_opt ? std::max<uint64_t>(d->E, 1) : 0, split);
+    begin(ctl_begin(V, delta, defer, dir_opt ? std::max<uint64_t>(d->E, 1) : 0, split));
+    RunBlock *const h = d->fr.h_blk;
     if (!staged) {
-        const EagerSpan eager{d, tm};
-        eager(kClsFront, s, [&] { frontier_compact(d, d->fr, s, nf_val, false, pm); });
         // one batch: kRoundBatch x (static || dynamic relax, after, compaction),
         // then the traversal state to the host
         // With both regions the static and dynamic relax of a round run as
@@ -2173,6 +2225,14 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
         const bool overlap = has_dyn && !(d->flags & OG_PLAN_NO_OVERLAP);
         const bool fuse = overlap && !(d->flags & OG_PLAN_NO_FUSE);
         const bool fuse_static = !has_dyn && !(d->flags & OG_PLAN_NO_FUSE);
+        // One launch per round and region is timed by the device's clock, the
+        // two-stream and separate launches by events.
+        const bool clocked = fuse || fuse_static;
+        RoundClock *const clk = clocked ? d->fr.clk : nullptr;
+        const EagerSpan eager{d, tm};
+        auto first = [&] { frontier_compact(d, d->fr, s, nf_val, false, pm, clk, kClkOther); };
+        if (clocked) first();
+        else eager(kClsFront, s, first);
         auto batch = [&](const auto &span, int rounds) {
             for (int r = 0; r < rounds; ++r) {
                 bool joined = false;
@@ -2200,11 +2260,18 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
                         OG_HIP(hipGetLastError());
                     });
                 if (joined) OG_HIP(hipStreamWaitEvent(s, d->ev_static, 0));
-                after();
-                span(kClsFront, s, [&] { frontier_compact(d, d->fr, s, nf_val, false, pm); });
+                after(clk);
+                span(kClsFront, s,
+                     [&] { frontier_compact(d, d->fr, s, nf_val, false, pm, clk, quiet_after ? kClkRelax : kClkOther); });
             }
-            OG_HIP(hipMemcpyAsync(d->fr.h_ctl, d->fr.ctl, sizeof(RoundCtl), hipMemcpyDeviceToHost, s));
+            OG_HIP(hipMemcpyAsync(h, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
         };
+        const NoSpan untimed;
+        auto enqueue = [&](const auto &span, int rounds) {
+            if (clocked) batch(untimed, rounds);
+            else batch(span, rounds);
+        };
+        uint64_t enqueued = 0;
         if (!(d->flags & OG_PLAN_NO_GRAPH)) {
             // first batch: exactly the pairs the previous run took (a 6-round
             // BFS replayed 8 rounds when this was rounded up to a multiple of
@@ -2216,10 +2283,9 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
                                      (uint64_t)has_dyn << 6 | (uint64_t)dir_opt << 7 | (uint64_t)split << 16 |
                                      (uint64_t)rounds << 8;
                 RoundGraph *rg = round_graph_for(d, key, [&](RoundGraph *n) {
-                    GraphSpan gs{n};
-                    gs.chain = (fuse || fuse_static) && quiet_after;  // one stream: relax span(s), then compaction
-                    batch(gs, rounds);
+                    enqueue(GraphSpan{n}, rounds);
                 });
+                enqueued += rounds;
                 rounds = kRoundBatch;
                 OG_HIP(hipGraphLaunch(rg->exec, s));
                 OG_HIP(hipStreamSynchronize(s));
@@ -2232,16 +2298,22 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
                         (void)hipGetLastError();
                     }
                 }
-                if (!d->fr.h_ctl->live) break;
+                if (!h->ctl.live) break;
             }
             // relax + compaction pairs of this run, for the next run's first batch
-            d->last_pairs[ALGO] = d->fr.h_ctl->compactions ? d->fr.h_ctl->compactions - 1 : 0;
+            d->last_pairs[ALGO] = h->ctl.compactions ? h->ctl.compactions - 1 : 0;
         } else {
             for (;;) {
-                batch(eager, kRoundBatch);
+                enqueue(eager, kRoundBatch);
+                enqueued += kRoundBatch;
                 OG_HIP(hipStreamSynchronize(s));
-                if (!d->fr.h_ctl->live) break;
+                if (!h->ctl.live) break;
             }
+        }
+        if (clocked) {  // their times come with the run block, once the run's last kernel has left the compaction
+            (fuse ? tm.dyn : tm.stat).launches += enqueued * (dir_opt ? 2 : 1);
+            tm.front.launches += enqueued + 1;
+            tm.clocked = fuse ? kClsDyn : kClsStat;
         }
     } else {
         {
@@ -2263,7 +2335,7 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
                     overload_wall += ow.ms();
                 }
                 if (joined) OG_HIP(hipStreamWaitEvent(s, d->ev_static, 0));
-                after();
+                after(nullptr);
             }
             {
                 EventSpan span(d, &tm.front, s);
@@ -2271,10 +2343,10 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
             }
             OG_HIP(hipStreamSynchronize(s));
         }
-        OG_HIP(hipMemcpyAsync(d->fr.h_ctl, d->fr.ctl, sizeof(RoundCtl), hipMemcpyDeviceToHost, s));
+        OG_HIP(hipMemcpyAsync(h, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
         OG_HIP(hipStreamSynchronize(s));
     }
-    const RoundCtl c = *d->fr.h_ctl;
+    const RoundCtl c = h->ctl;
     if (c.overflow) raise(OG_EUNSUPPORTED, "multi-source BFS deeper than 254 levels");
     st.iterations += c.rounds;
     st.node_sum += c.node_sum;
@@ -2293,8 +2365,15 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
     }
 }
 
-static void finish_stats(og_run_stats &st, RunTimers &tm, double gather_ms, double overload_wall,
-                         const unsigned long long *ctr, uint64_t upd_bytes, uint64_t link_eb) {
+static void finish_stats(og_run_stats &st, RunTimers &tm, double gather_ms, double overload_wall, const DeviceState *d,
+                         uint64_t upd_bytes) {
+    const RunBlock &h = *d->fr.h_blk;
+    const unsigned long long *ctr = h.counters;
+    const uint64_t link_eb = d->deb;
+    if (tm.clocked >= 0) {
+        tm.at(tm.clocked).ms += (double)(int64_t)h.clk.acc[kClkRelax] / d->clock_khz;
+        tm.front.ms += (double)(int64_t)h.clk.acc[kClkFront] / d->clock_khz;
+    }
     st.updates = ctr[0] + ctr[1];
     // dynamic edges served from the HBM-resident head did not cross the link
     st.h2d_bytes -= std::min<uint64_t>(st.h2d_bytes, ctr[5] * link_eb);
@@ -2329,38 +2408,25 @@ static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats 
     OG_HIP(hipStreamSynchronize(d->s_static));
     OG_HIP(hipStreamSynchronize(s));
     Stopwatch total;
-    OG_HIP(hipMemsetAsync(d->fr.counters, 0, 16 * sizeof(unsigned long long), s));
-    if (ALGO == ALGO_CC) {
-        hipLaunchKernelGGL(k_iota, dim3(fill_grid(V)), dim3(256), 0, s, d->d_val, V);
-        hipLaunchKernelGGL(k_fill_u8, dim3(fill_grid(V)), dim3(256), 0, s, d->fr.flag, V, (uint8_t)1);
-    } else {
-        hipLaunchKernelGGL(k_fill_u8, dim3(fill_grid(d->Vpad)), dim3(256), 0, s, d->fr.flag, d->Vpad, (uint8_t)0);
-        hipLaunchKernelGGL(k_fill_u32, dim3(fill_grid(V)), dim3(256), 0, s, d->d_val, V, OG_UNREACHED);
-        hipLaunchKernelGGL(k_set_source, dim3(1), dim3(1), 0, s, d->d_val, d->fr.flag, src);
-    }
-    OG_HIP(hipGetLastError());
-    frontier_loop<ALGO, W>(g, d, st, tm, gather_ms, overload_wall, []() {}, true);
+    auto begin = [&](const RoundCtl &c) {
+        hipLaunchKernelGGL((k_run_init<ALGO == ALGO_CC>), dim3(fill_grid(d->Vpad / 4)), dim3(kBlock), 0, s, d->d_val,
+                           d->fr.flag, V, d->Vpad, src, d->fr.blk, c);
+        OG_HIP(hipGetLastError());
+    };
+    frontier_loop<ALGO, W>(g, d, st, tm, gather_ms, overload_wall, begin, [](RoundClock *) {}, true);
     OG_HIP(hipStreamSynchronize(s));
     st.total_ms = total.ms();
 
-    {
-        // one lane per four vertices with the degree table, at most 2048
-        // workgroups (three atomics each on the same three counters: 16384
-        // workgroups spent 0.6 ms on them)
-        const uint64_t lanes = d->d_deg ? (V + 3) / 4 : V;
-        const unsigned grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(2048, (lanes + kBlock - 1) / kBlock));
-        hipLaunchKernelGGL(k_reach_stats, dim3(grid), dim3(kBlock), 0, s, d->d_val, d->d_ptr, d->d_deg,
-                           d->deg_heavy(), V,
-                           d->fr.counters + 2);
-    }
+    hipLaunchKernelGGL(k_reach_stats, dim3(stats_grid(V)), dim3(kStatsBlock), 0, s, d->d_val, d->d_ptr, d->d_deg,
+                       d->deg_heavy(), V, d->fr.counters + 2, tm.clocked >= 0 ? d->fr.clk : nullptr);
     OG_HIP(hipGetLastError());
-    OG_HIP(hipMemcpyAsync(d->fr.h_counters, d->fr.counters, 16 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    OG_HIP(hipMemcpyAsync(d->fr.h_blk, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
     if (out) copy_to_host(d, out, d->d_val, V * sizeof(uint32_t), s);
     OG_HIP(hipStreamSynchronize(s));
-    st.reached = d->fr.h_counters[2];
-    st.traversed_edges = d->fr.h_counters[3];
-    st.checksum = d->fr.h_counters[4];
-    finish_stats(st, tm, gather_ms, overload_wall, d->fr.h_counters, 8, d->deb);
+    st.reached = d->fr.h_blk->counters[2];
+    st.traversed_edges = d->fr.h_blk->counters[3];
+    st.checksum = d->fr.h_blk->counters[4];
+    finish_stats(st, tm, gather_ms, overload_wall, d, 8);
     if (stats) *stats = st;
 }
 
@@ -2391,7 +2457,7 @@ static void run_msbfs(og_graph *g, const uint32_t *sources, uint32_t n, uint32_t
     OG_HIP(hipStreamSynchronize(d->s_static));
     OG_HIP(hipStreamSynchronize(s));
     Stopwatch total;
-    OG_HIP(hipMemsetAsync(d->fr.counters, 0, 16 * sizeof(unsigned long long), s));
+    OG_HIP(hipMemsetAsync(d->fr.blk, 0, sizeof(RunBlock), s));
     double device_ms = 0;
     for (uint32_t b0 = 0; b0 < n; b0 += kMsWidth) {
         const uint32_t nb = std::min<uint32_t>(kMsWidth, n - b0);
@@ -2405,14 +2471,19 @@ static void run_msbfs(og_graph *g, const uint32_t *sources, uint32_t n, uint32_t
                            d->fr.flag, d->d_mlvl);
         OG_HIP(hipGetLastError());
         const unsigned cgrid = (unsigned)std::min<uint64_t>(4096, (V + kBlock - 1) / kBlock);
-        frontier_loop<ALGO_MSBFS, W>(g, d, st, tm, gather_ms, overload_wall, [&]() {
+        auto begin = [&](const RoundCtl &c) {
+            hipLaunchKernelGGL(k_ctl_set, dim3(1), dim3(1), 0, s, d->fr.ctl, c);
+            OG_HIP(hipGetLastError());
+        };
+        frontier_loop<ALGO_MSBFS, W>(g, d, st, tm, gather_ms, overload_wall, begin, [&](RoundClock *clk) {
             hipLaunchKernelGGL(k_ms_commit, dim3(cgrid), dim3(kBlock), 0, s, d->fr.flag, V, d->d_visit, d->d_front,
-                               d->d_next, d->d_mlvl, d->fr.ctl);
+                               d->d_next, d->d_mlvl, d->fr.ctl, clk);
             OG_HIP(hipGetLastError());
         }, false);
         OG_HIP(hipMemsetAsync(d->d_msum, 0, 3 * kMsWidth * 8, s));
         hipLaunchKernelGGL(k_ms_digest, dim3((unsigned)std::min<uint64_t>(1024, (V + kBlock - 1) / kBlock)),
-                           dim3(kBlock), 0, s, d->d_mlvl, d->d_ptr, V, d->d_msum);
+                           dim3(kBlock), 0, s, d->d_mlvl, d->d_ptr, V, d->d_msum,
+                           tm.clocked >= 0 ? d->fr.clk : nullptr);
         OG_HIP(hipGetLastError());
         OG_HIP(hipMemcpyAsync(hsum.data(), d->d_msum, 3 * kMsWidth * 8, hipMemcpyDeviceToHost, s));
         OG_HIP(hipStreamSynchronize(s));
@@ -2435,9 +2506,9 @@ static void run_msbfs(og_graph *g, const uint32_t *sources, uint32_t n, uint32_t
         }
     }
     st.total_ms = device_ms;
-    OG_HIP(hipMemcpyAsync(d->fr.h_counters, d->fr.counters, 16 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    OG_HIP(hipMemcpyAsync(d->fr.h_blk, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
     OG_HIP(hipStreamSynchronize(s));
-    finish_stats(st, tm, gather_ms, overload_wall, d->fr.h_counters, 9, d->deb);
+    finish_stats(st, tm, gather_ms, overload_wall, d, 9);
     if (stats) *stats = st;
 }
 
@@ -2448,6 +2519,7 @@ DeviceState *lane_state_create(og_graph *g, uint32_t delta) {
     // the graph as prepared (read only: every array below belongs to g->dev)
     l->approach = d->approach;
     l->device = d->device;
+    l->clock_khz = d->clock_khz;
     l->V = d->V;
     l->E = d->E;
     l->Vpad = d->Vpad;
@@ -2490,10 +2562,10 @@ uint64_t lane_state_bytes(const og_graph *g) {
     const uint64_t hub = std::max<uint64_t>(hub_capacity(g, d->plan.vsplit, d->tune), 1);
     // what lane_state_create and frontier_alloc request: values, flags (and
     // the heavy-round flags with the split), bin lists, degree prefix, the
-    // (empty) dynamic chunk table, compaction totals, round summary, control
-    // block, counters and hub tiles
+    // (empty) dynamic chunk table, compaction totals, round summary, run
+    // block and hub tiles
     return 4 * Vpad + Vpad * (d->d_pmid ? 2 : 1) + 4 * V + 8 * (V + 1) + 4 * 2 + 8 * totals_words(nblk) +
-           sizeof(FrontierInfo) + sizeof(RoundCtl) + 16 * 8 + 8 * hub;
+           sizeof(FrontierInfo) + sizeof(RunBlock) + 8 * hub;
 }
 
 void lane_run_sssp(og_graph *g, DeviceState *lane, uint32_t src, uint32_t *out, og_run_stats *st) {
@@ -3019,13 +3091,13 @@ static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t 
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, (uint32_t *)ctr, (uint64_t)32, 0u);
     hipLaunchKernelGGL(k_fill_u32, dim3(fill_grid(V)), dim3(256), 0, s, d_levels, V, OG_UNREACHED);
     hipLaunchKernelGGL(k_set_source, dim3(1), dim3(1), 0, s, d_levels, flag, src);
-    hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(1), 0, s, ctl, 0u, 0u, (uint64_t)0, V, 0u);
+    hipLaunchKernelGGL(k_ctl_set, dim3(1), dim3(1), 0, s, ctl, ctl_begin(V, 0, 0, 0, false));
     hipLaunchKernelGGL(k_totals_init, dim3(fill_grid(totals_words(nblk))), dim3(256), 0, s, ct.t, totals_words(nblk));
     auto compact = [&] {
         hipLaunchKernelGGL(k_frontier_compact<1>, dim3(nblk), dim3(kCompactBlock), 0, s, flag, (uint8_t *)nullptr, Vpad, V,
                            d_ptr, (const uint64_t *)nullptr, (const uint32_t *)nullptr, (const uint32_t *)nullptr, tn,
                            (const uint32_t *)nullptr, ctl, ct, info, list, hub, kNoAllocHubCap, doff,
-                           (uint32_t *)nullptr, (uint64_t)0);
+                           (uint32_t *)nullptr, (uint64_t)0, (RoundClock *)nullptr, (int)kClkOther);
     };
     RoundRelax r{};
     r.list = list;
@@ -3055,9 +3127,8 @@ static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t 
         if (!h.live) break;
     }
     const double ms = total.ms();
-    hipLaunchKernelGGL(k_reach_stats, dim3((unsigned)std::min<uint64_t>(2048, (V + kBlock - 1) / kBlock)),
-                       dim3(kBlock), 0, s, d_levels, d_ptr, (const uint32_t *)nullptr, (const uint32_t *)nullptr, V,
-                       ctr + 2);
+    hipLaunchKernelGGL(k_reach_stats, dim3(stats_grid(V)), dim3(kStatsBlock), 0, s, d_levels, d_ptr,
+                       (const uint32_t *)nullptr, (const uint32_t *)nullptr, V, ctr + 2, (RoundClock *)nullptr);
     OG_HIP(hipGetLastError());
     unsigned long long hc[16];
     OG_HIP(hipMemcpyAsync(hc, ctr, sizeof hc, hipMemcpyDeviceToHost, s));

@@ -293,6 +293,15 @@ struct MemPool {
     }
 };
 
+// PageRank's scalars on the device: what an iteration leaves for the next.
+struct PrState {
+    double dangling;      // rank mass of the vertices without out-edges
+    double l1;            // residual of the last iteration
+    double tolerance;
+    uint32_t iterations;
+    uint32_t done;        // the residual fell below the tolerance: later iterations do nothing
+};
+
 struct DeviceState {
     og_approach approach = OG_ASCETIC;
     int device = 0;
@@ -335,6 +344,13 @@ struct DeviceState {
     // V - vsplit + 1 entries
     uint64_t *d_lpos = nullptr;
     uint64_t split_nl = 0;           // light edges of the dynamic region
+    // Link format: when an edge word (id, or id << wbits | weight) fits lbits
+    // <= kLinkBitsMax bits, the dynamic region crosses the link as a stream of
+    // lbits-bit words (edge i of the host layout at bit i * lbits): zero-copy
+    // reads and PageRank's chunks.  0: the 4- or 8-byte edges.
+    uint32_t lbits = 0;
+    const uint32_t *h_link = nullptr;   // pinned
+    const void *hd_link = nullptr;      // the same, as a device address
     uint64_t dyn_resident = 0;       // zero-copy: dynamic edges held in d_staging (whole chunks)
     int64_t *d_rdelta = nullptr;     // zero-copy: per chunk of kResChunk vertices (index v >> kResChunkShift),
                                      // d_staging index - host-array position, or kNotResident; two per
@@ -373,19 +389,20 @@ struct DeviceState {
     uint32_t *d_in_cols = nullptr;   // E in-neighbours
 
     // PageRank state (allocated on first use)
-    void *d_rank[2] = {nullptr, nullptr};
-    void *d_contrib = nullptr;
+    void *d_rank = nullptr;
+    void *d_contrib[2] = {nullptr, nullptr};  // read / written in turn
     uint32_t *d_outdeg = nullptr;
-    double *d_partial = nullptr;     // per-block residual / dangling partials
-    double *d_scalars = nullptr;     // [0] dangling, [1] l1
-    double *h_scalars = nullptr;
-    uint64_t pr_partial_cap = 0;     // entries of d_partial
-    bool pr_fp64 = false;
-    std::shared_ptr<void> pr_plan;
+    double *d_partial = nullptr;     // per-block residual and dangling partials
+    unsigned long long *d_prtot = nullptr;  // arrivals of the pull's workgroups
+    uint64_t pr_partial_cap = 0;     // workgroups that d_partial and d_prtot are sized for
+    PrState *d_prstate = nullptr;
+    PrState *h_prstate = nullptr;    // pinned
+    unsigned long long *h_progress = nullptr;  // pinned, written by the device: iterations << 1 | done
+    std::shared_ptr<void> pr_plan;   // PageRank rows and chunk ranges (pagerank.hip)
     std::shared_ptr<void> round_graph;  // captured batches of device-driven rounds (engine.hip)
     void *h_out[2] = {nullptr, nullptr};  // pinned staging chunks of result copy-backs (copy_to_host)
     hipEvent_t ev_out[2] = {nullptr, nullptr};
-    uint32_t last_pairs[8] = {};        // relax + compaction pairs of the last device-driven run, per algorithm   // PageRank bins and chunk ranges (pagerank.hip)
+    uint32_t last_pairs[8] = {};        // relax + compaction pairs of the last device-driven run, per algorithm
 
     MemPool mem;                     // device + pinned allocations of this preparation
 
@@ -395,6 +412,28 @@ struct DeviceState {
 };
 
 // ------------------------------------------------------------ wave helpers
+
+// Waits until the wave's memory operations, atomics among them, are done.
+// With device-scope atomics on both sides (performed at one place for the
+// whole device) this orders a workgroup's reservations before its arrival
+// without a release fence, which on gfx950 writes the whole L2 of the XCD
+// back.
+__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// True in the workgroup that arrives last (called by one thread of each).
+// Arrivals are counted in two levels, kTotGroup workgroups per first-level
+// counter: same-address atomics take about 12 ns each.
+__device__ __forceinline__ bool arrive_last(const CompactTotals &ct) {
+    const uint32_t g = blockIdx.x / kTotGroup, ng = (ct.nblk + kTotGroup - 1) / kTotGroup;
+    unsigned long long *at = ct.t + kTotArrive + (uint64_t)g * kTotLine;
+    if (atomicAdd(at, 1ull) + 1 != min(kTotGroup, ct.nblk - g * kTotGroup)) return false;
+    atomicExch(at, 0ull);
+    if (ng > 1) {
+        if (atomicAdd(ct.t + kTotRoot, 1ull) + 1 != ng) return false;
+        atomicExch(ct.t + kTotRoot, 0ull);
+    }
+    return true;
+}
 
 __device__ __forceinline__ uint64_t shfl_up_u64(uint64_t x, int d) {
     uint32_t lo = (uint32_t)x, hi = (uint32_t)(x >> 32);
@@ -543,6 +582,21 @@ __device__ __forceinline__ void load_edge(const void *__restrict__ edges, uint64
     }
 }
 
+// Narrowest saving worth a second copy of the dynamic region in host memory:
+// an eighth of the link's bytes.
+constexpr uint32_t kLinkBitsMax = 28;
+
+// Word i of a stream of `bits`-bit words that starts `first` bits into p: one
+// 8-byte load (the stream is padded by a word), so that a wave's lanes touch
+// each link line once.
+__device__ __forceinline__ uint32_t link_word(const uint32_t *__restrict__ p, uint64_t i, uint32_t bits, uint32_t first = 0) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2), aligned(4)));
+    const uint64_t at = i * bits + first;
+    const u32x2 x = *(const u32x2 *)(p + (at >> 5));
+    const uint64_t w = ((uint64_t)x.y << 32 | x.x) >> (at & 31);
+    return (uint32_t)w & (uint32_t)((1ull << bits) - 1);
+}
+
 // ------------------------------------------------------------- host timing
 
 struct Stopwatch {
@@ -579,6 +633,10 @@ inline double sum_ms(const TimedClass &c) {
     }
     return t;
 }
+
+// Waits until the device has raised the pinned word *p (which it writes with
+// system scope while it runs) to at least `want`, or the stream has drained.
+void wait_progress(const unsigned long long *p, unsigned long long want, hipStream_t s);
 
 // Copies n bytes of device memory at src to host memory at dst (pageable or
 // not) on stream s and returns when they are there.  Large copies go through

@@ -24,6 +24,7 @@
 #include <vector>
 #include <cstdio>
 #include <cstring>
+#include <thread>
 
 #include "device.h"
 
@@ -100,13 +101,6 @@ __device__ __forceinline__ int bin_of(bool far, bool hold, uint64_t v, uint64_t 
     return 2;
 }
 
-// Waits until the wave's memory operations, atomics among them, are done.
-// With device-scope atomics on both sides (performed at one place for the
-// whole device) this orders a workgroup's reservations before its arrival
-// without a release fence, which on gfx950 writes the whole L2 of the XCD
-// back.
-__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
 // Reserves n entries with dd edges at the end of the dynamic list; the two
 // counts move together, so the list's degree prefix rises with the list.
 // One word holds both when they fit (count in the low dsh bits); else a lock
@@ -124,21 +118,6 @@ __device__ __forceinline__ void reserve_dyn(const CompactTotals &ct, uint64_t n,
     pd = atomicAdd(t + kTotWide + 2, (unsigned long long)dd);
     wait_vmem();
     atomicExch(t + kTotWide, 0ull);
-}
-
-// True in the workgroup that arrives last (called by one thread of each).
-// Arrivals are counted in two levels, kTotGroup workgroups per first-level
-// counter: same-address atomics take about 12 ns each.
-__device__ __forceinline__ bool arrive_last(const CompactTotals &ct) {
-    const uint32_t g = blockIdx.x / kTotGroup, ng = (ct.nblk + kTotGroup - 1) / kTotGroup;
-    unsigned long long *at = ct.t + kTotArrive + (uint64_t)g * kTotLine;
-    if (atomicAdd(at, 1ull) + 1 != min(kTotGroup, ct.nblk - g * kTotGroup)) return false;
-    atomicExch(at, 0ull);
-    if (ng > 1) {
-        if (atomicAdd(ct.t + kTotRoot, 1ull) + 1 != ng) return false;
-        atomicExch(ct.t + kTotRoot, 0ull);
-    }
-    return true;
 }
 
 // Totals between compactions: zero, each slot's smallest held-back value all
@@ -758,8 +737,9 @@ __global__ __launch_bounds__(kBlock) void k_relax_hub(const uint64_t *__restrict
 // x = ptr[u] + (q - doff[i]); when u's chunk of kResChunk vertices is
 // resident in HBM (rdelta[u >> kResChunkShift] != kNotResident) it is read
 // from `resident` at x + rdelta, else in place from the pinned host array
-// through its device mapping (`stage`, at x - dbase); reads served from HBM
-// are counted in *hits.  (Storing the host rows in
+// through its device mapping (`stage`, at x - dbase, whole edges or with
+// lbits a stream of lbits-bit words); reads served from HBM are counted in
+// *hits.  (Storing the host rows in
 // order of distance from a hub instead of vertex order was measured slower
 // on R-MAT: the active list stays in vertex order, so neighbouring lanes then
 // read scattered rows.)
@@ -785,7 +765,7 @@ __device__ __forceinline__ uint32_t relax_dyn_body(const uint32_t *__restrict__ 
                                                    const int64_t *__restrict__ rdelta, uint32_t wbits,
                                                    const RelaxArgs &a, const uint64_t *__restrict__ lpos,
                                                    uint64_t nl, uint64_t vsplit, const uint32_t *__restrict__ dchunk,
-                                                   DynLds &L, uint32_t bid, uint32_t nb, uint32_t &hits) {
+                                                   uint32_t lbits, DynLds &L, uint32_t bid, uint32_t nb, uint32_t &hits) {
     uint64_t *s_off = L.off;
     uint32_t *s_i = L.i;
     const uint32_t ndyn = info->n[3];
@@ -858,6 +838,10 @@ __device__ __forceinline__ uint32_t relax_dyn_body(const uint32_t *__restrict__ 
                     if (dl != kNotResident) {
                         load_edge<W, PACKED>(resident, (uint64_t)((int64_t)hp + dl), wbits, to[j], wt[j]);
                         ++h;
+                    } else if (lbits) {
+                        const uint32_t x = link_word((const uint32_t *)stage, hp, lbits);
+                        to[j] = W ? x >> wbits : x;
+                        wt[j] = W ? x & ((1u << wbits) - 1u) : 1u;
                     } else {
                         load_edge<W, PACKED>(stage, hp, wbits, to[j], wt[j]);
                     }
@@ -888,11 +872,12 @@ __global__ __launch_bounds__(kBlock) void k_relax_dyn(const uint32_t *__restrict
                                                       const int64_t *__restrict__ rdelta,
                                                       uint32_t wbits, RelaxArgs a, const uint64_t *__restrict__ lpos,
                                                       uint64_t nl, uint64_t vsplit, const uint32_t *__restrict__ dchunk,
-                                                      unsigned long long *upd, unsigned long long *hits) {
+                                                      uint32_t lbits, unsigned long long *upd,
+                                                      unsigned long long *hits) {
     __shared__ DynLds L;
     uint32_t h = 0;
     const uint32_t c = relax_dyn_body<ALGO, W, PACKED, DIRECT>(list, info, doff, stage, c0, c1max, ptr, dbase, resident,
-                                                               rdelta, wbits, a, lpos, nl, vsplit, dchunk, L,
+                                                               rdelta, wbits, a, lpos, nl, vsplit, dchunk, lbits, L,
                                                                blockIdx.x, gridDim.x, h);
     wave_add(upd, c);
     if (DIRECT) wave_add(hits, h);
@@ -924,6 +909,7 @@ struct RoundRelax {
     const int64_t *rdelta;
     const uint64_t *lpos;       // split layout of the host copy (null: rows whole)
     const uint32_t *dchunk;     // chunk table of the dynamic edge space
+    uint32_t lbits;             // bits per edge of the dynamic region in host memory (0: whole edges)
     uint64_t nl, vsplit;
     unsigned long long *counters;  // [0] static updates, [1] dynamic updates, [5] HBM-served dynamic edges
     RoundClock *clk;            // null: not timed
@@ -950,7 +936,7 @@ __global__ __launch_bounds__(kBlock) void k_relax_round(RoundRelax r, RelaxArgs 
         uint32_t h = 0;
         const uint32_t c = relax_dyn_body<ALGO, W, PK, true>(r.list, r.info, r.doff, r.stage, 0, ~0ull, r.ptr, r.dbase,
                                                              r.resident, r.rdelta, a.wbits, a, r.lpos, r.nl, r.vsplit,
-                                                             r.dchunk, *(DynLds *)s_fuse, r.cd * k + (j - kFuseStatic),
+                                                             r.dchunk, r.lbits, *(DynLds *)s_fuse, r.cd * k + (j - kFuseStatic),
                                                              r.cd * K, h);
         wave_add(r.counters + 1, c);
         wave_add(r.counters + 5, h);
@@ -1199,6 +1185,20 @@ __global__ void k_ms_extract(const uint8_t *__restrict__ lvl, uint64_t V, uint32
 // ============================================================ host driver
 
 static unsigned fill_grid(uint64_t n) { return (unsigned)std::min<uint64_t>(8192, std::max<uint64_t>(1, (n + 255) / 256)); }
+
+void wait_progress(const unsigned long long *p, unsigned long long want, hipStream_t s) {
+    for (uint64_t i = 1;; ++i) {
+        if (__atomic_load_n(p, __ATOMIC_ACQUIRE) >= want) return;
+        if (i % 1024) {
+            __builtin_ia32_pause();
+            continue;
+        }
+        const hipError_t e = hipStreamQuery(s);  // about every 40 us: also how a device error ends the wait
+        if (e == hipSuccess) return;
+        if (e != hipErrorNotReady) OG_HIP(e);
+        if (i >= (1u << 16)) std::this_thread::sleep_for(std::chrono::microseconds(20));
+    }
+}
 
 static unsigned stats_grid(uint64_t V) {
     return (unsigned)std::min<uint64_t>(256, std::max<uint64_t>(1, (V + 8 * kStatsBlock - 1) / (8 * kStatsBlock)));
@@ -1525,6 +1525,44 @@ static void stage_resident(DeviceState *d, const og_graph *g, uint64_t vsplit, u
     OG_HIP(hipStreamSynchronize(d->s_compute));
 }
 
+// Link format of the dynamic region (DeviceState::lbits): packs the host
+// layout's words `src` into a pinned stream of lbits-bit words, when they are
+// narrow enough.  Edge targets need the bits of V - 1, weighted words wbits
+// more; with V of a few million a quarter to a third of the bytes go (ER 3 M
+// x 32, 22 bits: PageRank 66 -> 46 ms, CC 7.9 -> 6.6 ms; preparing the
+// packed copy takes 12 ms more).
+static void pack_link(DeviceState *d, const og_graph *g, const uint32_t *src, uint64_t n) {
+    const uint32_t bits = std::max(bits_of(g->V - 1), 1u) + (d->packed ? d->wbits : 0);
+    if (bits > kLinkBitsMax || !n) return;
+    const uint64_t words = (n * bits + 31) / 32 + 2;
+    uint32_t *dst = (uint32_t *)d->palloc(words * 4);
+    dst[words - 1] = dst[words - 2] = 0;
+    // groups of 32 edges fill `bits` whole words
+    parallel_for((n + 31) / 32, 1 << 15, 0, [&](uint64_t b, uint64_t e, unsigned) {
+        for (uint64_t k = b; k < e; ++k) {
+            const uint64_t i1 = std::min(n, 32 * (k + 1));
+            uint32_t *out = dst + k * bits;
+            uint64_t acc = 0;
+            uint32_t have = 0;
+            for (uint64_t i = 32 * k; i < i1; ++i) {
+                acc |= (uint64_t)src[i] << have;
+                have += bits;
+                if (have >= 32) {
+                    *out++ = (uint32_t)acc;
+                    acc >>= 32;
+                    have -= 32;
+                }
+            }
+            if (have) *out = (uint32_t)acc;
+        }
+    });
+    void *hd = nullptr;
+    OG_HIP(hipHostGetDevicePointer(&hd, dst, 0));
+    d->lbits = bits;
+    d->h_link = dst;
+    d->hd_link = hd;
+}
+
 // The compaction's degree table (DeviceState::d_deg): 4 bytes per vertex
 // and range in place of two 8-byte row bounds.  Not built when a degree
 // exceeds 32 bits (the passes then read the row bounds).
@@ -1745,6 +1783,9 @@ static void prepare_impl(og_graph *g, og_approach approach, const og_plan_params
                 // resident in HBM instead.
                 stage_resident(d.get(), g, pl.vsplit, pl.staging_edges, lpos);
             }
+            // (a weighted graph that is not packed keeps its 8-byte edges)
+            if ((zc || g->kind == OG_KIND_PULL) && (g->kind != OG_KIND_WEIGHTED || d->packed))
+                pack_link(d.get(), g, (const uint32_t *)d->h_dyn, nd);
         }
     }
 
@@ -2006,7 +2047,7 @@ static void launch_dyn(DeviceState *d, unsigned grid, const void *src, uint64_t 
                        d->fr.info, d->fr.doff, src, c0, c1, d->d_ptr, d->dyn_base, (const void *)d->d_staging,
                        DIRECT ? (const int64_t *)d->d_rdelta : nullptr, d->wbits, relax_args(d),
                        DIRECT ? (const uint64_t *)d->d_lpos : nullptr, d->split_nl, d->plan.vsplit,
-                       DIRECT && c0 == 0 ? (const uint32_t *)d->fr.dchunk : nullptr, d->fr.counters + 1,
+                       DIRECT && c0 == 0 ? (const uint32_t *)d->fr.dchunk : nullptr, DIRECT ? d->lbits : 0u, d->fr.counters + 1,
                        d->fr.counters + 5);
 }
 
@@ -2034,7 +2075,8 @@ static void launch_round_fmt(DeviceState *d, bool with_dyn) {
     r.tile = d->tune.tile;
     r.cd = with_dyn ? (dyn + kHubGridCap - 1) / kHubGridCap : 0;
     r.doff = d->fr.doff;
-    r.stage = d->hd_dyn;
+    r.stage = d->lbits ? d->hd_link : d->hd_dyn;
+    r.lbits = d->lbits;
     r.dbase = d->dyn_base;
     r.resident = d->d_staging;
     r.rdelta = d->d_rdelta;
@@ -2242,7 +2284,7 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
                     span(kClsStat, s, [&] { launch_round_relax<ALGO, W>(d, false); });
                 } else if (overlap) {
                     OG_HIP(hipEventRecord(d->ev_fork, s));
-                    span(kClsDyn, s, [&] { launch_dyn_any<ALGO, W>(d, d->hd_dyn, 0, ~0ull, 0, true); });
+                    span(kClsDyn, s, [&] { launch_dyn_any<ALGO, W>(d, d->lbits ? d->hd_link : d->hd_dyn, 0, ~0ull, 0, true); });
                     OG_HIP(hipStreamWaitEvent(d->s_static, d->ev_fork, 0));
                     span(kClsStat, d->s_static,
                          [&] { launch_static_relax<ALGO, W>(d, d->fr, nullptr, relax_args(d), d->s_static); });
@@ -2250,7 +2292,7 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
                     joined = true;
                 } else {
                     joined = launch_static<ALGO, W>(d, nullptr, span);
-                    if (has_dyn) span(kClsDyn, s, [&] { launch_dyn_any<ALGO, W>(d, d->hd_dyn, 0, ~0ull, 0, true); });
+                    if (has_dyn) span(kClsDyn, s, [&] { launch_dyn_any<ALGO, W>(d, d->lbits ? d->hd_link : d->hd_dyn, 0, ~0ull, 0, true); });
                 }
                 if (dir_opt)
                     span(kClsStat, s, [&] {
@@ -2359,8 +2401,8 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
     st.relax_static_bytes += 24ull * c.static_node_sum + per_edge * c.static_work_edges;
     st.relax_dynamic_bytes += 24ull * c.dyn_node_sum + per_edge * dyn_edges;
     st.frontier_bytes += 2ull * d->Vpad * c.compactions + 4ull * c.node_sum;
-    if (has_dyn && zero_copy) {  // every active dynamic edge read in place (HBM-resident ones subtracted later)
-        st.h2d_bytes += dyn_edges * d->deb;
+    if (has_dyn && zero_copy) {  // every active dynamic edge read in place (HBM-resident ones taken off later)
+        st.h2d_bytes += dyn_edges;
         st.chunks += c.dyn_rounds;
     }
 }
@@ -2369,14 +2411,17 @@ static void finish_stats(og_run_stats &st, RunTimers &tm, double gather_ms, doub
                          uint64_t upd_bytes) {
     const RunBlock &h = *d->fr.h_blk;
     const unsigned long long *ctr = h.counters;
-    const uint64_t link_eb = d->deb;
     if (tm.clocked >= 0) {
         tm.at(tm.clocked).ms += (double)(int64_t)h.clk.acc[kClkRelax] / d->clock_khz;
         tm.front.ms += (double)(int64_t)h.clk.acc[kClkFront] / d->clock_khz;
     }
     st.updates = ctr[0] + ctr[1];
-    // dynamic edges served from the HBM-resident head did not cross the link
-    st.h2d_bytes -= std::min<uint64_t>(st.h2d_bytes, ctr[5] * link_eb);
+    // zero-copy: h2d_bytes counts edges so far; those served from the
+    // HBM-resident blocks did not cross the link
+    if (d->flags & OG_PLAN_ZERO_COPY) {
+        const uint64_t crossed = st.h2d_bytes - std::min<uint64_t>(st.h2d_bytes, ctr[5]);
+        st.h2d_bytes = d->lbits ? (crossed * d->lbits + 7) / 8 : crossed * d->deb;
+    }
     st.relax_static_bytes += upd_bytes * ctr[0];
     st.relax_dynamic_bytes += upd_bytes * ctr[1];
     st.frontier_kernel_ms = sum_ms(tm.front);

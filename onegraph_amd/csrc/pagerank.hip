@@ -14,15 +14,23 @@
 //
 // Every vertex is active each iteration, so the dynamic region is the
 // contiguous in-edge range [ptr[vsplit], E): it is copied chunk by chunk
-// straight from the pinned host CSR (no gather) on the copy stream while the
-// previous chunk is being summed.
+// straight from pinned host memory (no gather) on two copy streams while
+// earlier chunks are being summed.
 #include <algorithm>
 
 #include "device.h"
 
 namespace og {
 
-constexpr int kPrLpv0 = 8;  // lanes per vertex for the low-degree bin
+constexpr int kPrLpv0 = 4;   // lanes per vertex for rows up to t1
+constexpr int kPrRangeLpv = 8;  // the same in the dynamic region, whose rows come in every length
+constexpr int kPrBatch = 8;  // in-edges per lane whose reads are in flight together
+
+// A static row: its in-edges and its vertex, one 16-byte load.
+struct PrRow {
+    uint64_t b;
+    uint32_t n, v;  // n = 0xFFFFFFFF: longer, read the row bounds
+};
 
 template <typename T>
 struct Acc {  // running sum with Kahan compensation: value = s - c
@@ -71,134 +79,221 @@ __device__ __forceinline__ double block_sum_f64(double x, double *lds) {
     return t;
 }
 
-// contrib[v] = rank[v] / outdeg[v]; per-block FP64 partials of the dangling mass.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_pr_contrib(const T *__restrict__ rank, const uint32_t *__restrict__ outdeg,
-                                                       T *__restrict__ contrib, uint64_t V, double *partial) {
-    __shared__ double lds[kBlock / kWave];
-    double dang = 0;
-    for (uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x; v < V; v += (uint64_t)gridDim.x * kBlock) {
-        const T r = rank[v];
-        const uint32_t od = outdeg[v];
-        contrib[v] = od ? r / (T)od : (T)0;
-        if (!od) dang += (double)r;
+// Sum of the contributions of a row's in-edges sub, sub + L, sub + 2 L, ...
+// (L lanes per row), kPrBatch edge reads and then their contributions in
+// flight: one at a time a lane waited two memory latencies per edge.
+// edge(i): the row's in-neighbour i.
+template <typename T, class Edge>
+__device__ __forceinline__ void pull_row(Acc<T> &a, Edge edge, uint64_t n, uint32_t sub, uint32_t L,
+                                         const T *__restrict__ contrib) {
+    for (uint64_t i = sub; i < n; i += (uint64_t)kPrBatch * L) {
+        uint32_t u[kPrBatch];
+        T x[kPrBatch];
+#pragma unroll
+        for (int k = 0; k < kPrBatch; ++k) u[k] = i + (uint64_t)k * L < n ? edge(i + (uint64_t)k * L) : 0u;
+#pragma unroll
+        for (int k = 0; k < kPrBatch; ++k) x[k] = i + (uint64_t)k * L < n ? contrib[u[k]] : (T)0;
+#pragma unroll
+        for (int k = 0; k < kPrBatch; ++k)
+            if (i + (uint64_t)k * L < n) a.add(x[k]);
     }
+}
+
+// The iteration's inputs and outputs.
+template <typename T>
+struct PrArgs {
+    const uint64_t *ptr;
+    const uint32_t *edges;      // static region
+    const T *contrib;           // rank / out-degree before the iteration
+    T *next;                    // and after it
+    T *rank;                    // updated in place: a row reads and writes its own vertex only
+    const uint32_t *outdeg;
+    PrState *st;
+    double damping, inv_n;
+    double *partial;            // two per workgroup of the iteration: residual, dangling mass
+};
+
+// New rank of v: stored with its contribution to the next iteration; adds
+// the residual and the dangling mass.
+template <typename T>
+__device__ __forceinline__ void pr_apply(const PrArgs<T> &p, uint32_t v, T sum, T base, double &res, double &dang) {
+    const T nv = base + (T)p.damping * sum;
+    const uint32_t od = p.outdeg[v];
+    res += fabs((double)nv - (double)p.rank[v]);
+    p.rank[v] = nv;
+    p.next[v] = od ? nv / (T)od : (T)0;
+    if (!od) dang += (double)nv;
+}
+
+// (1-d)/n + d * dangling / n, formed in FP64 then rounded once.
+template <typename T>
+__device__ __forceinline__ T pr_base(const PrArgs<T> &p) {
+    return (T)((1.0 - p.damping) * p.inv_n + p.damping * p.st->dangling * p.inv_n);
+}
+
+// A workgroup's partials, at slot i; device-scope stores, so that the
+// workgroup that finishes the iteration can read them in the same launch.
+__device__ __forceinline__ void pr_partial(double *partial, uint64_t i, double res, double dang, double *lds) {
+    res = block_sum_f64(res, lds);
     dang = block_sum_f64(dang, lds);
-    if (threadIdx.x == 0) partial[blockIdx.x] = dang;
-}
-
-// Sums n partials in a fixed order into *out.
-__global__ __launch_bounds__(1024) void k_reduce_partials(const double *partial, uint32_t n, double *out) {
-    __shared__ double lds[1024 / kWave];
-    double s = 0;
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) s += partial[i];
-    s = block_sum_f64(s, lds);
-    if (threadIdx.x == 0) *out = s;
-}
-
-template <typename T>
-__device__ __forceinline__ T pr_apply(T sum, const double *scal, double damping, double inv_n) {
-    // base = (1-d)/n + d * dangling / n, formed in FP64 then rounded once.
-    const double base = (1.0 - damping) * inv_n + damping * scal[0] * inv_n;
-    return (T)base + (T)damping * sum;
-}
-
-// Pull over a list of static vertices with LPV lanes each.  Residual
-// partials go to partial[blockIdx.x + poff].
-template <typename T, int LPV>
-__global__ __launch_bounds__(kBlock) void k_pr_pull_list(const uint32_t *__restrict__ list, uint32_t n,
-                                                         const uint64_t *__restrict__ ptr,
-                                                         const uint32_t *__restrict__ edges, uint64_t edge_base,
-                                                         const T *__restrict__ contrib, const T *__restrict__ rank,
-                                                         T *__restrict__ next, const double *scal, double damping,
-                                                         double inv_n, double *partial) {
-    __shared__ double lds[kBlock / kWave];
-    const uint64_t gid = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    const uint64_t item = gid / LPV;
-    const uint32_t sub = (uint32_t)(gid % LPV);
-    Acc<T> a;
-    uint32_t v = 0;
-    if (item < n) {
-        v = list[item];
-        const uint64_t b = ptr[v], e = ptr[v + 1];
-        for (uint64_t i = b + sub; i < e; i += LPV) a.add(contrib[edges[i - edge_base]]);
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(partial + 2 * i, res, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(partial + 2 * i + 1, dang, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    group_merge<T, LPV>(a);
-    double res = 0;
-    if (item < n && sub == 0) {
-        const T nv = pr_apply<T>(a.value(), scal, damping, inv_n);
-        res = fabs((double)nv - (double)rank[v]);
-        next[v] = nv;
+}
+
+// Sums n workgroups' partials in a fixed order and closes the iteration.
+// progress (pinned host memory): iterations so far << 1 | done.
+__device__ __forceinline__ void pr_finish(const double *partial, uint32_t n, PrState *st, unsigned long long *progress,
+                                          double *lds) {
+    double res = 0, dang = 0;
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
+        res += __hip_atomic_load(partial + 2 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        dang += __hip_atomic_load(partial + 2 * i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     res = block_sum_f64(res, lds);
-    if (threadIdx.x == 0) partial[blockIdx.x] = res;
+    dang = block_sum_f64(dang, lds);
+    if (threadIdx.x == 0) {
+        const uint32_t it = st->iterations + 1, done = res < st->tolerance ? 1u : 0u;
+        st->dangling = dang;
+        st->l1 = res;
+        st->iterations = it;
+        st->done = done;
+        __hip_atomic_store(progress, (unsigned long long)it << 1 | done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
-// Pull for one hub vertex per workgroup (deterministic block reduction).
+__global__ __launch_bounds__(1024) void k_pr_finish(const double *partial, uint32_t n, PrState *st,
+                                                    unsigned long long *progress) {
+    __shared__ double lds[1024 / kWave];
+    if (st->done) return;
+    pr_finish(partial, n, st, progress, lds);
+}
+
+// Start: uniform ranks and their contributions; the last workgroup sums the
+// dangling mass.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_pr_pull_hub(const uint32_t *__restrict__ list,
-                                                        const uint64_t *__restrict__ ptr,
-                                                        const uint32_t *__restrict__ edges, uint64_t edge_base,
-                                                        const T *__restrict__ contrib, const T *__restrict__ rank,
-                                                        T *__restrict__ next, const double *scal, double damping,
-                                                        double inv_n, double *partial) {
-    __shared__ T s_s[kBlock / kWave], s_c[kBlock / kWave];
-    const uint32_t v = list[blockIdx.x];
-    const uint64_t b = ptr[v], e = ptr[v + 1];
-    Acc<T> a;
-    for (uint64_t i = b + threadIdx.x; i < e; i += kBlock) a.add(contrib[edges[i - edge_base]]);
-    group_merge<T, kWave>(a);
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-    if (lane == 0) {
-        s_s[wid] = a.s;
-        s_c[wid] = a.c;
+__global__ __launch_bounds__(kBlock) void k_pr_init(PrArgs<T> p, uint64_t V, double tolerance, CompactTotals ct) {
+    __shared__ double lds[kBlock / kWave];
+    __shared__ uint32_t s_last;
+    const T r = (T)p.inv_n;
+    double dang = 0;
+    for (uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x; v < V; v += (uint64_t)gridDim.x * kBlock) {
+        const uint32_t od = p.outdeg[v];
+        p.rank[v] = r;
+        p.next[v] = od ? r / (T)od : (T)0;
+        if (!od) dang += (double)r;
+    }
+    pr_partial(p.partial, blockIdx.x, 0.0, dang, lds);
+    if (threadIdx.x == 0) {
+        wait_vmem();
+        s_last = arrive_last(ct) ? 1u : 0u;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        Acc<T> t;
-        t.s = s_s[0];
-        t.c = s_c[0];
-        for (int w = 1; w < kBlock / kWave; ++w) t.merge(s_s[w], s_c[w]);
-        const T nv = pr_apply<T>(t.value(), scal, damping, inv_n);
-        partial[blockIdx.x] = fabs((double)nv - (double)rank[v]);
-        next[v] = nv;
+    if (!s_last) return;
+    double d = 0;
+    for (uint32_t i = threadIdx.x; i < gridDim.x; i += kBlock)
+        d += __hip_atomic_load(p.partial + 2 * i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    d = block_sum_f64(d, lds);
+    if (threadIdx.x == 0) *p.st = PrState{d, 0.0, tolerance, 0u, 0u};
+}
+
+// Pull over the static region in one launch: workgroups [0, nh) take a hub
+// row each (first, as they run longest), the next g1 stride over the wave
+// rows (t1 < in-degree <= t2), the rest over the short rows, kPrLpv0 lanes
+// each.  With `progress` the workgroup that arrives last also closes the
+// iteration, so that an iteration of a graph wholly in HBM is one launch
+// (300 K vertices, 4.5 M edges, FP64: contribution pass, three pulls, two
+// reductions, a copy and a host round trip took 122 us).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_pr_pull(PrArgs<T> p, const PrRow *__restrict__ rows, uint32_t n0, uint32_t n1,
+                                                    uint32_t nh, uint32_t g1, CompactTotals ct,
+                                                    unsigned long long *progress) {
+    __shared__ double lds[kBlock / kWave];
+    __shared__ T s_s[kBlock / kWave], s_c[kBlock / kWave];
+    __shared__ uint32_t s_last;
+    if (p.st->done) return;
+    const T base = pr_base(p);
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    double res = 0, dang = 0;
+    auto row_at = [&](uint32_t i, uint64_t &n) {
+        const PrRow r = rows[i];
+        n = r.n != 0xFFFFFFFFu ? r.n : p.ptr[r.v + 1] - r.b;
+        return r;
+    };
+    if (blockIdx.x < nh) {
+        uint64_t n;
+        const PrRow r = row_at(n0 + n1 + blockIdx.x, n);
+        Acc<T> a;
+        pull_row(a, [e = p.edges + r.b](uint64_t i) { return e[i]; }, n, threadIdx.x, kBlock, p.contrib);
+        group_merge<T, kWave>(a);
+        if (lane == 0) {
+            s_s[wid] = a.s;
+            s_c[wid] = a.c;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            Acc<T> t;
+            t.s = s_s[0];
+            t.c = s_c[0];
+            for (int w = 1; w < kBlock / kWave; ++w) t.merge(s_s[w], s_c[w]);
+            pr_apply<T>(p, r.v, t.value(), base, res, dang);
+        }
+    } else if (blockIdx.x < nh + g1) {
+        for (uint32_t i = (blockIdx.x - nh) * (kBlock / kWave) + wid; i < n1; i += g1 * (kBlock / kWave)) {
+            uint64_t n;
+            const PrRow r = row_at(n0 + i, n);
+            Acc<T> a;
+            pull_row(a, [e = p.edges + r.b](uint64_t i) { return e[i]; }, n, lane, kWave, p.contrib);
+            group_merge<T, kWave>(a);
+            if (lane == 0) pr_apply<T>(p, r.v, a.value(), base, res, dang);
+        }
+    } else {
+        const uint32_t g0 = gridDim.x - nh - g1;
+        const uint32_t sub = threadIdx.x % kPrLpv0;
+        for (uint64_t i = ((uint64_t)(blockIdx.x - nh - g1) * kBlock + threadIdx.x) / kPrLpv0; i < n0;
+             i += (uint64_t)g0 * (kBlock / kPrLpv0)) {
+            uint64_t n;
+            const PrRow r = row_at((uint32_t)i, n);
+            Acc<T> a;
+            pull_row(a, [e = p.edges + r.b](uint64_t i) { return e[i]; }, n, sub, kPrLpv0, p.contrib);
+            group_merge<T, kPrLpv0>(a);
+            if (sub == 0) pr_apply<T>(p, r.v, a.value(), base, res, dang);
+        }
     }
+    pr_partial(p.partial, blockIdx.x, res, dang, lds);
+    if (!progress) return;
+    if (threadIdx.x == 0) {
+        wait_vmem();
+        s_last = arrive_last(ct) ? 1u : 0u;
+    }
+    __syncthreads();
+    if (s_last) pr_finish(p.partial, gridDim.x, p.st, progress, lds);
 }
 
 // Pull for the contiguous vertex range [va, vb) whose in-edges sit in `stage`
-// starting at edge ptr[va].
-template <typename T, int LPV>
-__global__ __launch_bounds__(kBlock) void k_pr_pull_range(uint32_t va, uint32_t vb, const uint64_t *__restrict__ ptr,
-                                                          const uint32_t *__restrict__ stage,
-                                                          const T *__restrict__ contrib, const T *__restrict__ rank,
-                                                          T *__restrict__ next, const double *scal, double damping,
-                                                          double inv_n, double *partial) {
-    __shared__ double lds[kBlock / kWave];
-    const uint64_t gid = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    const uint64_t item = gid / LPV;
-    const uint32_t sub = (uint32_t)(gid % LPV);
-    const uint64_t base = ptr[va];
-    Acc<T> a;
-    const uint64_t v = va + item;
-    if (v < vb) {
-        const uint64_t b = ptr[v] - base, e = ptr[v + 1] - base;
-        for (uint64_t i = b + sub; i < e; i += LPV) a.add(contrib[stage[i]]);
-    }
-    group_merge<T, LPV>(a);
-    double res = 0;
-    if (v < vb && sub == 0) {
-        const T nv = pr_apply<T>(a.value(), scal, damping, inv_n);
-        res = fabs((double)nv - (double)rank[v]);
-        next[v] = nv;
-    }
-    res = block_sum_f64(res, lds);
-    if (threadIdx.x == 0) partial[blockIdx.x] = res;
-}
-
+// starting at edge ptr[va]: whole ids, or with lbits a stream of lbits-bit
+// ones whose first starts `first` bits in; partials from slot poff on.
 template <typename T>
-__global__ void k_fill_t(T *a, uint64_t n, T v) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        a[i] = v;
+__global__ __launch_bounds__(kBlock) void k_pr_pull_range(PrArgs<T> p, uint32_t va, uint32_t vb,
+                                                          const uint32_t *__restrict__ stage, uint32_t lbits,
+                                                          uint32_t first, uint64_t poff) {
+    __shared__ double lds[kBlock / kWave];
+    const uint32_t sub = threadIdx.x % kPrRangeLpv;
+    const uint64_t e0 = p.ptr[va];
+    const uint64_t v = va + ((uint64_t)blockIdx.x * kBlock + threadIdx.x) / kPrRangeLpv;
+    double res = 0, dang = 0;
+    if (v < vb) {  // the lanes of a row go together
+        const uint64_t b = p.ptr[v] - e0, n = p.ptr[v + 1] - e0 - b;
+        Acc<T> a;
+        if (lbits)
+            pull_row(a, [=](uint64_t i) { return link_word(stage, b + i, lbits, first); }, n, sub, kPrRangeLpv, p.contrib);
+        else
+            pull_row(a, [=](uint64_t i) { return stage[b + i]; }, n, sub, kPrRangeLpv, p.contrib);
+        group_merge<T, kPrRangeLpv>(a);
+        if (sub == 0) pr_apply<T>(p, (uint32_t)v, a.value(), pr_base(p), res, dang);
+    }
+    pr_partial(p.partial, poff + blockIdx.x, res, dang, lds);
 }
 
 // --------------------------------------------------------------- host
@@ -206,15 +301,44 @@ __global__ void k_fill_t(T *a, uint64_t n, T v) {
 namespace {
 
 struct PrPlan {
-    std::vector<uint32_t> bin0, bin1, hub;            // static vertices by in-degree
-    std::vector<std::pair<uint32_t, uint32_t>> chunks;  // dynamic vertex ranges
-    uint32_t *d_bins = nullptr;
-    uint64_t partial_cap = 0;
+    uint32_t n0 = 0, n1 = 0, nh = 0;  // static rows: up to t1, up to t2, hubs
+    unsigned g0 = 0, g1 = 0;          // workgroups of the first two
+    // The dynamic region crosses the link in chunks of whole rows through a
+    // ring of `ring` slots of `slot` words, all in the staging share.
+    struct Chunk {
+        uint32_t va, vb;
+        uint64_t word, words;  // of the host source
+        uint32_t first;        // bits before the first edge
+    };
+    std::vector<Chunk> chunks;
+    uint32_t ring = 0;
+    uint32_t lbits = 0;  // bits per edge on the link, 0: whole ids
+    uint64_t slot = 0;
+    const uint32_t *src = nullptr;
+    std::vector<hipEvent_t> ev_h2d, ev_pull;  // copy into / pull out of the slot finished
+    ~PrPlan() {
+        for (hipEvent_t e : ev_h2d) (void)hipEventDestroy(e);
+        for (hipEvent_t e : ev_pull) (void)hipEventDestroy(e);
+    }
+    PrRow *d_rows = nullptr;
+    uint64_t blocks = 0;              // workgroups of an iteration
+    unsigned static_grid() const { return nh + g1 + g0; }
 };
 
 unsigned grid_of(uint64_t threads) {
     return (unsigned)std::max<uint64_t>(1, (threads + kBlock - 1) / kBlock);
 }
+
+// Workgroups of the short and the wave rows at most: enough to fill the chip
+// (eight of 256 lanes per CU), few enough that the last one sums their
+// partials quickly.
+constexpr unsigned kPrGridCap = 2048;
+
+// Slots of the chunk ring: small enough that a few are on their way while
+// others are pulled, large enough that a copy takes longer than its hand-over
+// (4 MiB: 73 us on the link).
+constexpr uint64_t kPrSlotBytes = 4ull << 20;
+constexpr uint32_t kPrRing = 8;
 
 }  // namespace
 
@@ -223,44 +347,59 @@ static PrPlan &pr_plan(DeviceState *d, const og_graph *g) {
     if (d->pr_plan) return *(PrPlan *)d->pr_plan.get();
     std::shared_ptr<PrPlan> p = std::make_shared<PrPlan>();
     const uint64_t vs = d->plan.vsplit;
+    auto bin = [&](uint64_t deg) { return deg <= d->tune.t1 ? 0 : deg <= d->tune.t2 ? 1 : 2; };
+    uint64_t cnt[3] = {0, 0, 0};
+    for (uint64_t v = 0; v < vs; ++v) cnt[bin(g->ptr[v + 1] - g->ptr[v])]++;
+    std::vector<PrRow> rows(vs);
+    uint64_t at[3] = {0, cnt[0], cnt[0] + cnt[1]};
     for (uint64_t v = 0; v < vs; ++v) {
-        const uint64_t deg = g->ptr[v + 1] - g->ptr[v];
-        if (deg <= d->tune.t1) p->bin0.push_back((uint32_t)v);
-        else if (deg <= d->tune.t2) p->bin1.push_back((uint32_t)v);
-        else p->hub.push_back((uint32_t)v);
+        const uint64_t n = g->ptr[v + 1] - g->ptr[v];
+        rows[at[bin(n)]++] = PrRow{g->ptr[v], (uint32_t)std::min<uint64_t>(n, 0xFFFFFFFFull), (uint32_t)v};
+    }
+    p->n0 = (uint32_t)cnt[0];
+    p->n1 = (uint32_t)cnt[1];
+    p->nh = (uint32_t)cnt[2];
+    if (vs) {
+        p->g0 = p->n0 ? std::min(kPrGridCap, grid_of((uint64_t)p->n0 * kPrLpv0)) : 0;
+        p->g1 = p->n1 ? std::min(kPrGridCap, grid_of((uint64_t)p->n1 * kWave)) : 0;
+        p->d_rows = (PrRow *)d->dalloc(vs * sizeof(PrRow));
+        OG_HIP(hipMemcpy(p->d_rows, rows.data(), vs * sizeof(PrRow), hipMemcpyHostToDevice));
     }
     if (vs < d->V) {
-        const uint64_t C = d->slot_edges;
-        uint64_t va = vs;
-        while (va < d->V) {
-            uint64_t vb = va;
-            // greedy: extend while the range fits in one slot
+        uint64_t maxrow = 0;
+        for (uint64_t v = vs; v < d->V; ++v) maxrow = std::max(maxrow, g->ptr[v + 1] - g->ptr[v]);
+        if (maxrow > d->slot_edges)
+            raise(OG_EBUDGET, "a vertex has %llu in-edges, more than a staging slot (%llu)", (unsigned long long)maxrow,
+                  (unsigned long long)d->slot_edges);
+        const uint64_t total = (uint64_t)d->nslots * d->slot_edges;  // 4-byte words of the staging share
+        // the link format's rows start anywhere in a word and are read eight
+        // bytes at a time, so it takes slots of a few words more
+        p->lbits = d->lbits && (maxrow * d->lbits + 31) / 32 + 2 <= total / 2 ? d->lbits : 0;
+        const uint32_t bits = p->lbits ? p->lbits : 32;
+        auto words_of = [&](uint64_t n) { return (n * bits + 31) / 32 + (p->lbits ? 2 : 0); };
+        p->ring = (uint32_t)std::min<uint64_t>(kPrRing, std::max<uint64_t>(2, total * 4 / kPrSlotBytes));
+        while (p->ring > 2 && total / p->ring < words_of(maxrow)) --p->ring;
+        p->slot = total / p->ring;
+        p->src = p->lbits ? d->h_link : g->cols + d->dyn_base;
+        const uint64_t base = d->dyn_base;
+        for (uint64_t va = vs; va < d->V;) {
             uint64_t lo = va + 1, hi = d->V;
-            if (g->ptr[va + 1] - g->ptr[va] > C)
-                raise(OG_EBUDGET, "vertex %llu has %llu in-edges, more than a staging slot (%llu)",
-                      (unsigned long long)va, (unsigned long long)(g->ptr[va + 1] - g->ptr[va]),
-                      (unsigned long long)C);
-            while (lo < hi) {  // largest vb with ptr[vb] - ptr[va] <= C
-                uint64_t mid = (lo + hi + 1) / 2;
-                if (g->ptr[mid] - g->ptr[va] <= C) lo = mid; else hi = mid - 1;
+            while (lo < hi) {  // largest vb whose rows fit
+                const uint64_t mid = (lo + hi + 1) / 2;
+                if (words_of(g->ptr[mid] - g->ptr[va]) <= p->slot) lo = mid; else hi = mid - 1;
             }
-            vb = lo;
-            p->chunks.push_back({(uint32_t)va, (uint32_t)vb});
-            va = vb;
+            const uint64_t b0 = (g->ptr[va] - base) * bits, b1 = (g->ptr[lo] - base) * bits;
+            const uint64_t w0 = b0 / 32, w1 = (b1 + 31) / 32 + (p->lbits && b1 > b0 ? 1 : 0);
+            p->chunks.push_back({(uint32_t)va, (uint32_t)lo, w0, b1 > b0 ? w1 - w0 : 0, (uint32_t)(b0 % 32)});
+            va = lo;
         }
+        p->ev_h2d.assign(p->ring, nullptr);
+        p->ev_pull.assign(p->ring, nullptr);
+        for (auto &e : p->ev_h2d) OG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        for (auto &e : p->ev_pull) OG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
-    const uint64_t nb = p->bin0.size() + p->bin1.size() + p->hub.size();
-    p->d_bins = (uint32_t *)d->dalloc(std::max<uint64_t>(nb, 1) * 4);
-    std::vector<uint32_t> all;
-    all.reserve(nb);
-    all.insert(all.end(), p->bin0.begin(), p->bin0.end());
-    all.insert(all.end(), p->bin1.begin(), p->bin1.end());
-    all.insert(all.end(), p->hub.begin(), p->hub.end());
-    if (nb) OG_HIP(hipMemcpy(p->d_bins, all.data(), nb * 4, hipMemcpyHostToDevice));
-    // partial slots: one per block of every launch in an iteration
-    uint64_t cap = grid_of(p->bin0.size() * (uint64_t)kPrLpv0) + grid_of(p->bin1.size() * 64ull) + p->hub.size();
-    for (auto &c : p->chunks) cap += grid_of((uint64_t)(c.second - c.first) * kPrLpv0);
-    p->partial_cap = std::max<uint64_t>(cap, grid_of(d->V));
+    p->blocks = p->static_grid();
+    for (auto &c : p->chunks) p->blocks += grid_of((uint64_t)(c.vb - c.va) * kPrRangeLpv);
     d->pr_plan = p;
     return *p;
 }
@@ -271,137 +410,156 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
     const uint64_t V = d->V;
     PrPlan &pp = pr_plan(d, g);
     hipStream_t s = d->s_compute;
-    const bool f64 = sizeof(T) == 8;
+    const unsigned igrid = (unsigned)std::min<uint64_t>(1024, grid_of(V));
+    const uint64_t cap = std::max<uint64_t>(pp.blocks, igrid);
     if (!d->d_outdeg) {
         d->d_outdeg = (uint32_t *)d->dalloc(V * 4);
         OG_HIP(hipMemcpy(d->d_outdeg, g->out_degree, V * 4, hipMemcpyHostToDevice));
-        d->d_scalars = (double *)d->dalloc(4 * sizeof(double));
-        d->h_scalars = (double *)d->palloc(4 * sizeof(double));
-    }
-    if (pp.partial_cap > d->pr_partial_cap) {
-        d->d_partial = (double *)d->dalloc(pp.partial_cap * sizeof(double));
-        d->pr_partial_cap = pp.partial_cap;
-    }
-    if (!d->d_rank[0] || d->pr_fp64 != f64) {
+        d->d_prstate = (PrState *)d->dalloc(sizeof(PrState));
+        d->h_prstate = (PrState *)d->palloc(sizeof(PrState));
+        d->h_progress = (unsigned long long *)d->palloc(sizeof(unsigned long long));
         // sized for double so either precision fits
-        if (!d->d_rank[0]) {
-            d->d_rank[0] = d->dalloc(V * 8);
-            d->d_rank[1] = d->dalloc(V * 8);
-            d->d_contrib = d->dalloc(V * 8);
-        }
-        d->pr_fp64 = f64;
+        d->d_rank = d->dalloc(V * 8);
+        for (auto &c : d->d_contrib) c = d->dalloc(V * 8);
     }
-    T *rank = (T *)d->d_rank[0], *next = (T *)d->d_rank[1], *contrib = (T *)d->d_contrib;
-    const double inv_n = 1.0 / (double)V, damping = prm.damping;
-    const uint32_t *edges = (const uint32_t *)d->d_static;
-    TimedClass tc_contrib, tc_static, tc_dyn, tc_copy;
+    if (cap > d->pr_partial_cap) {
+        d->d_partial = (double *)d->dalloc(cap * 2 * sizeof(double));
+        d->d_prtot = (unsigned long long *)d->dalloc(totals_words(cap) * 8);
+        OG_HIP(hipMemset(d->d_prtot, 0, totals_words(cap) * 8));
+        d->pr_partial_cap = cap;
+    }
+    T *contrib[2] = {(T *)d->d_contrib[0], (T *)d->d_contrib[1]};
+    PrArgs<T> a{d->d_ptr, (const uint32_t *)d->d_static, nullptr, contrib[0], (T *)d->d_rank, d->d_outdeg, d->d_prstate,
+                prm.damping, 1.0 / (double)V, d->d_partial};
+    TimedClass tc_init, tc_static, tc_dyn, tc_copy;
     d->events.reset();
     og_pr_stats st{};
     st.run.approach = (uint32_t)d->approach;
 
     OG_HIP(hipStreamSynchronize(d->s_copy));
+    OG_HIP(hipStreamSynchronize(d->s_static));
     OG_HIP(hipStreamSynchronize(s));
     Stopwatch total;
-    hipLaunchKernelGGL(k_fill_t<T>, dim3(2048), dim3(256), 0, s, rank, V, (T)(1.0 / (double)V));
-    OG_HIP(hipGetLastError());
-    const unsigned cgrid = (unsigned)std::min<uint64_t>(2048, grid_of(V));
-    const uint32_t n0 = (uint32_t)pp.bin0.size(), n1 = (uint32_t)pp.bin1.size(), nh = (uint32_t)pp.hub.size();
-    const uint64_t eb = 4, C = d->slot_edges;
-    double l1 = 0;
-    uint32_t it = 0;
-    const uint64_t vb_bytes = f64 ? 8 : 4;
-    while (it < prm.max_iterations) {
-        {
-            EventSpan span(d, &tc_contrib, s);
-            hipLaunchKernelGGL(k_pr_contrib<T>, dim3(cgrid), dim3(kBlock), 0, s, rank, d->d_outdeg, contrib, V,
-                               d->d_partial);
-            hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, s, d->d_partial, cgrid, d->d_scalars + 0);
-            OG_HIP(hipGetLastError());
-        }
-        st.run.frontier_bytes += V * (4 + 2 * vb_bytes);
-        uint64_t poff = 0;
-        {
-            if (n0 | n1 | nh) {
-                EventSpan span(d, &tc_static, s);
-                if (n0) {
-                    const unsigned gr = grid_of((uint64_t)n0 * kPrLpv0);
-                    hipLaunchKernelGGL((k_pr_pull_list<T, kPrLpv0>), dim3(gr), dim3(kBlock), 0, s, pp.d_bins, n0,
-                                       d->d_ptr, edges, 0ull, contrib, rank, next, d->d_scalars, damping, inv_n,
-                                       d->d_partial + poff);
-                    poff += gr;
-                }
-                if (n1) {
-                    const unsigned gr = grid_of((uint64_t)n1 * 64);
-                    hipLaunchKernelGGL((k_pr_pull_list<T, 64>), dim3(gr), dim3(kBlock), 0, s, pp.d_bins + n0, n1,
-                                       d->d_ptr, edges, 0ull, contrib, rank, next, d->d_scalars, damping, inv_n,
-                                       d->d_partial + poff);
-                    poff += gr;
-                }
-                if (nh) {
-                    hipLaunchKernelGGL((k_pr_pull_hub<T>), dim3(nh), dim3(kBlock), 0, s, pp.d_bins + n0 + n1,
-                                       d->d_ptr, edges, 0ull, contrib, rank, next, d->d_scalars, damping, inv_n,
-                                       d->d_partial + poff);
-                    poff += nh;
-                }
-                OG_HIP(hipGetLastError());
-            }
-        }
-        const uint64_t sedges = d->plan.vsplit ? g->ptr[d->plan.vsplit] : 0;
-        st.run.relax_static_bytes += (16 + 2 * vb_bytes) * d->plan.vsplit + (4 + vb_bytes) * sedges;
-        st.run.static_work_edges += sedges;
-        for (size_t c = 0; c < pp.chunks.size(); ++c) {
-            const uint32_t va = pp.chunks[c].first, vb = pp.chunks[c].second;
-            const uint64_t e0 = g->ptr[va], e1 = g->ptr[vb];
-            const int slot = (int)(c % d->nslots);
-            uint8_t *dslot = (uint8_t *)d->d_staging + (uint64_t)slot * C * eb;
-            if (d->slot_relax_pending[slot]) OG_HIP(hipStreamWaitEvent(d->s_copy, d->ev_relax[slot], 0));
-            if (e1 > e0) {
-                EventSpan span(d, &tc_copy, d->s_copy);
-                OG_HIP(hipMemcpyAsync(dslot, g->cols + e0, (e1 - e0) * eb, hipMemcpyHostToDevice, d->s_copy));
-            }
-            OG_HIP(hipEventRecord(d->ev_h2d[slot], d->s_copy));
-            OG_HIP(hipStreamWaitEvent(s, d->ev_h2d[slot], 0));
-            {
-                EventSpan span(d, &tc_dyn, s);
-                const unsigned gr = grid_of((uint64_t)(vb - va) * kPrLpv0);
-                hipLaunchKernelGGL((k_pr_pull_range<T, kPrLpv0>), dim3(gr), dim3(kBlock), 0, s, va, vb, d->d_ptr,
-                                   (const uint32_t *)dslot, contrib, rank, next, d->d_scalars, damping, inv_n,
-                                   d->d_partial + poff);
-                OG_HIP(hipGetLastError());
-                poff += gr;
-            }
-            OG_HIP(hipEventRecord(d->ev_relax[slot], s));
-            d->slot_relax_pending[slot] = true;
-            st.run.h2d_bytes += (e1 - e0) * eb;
-            st.run.chunks++;
-            st.run.relax_dynamic_bytes += (16 + 2 * vb_bytes) * (vb - va) + (4 + vb_bytes) * (e1 - e0);
-        }
-        hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, s, d->d_partial, (uint32_t)poff,
-                           d->d_scalars + 1);
+    __atomic_store_n(d->h_progress, 0ull, __ATOMIC_RELEASE);
+    {
+        EventSpan span(d, &tc_init, s);
+        hipLaunchKernelGGL(k_pr_init<T>, dim3(igrid), dim3(kBlock), 0, s, a, V, prm.tolerance,
+                           CompactTotals{d->d_prtot, igrid, 0});
         OG_HIP(hipGetLastError());
-        OG_HIP(hipMemcpyAsync(d->h_scalars, d->d_scalars, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
-        OG_HIP(hipStreamSynchronize(s));
-        l1 = d->h_scalars[1];
-        std::swap(rank, next);
-        ++it;
-        st.run.work_edges += g->E;
-        if (l1 < prm.tolerance) break;
     }
-    OG_HIP(hipStreamSynchronize(s));
+    const uint64_t vb_bytes = sizeof(T);
+    const unsigned sgrid = pp.static_grid();
+    // the iteration's arrays: contributions of the last one in, its own out
+    auto turn = [&](uint32_t it) {
+        a.contrib = contrib[it & 1];
+        a.next = contrib[(it + 1) & 1];
+    };
+    auto pull_static = [&](hipStream_t on, unsigned long long *progress) {
+        hipLaunchKernelGGL(k_pr_pull<T>, dim3(sgrid), dim3(kBlock), 0, on, a, pp.d_rows, pp.n0, pp.n1, pp.nh, pp.g1,
+                           CompactTotals{d->d_prtot, sgrid, 0}, progress);
+        OG_HIP(hipGetLastError());
+    };
+    uint32_t it = 0;
+    if (pp.chunks.empty()) {
+        // One launch per iteration, enqueued a few ahead of the device:
+        // iterations past the last one return at once.
+        constexpr uint32_t kAhead = 4;
+        EventSpan span(d, &tc_static, s);
+        for (uint32_t k = 0; k < prm.max_iterations; ++k) {
+            if (k >= kAhead) wait_progress(d->h_progress, (unsigned long long)(k - kAhead + 1) << 1, s);
+            if (__atomic_load_n(d->h_progress, __ATOMIC_ACQUIRE) & 1) break;
+            turn(k);
+            pull_static(s, d->h_progress);
+        }
+        OG_HIP(hipMemcpyAsync(d->h_prstate, d->d_prstate, sizeof(PrState), hipMemcpyDeviceToHost, s));
+        OG_HIP(hipStreamSynchronize(s));
+        it = d->h_prstate->iterations;
+    } else {
+        // Chunk c of every iteration goes through slot (running number) % ring.
+        // The copies run ahead of the pulls by the ring, into the next
+        // iteration too (its edges are the same whatever the ranks are), so
+        // the link does not wait for the end of an iteration nor, while the
+        // ring fills, for the static pull.  Consecutive copies alternate
+        // between two streams: the hand-over from a copy to the next one's
+        // wait costs about 30 us, hidden behind the other stream's copy.
+        const uint64_t nc = pp.chunks.size();
+        uint64_t copied = 0, pulled = 0;
+        auto copy_next = [&] {
+            const PrPlan::Chunk &ch = pp.chunks[copied % nc];
+            const uint32_t slot = (uint32_t)(copied % pp.ring);
+            uint32_t *dslot = (uint32_t *)d->d_staging + slot * pp.slot;
+            const hipStream_t on = copied & 1 ? d->s_static : d->s_copy;
+            if (copied >= pp.ring) OG_HIP(hipStreamWaitEvent(on, pp.ev_pull[slot], 0));
+            if (ch.words)
+                OG_HIP(hipMemcpyAsync(dslot, pp.src + ch.word, ch.words * 4, hipMemcpyHostToDevice, on));
+            OG_HIP(hipEventRecord(pp.ev_h2d[slot], on));
+            st.run.h2d_bytes += ch.words * 4;
+            st.run.chunks++;
+            ++copied;
+        };
+        {
+            EventSpan copies(d, &tc_copy, d->s_copy);  // first copy to last: the link is busy throughout
+            while (it < prm.max_iterations) {
+                turn(it);
+                // the copies first: what the ring holds crosses the link beside the static pull
+                while (copied < pulled + std::min<uint64_t>(pp.ring, nc)) copy_next();
+                if (sgrid) {
+                    EventSpan span(d, &tc_static, s);
+                    pull_static(s, nullptr);
+                }
+                uint64_t poff = sgrid;
+                for (uint64_t c = 0; c < nc; ++c, ++pulled) {
+                    const PrPlan::Chunk &ch = pp.chunks[c];
+                    const uint32_t slot = (uint32_t)(pulled % pp.ring);
+                    OG_HIP(hipStreamWaitEvent(s, pp.ev_h2d[slot], 0));
+                    const unsigned gr = grid_of((uint64_t)(ch.vb - ch.va) * kPrRangeLpv);
+                    {
+                        EventSpan span(d, &tc_dyn, s);
+                        hipLaunchKernelGGL(k_pr_pull_range<T>, dim3(gr), dim3(kBlock), 0, s, a, ch.va, ch.vb,
+                                           (const uint32_t *)d->d_staging + slot * pp.slot, pp.lbits, ch.first, poff);
+                        OG_HIP(hipGetLastError());
+                    }
+                    poff += gr;
+                    OG_HIP(hipEventRecord(pp.ev_pull[slot], s));
+                    // the slots that are free, the one this chunk leaves among them
+                    const bool last = it + 1 == prm.max_iterations;
+                    while (copied < pulled + 1 + pp.ring && !(last && copied % nc == 0 && copied > pulled)) copy_next();
+                }
+                hipLaunchKernelGGL(k_pr_finish, dim3(1), dim3(1024), 0, s, d->d_partial, (uint32_t)poff, d->d_prstate,
+                                   d->h_progress);
+                OG_HIP(hipGetLastError());
+                ++it;
+                wait_progress(d->h_progress, (unsigned long long)it << 1, s);
+                if (__atomic_load_n(d->h_progress, __ATOMIC_ACQUIRE) & 1) break;
+            }
+        }
+        OG_HIP(hipMemcpyAsync(d->h_prstate, d->d_prstate, sizeof(PrState), hipMemcpyDeviceToHost, s));
+        OG_HIP(hipStreamSynchronize(s));
+        OG_HIP(hipStreamSynchronize(d->s_copy));
+        OG_HIP(hipStreamSynchronize(d->s_static));
+    }
     st.run.total_ms = total.ms();
-    if (out) copy_to_host(d, out, rank, V * sizeof(T), s);
-    // keep rank buffer order stable for the next call
-    if (rank != (T *)d->d_rank[0]) std::swap(d->d_rank[0], d->d_rank[1]);
+    if (out) copy_to_host(d, out, d->d_rank, V * sizeof(T), s);
+    const uint64_t sedges = d->plan.vsplit ? g->ptr[d->plan.vsplit] : 0;
+    // a row's bounds, rank (read and written), out-degree and contribution; an
+    // edge and its contribution
+    const uint64_t row = 16 + 2 * vb_bytes + 4 + vb_bytes;
+    st.run.frontier_bytes = V * (4 + 2 * vb_bytes);
+    st.run.relax_static_bytes = it * (row * d->plan.vsplit + (4 + vb_bytes) * sedges);
+    st.run.static_work_edges = it * sedges;
+    st.run.relax_dynamic_bytes = it * (row * (V - d->plan.vsplit) + (4 + vb_bytes) * (g->E - sedges));
+    if (pp.chunks.empty()) st.run.relax_dynamic_bytes = 0;
+    st.run.work_edges = (uint64_t)it * g->E;
     st.iterations = it;
-    st.final_l1 = l1;
+    st.final_l1 = d->h_prstate->l1;
     st.run.iterations = it;
     st.run.reached = V;
     st.run.traversed_edges = g->E;
     st.run.node_sum = (uint64_t)it * V;
-    st.run.frontier_kernel_ms = sum_ms(tc_contrib);
-    st.run.frontier_launches = tc_contrib.launches;
+    st.run.frontier_kernel_ms = sum_ms(tc_init);
+    st.run.frontier_launches = tc_init.launches;
     st.run.relax_static_kernel_ms = sum_ms(tc_static);
-    st.run.relax_static_launches = tc_static.launches;
+    st.run.relax_static_launches = pp.chunks.empty() ? it : tc_static.launches;
     st.run.relax_dynamic_kernel_ms = sum_ms(tc_dyn);
     st.run.relax_dynamic_launches = tc_dyn.launches;
     st.run.copy_ms = sum_ms(tc_copy);

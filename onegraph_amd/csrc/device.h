@@ -50,9 +50,8 @@ constexpr int kMsWidth = 64;            // sources per multi-source batch (bits 
 struct RelaxArgs {
     uint32_t *val;        // BFS level / SSSP distance / CC label
     uint8_t *flag;        // next-frontier flags
-    uint64_t *visit;      // multi-source: sources that reached v
+    ulonglong2 *vn;       // multi-source: x sources that reached v, y sources offered to v this round
     const uint64_t *front;// multi-source: sources whose frontier holds v
-    uint64_t *next;       // multi-source: sources offered to v this round
     uint32_t wbits;       // packed weighted edges: bits of the weight field
     const uint64_t *pull; // multi-source, optional: sources relaxed bottom-up this round
                           // (left out of the top-down relax)
@@ -379,11 +378,14 @@ struct DeviceState {
     std::unique_ptr<WorkerPool> pool;
 
     // multi-source BFS state (allocated on first use)
-    uint64_t *d_visit = nullptr, *d_front = nullptr, *d_next = nullptr;  // V each
-    uint8_t *d_mlvl = nullptr;       // V x 64 levels, vertex-major (0 = unreached)
+    ulonglong2 *d_vn = nullptr;      // V: sources that reached v, sources offered to v this round
+    uint64_t *d_front = nullptr;     // V: sources whose frontier holds v
+    uint8_t *d_mlvl = nullptr;       // V x 64 levels, vertex-major (0 = unreached); only when levels are asked for
+    unsigned long long *d_mpart = nullptr;  // per commit workgroup: digest, reached, traversed of the 64 sources
     uint32_t *d_msrc = nullptr;      // 64 sources of the batch
     unsigned long long *d_msum = nullptr;  // 2 x 64: checksum, reached per source
-    uint32_t *d_extract = nullptr;   // V scratch for one source's u32 levels
+    uint32_t *d_extract = nullptr;   // u32 levels of extract_cap sources on their way to the host
+    uint32_t extract_cap = 0;
     // direction-optimising BFS: in-edge CSR (OG_PLAN_DIRECTION_OPT)
     uint64_t *d_in_ptr = nullptr;    // V + 1
     uint32_t *d_in_cols = nullptr;   // E in-neighbours
@@ -685,8 +687,8 @@ struct SrvPull {
     const uint64_t *in_ptr;
     const uint32_t *in_cols;
     uint64_t V;
-    const uint64_t *visit, *front;
-    uint64_t *next;
+    ulonglong2 *vn;
+    const uint64_t *front;
     uint8_t *flag;
     const unsigned long long *pull;  // bit j: slot j scans bottom-up this round
 };

@@ -578,7 +578,10 @@ __device__ __forceinline__ typename SrcOf<ALGO>::T load_src(const RelaxArgs &a, 
 // atomic that finds nothing to do but never loses an update.
 template <int ALGO>
 __device__ __forceinline__ typename SrcOf<ALGO>::T peek(const RelaxArgs &a, uint32_t to) {
-    if constexpr (ALGO == ALGO_MSBFS) return a.visit[to];
+    if constexpr (ALGO == ALGO_MSBFS) {
+        const ulonglong2 x = a.vn[to];
+        return x.x | x.y;
+    }
     else return a.val[to];
 }
 
@@ -587,15 +590,19 @@ __device__ __forceinline__ typename SrcOf<ALGO>::T peek(const RelaxArgs &a, uint
 // store is race-free (a visited bitmap claimed with atomicOr, one writer per
 // vertex, was measured slower on R-MAT 20: 14.7 vs 17.2 GTEPS); SSSP/CC use atomicMin so no smaller offer is lost
 // (the reference's check-then-write in K7/K11 can lose one).  Multi-source:
-// the sources of u's frontier that have not reached `to` are OR-ed into
-// next[to] (one 64-bit atomic for all 64 searches).
+// the sources of u's frontier that have neither reached `to` nor been offered
+// to it are OR-ed into vn[to].y (one 64-bit atomic for all 64 searches).  The
+// two masks share a 16-byte load: with the offers unseen, every edge of a dense
+// round into a well-connected vertex repeated its atomic (R-MAT 4 M vertices,
+// 64 sources, the three dense rounds: 3.75, 2.43, 1.69 -> 1.86, 1.84, 1.70 ms,
+// the last ones the link's).
 template <int ALGO>
 __device__ __forceinline__ uint32_t commit(const RelaxArgs &a, typename SrcOf<ALGO>::T s, uint32_t to, uint32_t wt,
                                            typename SrcOf<ALGO>::T seen) {
     if constexpr (ALGO == ALGO_MSBFS) {
         const uint64_t m = s & ~seen;
         if (!m) return 0;
-        atomicOr((unsigned long long *)(a.next + to), (unsigned long long)m);
+        atomicOr(&a.vn[to].y, (unsigned long long)m);
         a.flag[to] = 1;
         return 1;
     } else {
@@ -947,12 +954,12 @@ __global__ __launch_bounds__(kBlock) void k_relax_round(RoundRelax r, RelaxArgs 
 // pulling slots P = *pull.  Every vertex that some slot of P has not reached
 // scans its in-edges, ORing the frontier masks of its in-neighbours
 // (restricted to those slots), and stops once every such slot is found.
-// Found slots are offered through next[v] like a top-down relax.
+// Found slots are offered through vn[v].y like a top-down relax.
 __device__ __forceinline__ void srv_pull_body(const SrvPull &p, uint32_t bid, uint32_t nb) {
     const uint64_t P = *p.pull;
     if (!P) return;
     for (uint64_t v = (uint64_t)bid * kBlock + threadIdx.x; v < p.V; v += (uint64_t)nb * kBlock) {
-        const uint64_t need = P & ~p.visit[v];
+        const uint64_t need = P & ~p.vn[v].x;
         if (!need) continue;
         uint64_t acc = 0;
         const uint64_t b = p.in_ptr[v], e = p.in_ptr[v + 1];
@@ -965,7 +972,7 @@ __device__ __forceinline__ void srv_pull_body(const SrvPull &p, uint32_t bid, ui
                 if (i + k < e) acc |= p.front[u[k]] & need;
         }
         if (acc) {
-            atomicOr((unsigned long long *)(p.next + v), (unsigned long long)acc);
+            atomicOr(&p.vn[v].y, (unsigned long long)acc);
             p.flag[v] = 1;
         }
     }
@@ -974,7 +981,8 @@ __device__ __forceinline__ void srv_pull_body(const SrvPull &p, uint32_t bid, ui
 // A served BFS round's relax in one launch: the top-down slots through the
 // static bins (as k_relax_round with cd = 0) and, beside them, the bottom-up
 // scan of the pulling slots (cp workgroups per period of kFuseStatic + cp).
-// The two only read visit / front and only OR into next and set flags, so
+// The two only read the reached and frontier masks and only OR into the offers
+// and set flags, so
 // they may run side by side.
 template <bool W, bool PK, int LPV>
 __global__ __launch_bounds__(kBlock) void k_srv_round(RoundRelax r, RelaxArgs a, SrvPull p, uint32_t cp) {
@@ -1106,79 +1114,167 @@ __global__ __launch_bounds__(kStatsBlock) void k_reach_stats(const uint32_t *__r
 
 // ------------------------------------------------------- multi-source BFS
 
-// Seeds up to 64 sources: bit j of visit/front at source j, level 1.
-__global__ void k_ms_init(const uint32_t *__restrict__ src, uint32_t n, uint64_t *visit, uint64_t *front,
-                          uint8_t *flag, uint8_t *lvl) {
+// Workgroups of the commit sweep at most: each keeps its own partial sums.
+constexpr unsigned kMsCommitGrid = 2048;
+// A wave's reached vertices (< 2^20 of them each round: V < 2^32 over at least
+// the grid's waves) and their degrees share a word; a graph has under 2^44 edges.
+constexpr int kMsFcShift = 44;
+constexpr int kMsGroups = 4;  // groups of 64 vertices per wave whose reads are in flight together
+constexpr int kMsSums = 3 * kMsWidth;  // digest, reached, traversed per source
+
+// Start of a batch, one launch: masks, flags and partial sums cleared, the
+// traversal state set (levels, when kept, are cleared apart).
+__global__ __launch_bounds__(kBlock) void k_ms_clear(ulonglong2 *__restrict__ vn, uint64_t *__restrict__ front,
+                                                     uint8_t *__restrict__ flag, uint64_t V, uint64_t Vpad,
+                                                     unsigned long long *__restrict__ part, uint64_t nparts,
+                                                     RoundCtl *ctl, RoundCtl c) {
+    const uint64_t tid = (uint64_t)blockIdx.x * kBlock + threadIdx.x, nth = (uint64_t)gridDim.x * kBlock;
+    if (tid == 0) *ctl = c;
+    for (uint64_t v = tid; v < V; v += nth) {
+        vn[v] = make_ulonglong2(0, 0);
+        front[v] = 0;
+    }
+    for (uint64_t i = tid; i < Vpad / 16; i += nth) ((uint4 *)flag)[i] = make_uint4(0, 0, 0, 0);
+    for (uint64_t i = tid; i < nparts; i += nth) part[i] = 0;
+}
+
+// Seeds up to 64 sources: bit j of the masks of source j, level 1, and its
+// terms in the sums of the first workgroup.
+__global__ void k_ms_init(const uint32_t *__restrict__ src, uint32_t n, ulonglong2 *vn, uint64_t *front, uint8_t *flag,
+                          uint8_t *lvl, const uint64_t *__restrict__ ptr, unsigned long long *part) {
     const uint32_t j = threadIdx.x;
     if (j < n) {
         const uint32_t s = src[j];
-        atomicOr((unsigned long long *)(visit + s), 1ull << j);
+        atomicOr(&vn[s].x, 1ull << j);
         atomicOr((unsigned long long *)(front + s), 1ull << j);
         flag[s] = 1;
-        lvl[(uint64_t)s * kMsWidth + j] = 1;
+        if (lvl) lvl[(uint64_t)s * kMsWidth + j] = 1;
+        part[j] = d_mix64(((uint64_t)s << 32) | 1u);
+        part[kMsWidth + j] = 1;
+        part[2 * kMsWidth + j] = ptr[s + 1] - ptr[s];
     }
 }
 
 // After a round: for every flagged vertex, the offered sources it had not
 // seen become its new frontier mask and get the round's level (rounds with
 // active vertices so far + 1, read from the device state; a level past 255
-// sets ctl->overflow); vertices with nothing new leave the frontier.
-__global__ __launch_bounds__(kBlock) void k_ms_commit(uint8_t *__restrict__ flag, uint64_t V, uint64_t *visit,
-                                                      uint64_t *front, uint64_t *next, uint8_t *lvl, RoundCtl *ctl,
-                                                      RoundClock *clk) {
+// sets ctl->overflow); vertices with nothing new leave the frontier.  A wave
+// takes 64 vertices; the new sources of one vertex are handled side by side,
+// lane = source: the lane adds the vertex to its source's digest, reached and
+// traversed sums (so the results need no pass over the levels) and, when the
+// caller wants levels, the row of 64 is stored as one line.  What bounds a
+// dense round is the instructions per vertex: its digest term, the same for
+// every source, is computed with lane = vertex, and its mask of new sources is
+// the lanes that add it (R-MAT 4 M vertices, 64 sources, a dense round: 290 us
+// with the terms per source, 172 now; one lane per vertex with a loop over
+// its sources and byte stores took 640, and a digest pass at the end 757).  The sums of a
+// workgroup go to its own slots of `part`.
+template <bool LEVELS>
+__global__ __launch_bounds__(kBlock) void k_ms_commit(uint8_t *__restrict__ flag, uint64_t V, ulonglong2 *__restrict__ vn,
+                                                      uint64_t *__restrict__ front, uint8_t *__restrict__ lvl,
+                                                      const uint64_t *__restrict__ ptr,
+                                                      const uint32_t *__restrict__ deg,
+                                                      const uint32_t *__restrict__ hdeg, RoundCtl *ctl,
+                                                      unsigned long long *__restrict__ part, RoundClock *clk) {
+    __shared__ unsigned long long s_sum[kMsSums];
     clock_stamp(clk, kClkRelax, kClkOther);
+    for (int i = threadIdx.x; i < kMsSums; i += kBlock) s_sum[i] = 0;
     const uint32_t lv32 = ctl->rounds + 1;
-    const uint8_t level = (uint8_t)min(lv32, 255u);
-    for (uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x; v < V; v += (uint64_t)gridDim.x * kBlock) {
-        if (!flag[v]) continue;
-        const uint64_t vis = visit[v];
-        const uint64_t nw = next[v] & ~vis;
-        next[v] = 0;
-        front[v] = nw;
-        if (nw) {
-            if (lv32 > 255) ctl->overflow = 1;
-            visit[v] = vis | nw;
-            uint64_t m = nw;
-            while (m) {
-                const int j = __builtin_ctzll(m);
-                m &= m - 1;
-                lvl[v * kMsWidth + j] = level;
-            }
-        } else {
-            flag[v] = 0;
-        }
-    }
-}
-
-// Per-source reached count, traversed edges and digest over the vertex-major
-// level array: lane j of each wave handles source j (one 64-byte line per
-// vertex), partial sums leave with one atomic per lane per block.
-__global__ __launch_bounds__(kBlock) void k_ms_digest(const uint8_t *__restrict__ lvl,
-                                                      const uint64_t *__restrict__ ptr, uint64_t V,
-                                                      unsigned long long *out /* 3 x 64 */, RoundClock *clk) {
-    clock_stamp(clk, kClkFront, kClkOther);
+    const uint32_t level = min(lv32, 255u);
     const int lane = threadIdx.x & (kWave - 1);
-    const uint64_t wave = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
-    const uint64_t nwaves = (uint64_t)gridDim.x * kBlock / kWave;
-    uint64_t r = 0, t = 0, h = 0;
-    for (uint64_t v = wave; v < V; v += nwaves) {
-        const uint32_t x = lvl[v * kMsWidth + lane];
-        if (x) {
-            ++r;
-            t += ptr[v + 1] - ptr[v];
-            h += d_mix64((v << 32) | x);
+    const uint64_t nwaves = (uint64_t)gridDim.x * (kBlock / kWave);
+    uint64_t h = 0, fc = 0;  // digest; reached << kMsFcShift | traversed
+    __syncthreads();
+    for (uint64_t g0 = (uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; g0 * kWave < V;
+         g0 += kMsGroups * nwaves) {
+        bool on[kMsGroups];
+        uint64_t nw[kMsGroups], dv[kMsGroups], mix[kMsGroups];
+#pragma unroll
+        for (int k = 0; k < kMsGroups; ++k) {
+            const uint64_t v = (g0 + k * nwaves) * kWave + lane;
+            on[k] = v < V && flag[v];
+        }
+        ulonglong2 x[kMsGroups];
+#pragma unroll
+        for (int k = 0; k < kMsGroups; ++k) {
+            const uint64_t v = (g0 + k * nwaves) * kWave + lane;
+            x[k] = on[k] ? vn[v] : make_ulonglong2(0, 0);
+            dv[k] = on[k] ? round_deg(deg, hdeg, ptr, nullptr, false, v) : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < kMsGroups; ++k) {
+            const uint64_t v = (g0 + k * nwaves) * kWave + lane;
+            nw[k] = x[k].y & ~x[k].x;
+            mix[k] = d_mix64((v << 32) | level);
+            dv[k] |= 1ull << kMsFcShift;
+            if (!on[k]) continue;
+            vn[v] = make_ulonglong2(x[k].x | nw[k], 0);
+            front[v] = nw[k];
+            if (!nw[k]) flag[v] = 0;
+        }
+#pragma unroll
+        for (int k = 0; k < kMsGroups; ++k) {
+            uint64_t todo = __ballot(nw[k] != 0);
+            if (todo && lv32 > 255) ctl->overflow = 1;
+            while (todo) {
+                const int l = __builtin_ctzll(todo);
+                todo &= todo - 1;
+                const uint64_t m = wave_read_u64(nw[k], l), d = wave_read_u64(dv[k], l), z = wave_read_u64(mix[k], l);
+                if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+                    h += z;
+                    fc += d;
+                    if (LEVELS) lvl[((g0 + k * nwaves) * kWave + l) * kMsWidth + lane] = (uint8_t)level;
+                }
+            }
         }
     }
-    atomicAdd(out + lane, (unsigned long long)h);
-    atomicAdd(out + kMsWidth + lane, (unsigned long long)r);
-    atomicAdd(out + 2 * kMsWidth + lane, (unsigned long long)t);
+    if (__ballot(fc != 0)) {
+        atomicAdd(&s_sum[lane], (unsigned long long)h);
+        atomicAdd(&s_sum[kMsWidth + lane], (unsigned long long)(fc >> kMsFcShift));
+        atomicAdd(&s_sum[2 * kMsWidth + lane], (unsigned long long)(fc & ((1ull << kMsFcShift) - 1)));
+    }
+    __syncthreads();
+    if (threadIdx.x < kMsSums && s_sum[threadIdx.x]) part[(uint64_t)blockIdx.x * kMsSums + threadIdx.x] += s_sum[threadIdx.x];
 }
 
-// Levels of source j as u32 in the single-source convention.
-__global__ void k_ms_extract(const uint8_t *__restrict__ lvl, uint64_t V, uint32_t j, uint32_t *out) {
-    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t x = lvl[v * kMsWidth + j];
-        out[v] = x ? x : OG_UNREACHED;
+// The sources' sums over the commit's workgroups.
+__global__ __launch_bounds__(1024) void k_ms_sum(const unsigned long long *__restrict__ part, uint32_t n,
+                                                 unsigned long long *out, RoundClock *clk) {
+    __shared__ uint64_t s[1024];
+    clock_stamp(clk, kClkFront, kClkOther);
+    const uint32_t col = blockIdx.x * kMsWidth + threadIdx.x % kMsWidth;
+    uint64_t x = 0;
+    for (uint32_t b = threadIdx.x / kMsWidth; b < n; b += 1024 / kMsWidth) x += part[(uint64_t)b * kMsSums + col];
+    s[threadIdx.x] = x;
+    __syncthreads();
+    if (threadIdx.x < kMsWidth) {
+        for (int k = 1; k < 1024 / kMsWidth; ++k) x += s[threadIdx.x + k * kMsWidth];
+        out[col] = x;
+    }
+}
+
+// Levels of sources j0 .. j0 + nj - 1 as u32 in the single-source convention,
+// one row of V per source: a workgroup turns the 64-byte rows of 64 vertices
+// through LDS, so that both sides move whole lines (a pass per source read
+// every row's line for one byte of it).
+__global__ __launch_bounds__(kBlock) void k_ms_extract(const uint8_t *__restrict__ lvl, uint64_t V, uint32_t j0, uint32_t nj,
+                                                       uint32_t *__restrict__ out) {
+    __shared__ uint32_t s_row[kWave][kMsWidth / 4 + 1];
+    for (uint64_t v0 = (uint64_t)blockIdx.x * kWave; v0 < V; v0 += (uint64_t)gridDim.x * kWave) {
+        const uint32_t r = threadIdx.x / 4, q = threadIdx.x % 4;
+        const uint4 x = v0 + r < V ? ((const uint4 *)(lvl + (v0 + r) * kMsWidth))[q] : make_uint4(0, 0, 0, 0);
+        s_row[r][4 * q + 0] = x.x;
+        s_row[r][4 * q + 1] = x.y;
+        s_row[r][4 * q + 2] = x.z;
+        s_row[r][4 * q + 3] = x.w;
+        __syncthreads();
+        const uint64_t v = v0 + threadIdx.x % kWave;
+        for (uint32_t j = threadIdx.x / kWave; j < nj; j += kBlock / kWave) {
+            const uint32_t js = j0 + j;
+            const uint32_t l = (s_row[threadIdx.x % kWave][js / 4] >> (8 * (js % 4))) & 0xFFu;
+            if (v < V) out[(uint64_t)j * V + v] = l ? l : OG_UNREACHED;
+        }
+        __syncthreads();
     }
 }
 
@@ -1965,7 +2061,7 @@ static void gather(DeviceState *d, const og_graph *g, uint32_t ndyn, uint64_t c0
 }
 
 static RelaxArgs relax_args(DeviceState *d) {
-    return RelaxArgs{d->d_val, d->fr.flag, d->d_visit, d->d_front, d->d_next, d->wbits, nullptr, d->run_pmid};
+    return RelaxArgs{d->d_val, d->fr.flag, d->d_vn, d->d_front, d->wbits, nullptr, d->run_pmid};
 }
 
 // Grids of device-count launches: the kernels stride over whatever count
@@ -2227,9 +2323,10 @@ constexpr int kRoundBatchMax = 64;  // largest first batch (sized from the previ
 // round's summary.
 // quiet_after: after() enqueues nothing (the compaction follows the relax).
 // begin(ctl): enqueues the start of the run with that traversal state.
+// variant: tells runs apart whose after() captures other work.
 template <int ALGO, bool W, class Begin, class After>
 static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTimers &tm, double &gather_ms,
-                          double &overload_wall, Begin begin, After after, bool quiet_after) {
+                          double &overload_wall, Begin begin, After after, bool quiet_after, bool variant = false) {
     hipStream_t s = d->s_compute;
     const uint64_t V = d->V;
     // SSSP near-far order: only vertices below the threshold relax in a
@@ -2323,7 +2420,7 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
             for (;;) {
                 const uint64_t key = (uint64_t)ALGO | (uint64_t)W << 4 | (uint64_t)(delta != 0) << 5 |
                                      (uint64_t)has_dyn << 6 | (uint64_t)dir_opt << 7 | (uint64_t)split << 16 |
-                                     (uint64_t)rounds << 8;
+                                     (uint64_t)variant << 17 | (uint64_t)rounds << 8;
                 RoundGraph *rg = round_graph_for(d, key, [&](RoundGraph *n) {
                     enqueue(GraphSpan{n}, rounds);
                 });
@@ -2476,23 +2573,33 @@ static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats 
 }
 
 // Multi-source BFS: sources in batches of 64; per vertex, u64 masks of the
-// sources that reached it (visit), whose frontier holds it (front) and that
-// were offered to it this round (next); levels as u8 per (vertex, source).
+// sources that reached it, that were offered to it this round (side by side)
+// and whose frontier holds it; levels as u8 per (vertex, source) when the
+// caller wants them.
+constexpr uint64_t kExtractBytes = 256ull << 20;  // device buffer of levels on their way to the host, at most
+
 template <bool W>
 static void run_msbfs(og_graph *g, const uint32_t *sources, uint32_t n, uint32_t *levels, uint64_t *checksums,
                       uint64_t *reached, og_run_stats *stats) {
     DeviceState *d = g->dev;
     const uint64_t V = d->V;
     hipStream_t s = d->s_compute;
-    if (!d->d_visit) {
-        d->d_visit = (uint64_t *)d->dalloc(V * 8);
+    const unsigned cgrid =
+        (unsigned)std::min<uint64_t>(kMsCommitGrid, std::max<uint64_t>(1, (V + kBlock - 1) / kBlock));
+    if (!d->d_vn) {
+        d->d_vn = (ulonglong2 *)d->dalloc(V * 16);
         d->d_front = (uint64_t *)d->dalloc(V * 8);
-        d->d_next = (uint64_t *)d->dalloc(V * 8);
-        d->d_mlvl = (uint8_t *)d->dalloc(V * kMsWidth);
         d->d_msrc = (uint32_t *)d->dalloc(kMsWidth * 4);
-        d->d_msum = (unsigned long long *)d->dalloc(3 * kMsWidth * 8);
+        d->d_msum = (unsigned long long *)d->dalloc(kMsSums * 8);
+        d->d_mpart = (unsigned long long *)d->dalloc((uint64_t)cgrid * kMsSums * 8);
     }
-    std::vector<unsigned long long> hsum(3 * kMsWidth);
+    if (levels && !d->d_mlvl) {
+        d->d_mlvl = (uint8_t *)d->dalloc(V * kMsWidth);
+        d->extract_cap = (uint32_t)std::min<uint64_t>(kMsWidth, std::max<uint64_t>(1, kExtractBytes / (V * 4)));
+        d->d_extract = (uint32_t *)d->dalloc((uint64_t)d->extract_cap * V * 4);
+    }
+    uint8_t *const lvl = levels ? d->d_mlvl : nullptr;
+    std::vector<unsigned long long> hsum(kMsSums);
     og_run_stats st{};
     st.approach = (uint32_t)d->approach;
     RunTimers tm;
@@ -2506,31 +2613,29 @@ static void run_msbfs(og_graph *g, const uint32_t *sources, uint32_t n, uint32_t
     double device_ms = 0;
     for (uint32_t b0 = 0; b0 < n; b0 += kMsWidth) {
         const uint32_t nb = std::min<uint32_t>(kMsWidth, n - b0);
-        OG_HIP(hipMemsetAsync(d->d_visit, 0, V * 8, s));
-        OG_HIP(hipMemsetAsync(d->d_front, 0, V * 8, s));
-        OG_HIP(hipMemsetAsync(d->d_next, 0, V * 8, s));
-        OG_HIP(hipMemsetAsync(d->d_mlvl, 0, V * kMsWidth, s));
-        OG_HIP(hipMemsetAsync(d->fr.flag, 0, d->Vpad, s));
+        if (lvl) OG_HIP(hipMemsetAsync(lvl, 0, V * kMsWidth, s));
         OG_HIP(hipMemcpyAsync(d->d_msrc, sources + b0, nb * 4, hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(k_ms_init, dim3(1), dim3(kMsWidth), 0, s, d->d_msrc, nb, d->d_visit, d->d_front,
-                           d->fr.flag, d->d_mlvl);
-        OG_HIP(hipGetLastError());
-        const unsigned cgrid = (unsigned)std::min<uint64_t>(4096, (V + kBlock - 1) / kBlock);
         auto begin = [&](const RoundCtl &c) {
-            hipLaunchKernelGGL(k_ctl_set, dim3(1), dim3(1), 0, s, d->fr.ctl, c);
+            hipLaunchKernelGGL(k_ms_clear, dim3(fill_grid(V)), dim3(kBlock), 0, s, d->d_vn, d->d_front, d->fr.flag, V,
+                               d->Vpad, d->d_mpart, (uint64_t)cgrid * kMsSums, d->fr.ctl, c);
+            hipLaunchKernelGGL(k_ms_init, dim3(1), dim3(kMsWidth), 0, s, d->d_msrc, nb, d->d_vn, d->d_front,
+                               d->fr.flag, lvl, d->d_ptr, d->d_mpart);
             OG_HIP(hipGetLastError());
         };
-        frontier_loop<ALGO_MSBFS, W>(g, d, st, tm, gather_ms, overload_wall, begin, [&](RoundClock *clk) {
-            hipLaunchKernelGGL(k_ms_commit, dim3(cgrid), dim3(kBlock), 0, s, d->fr.flag, V, d->d_visit, d->d_front,
-                               d->d_next, d->d_mlvl, d->fr.ctl, clk);
+        auto commit = [&](RoundClock *clk) {
+            if (lvl)
+                hipLaunchKernelGGL(k_ms_commit<true>, dim3(cgrid), dim3(kBlock), 0, s, d->fr.flag, V, d->d_vn,
+                                   d->d_front, lvl, d->d_ptr, d->d_deg, d->deg_heavy(), d->fr.ctl, d->d_mpart, clk);
+            else
+                hipLaunchKernelGGL(k_ms_commit<false>, dim3(cgrid), dim3(kBlock), 0, s, d->fr.flag, V, d->d_vn,
+                                   d->d_front, lvl, d->d_ptr, d->d_deg, d->deg_heavy(), d->fr.ctl, d->d_mpart, clk);
             OG_HIP(hipGetLastError());
-        }, false);
-        OG_HIP(hipMemsetAsync(d->d_msum, 0, 3 * kMsWidth * 8, s));
-        hipLaunchKernelGGL(k_ms_digest, dim3((unsigned)std::min<uint64_t>(1024, (V + kBlock - 1) / kBlock)),
-                           dim3(kBlock), 0, s, d->d_mlvl, d->d_ptr, V, d->d_msum,
+        };
+        frontier_loop<ALGO_MSBFS, W>(g, d, st, tm, gather_ms, overload_wall, begin, commit, false, lvl != nullptr);
+        hipLaunchKernelGGL(k_ms_sum, dim3(3), dim3(1024), 0, s, d->d_mpart, cgrid, d->d_msum,
                            tm.clocked >= 0 ? d->fr.clk : nullptr);
         OG_HIP(hipGetLastError());
-        OG_HIP(hipMemcpyAsync(hsum.data(), d->d_msum, 3 * kMsWidth * 8, hipMemcpyDeviceToHost, s));
+        OG_HIP(hipMemcpyAsync(hsum.data(), d->d_msum, kMsSums * 8, hipMemcpyDeviceToHost, s));
         OG_HIP(hipStreamSynchronize(s));
         device_ms = total.ms();
         for (uint32_t j = 0; j < nb; ++j) {
@@ -2540,15 +2645,15 @@ static void run_msbfs(og_graph *g, const uint32_t *sources, uint32_t n, uint32_t
             st.traversed_edges += hsum[2 * kMsWidth + j];
             st.checksum += hsum[j];
         }
-        if (levels) {
-            if (!d->d_extract) d->d_extract = (uint32_t *)d->dalloc(V * 4);
-            for (uint32_t j = 0; j < nb; ++j) {
-                hipLaunchKernelGGL(k_ms_extract, dim3(fill_grid(V)), dim3(256), 0, s, d->d_mlvl, V, j, d->d_extract);
+        if (levels)
+            for (uint32_t j = 0; j < nb; j += d->extract_cap) {
+                const uint32_t nj = std::min(d->extract_cap, nb - j);
+                hipLaunchKernelGGL(k_ms_extract,
+                                   dim3((unsigned)std::min<uint64_t>(8192, (V + kWave - 1) / kWave)), dim3(kBlock), 0, s,
+                                   lvl, V, j, nj, d->d_extract);
                 OG_HIP(hipGetLastError());
-                copy_to_host(d, levels + (uint64_t)(b0 + j) * V, d->d_extract, V * 4, s);
+                copy_to_host(d, levels + (uint64_t)(b0 + j) * V, d->d_extract, (uint64_t)nj * V * 4, s);
             }
-            OG_HIP(hipStreamSynchronize(s));
-        }
     }
     st.total_ms = device_ms;
     OG_HIP(hipMemcpyAsync(d->fr.h_blk, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
@@ -3155,7 +3260,7 @@ static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t 
     r.cd = 0;  // the whole graph is static: three bins in one launch
     r.vsplit = V;
     r.counters = ctr;
-    const RelaxArgs a{d_levels, flag, nullptr, nullptr, nullptr, 0, nullptr, nullptr};
+    const RelaxArgs a{d_levels, flag, nullptr, nullptr, 0, nullptr, nullptr};
     static_assert(Tuning{}.lpv0 == 8, "the relax below is instantiated for 8 lanes per bin-0 vertex");
     compact();
     OG_HIP(hipGetLastError());

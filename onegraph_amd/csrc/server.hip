@@ -4,7 +4,7 @@
 //
 // BFS: every graph has one batch engine with 64 query slots, its own HIP
 // stream, frontier buffers and host thread.  A slot is one bit of the
-// per-vertex u64 masks visit / front / next.  The host waits once per round,
+// per-vertex u64 masks visit / next (side by side) / front.  The host waits once per round,
 // for the commit's summary (step 2), and enqueues the next round while the
 // rest of this one runs:
 //   1. admit pending queries into free slots: the source's bit goes into
@@ -81,12 +81,12 @@ __device__ __forceinline__ uint64_t wave_or(uint64_t x) {
 // slot's explored-edge count and its sums (digest, reached, traversed in
 // acc[j], acc[64 + j], acc[128 + j]) restart: a finished slot keeps its last
 // sums until it takes another query, and nothing adds to an unused slot's.
-__global__ void k_srv_seed(SeedList sl, uint64_t *next, uint8_t *flag, unsigned long long *explored,
+__global__ void k_srv_seed(SeedList sl, ulonglong2 *vn, uint8_t *flag, unsigned long long *explored,
                            unsigned long long *acc) {
     const uint32_t i = threadIdx.x;
     if (i < sl.n) {
         const uint32_t j = sl.slot[i];
-        atomicOr((unsigned long long *)(next + sl.src[i]), 1ull << j);
+        atomicOr(&vn[sl.src[i]].y, 1ull << j);
         flag[sl.src[i]] = 1;
         explored[j] = 0;
         acc[j] = acc[64 + j] = acc[128 + j] = 0;
@@ -118,8 +118,8 @@ constexpr int kFcShift = 40;
 __global__ __launch_bounds__(kBlock) void k_srv_commit(uint8_t *__restrict__ flag, uint64_t V,
                                                        const uint64_t *__restrict__ ptr,
                                                        const uint32_t *__restrict__ deg,
-                                                       const uint32_t *__restrict__ hdeg, uint64_t *__restrict__ visit,
-                                                       uint64_t *__restrict__ front, uint64_t *__restrict__ next,
+                                                       const uint32_t *__restrict__ hdeg, ulonglong2 *__restrict__ vn,
+                                                       uint64_t *__restrict__ front,
                                                        SlotLevels L, KeepList keep, unsigned long long *acc,
                                                        unsigned long long *fstat, unsigned long long *alive) {
     __shared__ unsigned long long sdig[kCommitCopies * kCommitStride], sfe[kCommitCopies * kCommitStride];
@@ -142,14 +142,13 @@ __global__ __launch_bounds__(kBlock) void k_srv_commit(uint8_t *__restrict__ fla
         const bool on = v < V && flag[v];
         if (!__ballot(on)) continue;  // b is the same for the whole wave
         if (on) {
-            const uint64_t vis = visit[v];
-            const uint64_t nw = next[v] & ~vis;
-            next[v] = 0;
+            const ulonglong2 x = vn[v];
+            const uint64_t nw = x.y & ~x.x;
+            vn[v] = make_ulonglong2(x.x | nw, 0);
             const uint64_t dv = round_deg(deg, hdeg, ptr, nullptr, false, v);
             if (nw) {
                 // each slot that reaches v: digest term, one more reached
                 // vertex, deg more traversed edges (= its frontier edges)
-                visit[v] = vis | nw;
                 uint64_t m = nw;
                 while (m) {
                     const int j = __builtin_ctzll(m);
@@ -235,10 +234,10 @@ __global__ __launch_bounds__(kBlock) void k_srv_clear_front(const uint32_t *__re
 }
 
 // Clears the visit bits of finished slots (before the slots are reused).
-__global__ __launch_bounds__(kBlock) void k_srv_clear_visit(uint64_t V, uint64_t dirty, uint64_t *visit) {
+__global__ __launch_bounds__(kBlock) void k_srv_clear_visit(uint64_t V, uint64_t dirty, ulonglong2 *vn) {
     for (uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x; v < V; v += (uint64_t)gridDim.x * kBlock) {
-        const uint64_t x = visit[v];
-        if (x & dirty) visit[v] = x & ~dirty;
+        const uint64_t x = vn[v].x;
+        if (x & dirty) vn[v].x = x & ~dirty;
     }
 }
 
@@ -767,7 +766,8 @@ struct BfsEngine {
     Frontier f;
     hipStream_t s = nullptr;
     hipEvent_t ev_summary = nullptr;  // the round's alive mask and slot sums are on the host
-    uint64_t *visit = nullptr, *front = nullptr, *next = nullptr;
+    ulonglong2 *vn = nullptr;  // slots that reached the vertex, slots offered to it this round
+    uint64_t *front = nullptr;
     // round summary: [0] alive slots (the commit ORs into it), [1] pulling
     // slots, [2] the round's alive slots, [3, 195) slot sums (acc); the host
     // copy h_sum receives [1, 195) each round
@@ -1002,7 +1002,7 @@ void BfsEngine::step() {
         const uint32_t clean = kSlots - (uint32_t)__builtin_popcountll(used | dirty);
         if (dirty && (pending->size() > clean || __builtin_popcountll(dirty) >= (int)kSlots / 2)) {
             hipLaunchKernelGGL(k_srv_clear_visit, dim3(sweep_grid(d->V, 16384)), dim3(kBlock), 0, s, d->V, dirty,
-                               visit);
+                               vn);
             OG_HIP(hipGetLastError());
             dirty = 0;  // stream order: the sweep runs before this round's seeds and commit
         }
@@ -1037,14 +1037,14 @@ void BfsEngine::step() {
         if (kb >= 0) OG_HIP(hipMemsetAsync(keep_buf[kb], 0xFF, V * 4, s));
     }
     if (sl.n) {
-        hipLaunchKernelGGL(k_srv_seed, dim3(1), dim3(64), 0, s, sl, next, f.flag, d_explored, d_acc);
+        hipLaunchKernelGGL(k_srv_seed, dim3(1), dim3(64), 0, s, sl, vn, f.flag, d_explored, d_acc);
         OG_HIP(hipGetLastError());
     }
     const bool dir_opt = d->d_in_ptr != nullptr;
     SlotLevels L{};
     for (uint32_t j = 0; j < kSlots; ++j) L.lv[j] = round - slots[j].start_round + 1;
     hipLaunchKernelGGL(k_srv_commit, dim3(sweep_grid(V, 4096)), dim3(kBlock), 0, s, f.flag, V,
-                       d->d_ptr, d->d_deg, d->deg_heavy(), visit, front, next, L, keep_list(used), d_acc, d_fstat,
+                       d->d_ptr, d->d_deg, d->deg_heavy(), vn, front, L, keep_list(used), d_acc, d_fstat,
                        d_alive);
     OG_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_srv_direction, dim3(1), dim3(64), 0, s, used, V, d->E, dir_opt ? 1 : 0, d_fstat,
@@ -1056,8 +1056,8 @@ void BfsEngine::step() {
     // Counts stay on the device: the compaction, relax and clear kernels read
     // them from f.info, so the round needs no host round trip before its end.
     frontier_compact(d, f, s, nullptr, false);
-    RelaxArgs a{nullptr, f.flag, visit, front, next, d->wbits, dir_opt ? (const uint64_t *)d_pull : nullptr};
-    const SrvPull pl{d->d_in_ptr, d->d_in_cols, V, visit, front, next, f.flag, d_pull};
+    RelaxArgs a{nullptr, f.flag, vn, front, d->wbits, dir_opt ? (const uint64_t *)d_pull : nullptr};
+    const SrvPull pl{d->d_in_ptr, d->d_in_cols, V, vn, front, f.flag, d_pull};
     launch_srv_round(d, f, a, s, dir_opt ? &pl : nullptr, g->kind == OG_KIND_WEIGHTED);
     hipLaunchKernelGGL(k_srv_clear_front, dim3(1024), dim3(kBlock), 0, s, f.list, d->plan.vsplit, f.hub,
                        f.hub_cap, f.info, front);
@@ -1476,13 +1476,11 @@ extern "C" og_status og_server_create(og_graph *const *graphs, uint32_t num_grap
             OG_HIP(hipStreamCreateWithFlags(&e->s, hipStreamNonBlocking));
             OG_HIP(hipEventCreateWithFlags(&e->ev_summary, hipEventDisableTiming));
             frontier_alloc(g->dev, g, e->f, e->mem);
-            e->visit = (uint64_t *)e->mem.dalloc(V * 8);
+            e->vn = (ulonglong2 *)e->mem.dalloc(V * 16);
             e->front = (uint64_t *)e->mem.dalloc(V * 8);
-            e->next = (uint64_t *)e->mem.dalloc(V * 8);
             for (auto &kb : e->keep_buf) kb = (uint32_t *)e->mem.dalloc(V * 4);
-            OG_HIP(hipMemset(e->visit, 0, V * 8));
+            OG_HIP(hipMemset(e->vn, 0, V * 16));
             OG_HIP(hipMemset(e->front, 0, V * 8));
-            OG_HIP(hipMemset(e->next, 0, V * 8));
             e->d_sum = (unsigned long long *)e->mem.dalloc((3 + 3 * 64) * 8);
             e->h_sum = (unsigned long long *)e->mem.palloc((3 + 3 * 64) * 8);
             OG_HIP(hipMemset(e->d_sum, 0, (3 + 3 * 64) * 8));

@@ -225,6 +225,7 @@ struct Frontier {
     RoundCtl *ctl = nullptr;         // parts of blk
     unsigned long long *counters = nullptr;
     RoundClock *clk = nullptr;
+    unsigned long long *spread = nullptr;  // kSpreadWords: the relax kernels' counters on their way to blk
 };
 
 // Timing of one class of launches: pairs of events on the launching stream.
@@ -555,12 +556,32 @@ __device__ __forceinline__ uint64_t block_sum(uint64_t x, uint64_t *lds) {
     return t;
 }
 
-// Adds the wave's per-lane counts to *ctr with one atomic per wave.
-__device__ __forceinline__ void wave_add(unsigned long long *ctr, uint32_t v) {
-    uint64_t s = v;
+// Work counters of a run's relax kernels, spread over kSpread lines of 16
+// words: every wave of a launch adds to one, and on a single line those
+// atomics queued at about 12 ns each (20480 waves of a round: 230 us, which is
+// what a dense round took whatever it relaxed).  The run's last kernel folds
+// them (fold_spread).
+constexpr uint32_t kSpread = 128;
+constexpr uint32_t kSpreadWords = kSpread * 16;
+enum SpreadWord { kUpdStatic = 0, kUpdDynamic = 1, kHbmEdges = 5 };  // word of a line = index in RunBlock::counters
+
+// Adds the wave's per-lane counts with one atomic per wave.
+__device__ __forceinline__ void wave_count(unsigned long long *spread, int word, uint32_t v) {
+    const uint32_t s = wave_scan_u32(v);
+    const uint32_t line = (blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave) % kSpread;
+    if ((threadIdx.x & (kWave - 1)) == kWave - 1 && s) atomicAdd(spread + line * 16 + word, (unsigned long long)s);
+}
+
+// counters[w] += the lines' words w, which restart at zero (one workgroup of
+// at least kSpread threads).
+__device__ __forceinline__ void fold_spread(unsigned long long *spread, unsigned long long *counters) {
+    if (threadIdx.x >= kSpread) return;
+    const int words[3] = {kUpdStatic, kUpdDynamic, kHbmEdges};
 #pragma unroll
-    for (int m = 1; m < kWave; m <<= 1) s += shfl_xor_u64(s, m);
-    if ((threadIdx.x & (kWave - 1)) == 0 && s) atomicAdd(ctr, (unsigned long long)s);
+    for (int i = 0; i < 3; ++i) {
+        const uint64_t s = wave_scan_u64(atomicExch(spread + threadIdx.x * 16 + words[i], 0ull));
+        if ((threadIdx.x & (kWave - 1)) == kWave - 1 && s) atomicAdd(counters + words[i], (unsigned long long)s);
+    }
 }
 
 constexpr int kRelaxBatch = 4;  // edges per lane whose reads are issued together

@@ -66,12 +66,13 @@ __device__ __forceinline__ void clock_stamp(RoundClock *clk, int prev, int kind)
 template <bool IOTA>
 __global__ __launch_bounds__(kBlock) void k_run_init(uint32_t *__restrict__ val, uint8_t *__restrict__ flag, uint64_t V,
                                                      uint64_t Vpad, uint32_t src, RunBlock *__restrict__ blk,
-                                                     RoundCtl c) {
+                                                     unsigned long long *__restrict__ spread, RoundCtl c) {
     const uint64_t tid = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
     if (blockIdx.x == 0) {
         if (threadIdx.x < 16) blk->counters[threadIdx.x] = 0;
         if (threadIdx.x < 3) blk->clk.acc[threadIdx.x] = 0;
         if (threadIdx.x == 0) blk->ctl = c;
+        for (uint32_t i = threadIdx.x; i < kSpreadWords; i += kBlock) spread[i] = 0;
     }
     for (uint64_t i = tid; i < Vpad / 4; i += (uint64_t)gridDim.x * kBlock) {
         const uint64_t v = 4 * i;
@@ -573,8 +574,8 @@ __device__ __forceinline__ typename SrcOf<ALGO>::T load_src(const RelaxArgs &a, 
 
 // Relaxing an edge (u -> to, wt) is split in two so that a lane can keep the
 // reads of several edges in flight before its first atomic: peek() reads the
-// target's state, commit() compares u's offer with what peek saw and applies
-// it.  Values only decrease (masks only grow), so a stale peek can cost an
+// target's state, commit() compares the offers with what peek saw and applies
+// them.  Values only decrease (masks only grow), so a stale peek can cost an
 // atomic that finds nothing to do but never loses an update.
 template <int ALGO>
 __device__ __forceinline__ typename SrcOf<ALGO>::T peek(const RelaxArgs &a, uint32_t to) {
@@ -585,41 +586,78 @@ __device__ __forceinline__ typename SrcOf<ALGO>::T peek(const RelaxArgs &a, uint
     else return a.val[to];
 }
 
-// Returns 1 when `to` improved (and is flagged for the next frontier).
+// Applies N offers of a lane (edge k valid when bit k of `ok` is set, its
+// source's state src(k)) and returns how many improved their target (which is
+// then flagged for the next frontier).
 // BFS writes the same level from every writer in an iteration, so a plain
 // store is race-free (a visited bitmap claimed with atomicOr, one writer per
-// vertex, was measured slower on R-MAT 20: 14.7 vs 17.2 GTEPS); SSSP/CC use atomicMin so no smaller offer is lost
-// (the reference's check-then-write in K7/K11 can lose one).  Multi-source:
-// the sources of u's frontier that have neither reached `to` nor been offered
-// to it are OR-ed into vn[to].y (one 64-bit atomic for all 64 searches).  The
-// two masks share a 16-byte load: with the offers unseen, every edge of a dense
-// round into a well-connected vertex repeated its atomic (R-MAT 4 M vertices,
-// 64 sources, the three dense rounds: 3.75, 2.43, 1.69 -> 1.86, 1.84, 1.70 ms,
-// the last ones the link's).
-template <int ALGO>
-__device__ __forceinline__ uint32_t commit(const RelaxArgs &a, typename SrcOf<ALGO>::T s, uint32_t to, uint32_t wt,
-                                           typename SrcOf<ALGO>::T seen) {
+// vertex, was measured slower on R-MAT 20: 14.7 vs 17.2 GTEPS); SSSP/CC use
+// atomicMin so no smaller offer is lost (the reference's check-then-write in
+// K7/K11 can lose one).  With AGAIN a lane first reads the targets that its
+// peeks would improve once more, at the place where the device's atomics are
+// performed: a peek may come from a copy in this XCD's L2 that keeps the value
+// of the kernel's start, and atomics on one line queue at about 12 ns each.
+// It pays beside the link's latency, in the dynamic region (out-of-memory SSSP
+// R-MAT 16.7 M 16.75 -> 16.05 ms, CC 3 M 6.55 -> 6.32 ms), and costs a round trip
+// elsewhere (SSSP in memory 0.77 -> 0.83 ms).  Multi-source: the sources of u's frontier that have neither reached `to`
+// nor been offered to it are OR-ed into vn[to].y (one 64-bit atomic for all 64
+// searches).  The two masks share a 16-byte load: with the offers unseen, every
+// edge of a dense round into a well-connected vertex repeated its atomic (R-MAT
+// 4 M vertices, 64 sources, the three dense rounds: 3.75, 2.43, 1.69 -> 1.86,
+// 1.84, 1.70 ms, the last ones the link's).
+template <int ALGO, int N, bool AGAIN = false, class Src>
+__device__ __forceinline__ uint32_t commit(const RelaxArgs &a, Src src, const uint32_t (&to)[N], const uint32_t (&wt)[N],
+                                           const typename SrcOf<ALGO>::T (&seen)[N], uint32_t ok) {
+    uint32_t c = 0;
     if constexpr (ALGO == ALGO_MSBFS) {
-        const uint64_t m = s & ~seen;
-        if (!m) return 0;
-        atomicOr(&a.vn[to].y, (unsigned long long)m);
-        a.flag[to] = 1;
-        return 1;
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const uint64_t m = (ok >> k) & 1 ? src(k) & ~seen[k] : 0;
+            if (!m) continue;
+            atomicOr(&a.vn[to[k]].y, (unsigned long long)m);
+            a.flag[to[k]] = 1;
+            ++c;
+        }
+    } else if constexpr (ALGO == ALGO_BFS) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const uint32_t nd = offer<ALGO>(src(k), wt[k]);
+            if (!((ok >> k) & 1) || nd >= seen[k]) continue;
+            a.val[to[k]] = nd;
+            a.flag[to[k]] = 1;
+            ++c;
+        }
     } else {
-        const uint32_t nd = offer<ALGO>(s, wt);
-        if (nd >= seen) return 0;
-        if (ALGO == ALGO_BFS) {
-            a.val[to] = nd;
-            a.flag[to] = 1;
-            return 1;
+        uint32_t nd[N], x[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            nd[k] = offer<ALGO>(src(k), wt[k]);
+            if (nd[k] >= seen[k]) ok &= ~(1u << k);
         }
-        const uint32_t old = atomicMin(a.val + to, nd);
-        if (nd < old) {
-            a.flag[to] = 1;
-            return 1;
+        if (!ok) return 0;
+        if constexpr (AGAIN) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                x[k] = 0;
+                if ((ok >> k) & 1) x[k] = __hip_atomic_load(a.val + to[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+#pragma unroll
+            for (int k = 0; k < N; ++k)
+                if (nd[k] >= x[k]) ok &= ~(1u << k);
+            if (!ok) return 0;
         }
-        return 0;
+        // all atomics before the first result is used
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            if ((ok >> k) & 1) x[k] = atomicMin(a.val + to[k], nd[k]);
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            if (((ok >> k) & 1) && nd[k] < x[k]) {
+                a.flag[to[k]] = 1;
+                ++c;
+            }
     }
+    return c;
 }
 
 // The relax kernels read their work counts from the round's FrontierInfo on
@@ -657,12 +695,16 @@ __device__ __forceinline__ uint32_t relax_group_body(const uint32_t *__restrict_
                 wt[k] = 0;
                 if (i + (uint64_t)k * LPV < e) load_edge<W, PK>(edges, i + (uint64_t)k * LPV, a.wbits, to[k], wt[k]);
             }
+            uint32_t ok = 0;
 #pragma unroll
-            for (int k = 0; k < kRelaxBatch; ++k)
-                if (i + (uint64_t)k * LPV < e) seen[k] = peek<ALGO>(a, to[k]);
-#pragma unroll
-            for (int k = 0; k < kRelaxBatch; ++k)
-                if (i + (uint64_t)k * LPV < e) cnt += commit<ALGO>(a, s, to[k], wt[k], seen[k]);
+            for (int k = 0; k < kRelaxBatch; ++k) {
+                seen[k] = 0;
+                if (i + (uint64_t)k * LPV < e) {
+                    seen[k] = peek<ALGO>(a, to[k]);
+                    ok |= 1u << k;
+                }
+            }
+            cnt += commit<ALGO, kRelaxBatch>(a, [&](int) { return s; }, to, wt, seen, ok);
         }
     }
     return cnt;
@@ -673,8 +715,8 @@ __global__ __launch_bounds__(kBlock) void k_relax_group(const uint32_t *__restri
                                                         const FrontierInfo *__restrict__ info,
                                                         const uint64_t *__restrict__ ptr,
                                                         const void *__restrict__ edges, RelaxArgs a,
-                                                        unsigned long long *upd) {
-    wave_add(upd, relax_group_body<ALGO, W, PK, LPV>(list, vsplit, bin, info, ptr, edges, a, blockIdx.x, gridDim.x));
+                                                        unsigned long long *spread) {
+    wave_count(spread, kUpdStatic, relax_group_body<ALGO, W, PK, LPV>(list, vsplit, bin, info, ptr, edges, a, blockIdx.x, gridDim.x));
 }
 
 template <int ALGO, bool W, bool PK>
@@ -712,12 +754,16 @@ __device__ __forceinline__ uint32_t relax_hub_body(const uint64_t *__restrict__ 
                 wt[j] = 0;
                 if (k0 + j * kBlock < cnt) load_edge<W, PK>(s_edges, k0 + j * kBlock, a.wbits, to[j], wt[j]);
             }
+            uint32_t ok = 0;
 #pragma unroll
-            for (int j = 0; j < kRelaxBatch; ++j)
-                if (k0 + j * kBlock < cnt) seen[j] = peek<ALGO>(a, to[j]);
-#pragma unroll
-            for (int j = 0; j < kRelaxBatch; ++j)
-                if (k0 + j * kBlock < cnt) c += commit<ALGO>(a, s, to[j], wt[j], seen[j]);
+            for (int j = 0; j < kRelaxBatch; ++j) {
+                seen[j] = 0;
+                if (k0 + j * kBlock < cnt) {
+                    seen[j] = peek<ALGO>(a, to[j]);
+                    ok |= 1u << j;
+                }
+            }
+            c += commit<ALGO, kRelaxBatch>(a, [&](int) { return s; }, to, wt, seen, ok);
         }
         __syncthreads();  // the tile buffer is reused by the next tile
     }
@@ -732,9 +778,9 @@ __global__ __launch_bounds__(kBlock) void k_relax_hub(const uint64_t *__restrict
                                                       const FrontierInfo *__restrict__ info, uint32_t tile,
                                                       const uint64_t *__restrict__ ptr,
                                                       const void *__restrict__ edges, RelaxArgs a,
-                                                      unsigned long long *upd) {
+                                                      unsigned long long *spread) {
     extern __shared__ uint32_t s_edges[];
-    wave_add(upd, relax_hub_body<ALGO, W, PK>(hub, hub_cap, info, tile, ptr, edges, a, s_edges, blockIdx.x, gridDim.x));
+    wave_count(spread, kUpdStatic, relax_hub_body<ALGO, W, PK>(hub, hub_cap, info, tile, ptr, edges, a, s_edges, blockIdx.x, gridDim.x));
 }
 
 // Dynamic region, edges [c0, min(c1, D)) of the concatenated active dynamic
@@ -857,12 +903,16 @@ __device__ __forceinline__ uint32_t relax_dyn_body(const uint32_t *__restrict__ 
                 }
             }
         }
+        uint32_t ok = 0;
 #pragma unroll
-        for (int j = 0; j < kDynEdgesPerThread; ++j)
-            if (q0 + threadIdx.x + (uint64_t)j * kBlock < q1) seen[j] = peek<ALGO>(a, to[j]);
-#pragma unroll
-        for (int j = 0; j < kDynEdgesPerThread; ++j)
-            if (q0 + threadIdx.x + (uint64_t)j * kBlock < q1) c += commit<ALGO>(a, sv[j], to[j], wt[j], seen[j]);
+        for (int j = 0; j < kDynEdgesPerThread; ++j) {
+            seen[j] = 0;
+            if (q0 + threadIdx.x + (uint64_t)j * kBlock < q1) {
+                seen[j] = peek<ALGO>(a, to[j]);
+                ok |= 1u << j;
+            }
+        }
+        c += commit<ALGO, kDynEdgesPerThread, true>(a, [&](int j) { return sv[j]; }, to, wt, seen, ok);
         __syncthreads();  // s_off / s_i are reloaded for the next chunk
     }
     hits = h;
@@ -879,15 +929,14 @@ __global__ __launch_bounds__(kBlock) void k_relax_dyn(const uint32_t *__restrict
                                                       const int64_t *__restrict__ rdelta,
                                                       uint32_t wbits, RelaxArgs a, const uint64_t *__restrict__ lpos,
                                                       uint64_t nl, uint64_t vsplit, const uint32_t *__restrict__ dchunk,
-                                                      uint32_t lbits, unsigned long long *upd,
-                                                      unsigned long long *hits) {
+                                                      uint32_t lbits, unsigned long long *spread) {
     __shared__ DynLds L;
     uint32_t h = 0;
     const uint32_t c = relax_dyn_body<ALGO, W, PACKED, DIRECT>(list, info, doff, stage, c0, c1max, ptr, dbase, resident,
                                                                rdelta, wbits, a, lpos, nl, vsplit, dchunk, lbits, L,
                                                                blockIdx.x, gridDim.x, h);
-    wave_add(upd, c);
-    if (DIRECT) wave_add(hits, h);
+    wave_count(spread, kUpdDynamic, c);
+    if (DIRECT) wave_count(spread, kHbmEdges, h);
 }
 
 // One round's relax in a single launch: static bins 0 and 1, hub tiles and
@@ -918,7 +967,7 @@ struct RoundRelax {
     const uint32_t *dchunk;     // chunk table of the dynamic edge space
     uint32_t lbits;             // bits per edge of the dynamic region in host memory (0: whole edges)
     uint64_t nl, vsplit;
-    unsigned long long *counters;  // [0] static updates, [1] dynamic updates, [5] HBM-served dynamic edges
+    unsigned long long *spread;  // work counters
     RoundClock *clk;            // null: not timed
 };
 constexpr uint32_t kFuseStatic = 5;
@@ -931,13 +980,13 @@ __global__ __launch_bounds__(kBlock) void k_relax_round(RoundRelax r, RelaxArgs 
     const uint32_t K = gridDim.x / P;
     const uint32_t k = blockIdx.x / P, j = blockIdx.x - k * P;
     if (j < 2) {
-        wave_add(r.counters + 0,
+        wave_count(r.spread, kUpdStatic,
                  relax_group_body<ALGO, W, PK, LPV>(r.list, r.vsplit, 0, r.info, r.ptr, r.sedges, a, 2 * k + j, 2 * K));
     } else if (j < 4) {
-        wave_add(r.counters + 0,
+        wave_count(r.spread, kUpdStatic,
                  relax_group_body<ALGO, W, PK, 64>(r.list, r.vsplit, 1, r.info, r.ptr, r.sedges, a, 2 * k + j - 2, 2 * K));
     } else if (j == 4) {
-        wave_add(r.counters + 0, relax_hub_body<ALGO, W, PK>(r.hub, r.hub_cap, r.info, r.tile, r.ptr, r.sedges, a,
+        wave_count(r.spread, kUpdStatic, relax_hub_body<ALGO, W, PK>(r.hub, r.hub_cap, r.info, r.tile, r.ptr, r.sedges, a,
                                                               (uint32_t *)s_fuse, k, K));
     } else {
         uint32_t h = 0;
@@ -945,8 +994,8 @@ __global__ __launch_bounds__(kBlock) void k_relax_round(RoundRelax r, RelaxArgs 
                                                              r.resident, r.rdelta, a.wbits, a, r.lpos, r.nl, r.vsplit,
                                                              r.dchunk, r.lbits, *(DynLds *)s_fuse, r.cd * k + (j - kFuseStatic),
                                                              r.cd * K, h);
-        wave_add(r.counters + 1, c);
-        wave_add(r.counters + 5, h);
+        wave_count(r.spread, kUpdDynamic, c);
+        wave_count(r.spread, kHbmEdges, h);
     }
 }
 
@@ -991,13 +1040,13 @@ __global__ __launch_bounds__(kBlock) void k_srv_round(RoundRelax r, RelaxArgs a,
     const uint32_t K = gridDim.x / P;
     const uint32_t k = blockIdx.x / P, j = blockIdx.x - k * P;
     if (j < 2) {
-        wave_add(r.counters + 0, relax_group_body<ALGO_MSBFS, W, PK, LPV>(r.list, r.vsplit, 0, r.info, r.ptr, r.sedges, a,
+        wave_count(r.spread, kUpdStatic, relax_group_body<ALGO_MSBFS, W, PK, LPV>(r.list, r.vsplit, 0, r.info, r.ptr, r.sedges, a,
                                                                          2 * k + j, 2 * K));
     } else if (j < 4) {
-        wave_add(r.counters + 0, relax_group_body<ALGO_MSBFS, W, PK, 64>(r.list, r.vsplit, 1, r.info, r.ptr, r.sedges, a,
+        wave_count(r.spread, kUpdStatic, relax_group_body<ALGO_MSBFS, W, PK, 64>(r.list, r.vsplit, 1, r.info, r.ptr, r.sedges, a,
                                                                         2 * k + j - 2, 2 * K));
     } else if (j == 4) {
-        wave_add(r.counters + 0, relax_hub_body<ALGO_MSBFS, W, PK>(r.hub, r.hub_cap, r.info, r.tile, r.ptr, r.sedges,
+        wave_count(r.spread, kUpdStatic, relax_hub_body<ALGO_MSBFS, W, PK>(r.hub, r.hub_cap, r.info, r.tile, r.ptr, r.sedges,
                                                                     a, (uint32_t *)s_fuse, k, K));
     } else {
         srv_pull_body(p, cp * k + (j - kFuseStatic), cp * K);
@@ -1013,7 +1062,7 @@ __global__ __launch_bounds__(kBlock) void k_bfs_pull(const uint64_t *__restrict_
                                                      const uint32_t *__restrict__ in_cols, uint64_t V,
                                                      const FrontierInfo *__restrict__ info,
                                                      const RoundCtl *__restrict__ ctl, uint32_t *val,
-                                                     uint8_t *__restrict__ flag, unsigned long long *upd) {
+                                                     uint8_t *__restrict__ flag, unsigned long long *spread) {
     if (!info->pull) return;
     const uint32_t L = ctl->rounds;
     uint32_t c = 0;
@@ -1035,7 +1084,7 @@ __global__ __launch_bounds__(kBlock) void k_bfs_pull(const uint64_t *__restrict_
             }
         }
     }
-    wave_add(upd, c);
+    wave_count(spread, kUpdStatic, c);
 }
 
 // Order-independent digest of a result array: the sum (mod 2^64) of
@@ -1046,8 +1095,8 @@ __device__ __forceinline__ uint64_t d_mix64(uint64_t z) {
     return z ^ (z >> 31);
 }
 
-// reached = #{v : val[v] != UNREACHED}, traversed = sum of their degrees,
-// checksum = digest of val.
+// counters[2..4]: reached = #{v : val[v] != UNREACHED}, traversed = sum of
+// their degrees, checksum = digest of val; folds the run's work counters.
 // deg / hdeg: the degree table (hdeg: heavy degrees with the split, else
 // null), or null for the row bounds.  With the table, each lane reads four
 // values and four degrees per 16-byte load.  Few, large workgroups
@@ -1058,7 +1107,8 @@ __global__ __launch_bounds__(kStatsBlock) void k_reach_stats(const uint32_t *__r
                                                         const uint64_t *__restrict__ ptr,
                                                         const uint32_t *__restrict__ deg,
                                                         const uint32_t *__restrict__ hdeg, uint64_t V,
-                                                        unsigned long long *out, RoundClock *clk) {
+                                                        unsigned long long *counters, unsigned long long *spread,
+                                                             RoundClock *clk) {
     __shared__ unsigned long long s_sum[3];
     if (threadIdx.x < 3) s_sum[threadIdx.x] = 0;
     clock_stamp(clk, kClkFront, kClkOther);
@@ -1109,7 +1159,8 @@ __global__ __launch_bounds__(kStatsBlock) void k_reach_stats(const uint32_t *__r
 #pragma unroll
         for (int i = 0; i < 3; ++i) atomicAdd(&s_sum[i], (unsigned long long)w[i]);
     __syncthreads();
-    if (threadIdx.x < 3 && s_sum[threadIdx.x]) atomicAdd(out + threadIdx.x, s_sum[threadIdx.x]);
+    if (threadIdx.x < 3 && s_sum[threadIdx.x]) atomicAdd(counters + 2 + threadIdx.x, s_sum[threadIdx.x]);
+    if (blockIdx.x == 0) fold_spread(spread, counters);
 }
 
 // ------------------------------------------------------- multi-source BFS
@@ -1237,12 +1288,15 @@ __global__ __launch_bounds__(kBlock) void k_ms_commit(uint8_t *__restrict__ flag
     if (threadIdx.x < kMsSums && s_sum[threadIdx.x]) part[(uint64_t)blockIdx.x * kMsSums + threadIdx.x] += s_sum[threadIdx.x];
 }
 
-// The sources' sums over the commit's workgroups.
+// The sources' sums over the commit's workgroups; folds the batch's work
+// counters.
 __global__ __launch_bounds__(1024) void k_ms_sum(const unsigned long long *__restrict__ part, uint32_t n,
-                                                 unsigned long long *out, RoundClock *clk) {
+                                                 unsigned long long *out, unsigned long long *counters,
+                                                 unsigned long long *spread, RoundClock *clk) {
     __shared__ uint64_t s[1024];
     clock_stamp(clk, kClkFront, kClkOther);
     const uint32_t col = blockIdx.x * kMsWidth + threadIdx.x % kMsWidth;
+    if (blockIdx.x == 0) fold_spread(spread, counters);
     uint64_t x = 0;
     for (uint32_t b = threadIdx.x / kMsWidth; b < n; b += 1024 / kMsWidth) x += part[(uint64_t)b * kMsSums + col];
     s[threadIdx.x] = x;
@@ -1395,6 +1449,8 @@ void frontier_alloc(DeviceState *d, const og_graph *g, Frontier &f, MemPool &m) 
     f.ctl = &f.blk->ctl;
     f.clk = &f.blk->clk;
     f.counters = f.blk->counters;
+    f.spread = (unsigned long long *)m.dalloc(kSpreadWords * 8);
+    OG_HIP(hipMemset(f.spread, 0, kSpreadWords * 8));
     f.h_info = (FrontierInfo *)m.palloc(sizeof(FrontierInfo));
     f.h_blk = (RunBlock *)m.palloc(sizeof(RunBlock));
     const uint64_t cap = std::max<uint64_t>(hub_capacity(g, d->plan.vsplit, d->tune), 1);
@@ -2079,7 +2135,7 @@ template <int ALGO, bool W, bool PK>
 static void launch_static_relax_fmt(DeviceState *d, Frontier &f, const FrontierInfo *hfi, const RelaxArgs &a,
                                     hipStream_t s) {
     const void *edges = d->d_static;
-    unsigned long long *upd = f.counters + 0;
+    unsigned long long *upd = f.spread;
     const uint32_t lpv0 = d->tune.lpv0;
     if (!hfi || hfi->n[0]) {
         const dim3 gr(hfi ? capped(((uint64_t)hfi->n[0] * lpv0 + kBlock - 1) / kBlock, kGroupGridCap) : kGroupGridCap);
@@ -2143,8 +2199,7 @@ static void launch_dyn(DeviceState *d, unsigned grid, const void *src, uint64_t 
                        d->fr.info, d->fr.doff, src, c0, c1, d->d_ptr, d->dyn_base, (const void *)d->d_staging,
                        DIRECT ? (const int64_t *)d->d_rdelta : nullptr, d->wbits, relax_args(d),
                        DIRECT ? (const uint64_t *)d->d_lpos : nullptr, d->split_nl, d->plan.vsplit,
-                       DIRECT && c0 == 0 ? (const uint32_t *)d->fr.dchunk : nullptr, DIRECT ? d->lbits : 0u, d->fr.counters + 1,
-                       d->fr.counters + 5);
+                       DIRECT && c0 == 0 ? (const uint32_t *)d->fr.dchunk : nullptr, DIRECT ? d->lbits : 0u, d->fr.spread);
 }
 
 // The fused round relax (k_relax_round) of a device-driven round on the
@@ -2180,7 +2235,7 @@ static void launch_round_fmt(DeviceState *d, bool with_dyn) {
     r.dchunk = d->fr.dchunk;
     r.nl = d->split_nl;
     r.vsplit = d->plan.vsplit;
-    r.counters = d->fr.counters;
+    r.spread = d->fr.spread;
     r.clk = d->fr.clk;
     const unsigned grid = (kFuseStatic + r.cd) * kHubGridCap;
     const size_t lds = std::max<size_t>(with_dyn ? sizeof(DynLds) : 0, (size_t)d->tune.tile * d->eb);
@@ -2213,7 +2268,7 @@ static void launch_srv_round_fmt(DeviceState *d, Frontier &f, const RelaxArgs &a
     r.hub_cap = f.hub_cap;
     r.tile = d->tune.tile;
     r.vsplit = d->plan.vsplit;
-    r.counters = f.counters;
+    r.spread = f.spread;
     SrvPull p{};
     if (pull) p = *pull;
     const uint32_t cp = pull ? kDynGridCap / kHubGridCap : 0;  // the separate pull's 8192 workgroups
@@ -2395,7 +2450,7 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
                     span(kClsStat, s, [&] {
                         hipLaunchKernelGGL(k_bfs_pull, dim3(capped((d->V + kBlock - 1) / kBlock, kGroupGridCap)),
                                            dim3(kBlock), 0, s, d->d_in_ptr, d->d_in_cols, d->V, d->fr.info,
-                                           d->fr.ctl, d->d_val, d->fr.flag, d->fr.counters + 0);
+                                           d->fr.ctl, d->d_val, d->fr.flag, d->fr.spread);
                         OG_HIP(hipGetLastError());
                     });
                 if (joined) OG_HIP(hipStreamWaitEvent(s, d->ev_static, 0));
@@ -2552,7 +2607,7 @@ static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats 
     Stopwatch total;
     auto begin = [&](const RoundCtl &c) {
         hipLaunchKernelGGL((k_run_init<ALGO == ALGO_CC>), dim3(fill_grid(d->Vpad / 4)), dim3(kBlock), 0, s, d->d_val,
-                           d->fr.flag, V, d->Vpad, src, d->fr.blk, c);
+                           d->fr.flag, V, d->Vpad, src, d->fr.blk, d->fr.spread, c);
         OG_HIP(hipGetLastError());
     };
     frontier_loop<ALGO, W>(g, d, st, tm, gather_ms, overload_wall, begin, [](RoundClock *) {}, true);
@@ -2560,7 +2615,7 @@ static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats 
     st.total_ms = total.ms();
 
     hipLaunchKernelGGL(k_reach_stats, dim3(stats_grid(V)), dim3(kStatsBlock), 0, s, d->d_val, d->d_ptr, d->d_deg,
-                       d->deg_heavy(), V, d->fr.counters + 2, tm.clocked >= 0 ? d->fr.clk : nullptr);
+                       d->deg_heavy(), V, d->fr.counters, d->fr.spread, tm.clocked >= 0 ? d->fr.clk : nullptr);
     OG_HIP(hipGetLastError());
     OG_HIP(hipMemcpyAsync(d->fr.h_blk, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
     if (out) copy_to_host(d, out, d->d_val, V * sizeof(uint32_t), s);
@@ -2610,6 +2665,7 @@ static void run_msbfs(og_graph *g, const uint32_t *sources, uint32_t n, uint32_t
     OG_HIP(hipStreamSynchronize(s));
     Stopwatch total;
     OG_HIP(hipMemsetAsync(d->fr.blk, 0, sizeof(RunBlock), s));
+    OG_HIP(hipMemsetAsync(d->fr.spread, 0, kSpreadWords * 8, s));
     double device_ms = 0;
     for (uint32_t b0 = 0; b0 < n; b0 += kMsWidth) {
         const uint32_t nb = std::min<uint32_t>(kMsWidth, n - b0);
@@ -2633,7 +2689,7 @@ static void run_msbfs(og_graph *g, const uint32_t *sources, uint32_t n, uint32_t
         };
         frontier_loop<ALGO_MSBFS, W>(g, d, st, tm, gather_ms, overload_wall, begin, commit, false, lvl != nullptr);
         hipLaunchKernelGGL(k_ms_sum, dim3(3), dim3(1024), 0, s, d->d_mpart, cgrid, d->d_msum,
-                           tm.clocked >= 0 ? d->fr.clk : nullptr);
+                           d->fr.counters, d->fr.spread, tm.clocked >= 0 ? d->fr.clk : nullptr);
         OG_HIP(hipGetLastError());
         OG_HIP(hipMemcpyAsync(hsum.data(), d->d_msum, kMsSums * 8, hipMemcpyDeviceToHost, s));
         OG_HIP(hipStreamSynchronize(s));
@@ -2713,9 +2769,9 @@ uint64_t lane_state_bytes(const og_graph *g) {
     // what lane_state_create and frontier_alloc request: values, flags (and
     // the heavy-round flags with the split), bin lists, degree prefix, the
     // (empty) dynamic chunk table, compaction totals, round summary, run
-    // block and hub tiles
+    // block, work counters and hub tiles
     return 4 * Vpad + Vpad * (d->d_pmid ? 2 : 1) + 4 * V + 8 * (V + 1) + 4 * 2 + 8 * totals_words(nblk) +
-           sizeof(FrontierInfo) + sizeof(RunBlock) + 8 * hub;
+           sizeof(FrontierInfo) + sizeof(RunBlock) + 8 * kSpreadWords + 8 * hub;
 }
 
 void lane_run_sssp(og_graph *g, DeviceState *lane, uint32_t src, uint32_t *out, og_run_stats *st) {
@@ -3183,7 +3239,8 @@ constexpr uint64_t kNaTot = kNaDoff + na_up(8 * 16);
 constexpr uint64_t kNaInfo = kNaTot + na_up(8 * totals_words(kNoAllocMaxBlk));
 constexpr uint64_t kNaCtl = kNaInfo + na_up(sizeof(FrontierInfo));
 constexpr uint64_t kNaCounters = kNaCtl + na_up(sizeof(RoundCtl));
-constexpr uint64_t kNoAllocScratchBytes = kNaCounters + na_up(16 * 8);
+constexpr uint64_t kNaSpread = kNaCounters + na_up(16 * 8);
+constexpr uint64_t kNoAllocScratchBytes = kNaSpread + na_up(8 * kSpreadWords);
 
 // The scratch memory of og_bfs_device_noalloc.  In host code `scratch` is a
 // stand-in for the symbol, not a device address: kernels get the address
@@ -3233,12 +3290,14 @@ static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t 
     FrontierInfo *info = (FrontierInfo *)(base + kNaInfo);
     RoundCtl *ctl = (RoundCtl *)(base + kNaCtl);
     unsigned long long *ctr = (unsigned long long *)(base + kNaCounters);
+    unsigned long long *spread = (unsigned long long *)(base + kNaSpread);
     const Tuning tn;  // default bins: the hub bound above assumes its t2 and tile
     static_assert(Tuning{}.t2 == 4096 && Tuning{}.tile == 2048, "hub capacity bound follows the default tuning");
     Stopwatch total;
     // clear what must start at zero: fill kernels (no memset nodes)
     hipLaunchKernelGGL(k_fill_u8, dim3(fill_grid(Vpad)), dim3(256), 0, s, flag, Vpad, (uint8_t)0);
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, (uint32_t *)ctr, (uint64_t)32, 0u);
+    static_assert(kNaSpread == kNaCounters + 16 * 8 + 128, "cleared together");
+    hipLaunchKernelGGL(k_fill_u32, dim3(16), dim3(256), 0, s, (uint32_t *)ctr, (uint64_t)(kNoAllocScratchBytes - kNaCounters) / 4, 0u);
     hipLaunchKernelGGL(k_fill_u32, dim3(fill_grid(V)), dim3(256), 0, s, d_levels, V, OG_UNREACHED);
     hipLaunchKernelGGL(k_set_source, dim3(1), dim3(1), 0, s, d_levels, flag, src);
     hipLaunchKernelGGL(k_ctl_set, dim3(1), dim3(1), 0, s, ctl, ctl_begin(V, 0, 0, 0, false));
@@ -3259,7 +3318,7 @@ static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t 
     r.tile = tn.tile;
     r.cd = 0;  // the whole graph is static: three bins in one launch
     r.vsplit = V;
-    r.counters = ctr;
+    r.spread = spread;
     const RelaxArgs a{d_levels, flag, nullptr, nullptr, 0, nullptr, nullptr};
     static_assert(Tuning{}.lpv0 == 8, "the relax below is instantiated for 8 lanes per bin-0 vertex");
     compact();
@@ -3278,7 +3337,7 @@ static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t 
     }
     const double ms = total.ms();
     hipLaunchKernelGGL(k_reach_stats, dim3(stats_grid(V)), dim3(kStatsBlock), 0, s, d_levels, d_ptr,
-                       (const uint32_t *)nullptr, (const uint32_t *)nullptr, V, ctr + 2, (RoundClock *)nullptr);
+                       (const uint32_t *)nullptr, (const uint32_t *)nullptr, V, ctr, spread, (RoundClock *)nullptr);
     OG_HIP(hipGetLastError());
     unsigned long long hc[16];
     OG_HIP(hipMemcpyAsync(hc, ctr, sizeof hc, hipMemcpyDeviceToHost, s));

@@ -225,6 +225,7 @@ struct Frontier {
     RoundCtl *ctl = nullptr;         // parts of blk
     unsigned long long *counters = nullptr;
     RoundClock *clk = nullptr;
+    unsigned long long *h_progress = nullptr;  // pinned, written by the device: compactions << 1 | ended
     unsigned long long *spread = nullptr;  // kSpreadWords: the relax kernels' counters on their way to blk
 };
 
@@ -403,8 +404,15 @@ struct DeviceState {
     unsigned long long *h_progress = nullptr;  // pinned, written by the device: iterations << 1 | done
     std::shared_ptr<void> pr_plan;   // PageRank rows and chunk ranges (pagerank.hip)
     std::shared_ptr<void> round_graph;  // captured batches of device-driven rounds (engine.hip)
-    void *h_out[2] = {nullptr, nullptr};  // pinned staging chunks of result copy-backs (copy_to_host)
-    hipEvent_t ev_out[2] = {nullptr, nullptr};
+    // result copy-backs (copy_to_host): pinned staging, a word per slab that the device writes once the slab
+    // is there, the number of the last copy and the threads that copy slabs out; chunks of larger results
+    char *h_out = nullptr;
+    size_t out_bytes = 0;
+    unsigned long long *h_out_flag = nullptr;
+    unsigned long long out_seq = 0;
+    std::unique_ptr<WorkerPool> out_pool;
+    void *h_chunk[2] = {nullptr, nullptr};
+    hipEvent_t ev_chunk[2] = {nullptr, nullptr};
     uint32_t last_pairs[8] = {};        // relax + compaction pairs of the last device-driven run, per algorithm
 
     MemPool mem;                     // device + pinned allocations of this preparation
@@ -658,14 +666,13 @@ inline double sum_ms(const TimedClass &c) {
 }
 
 // Waits until the device has raised the pinned word *p (which it writes with
-// system scope while it runs) to at least `want`, or the stream has drained.
+// system scope while it runs: count << 1 | ended) to at least `want` or to an
+// ended one, or the stream has drained.
 void wait_progress(const unsigned long long *p, unsigned long long want, hipStream_t s);
 
-// Copies n bytes of device memory at src to host memory at dst (pageable or
-// not) on stream s and returns when they are there.  Large copies go through
-// two pinned staging chunks: chunk k + 1 crosses the link while the host
-// threads copy chunk k out, instead of HIP's staged copy into pageable
-// memory (~10 GB/s on the box for a 64 MB result against ~50 for pinned).
+// Copies n bytes (a multiple of 4) of device memory at src (16-byte aligned) to
+// host memory at dst, pageable or not, on stream s and returns when they are
+// there.
 void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStream_t s);
 
 // Allocates a frontier (device buffers + pinned summaries) sized for the
@@ -695,7 +702,7 @@ void lane_run_sssp(og_graph *g, DeviceState *lane, uint32_t src, uint32_t *out, 
 // the round's mode.  clk (optional): the run's clock, which leaves `prev`.
 void frontier_compact(DeviceState *d, Frontier &f, hipStream_t s, const uint32_t *val = nullptr,
                       bool to_host = true, const uint64_t *pmid = nullptr, RoundClock *clk = nullptr,
-                      int prev = kClkOther);
+                      int prev = kClkOther, unsigned long long *progress = nullptr);
 
 
 // Launches the static-region relax of the bins for op ALGO.  The kernels

@@ -135,9 +135,11 @@ __global__ void k_totals_init(unsigned long long *t, uint64_t n) {
 // publishes the round's summary and advances the traversal state: statistics,
 // liveness, the BFS direction and, when the near set is empty but vertices
 // are held back, the near-far threshold (min held-back value + delta) for
-// the next compaction.
+// the next compaction.  progress (pinned host memory, or null): compactions so
+// far << 1 | traversal ended.
 __device__ __forceinline__ void compact_finish(const CompactTotals &ct, FrontierInfo *__restrict__ info,
-                                               uint64_t *__restrict__ doff, RoundCtl *__restrict__ ctl) {
+                                               uint64_t *__restrict__ doff, RoundCtl *__restrict__ ctl,
+                                               unsigned long long *progress) {
     const uint32_t lane = threadIdx.x;
     RoundCtl c = *ctl;
     uint64_t zf = 0, sd = 0, lh = 0, mf = ~0ull, a01 = 0, ath = 0, dyn = 0, wn = 0, wd = 0;
@@ -245,6 +247,9 @@ __device__ __forceinline__ void compact_finish(const CompactTotals &ct, Frontier
     else c.hold = c.defer == 1 && !was_heavy && active ? 1u : 0u;
     c.mode = heavy_next ? 1u : 0u;
     *ctl = c;
+    if (progress)
+        __hip_atomic_store(progress, (unsigned long long)c.compactions << 1 | (fi.live ? 0u : 1u), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Frontier compaction, one launch: flags -> bin lists, hub tiles, the dynamic
@@ -276,7 +281,8 @@ __global__ __launch_bounds__(kCompactBlock) void k_frontier_compact(
     const uint64_t *__restrict__ ptr, const uint64_t *__restrict__ pmid, const uint32_t *__restrict__ deg,
     const uint32_t *__restrict__ hdeg, Tuning tn, const uint32_t *__restrict__ val_a, RoundCtl *ctl, CompactTotals ct,
     FrontierInfo *__restrict__ info, uint32_t *__restrict__ list, uint64_t *__restrict__ hub, uint64_t hub_cap,
-    uint64_t *__restrict__ doff, uint32_t *__restrict__ dchunk, uint64_t dchunk_cap, RoundClock *clk, int clk_prev) {
+    uint64_t *__restrict__ doff, uint32_t *__restrict__ dchunk, uint64_t dchunk_cap, RoundClock *clk, int clk_prev,
+    unsigned long long *progress) {
     constexpr int kWaves = kCompactBlock / kWave;
     static_assert(NW * kWaves <= kWave, "one lane per (window, wave)");
     __shared__ uint64_t s_cnt[NW * kWaves], s_deg[NW * kWaves];  // per window and wave: packed counts, degrees
@@ -306,7 +312,7 @@ __global__ __launch_bounds__(kCompactBlock) void k_frontier_compact(
     if (!__syncthreads_or(any != 0)) {  // no flags here (most blocks in a small round)
         if (threadIdx.x < kWave) {
             const bool last = threadIdx.x == 0 && arrive_last(ct);
-            if (__ballot(last)) compact_finish(ct, info, doff, ctl);
+            if (__ballot(last)) compact_finish(ct, info, doff, ctl, progress);
         }
         return;
     }
@@ -519,7 +525,7 @@ __global__ __launch_bounds__(kCompactBlock) void k_frontier_compact(
         // (the word belongs to this thread alone)
         if (mark && hw) *(uint32_t *)(hflag + v0 + q * kWin) |= hw;
     }
-    if (wid == 0 && __ballot(last)) compact_finish(ct, info, doff, ctl);
+    if (wid == 0 && __ballot(last)) compact_finish(ct, info, doff, ctl, progress);
 }
 
 // Traversal state at the start: near-far width `delta` with the first
@@ -1338,7 +1344,8 @@ static unsigned fill_grid(uint64_t n) { return (unsigned)std::min<uint64_t>(8192
 
 void wait_progress(const unsigned long long *p, unsigned long long want, hipStream_t s) {
     for (uint64_t i = 1;; ++i) {
-        if (__atomic_load_n(p, __ATOMIC_ACQUIRE) >= want) return;
+        const unsigned long long now = __atomic_load_n(p, __ATOMIC_ACQUIRE);
+        if (now >= want || (now & 1)) return;
         if (i % 1024) {
             __builtin_ia32_pause();
             continue;
@@ -1366,40 +1373,77 @@ void device_state_free(DeviceState *d) {
     if (d->s_copy && d->s_copy != d->s_compute) (void)hipStreamDestroy(d->s_copy);
     if (d->s_static && d->s_static != d->s_compute) (void)hipStreamDestroy(d->s_static);
     if (d->s_compute) (void)hipStreamDestroy(d->s_compute);
+    for (hipEvent_t e : d->ev_chunk)
+        if (e) (void)hipEventDestroy(e);
     if (d->ev_static) (void)hipEventDestroy(d->ev_static);
     if (d->ev_fork) (void)hipEventDestroy(d->ev_fork);
-    for (hipEvent_t e : d->ev_out)
-        if (e) (void)hipEventDestroy(e);
     delete d;
 }
 
-constexpr size_t kOutChunk = 8u << 20;  // bytes per pinned staging chunk of a result copy-back
+// Result copy-backs up to kOutMax bytes: the device writes slabs of kOutSlab
+// bytes into pinned staging, one workgroup each, and raises the slab's flag; host
+// threads copy slabs out while later ones cross the link.  (A copy into pageable
+// memory goes through the runtime's own staging, a megabyte at a time with about
+// 70 us between: 4 MB 236 us, this way 145.)  Larger results go through two
+// pinned chunks that the copy engine fills in turn (64 MB: 47 GB/s, the slabs 44).
+constexpr size_t kOutSlab = 32u << 10;
+constexpr size_t kOutMax = 8u << 20;
+constexpr size_t kOutChunk = 8u << 20;
 
-void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStream_t s) {
-    if (n <= kOutChunk) {  // one chunk: nothing to overlap
-        OG_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, s));
-        OG_HIP(hipStreamSynchronize(s));
-        return;
+__global__ __launch_bounds__(kBlock) void k_export(const uint32_t *__restrict__ src, uint64_t nwords,
+                                                   uint32_t *__restrict__ dst, unsigned long long *flag,
+                                                   unsigned long long seq) {
+    constexpr uint32_t kWords = kOutSlab / 4, kPer = kWords / 4 / kBlock;
+    const uint64_t w0 = (uint64_t)blockIdx.x * kWords;
+    const uint32_t n = (uint32_t)min((uint64_t)kWords, nwords - w0);
+    const uint4 *from = (const uint4 *)(src + w0);
+    uint4 *to = (uint4 *)(dst + w0);
+    uint4 x[kPer];
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k)
+        if (threadIdx.x + k * kBlock < n / 4) x[k] = from[threadIdx.x + k * kBlock];
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k)
+        if (threadIdx.x + k * kBlock < n / 4) to[threadIdx.x + k * kBlock] = x[k];
+    if (threadIdx.x < n % 4) dst[w0 + n / 4 * 4 + threadIdx.x] = src[w0 + n / 4 * 4 + threadIdx.x];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag + blockIdx.x, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Pinned staging for results of n bytes (at most kOutMax).
+static void out_reserve(DeviceState *d, size_t n) {
+    const size_t want = (n + kOutSlab - 1) / kOutSlab * kOutSlab;
+    if (want > d->out_bytes) {
+        d->h_out = (char *)d->palloc(want);
+        d->out_bytes = want;
     }
-    if (!d->h_out[0]) {
-        for (auto &p : d->h_out) p = d->palloc(kOutChunk);
-        for (auto &e : d->ev_out) OG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (!d->h_out_flag) {
+        d->h_out_flag = (unsigned long long *)d->palloc(kOutMax / kOutSlab * sizeof(unsigned long long));
+        std::memset(d->h_out_flag, 0, kOutMax / kOutSlab * sizeof(unsigned long long));
+    }
+}
+
+static void copy_chunks_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStream_t s) {
+    if (!d->h_chunk[0]) {
+        for (auto &p : d->h_chunk) p = d->palloc(kOutChunk);
+        for (auto &e : d->ev_chunk) OG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
     if (!d->pool) d->pool.reset(new WorkerPool(d->host_threads));
     const size_t nch = (n + kOutChunk - 1) / kOutChunk;
     auto issue = [&](size_t k) {
         const size_t off = k * kOutChunk, len = std::min(kOutChunk, n - off);
-        OG_HIP(hipMemcpyAsync(d->h_out[k & 1], (const char *)src + off, len, hipMemcpyDeviceToHost, s));
-        OG_HIP(hipEventRecord(d->ev_out[k & 1], s));
+        OG_HIP(hipMemcpyAsync(d->h_chunk[k & 1], (const char *)src + off, len, hipMemcpyDeviceToHost, s));
+        OG_HIP(hipEventRecord(d->ev_chunk[k & 1], s));
     };
     issue(0);
     for (size_t k = 0; k < nch; ++k) {
         // chunk k + 1 reuses the buffer chunk k - 1 left: its host copy ended
         // in the previous iteration
         if (k + 1 < nch) issue(k + 1);
-        OG_HIP(hipEventSynchronize(d->ev_out[k & 1]));
+        OG_HIP(hipEventSynchronize(d->ev_chunk[k & 1]));
         const size_t off = k * kOutChunk, len = std::min(kOutChunk, n - off);
-        const char *from = (const char *)d->h_out[k & 1];
+        const char *from = (const char *)d->h_chunk[k & 1];
         char *to = (char *)dst + off;
         const unsigned T = d->pool->size();
         d->pool->run([&](unsigned t) {
@@ -1407,6 +1451,51 @@ void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStrea
             std::memcpy(to + a, from + a, b - a);
         });
     }
+}
+
+void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStream_t s) {
+    if (!n) return;
+    if (n > kOutMax) return copy_chunks_to_host(d, dst, src, n, s);
+    out_reserve(d, n);
+    const size_t slabs = (n + kOutSlab - 1) / kOutSlab;
+    const unsigned long long seq = ++d->out_seq;
+    hipLaunchKernelGGL(k_export, dim3((unsigned)slabs), dim3(kBlock), 0, s, (const uint32_t *)src, (uint64_t)(n / 4),
+                       (uint32_t *)d->h_out, d->h_out_flag, seq);
+    OG_HIP(hipGetLastError());
+    std::atomic<size_t> next{0}, copied{0};
+    std::atomic<bool> failed{false};
+    // thread 0 asks the stream now and then: a device error ends every wait
+    auto pause = [&](unsigned t, uint64_t spins) {
+        if (spins % 2048) {
+            __builtin_ia32_pause();
+            return;
+        }
+        if (t == 0) {
+            const hipError_t e = hipStreamQuery(s);
+            if (e != hipSuccess && e != hipErrorNotReady) failed.store(true);
+        }
+        std::this_thread::yield();
+    };
+    auto work = [&](unsigned t) {
+        for (size_t i = next.fetch_add(1); i < slabs; i = next.fetch_add(1)) {
+            for (uint64_t spins = 1; __atomic_load_n(d->h_out_flag + i, __ATOMIC_ACQUIRE) != seq; ++spins) {
+                if (failed.load(std::memory_order_relaxed)) return;
+                pause(t, spins);
+            }
+            const size_t off = i * kOutSlab;
+            std::memcpy((char *)dst + off, d->h_out + off, std::min(kOutSlab, n - off));
+            copied.fetch_add(1);
+        }
+        if (t == 0)
+            for (uint64_t spins = 1; copied.load() < slabs && !failed.load(); ++spins) pause(t, spins);
+    };
+    if (n > (256u << 10) && d->host_threads > 1) {
+        if (!d->out_pool) d->out_pool.reset(new WorkerPool(std::min(4u, d->host_threads)));
+        d->out_pool->run(work);
+    } else {
+        work(0);
+    }
+    if (failed.load()) OG_HIP(hipStreamSynchronize(s));
 }
 
 // Largest number of hub tiles any frontier can produce for the current tuning.
@@ -1453,6 +1542,7 @@ void frontier_alloc(DeviceState *d, const og_graph *g, Frontier &f, MemPool &m) 
     OG_HIP(hipMemset(f.spread, 0, kSpreadWords * 8));
     f.h_info = (FrontierInfo *)m.palloc(sizeof(FrontierInfo));
     f.h_blk = (RunBlock *)m.palloc(sizeof(RunBlock));
+    f.h_progress = (unsigned long long *)m.palloc(sizeof(unsigned long long));
     const uint64_t cap = std::max<uint64_t>(hub_capacity(g, d->plan.vsplit, d->tune), 1);
     f.hub = (uint64_t *)m.dalloc(cap * sizeof(uint64_t));
     f.hub_cap = cap;
@@ -1463,18 +1553,18 @@ void frontier_alloc(DeviceState *d, const og_graph *g, Frontier &f, MemPool &m) 
 }
 
 void frontier_compact(DeviceState *d, Frontier &f, hipStream_t s, const uint32_t *val, bool to_host,
-                      const uint64_t *pmid, RoundClock *clk, int prev) {
+                      const uint64_t *pmid, RoundClock *clk, int prev, unsigned long long *progress) {
     // the degree table (a split round needs its light and heavy parts)
     const uint32_t *deg = d->d_deg && (!pmid || d->deg_split) ? d->d_deg : nullptr;
     const uint32_t *hdeg = deg ? d->deg_heavy() : nullptr;
     if (f.nw == 1)
         hipLaunchKernelGGL(k_frontier_compact<1>, dim3(f.nblk), dim3(kCompactBlock), 0, s, f.flag, f.hflag, d->Vpad,
                            d->plan.vsplit, d->d_ptr, pmid, deg, hdeg, d->tune, val, f.ctl, f.totals(), f.info, f.list,
-                           f.hub, f.hub_cap, f.doff, f.dchunk, f.dchunk_cap, clk, prev);
+                           f.hub, f.hub_cap, f.doff, f.dchunk, f.dchunk_cap, clk, prev, progress);
     else
         hipLaunchKernelGGL(k_frontier_compact<4>, dim3(f.nblk), dim3(kCompactBlock), 0, s, f.flag, f.hflag, d->Vpad,
                            d->plan.vsplit, d->d_ptr, pmid, deg, hdeg, d->tune, val, f.ctl, f.totals(), f.info, f.list,
-                           f.hub, f.hub_cap, f.doff, f.dchunk, f.dchunk_cap, clk, prev);
+                           f.hub, f.hub_cap, f.doff, f.dchunk, f.dchunk_cap, clk, prev, progress);
     OG_HIP(hipGetLastError());
     if (to_host) OG_HIP(hipMemcpyAsync(f.h_info, f.info, sizeof(FrontierInfo), hipMemcpyDeviceToHost, s));
 }
@@ -1977,6 +2067,7 @@ static void prepare_impl(og_graph *g, og_approach approach, const og_plan_params
     d->d_val = (uint32_t *)d->dalloc(d->Vpad * sizeof(uint32_t));
     OG_HIP(hipStreamSynchronize(d->s_compute));
     frontier_alloc(d.get(), g, d->fr, d->mem);
+    if (V * sizeof(uint32_t) <= kOutMax) out_reserve(d.get(), V * sizeof(uint32_t));
     pl.device_bytes = d->device_bytes();
     if (info) *info = pl;
     g->dev = d.release();
@@ -2360,6 +2451,7 @@ constexpr uint64_t edge_bytes_alg() {
 }
 
 constexpr int kRoundBatch = 4;     // device-driven rounds enqueued per host check
+constexpr uint64_t kRoundsAhead = 2;  // rounds enqueued before the device has reached them (OG_PLAN_NO_GRAPH)
 constexpr int kRoundBatchMax = 64;  // largest first batch (sized from the previous run)
 
 // Iterates compaction -> static relax || dynamic relax -> after() until no
@@ -2424,7 +2516,9 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
         const bool clocked = fuse || fuse_static;
         RoundClock *const clk = clocked ? d->fr.clk : nullptr;
         const EagerSpan eager{d, tm};
-        auto first = [&] { frontier_compact(d, d->fr, s, nf_val, false, pm, clk, kClkOther); };
+        unsigned long long *const progress = clocked && (d->flags & OG_PLAN_NO_GRAPH) ? d->fr.h_progress : nullptr;
+        auto first = [&] { frontier_compact(d, d->fr, s, nf_val, false, pm, clk, kClkOther, progress); };
+        if (progress) __atomic_store_n(progress, 0ull, __ATOMIC_RELEASE);
         if (clocked) first();
         else eager(kClsFront, s, first);
         auto batch = [&](const auto &span, int rounds) {
@@ -2456,9 +2550,12 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
                 if (joined) OG_HIP(hipStreamWaitEvent(s, d->ev_static, 0));
                 after(clk);
                 span(kClsFront, s,
-                     [&] { frontier_compact(d, d->fr, s, nf_val, false, pm, clk, quiet_after ? kClkRelax : kClkOther); });
+                     [&] {
+                         frontier_compact(d, d->fr, s, nf_val, false, pm, clk, quiet_after ? kClkRelax : kClkOther,
+                                          progress);
+                     });
             }
-            OG_HIP(hipMemcpyAsync(h, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
+            if (!progress) OG_HIP(hipMemcpyAsync(h, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
         };
         const NoSpan untimed;
         auto enqueue = [&](const auto &span, int rounds) {
@@ -2496,6 +2593,15 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
             }
             // relax + compaction pairs of this run, for the next run's first batch
             d->last_pairs[ALGO] = h->ctl.compactions ? h->ctl.compactions - 1 : 0;
+        } else if (progress) {
+            // rounds are enqueued kRoundsAhead ahead of the device, which
+            // tells how far it is: no host round trip between rounds, and that
+            // many empty ones (about 8 us each) at the end
+            for (;; ++enqueued) {
+                if (enqueued >= kRoundsAhead) wait_progress(progress, (enqueued + 1 - kRoundsAhead) << 1, s);
+                if (__atomic_load_n(progress, __ATOMIC_ACQUIRE) & 1) break;
+                enqueue(untimed, 1);
+            }
         } else {
             for (;;) {
                 enqueue(eager, kRoundBatch);
@@ -2537,10 +2643,15 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
             }
             OG_HIP(hipStreamSynchronize(s));
         }
-        OG_HIP(hipMemcpyAsync(h, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
-        OG_HIP(hipStreamSynchronize(s));
     }
-    const RoundCtl c = h->ctl;
+}
+
+// Adds a traversal's statistics, whose run block is on the host.
+template <int ALGO, bool W>
+static void collect_loop(DeviceState *d, og_run_stats &st) {
+    const RoundCtl c = d->fr.h_blk->ctl;
+    const bool zero_copy = (d->flags & OG_PLAN_ZERO_COPY) != 0;
+    const bool has_dyn = d->plan.vsplit < d->V;
     if (c.overflow) raise(OG_EUNSUPPORTED, "multi-source BFS deeper than 254 levels");
     st.iterations += c.rounds;
     st.node_sum += c.node_sum;
@@ -2611,7 +2722,6 @@ static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats 
         OG_HIP(hipGetLastError());
     };
     frontier_loop<ALGO, W>(g, d, st, tm, gather_ms, overload_wall, begin, [](RoundClock *) {}, true);
-    OG_HIP(hipStreamSynchronize(s));
     st.total_ms = total.ms();
 
     hipLaunchKernelGGL(k_reach_stats, dim3(stats_grid(V)), dim3(kStatsBlock), 0, s, d->d_val, d->d_ptr, d->d_deg,
@@ -2620,6 +2730,7 @@ static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats 
     OG_HIP(hipMemcpyAsync(d->fr.h_blk, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
     if (out) copy_to_host(d, out, d->d_val, V * sizeof(uint32_t), s);
     OG_HIP(hipStreamSynchronize(s));
+    collect_loop<ALGO, W>(d, st);
     st.reached = d->fr.h_blk->counters[2];
     st.traversed_edges = d->fr.h_blk->counters[3];
     st.checksum = d->fr.h_blk->counters[4];
@@ -2691,9 +2802,11 @@ static void run_msbfs(og_graph *g, const uint32_t *sources, uint32_t n, uint32_t
         hipLaunchKernelGGL(k_ms_sum, dim3(3), dim3(1024), 0, s, d->d_mpart, cgrid, d->d_msum,
                            d->fr.counters, d->fr.spread, tm.clocked >= 0 ? d->fr.clk : nullptr);
         OG_HIP(hipGetLastError());
+        OG_HIP(hipMemcpyAsync(d->fr.h_blk, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
         OG_HIP(hipMemcpyAsync(hsum.data(), d->d_msum, kMsSums * 8, hipMemcpyDeviceToHost, s));
         OG_HIP(hipStreamSynchronize(s));
         device_ms = total.ms();
+        collect_loop<ALGO_MSBFS, W>(d, st);
         for (uint32_t j = 0; j < nb; ++j) {
             if (checksums) checksums[b0 + j] = hsum[j];
             if (reached) reached[b0 + j] = hsum[kMsWidth + j];
@@ -2712,8 +2825,7 @@ static void run_msbfs(og_graph *g, const uint32_t *sources, uint32_t n, uint32_t
             }
     }
     st.total_ms = device_ms;
-    OG_HIP(hipMemcpyAsync(d->fr.h_blk, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
-    OG_HIP(hipStreamSynchronize(s));
+    if (!n) *d->fr.h_blk = RunBlock{};
     finish_stats(st, tm, gather_ms, overload_wall, d, 9);
     if (stats) *stats = st;
 }
@@ -3306,7 +3418,7 @@ static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t 
         hipLaunchKernelGGL(k_frontier_compact<1>, dim3(nblk), dim3(kCompactBlock), 0, s, flag, (uint8_t *)nullptr, Vpad, V,
                            d_ptr, (const uint64_t *)nullptr, (const uint32_t *)nullptr, (const uint32_t *)nullptr, tn,
                            (const uint32_t *)nullptr, ctl, ct, info, list, hub, kNoAllocHubCap, doff,
-                           (uint32_t *)nullptr, (uint64_t)0, (RoundClock *)nullptr, (int)kClkOther);
+                           (uint32_t *)nullptr, (uint64_t)0, (RoundClock *)nullptr, (int)kClkOther, (unsigned long long *)nullptr);
     };
     RoundRelax r{};
     r.list = list;

@@ -6,6 +6,7 @@
 
 #include <chrono>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "og_internal.h"
@@ -294,6 +295,23 @@ struct MemPool {
     }
 };
 
+// What result copy-backs go through (copy_to_host): pinned staging, a word per
+// slab that the device writes once the slab is there, and threads that copy
+// slabs out.  Shared by every preparation of the process and given back with the
+// last of them: a new graph's first result would otherwise wait for the threads
+// to start and for the link's page tables to learn 4 MB of new staging (about
+// 0.75 ms).  One copy uses it at a time; another that finds it taken goes
+// through the runtime.
+struct OutStage {
+    std::mutex use;
+    char *buf = nullptr;
+    size_t bytes = 0;
+    unsigned long long *flag = nullptr;
+    unsigned long long seq = 0;
+    std::unique_ptr<WorkerPool> pool;
+    ~OutStage();
+};
+
 // PageRank's scalars on the device: what an iteration leaves for the next.
 struct PrState {
     double dangling;      // rank mass of the vertices without out-edges
@@ -404,13 +422,8 @@ struct DeviceState {
     unsigned long long *h_progress = nullptr;  // pinned, written by the device: iterations << 1 | done
     std::shared_ptr<void> pr_plan;   // PageRank rows and chunk ranges (pagerank.hip)
     std::shared_ptr<void> round_graph;  // captured batches of device-driven rounds (engine.hip)
-    // result copy-backs (copy_to_host): pinned staging, a word per slab that the device writes once the slab
-    // is there, the number of the last copy and the threads that copy slabs out; chunks of larger results
-    char *h_out = nullptr;
-    size_t out_bytes = 0;
-    unsigned long long *h_out_flag = nullptr;
-    unsigned long long out_seq = 0;
-    std::unique_ptr<WorkerPool> out_pool;
+    std::shared_ptr<OutStage> out;        // result copy-backs up to kOutMax bytes
+    // and the two chunks of larger ones
     void *h_chunk[2] = {nullptr, nullptr};
     hipEvent_t ev_chunk[2] = {nullptr, nullptr};
     uint32_t last_pairs[8] = {};        // relax + compaction pairs of the last device-driven run, per algorithm

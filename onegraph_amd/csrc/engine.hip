@@ -1411,17 +1411,49 @@ __global__ __launch_bounds__(kBlock) void k_export(const uint32_t *__restrict__ 
     if (threadIdx.x == 0) __hip_atomic_store(flag + blockIdx.x, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Pinned staging for results of n bytes (at most kOutMax).
-static void out_reserve(DeviceState *d, size_t n) {
-    const size_t want = (n + kOutSlab - 1) / kOutSlab * kOutSlab;
-    if (want > d->out_bytes) {
-        d->h_out = (char *)d->palloc(want);
-        d->out_bytes = want;
+constexpr size_t kOutAlone = 256u << 10;  // results up to here are copied out by the calling thread alone
+
+OutStage::~OutStage() {
+    pool.reset();
+    if (buf) (void)hipHostFree(buf);
+    if (flag) (void)hipHostFree(flag);
+}
+
+// The staging, ready for results of n bytes (at most kOutMax) unless it is in
+// use (then it stays as it is).
+static std::shared_ptr<OutStage> out_stage(size_t n) {
+    static std::mutex mu;
+    static std::weak_ptr<OutStage> shared;
+    std::shared_ptr<OutStage> o;
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        o = shared.lock();
+        if (!o) shared = o = std::make_shared<OutStage>();
     }
-    if (!d->h_out_flag) {
-        d->h_out_flag = (unsigned long long *)d->palloc(kOutMax / kOutSlab * sizeof(unsigned long long));
-        std::memset(d->h_out_flag, 0, kOutMax / kOutSlab * sizeof(unsigned long long));
+    std::unique_lock<std::mutex> use(o->use, std::try_to_lock);
+    if (!use.owns_lock()) return o;
+    const size_t want = n <= kOutAlone ? kOutAlone : kOutMax;
+    if (want > o->bytes) {
+        char *p = nullptr;
+        if (hipHostMalloc((void **)&p, want, hipHostMallocDefault) != hipSuccess || !p) {
+            (void)hipGetLastError();
+            raise(OG_ENOMEM_HOST, "pinned host allocation of %zu bytes failed", want);
+        }
+        if (o->buf) (void)hipHostFree(o->buf);
+        o->buf = p;
+        o->bytes = want;
     }
+    if (!o->flag) {
+        const size_t fb = kOutMax / kOutSlab * sizeof(unsigned long long);
+        if (hipHostMalloc((void **)&o->flag, fb, hipHostMallocDefault) != hipSuccess || !o->flag) {
+            (void)hipGetLastError();
+            o->flag = nullptr;
+            raise(OG_ENOMEM_HOST, "pinned host allocation of %zu bytes failed", fb);
+        }
+        std::memset(o->flag, 0, fb);
+    }
+    if (n > kOutAlone && !o->pool) o->pool.reset(new WorkerPool(std::min(4u, default_threads())));
+    return o;
 }
 
 static void copy_chunks_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStream_t s) {
@@ -1456,11 +1488,18 @@ static void copy_chunks_to_host(DeviceState *d, void *dst, const void *src, size
 void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStream_t s) {
     if (!n) return;
     if (n > kOutMax) return copy_chunks_to_host(d, dst, src, n, s);
-    out_reserve(d, n);
+    if (!d->out || d->out->bytes < n) d->out = out_stage(n);
+    OutStage &o = *d->out;
+    std::unique_lock<std::mutex> use(o.use, std::try_to_lock);
+    if (!use.owns_lock() || o.bytes < n) {
+        OG_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, s));
+        OG_HIP(hipStreamSynchronize(s));
+        return;
+    }
     const size_t slabs = (n + kOutSlab - 1) / kOutSlab;
-    const unsigned long long seq = ++d->out_seq;
+    const unsigned long long seq = ++o.seq;
     hipLaunchKernelGGL(k_export, dim3((unsigned)slabs), dim3(kBlock), 0, s, (const uint32_t *)src, (uint64_t)(n / 4),
-                       (uint32_t *)d->h_out, d->h_out_flag, seq);
+                       (uint32_t *)o.buf, o.flag, seq);
     OG_HIP(hipGetLastError());
     std::atomic<size_t> next{0}, copied{0};
     std::atomic<bool> failed{false};
@@ -1478,23 +1517,19 @@ void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStrea
     };
     auto work = [&](unsigned t) {
         for (size_t i = next.fetch_add(1); i < slabs; i = next.fetch_add(1)) {
-            for (uint64_t spins = 1; __atomic_load_n(d->h_out_flag + i, __ATOMIC_ACQUIRE) != seq; ++spins) {
+            for (uint64_t spins = 1; __atomic_load_n(o.flag + i, __ATOMIC_ACQUIRE) != seq; ++spins) {
                 if (failed.load(std::memory_order_relaxed)) return;
                 pause(t, spins);
             }
             const size_t off = i * kOutSlab;
-            std::memcpy((char *)dst + off, d->h_out + off, std::min(kOutSlab, n - off));
+            std::memcpy((char *)dst + off, o.buf + off, std::min(kOutSlab, n - off));
             copied.fetch_add(1);
         }
         if (t == 0)
             for (uint64_t spins = 1; copied.load() < slabs && !failed.load(); ++spins) pause(t, spins);
     };
-    if (n > (256u << 10) && d->host_threads > 1) {
-        if (!d->out_pool) d->out_pool.reset(new WorkerPool(std::min(4u, d->host_threads)));
-        d->out_pool->run(work);
-    } else {
-        work(0);
-    }
+    if (n > kOutAlone && o.pool) o.pool->run(work);
+    else work(0);
     if (failed.load()) OG_HIP(hipStreamSynchronize(s));
 }
 
@@ -2067,7 +2102,7 @@ static void prepare_impl(og_graph *g, og_approach approach, const og_plan_params
     d->d_val = (uint32_t *)d->dalloc(d->Vpad * sizeof(uint32_t));
     OG_HIP(hipStreamSynchronize(d->s_compute));
     frontier_alloc(d.get(), g, d->fr, d->mem);
-    if (V * sizeof(uint32_t) <= kOutMax) out_reserve(d.get(), V * sizeof(uint32_t));
+    if (V * sizeof(uint32_t) <= kOutMax) d->out = out_stage(V * sizeof(uint32_t));
     pl.device_bytes = d->device_bytes();
     if (info) *info = pl;
     g->dev = d.release();

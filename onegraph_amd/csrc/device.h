@@ -295,6 +295,30 @@ struct MemPool {
     }
 };
 
+// The dynamic region as chunks of whole rows that cross the link in vertex
+// order, straight from the host copy (no gather), through a ring of `ring`
+// slots of `slot` words in the staging share: PageRank's iterations, and rounds
+// of the copy loader that relax much of the region.
+struct LinkRing {
+    struct Chunk {
+        uint32_t va, vb;       // vertices
+        uint64_t word, words;  // of the host source
+        uint32_t first;        // bits before the first edge
+        uint64_t tab = 0;      // its entries in DeviceState::d_ring_tab
+    };
+    std::vector<Chunk> chunks;
+    uint32_t ring = 0;
+    uint32_t lbits = 0;        // bits per edge on the link, 0: whole edges
+    uint64_t slot = 0;
+    uint64_t maxrow = 0;       // edges of the longest row
+    const uint32_t *src = nullptr;
+    std::vector<hipEvent_t> ev_h2d, ev_use;  // copy into / use of the slot finished
+    ~LinkRing() {
+        for (hipEvent_t e : ev_h2d) (void)hipEventDestroy(e);
+        for (hipEvent_t e : ev_use) (void)hipEventDestroy(e);
+    }
+};
+
 // What result copy-backs go through (copy_to_host): pinned staging, a word per
 // slab that the device writes once the slab is there, and threads that copy
 // slabs out.  Shared by every preparation of the process and given back with the
@@ -370,6 +394,9 @@ struct DeviceState {
     uint32_t lbits = 0;
     const uint32_t *h_link = nullptr;   // pinned
     const void *hd_link = nullptr;      // the same, as a device address
+    std::shared_ptr<LinkRing> link_ring;  // built on first use
+    uint8_t *d_mark = nullptr;       // V: vertices a ring round relaxes (zero between rounds)
+    uint32_t *d_ring_tab = nullptr;  // rows of the ring chunks' workgroups (k_relax_range)
     uint64_t dyn_resident = 0;       // zero-copy: dynamic edges held in d_staging (whole chunks)
     int64_t *d_rdelta = nullptr;     // zero-copy: per chunk of kResChunk vertices (index v >> kResChunkShift),
                                      // d_staging index - host-array position, or kNotResident; two per
@@ -682,6 +709,9 @@ inline double sum_ms(const TimedClass &c) {
 // system scope while it runs: count << 1 | ended) to at least `want` or to an
 // ended one, or the stream has drained.
 void wait_progress(const unsigned long long *p, unsigned long long want, hipStream_t s);
+
+// The preparation's chunk ring, or null when a row does not fit a slot.
+LinkRing *link_ring(DeviceState *d, const og_graph *g);
 
 // Copies n bytes (a multiple of 4) of device memory at src (16-byte aligned) to
 // host memory at dst, pageable or not, on stream s and returns when they are

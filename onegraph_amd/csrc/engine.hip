@@ -945,6 +945,72 @@ __global__ __launch_bounds__(kBlock) void k_relax_dyn(const uint32_t *__restrict
     if (DIRECT) wave_count(spread, kHbmEdges, h);
 }
 
+// Marks the dynamic list's vertices for k_relax_range (or unmarks them).
+__global__ void k_mark(const uint32_t *__restrict__ dlist, uint32_t n, uint8_t *__restrict__ mark, uint8_t x) {
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) mark[dlist[i]] = x;
+}
+
+// Ring chunk of a dynamic round: relaxes the edges [e0, e1) whose source is
+// marked.  The chunk's whole rows sit in `stage` (whole edges, or with lbits a
+// stream of lbits-bit words from bit `first` on).  Edge-parallel like
+// relax_dyn_body: a workgroup takes kDynEdgesPerBlock consecutive edges, whose
+// rows `tab` (the vertex of each workgroup's first edge, and of the chunk's
+// last) bounds, and finds an edge's row by binary search, in LDS unless empty
+// rows make the slice too long.  A chunk holds some 10^5 edges, so what bounds
+// it is the longest chain of dependent reads (rows by groups of lanes, long rows
+// by workgroups: 40-160 us per chunk of 660 K edges, this way 17-35).
+struct RangeLds {
+    uint64_t off[kDynEdgesPerBlock + 2];
+};
+template <int ALGO, bool W, bool PK>
+__global__ __launch_bounds__(kBlock) void k_relax_range(uint64_t e0, uint64_t e1, const uint32_t *__restrict__ tab,
+                                                        const FrontierInfo *__restrict__ info,
+                                                        const uint64_t *__restrict__ ptr,
+                                                        const uint32_t *__restrict__ stage, uint32_t lbits,
+                                                        uint32_t first, const uint8_t *__restrict__ mark, RelaxArgs a,
+                                                        unsigned long long *spread) {
+    __shared__ RangeLds L;
+    const bool heavy = info->heavy != 0;
+    const uint64_t x0 = e0 + (uint64_t)blockIdx.x * kDynEdgesPerBlock, x1 = min(x0 + kDynEdgesPerBlock, e1);
+    const uint32_t u0 = tab[blockIdx.x], nv = tab[blockIdx.x + 1] - u0 + 1;
+    const bool local = nv <= kDynEdgesPerBlock + 1;
+    if (local)
+        for (uint32_t k = threadIdx.x; k <= nv; k += kBlock) L.off[k] = ptr[(uint64_t)u0 + k];
+    __syncthreads();
+    uint32_t to[kDynEdgesPerThread], wt[kDynEdgesPerThread], ok = 0;
+    typename SrcOf<ALGO>::T sv[kDynEdgesPerThread], seen[kDynEdgesPerThread];
+#pragma unroll
+    for (int j = 0; j < kDynEdgesPerThread; ++j) {
+        const uint64_t x = x0 + threadIdx.x + (uint64_t)j * kBlock;
+        to[j] = 0;
+        wt[j] = 0;
+        sv[j] = 0;
+        seen[j] = 0;
+        if (x >= x1) continue;
+        uint32_t lo = 0, hi = nv;  // largest row that starts at or before x
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if ((local ? L.off[mid] : ptr[(uint64_t)u0 + mid]) <= x) lo = mid; else hi = mid;
+        }
+        const uint32_t u = u0 + lo;
+        if (!mark[u] || (a.pmid && (x >= a.pmid[u]) != heavy)) continue;
+        sv[j] = load_src<ALGO>(a, u);
+        ok |= 1u << j;
+        if (lbits) {
+            const uint32_t w = link_word(stage, x - e0, lbits, first);
+            to[j] = W ? w >> a.wbits : w;
+            wt[j] = W ? w & ((1u << a.wbits) - 1u) : 1u;
+        } else {
+            load_edge<W, PK>(stage, x - e0, a.wbits, to[j], wt[j]);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kDynEdgesPerThread; ++j)
+        if ((ok >> j) & 1) seen[j] = peek<ALGO>(a, to[j]);
+    const uint32_t c = commit<ALGO, kDynEdgesPerThread>(a, [&](int j) { return sv[j]; }, to, wt, seen, ok);
+    wave_count(spread, kUpdDynamic, c);
+}
+
 // One round's relax in a single launch: static bins 0 and 1, hub tiles and
 // the zero-copy dynamic region side by side, so a device-driven round needs
 // no second stream (the fork and join of which cost tens of microseconds per
@@ -1802,6 +1868,48 @@ static void stage_resident(DeviceState *d, const og_graph *g, uint64_t vsplit, u
     OG_HIP(hipStreamSynchronize(d->s_compute));
 }
 
+// Slots of the chunk ring: small enough that a few are on their way while
+// others are used, large enough that a copy takes longer than its hand-over
+// (4 MiB: 73 us on the link).
+constexpr uint64_t kRingSlotBytes = 4ull << 20;
+constexpr uint32_t kRing = 8;
+
+LinkRing *link_ring(DeviceState *d, const og_graph *g) {
+    if (d->link_ring) return d->link_ring->ring ? d->link_ring.get() : nullptr;
+    auto r = std::make_shared<LinkRing>();
+    d->link_ring = r;
+    const uint64_t vs = d->plan.vsplit, base = d->dyn_base;
+    for (uint64_t v = vs; v < d->V; ++v) r->maxrow = std::max(r->maxrow, g->ptr[v + 1] - g->ptr[v]);
+    if (r->maxrow > d->slot_edges) return nullptr;
+    const uint64_t total = (uint64_t)d->nslots * d->slot_edges * d->eb / 4;  // words of the staging share
+    // the link format's rows start anywhere in a word and are read eight bytes
+    // at a time, so it takes slots of a few words more
+    r->lbits = d->lbits && (r->maxrow * d->lbits + 31) / 32 + 2 <= total / 2 ? d->lbits : 0;
+    const uint64_t bits = r->lbits ? r->lbits : 8 * d->eb;
+    auto words_of = [&](uint64_t n) { return (n * bits + 31) / 32 + (r->lbits ? 2 : 0); };
+    uint32_t ring = (uint32_t)std::min<uint64_t>(kRing, std::max<uint64_t>(2, total * 4 / kRingSlotBytes));
+    while (ring > 2 && total / ring < words_of(r->maxrow)) --ring;
+    r->slot = total / ring;
+    r->src = r->lbits ? d->h_link : (const uint32_t *)d->h_dyn;
+    for (uint64_t va = vs; va < d->V;) {
+        uint64_t lo = va + 1, hi = d->V;
+        while (lo < hi) {  // largest vb whose rows fit
+            const uint64_t mid = (lo + hi + 1) / 2;
+            if (words_of(g->ptr[mid] - g->ptr[va]) <= r->slot) lo = mid; else hi = mid - 1;
+        }
+        const uint64_t b0 = (g->ptr[va] - base) * bits, b1 = (g->ptr[lo] - base) * bits;
+        const uint64_t w0 = b0 / 32, w1 = (b1 + 31) / 32 + (r->lbits && b1 > b0 ? 1 : 0);
+        r->chunks.push_back({(uint32_t)va, (uint32_t)lo, w0, b1 > b0 ? w1 - w0 : 0, (uint32_t)(b0 % 32)});
+        va = lo;
+    }
+    r->ev_h2d.assign(ring, nullptr);
+    r->ev_use.assign(ring, nullptr);
+    for (auto &e : r->ev_h2d) OG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    for (auto &e : r->ev_use) OG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    r->ring = ring;
+    return r.get();
+}
+
 // Link format of the dynamic region (DeviceState::lbits): packs the host
 // layout's words `src` into a pinned stream of lbits-bit words, when they are
 // narrow enough.  Edge targets need the bits of V - 1, weighted words wbits
@@ -2061,7 +2169,7 @@ static void prepare_impl(og_graph *g, og_approach approach, const og_plan_params
                 stage_resident(d.get(), g, pl.vsplit, pl.staging_edges, lpos);
             }
             // (a weighted graph that is not packed keeps its 8-byte edges)
-            if ((zc || g->kind == OG_KIND_PULL) && (g->kind != OG_KIND_WEIGHTED || d->packed))
+            if (g->kind != OG_KIND_WEIGHTED || d->packed)
                 pack_link(d.get(), g, (const uint32_t *)d->h_dyn, nd);
         }
     }
@@ -2223,7 +2331,7 @@ static void gather(DeviceState *d, const og_graph *g, uint32_t ndyn, uint64_t c0
     const unsigned T = d->pool->size();
     const unsigned use = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(T, n / 16384));
     const uint64_t L = (n + use - 1) / use;
-    d->pool->run([&](unsigned t) {
+    auto part = [&](unsigned t) {
         if (t >= use) return;
         const uint64_t p0 = c0 + (uint64_t)t * L;
         const uint64_t p1 = std::min(c1, p0 + L);
@@ -2239,7 +2347,9 @@ static void gather(DeviceState *d, const og_graph *g, uint32_t ndyn, uint64_t c0
             p = stop;
             ++i;
         }
-    });
+    };
+    if (use == 1) part(0);  // (waking the pool takes longer than this copy)
+    else d->pool->run(part);
 }
 
 static RelaxArgs relax_args(DeviceState *d) {
@@ -2435,6 +2545,86 @@ static void launch_dyn_any(DeviceState *d, const void *src, uint64_t c0, uint64_
     OG_HIP(hipGetLastError());
 }
 
+// A dynamic round of the copy loader that relaxes much of the region: its rows
+// cross the link whole, in vertex order, through the chunk ring, and the relax
+// picks the active ones.  Against the gather, which the host's threads build at
+// about 16 GB/s and a list and prefix copied back first, it moves the rest of the
+// region too, at the link's speed and in the link format: it pays from about
+// kRingShare of the region's edges on.  (BFS R-MAT 1 M, a quarter of the edges on
+// the device: 4.4 -> 3.0 ms.)  False: not such a round, or a row is too long.
+constexpr double kRingShare = 0.125;
+
+template <int ALGO, bool W>
+static bool run_ring(DeviceState *d, const og_graph *g, const FrontierInfo &fi, RunTimers &tm, og_run_stats &st) {
+    if ((d->flags & OG_PLAN_NO_OVERLAP) || (double)fi.dyn_deg < kRingShare * (double)(g->E - d->dyn_base)) return false;
+    LinkRing *lr = link_ring(d, g);
+    if (!lr) return false;
+    hipStream_t s = d->s_compute;
+    if (!d->d_mark) {
+        d->d_mark = (uint8_t *)d->dalloc(d->V);
+        hipLaunchKernelGGL(k_fill_u8, dim3(fill_grid(d->V)), dim3(256), 0, s, d->d_mark, d->V, (uint8_t)0);
+        // per chunk, the row of every kDynEdgesPerBlock-th edge and of the last
+        std::vector<uint32_t> tab;
+        for (LinkRing::Chunk &ch : lr->chunks) {
+            ch.tab = tab.size();
+            const uint64_t a0 = g->ptr[ch.va], a1 = g->ptr[ch.vb];
+            uint64_t v = ch.va;
+            for (uint64_t x = a0; x < a1; x += kDynEdgesPerBlock) {
+                while (g->ptr[v + 1] <= x) ++v;
+                tab.push_back((uint32_t)v);
+            }
+            if (a1 > a0) {
+                while (g->ptr[v + 1] < a1) ++v;
+                tab.push_back((uint32_t)v);
+            }
+        }
+        d->d_ring_tab = (uint32_t *)d->dalloc(std::max<size_t>(tab.size(), 1) * 4);
+        OG_HIP(hipMemcpy(d->d_ring_tab, tab.data(), tab.size() * 4, hipMemcpyHostToDevice));
+    }
+    const uint32_t *dlist = d->fr.list + d->plan.vsplit;
+    hipLaunchKernelGGL(k_mark, dim3(fill_grid(fi.n[3])), dim3(256), 0, s, dlist, fi.n[3], d->d_mark, (uint8_t)1);
+    OG_HIP(hipGetLastError());
+    const uint64_t nc = lr->chunks.size();
+    auto copy = [&](uint64_t k) {  // consecutive copies on two streams: one's hand-over hides behind the other
+        const LinkRing::Chunk &ch = lr->chunks[k];
+        const uint32_t slot = (uint32_t)(k % lr->ring);
+        const hipStream_t on = k & 1 ? d->s_static : d->s_copy;
+        if (k >= lr->ring) OG_HIP(hipStreamWaitEvent(on, lr->ev_use[slot], 0));
+        if (ch.words)
+            OG_HIP(hipMemcpyAsync((uint32_t *)d->d_staging + slot * lr->slot, lr->src + ch.word, ch.words * 4,
+                                  hipMemcpyHostToDevice, on));
+        OG_HIP(hipEventRecord(lr->ev_h2d[slot], on));
+        st.h2d_bytes += ch.words * 4;
+        st.chunks++;
+    };
+    // one pair of events per round: a pair per chunk stalls the stream as long
+    // as the chunk's copy takes
+    EventSpan copies(d, &tm.copy, d->s_copy), relaxes(d, &tm.dyn, s);
+    uint64_t copied = 0;
+    while (copied < std::min<uint64_t>(lr->ring, nc)) copy(copied++);
+    for (uint64_t k = 0; k < nc; ++k) {
+        const LinkRing::Chunk &ch = lr->chunks[k];
+        const uint32_t slot = (uint32_t)(k % lr->ring);
+        const uint32_t *stage = (const uint32_t *)d->d_staging + slot * lr->slot;
+        const uint64_t e0 = g->ptr[ch.va], e1 = g->ptr[ch.vb];
+        const unsigned grid = (unsigned)((e1 - e0 + kDynEdgesPerBlock - 1) / kDynEdgesPerBlock);
+        OG_HIP(hipStreamWaitEvent(s, lr->ev_h2d[slot], 0));
+        auto relax = [&](auto kernel) {
+            if (grid)
+                hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), 0, s, e0, e1, d->d_ring_tab + ch.tab, d->fr.info,
+                                   d->d_ptr, stage, lr->lbits, ch.first, d->d_mark, relax_args(d), d->fr.spread);
+        };
+        if (W && d->packed) relax(k_relax_range<ALGO, W, true>);
+        else relax(k_relax_range<ALGO, W, false>);
+        OG_HIP(hipGetLastError());
+        OG_HIP(hipEventRecord(lr->ev_use[slot], s));
+        if (copied < nc) copy(copied++);
+    }
+    hipLaunchKernelGGL(k_mark, dim3(fill_grid(fi.n[3])), dim3(256), 0, s, dlist, fi.n[3], d->d_mark, (uint8_t)0);
+    OG_HIP(hipGetLastError());
+    return true;
+}
+
 // Staged dynamic region of a round whose summary the host holds: the host
 // gathers the active edges into pinned slots and the copy stream moves them
 // while the other slot is relaxed.
@@ -2444,6 +2634,7 @@ static void run_dynamic(DeviceState *d, const og_graph *g, const FrontierInfo &f
     const uint32_t ndyn = fi.n[3];
     const uint64_t D = fi.dyn_deg;
     if (!ndyn || !D) return;
+    if (run_ring<ALGO, W>(d, g, fi, tm, st)) return;
     const uint32_t *d_dlist = d->fr.list + d->plan.vsplit;
     const uint64_t eb = d->deb;
     OG_HIP(hipMemcpyAsync(d->h_dlist, d_dlist, (size_t)ndyn * 4, hipMemcpyDeviceToHost, d->s_copy));

@@ -303,23 +303,7 @@ namespace {
 struct PrPlan {
     uint32_t n0 = 0, n1 = 0, nh = 0;  // static rows: up to t1, up to t2, hubs
     unsigned g0 = 0, g1 = 0;          // workgroups of the first two
-    // The dynamic region crosses the link in chunks of whole rows through a
-    // ring of `ring` slots of `slot` words, all in the staging share.
-    struct Chunk {
-        uint32_t va, vb;
-        uint64_t word, words;  // of the host source
-        uint32_t first;        // bits before the first edge
-    };
-    std::vector<Chunk> chunks;
-    uint32_t ring = 0;
-    uint32_t lbits = 0;  // bits per edge on the link, 0: whole ids
-    uint64_t slot = 0;
-    const uint32_t *src = nullptr;
-    std::vector<hipEvent_t> ev_h2d, ev_pull;  // copy into / pull out of the slot finished
-    ~PrPlan() {
-        for (hipEvent_t e : ev_h2d) (void)hipEventDestroy(e);
-        for (hipEvent_t e : ev_pull) (void)hipEventDestroy(e);
-    }
+    LinkRing *link = nullptr;         // the dynamic region's chunks (null: none)
     PrRow *d_rows = nullptr;
     uint64_t blocks = 0;              // workgroups of an iteration
     unsigned static_grid() const { return nh + g1 + g0; }
@@ -333,12 +317,6 @@ unsigned grid_of(uint64_t threads) {
 // (eight of 256 lanes per CU), few enough that the last one sums their
 // partials quickly.
 constexpr unsigned kPrGridCap = 2048;
-
-// Slots of the chunk ring: small enough that a few are on their way while
-// others are pulled, large enough that a copy takes longer than its hand-over
-// (4 MiB: 73 us on the link).
-constexpr uint64_t kPrSlotBytes = 4ull << 20;
-constexpr uint32_t kPrRing = 8;
 
 }  // namespace
 
@@ -366,40 +344,14 @@ static PrPlan &pr_plan(DeviceState *d, const og_graph *g) {
         OG_HIP(hipMemcpy(p->d_rows, rows.data(), vs * sizeof(PrRow), hipMemcpyHostToDevice));
     }
     if (vs < d->V) {
-        uint64_t maxrow = 0;
-        for (uint64_t v = vs; v < d->V; ++v) maxrow = std::max(maxrow, g->ptr[v + 1] - g->ptr[v]);
-        if (maxrow > d->slot_edges)
-            raise(OG_EBUDGET, "a vertex has %llu in-edges, more than a staging slot (%llu)", (unsigned long long)maxrow,
+        p->link = link_ring(d, g);
+        if (!p->link)
+            raise(OG_EBUDGET, "a vertex has more in-edges than a staging slot holds (%llu)",
                   (unsigned long long)d->slot_edges);
-        const uint64_t total = (uint64_t)d->nslots * d->slot_edges;  // 4-byte words of the staging share
-        // the link format's rows start anywhere in a word and are read eight
-        // bytes at a time, so it takes slots of a few words more
-        p->lbits = d->lbits && (maxrow * d->lbits + 31) / 32 + 2 <= total / 2 ? d->lbits : 0;
-        const uint32_t bits = p->lbits ? p->lbits : 32;
-        auto words_of = [&](uint64_t n) { return (n * bits + 31) / 32 + (p->lbits ? 2 : 0); };
-        p->ring = (uint32_t)std::min<uint64_t>(kPrRing, std::max<uint64_t>(2, total * 4 / kPrSlotBytes));
-        while (p->ring > 2 && total / p->ring < words_of(maxrow)) --p->ring;
-        p->slot = total / p->ring;
-        p->src = p->lbits ? d->h_link : g->cols + d->dyn_base;
-        const uint64_t base = d->dyn_base;
-        for (uint64_t va = vs; va < d->V;) {
-            uint64_t lo = va + 1, hi = d->V;
-            while (lo < hi) {  // largest vb whose rows fit
-                const uint64_t mid = (lo + hi + 1) / 2;
-                if (words_of(g->ptr[mid] - g->ptr[va]) <= p->slot) lo = mid; else hi = mid - 1;
-            }
-            const uint64_t b0 = (g->ptr[va] - base) * bits, b1 = (g->ptr[lo] - base) * bits;
-            const uint64_t w0 = b0 / 32, w1 = (b1 + 31) / 32 + (p->lbits && b1 > b0 ? 1 : 0);
-            p->chunks.push_back({(uint32_t)va, (uint32_t)lo, w0, b1 > b0 ? w1 - w0 : 0, (uint32_t)(b0 % 32)});
-            va = lo;
-        }
-        p->ev_h2d.assign(p->ring, nullptr);
-        p->ev_pull.assign(p->ring, nullptr);
-        for (auto &e : p->ev_h2d) OG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        for (auto &e : p->ev_pull) OG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
     p->blocks = p->static_grid();
-    for (auto &c : p->chunks) p->blocks += grid_of((uint64_t)(c.vb - c.va) * kPrRangeLpv);
+    if (p->link)
+        for (auto &c : p->link->chunks) p->blocks += grid_of((uint64_t)(c.vb - c.va) * kPrRangeLpv);
     d->pr_plan = p;
     return *p;
 }
@@ -460,7 +412,7 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
         OG_HIP(hipGetLastError());
     };
     uint32_t it = 0;
-    if (pp.chunks.empty()) {
+    if (!pp.link) {
         // One launch per iteration, enqueued a few ahead of the device:
         // iterations past the last one return at once.
         constexpr uint32_t kAhead = 4;
@@ -482,17 +434,18 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
         // ring fills, for the static pull.  Consecutive copies alternate
         // between two streams: the hand-over from a copy to the next one's
         // wait costs about 30 us, hidden behind the other stream's copy.
-        const uint64_t nc = pp.chunks.size();
+        LinkRing &lr = *pp.link;
+        const uint64_t nc = lr.chunks.size();
         uint64_t copied = 0, pulled = 0;
         auto copy_next = [&] {
-            const PrPlan::Chunk &ch = pp.chunks[copied % nc];
-            const uint32_t slot = (uint32_t)(copied % pp.ring);
-            uint32_t *dslot = (uint32_t *)d->d_staging + slot * pp.slot;
+            const LinkRing::Chunk &ch = lr.chunks[copied % nc];
+            const uint32_t slot = (uint32_t)(copied % lr.ring);
+            uint32_t *dslot = (uint32_t *)d->d_staging + slot * lr.slot;
             const hipStream_t on = copied & 1 ? d->s_static : d->s_copy;
-            if (copied >= pp.ring) OG_HIP(hipStreamWaitEvent(on, pp.ev_pull[slot], 0));
+            if (copied >= lr.ring) OG_HIP(hipStreamWaitEvent(on, lr.ev_use[slot], 0));
             if (ch.words)
-                OG_HIP(hipMemcpyAsync(dslot, pp.src + ch.word, ch.words * 4, hipMemcpyHostToDevice, on));
-            OG_HIP(hipEventRecord(pp.ev_h2d[slot], on));
+                OG_HIP(hipMemcpyAsync(dslot, lr.src + ch.word, ch.words * 4, hipMemcpyHostToDevice, on));
+            OG_HIP(hipEventRecord(lr.ev_h2d[slot], on));
             st.run.h2d_bytes += ch.words * 4;
             st.run.chunks++;
             ++copied;
@@ -502,28 +455,28 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
             while (it < prm.max_iterations) {
                 turn(it);
                 // the copies first: what the ring holds crosses the link beside the static pull
-                while (copied < pulled + std::min<uint64_t>(pp.ring, nc)) copy_next();
+                while (copied < pulled + std::min<uint64_t>(lr.ring, nc)) copy_next();
                 if (sgrid) {
                     EventSpan span(d, &tc_static, s);
                     pull_static(s, nullptr);
                 }
                 uint64_t poff = sgrid;
                 for (uint64_t c = 0; c < nc; ++c, ++pulled) {
-                    const PrPlan::Chunk &ch = pp.chunks[c];
-                    const uint32_t slot = (uint32_t)(pulled % pp.ring);
-                    OG_HIP(hipStreamWaitEvent(s, pp.ev_h2d[slot], 0));
+                    const LinkRing::Chunk &ch = lr.chunks[c];
+                    const uint32_t slot = (uint32_t)(pulled % lr.ring);
+                    OG_HIP(hipStreamWaitEvent(s, lr.ev_h2d[slot], 0));
                     const unsigned gr = grid_of((uint64_t)(ch.vb - ch.va) * kPrRangeLpv);
                     {
                         EventSpan span(d, &tc_dyn, s);
                         hipLaunchKernelGGL(k_pr_pull_range<T>, dim3(gr), dim3(kBlock), 0, s, a, ch.va, ch.vb,
-                                           (const uint32_t *)d->d_staging + slot * pp.slot, pp.lbits, ch.first, poff);
+                                           (const uint32_t *)d->d_staging + slot * lr.slot, lr.lbits, ch.first, poff);
                         OG_HIP(hipGetLastError());
                     }
                     poff += gr;
-                    OG_HIP(hipEventRecord(pp.ev_pull[slot], s));
+                    OG_HIP(hipEventRecord(lr.ev_use[slot], s));
                     // the slots that are free, the one this chunk leaves among them
                     const bool last = it + 1 == prm.max_iterations;
-                    while (copied < pulled + 1 + pp.ring && !(last && copied % nc == 0 && copied > pulled)) copy_next();
+                    while (copied < pulled + 1 + lr.ring && !(last && copied % nc == 0 && copied > pulled)) copy_next();
                 }
                 hipLaunchKernelGGL(k_pr_finish, dim3(1), dim3(1024), 0, s, d->d_partial, (uint32_t)poff, d->d_prstate,
                                    d->h_progress);
@@ -548,7 +501,7 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
     st.run.relax_static_bytes = it * (row * d->plan.vsplit + (4 + vb_bytes) * sedges);
     st.run.static_work_edges = it * sedges;
     st.run.relax_dynamic_bytes = it * (row * (V - d->plan.vsplit) + (4 + vb_bytes) * (g->E - sedges));
-    if (pp.chunks.empty()) st.run.relax_dynamic_bytes = 0;
+    if (!pp.link) st.run.relax_dynamic_bytes = 0;
     st.run.work_edges = (uint64_t)it * g->E;
     st.iterations = it;
     st.final_l1 = d->h_prstate->l1;
@@ -559,7 +512,7 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
     st.run.frontier_kernel_ms = sum_ms(tc_init);
     st.run.frontier_launches = tc_init.launches;
     st.run.relax_static_kernel_ms = sum_ms(tc_static);
-    st.run.relax_static_launches = pp.chunks.empty() ? it : tc_static.launches;
+    st.run.relax_static_launches = !pp.link ? it : tc_static.launches;
     st.run.relax_dynamic_kernel_ms = sum_ms(tc_dyn);
     st.run.relax_dynamic_launches = tc_dyn.launches;
     st.run.copy_ms = sum_ms(tc_copy);

@@ -65,3 +65,38 @@ def test_pagerank_chunk_ring(V, frac, fp64):
         assert abs(st["iterations"] - it) <= 1
     assert g.pagerank(fp64=fp64, max_iterations=3)[1]["iterations"] == 3
     g.close()
+
+
+@pytest.mark.parametrize("pack", [True, False])
+@pytest.mark.parametrize("approach", ["ascetic", "subway"])
+def test_copy_loader_ring(approach, pack):
+    """Rounds of the copy loader that relax much of the dynamic region (whole
+    rows through the chunk ring), on rows that a workgroup's slice cannot hold
+    in LDS (5000 empty rows in a stretch), that span several workgroups (9000
+    edges) and that end at chunk ends."""
+    V = 30001
+    rng = np.random.default_rng(5)
+    deg = rng.integers(0, 9, V)
+    deg[15000:20000] = 0
+    deg[21000] = 9000
+    ptr = np.zeros(V + 1, np.uint64)
+    ptr[1:] = np.cumsum(deg)
+    cols = rng.integers(0, V, int(ptr[-1])).astype(np.uint32)
+    w = rng.integers(1, 64, len(cols)).astype(np.uint32)
+    ptr = ptr[:-1].copy()
+    flags = 0 if pack else og.PLAN_NO_PACK
+    src = 21000
+    bfs, sssp, cc = oracle.bfs(ptr, cols, src)[0], oracle.sssp(ptr, cols, w, src), oracle.cc(ptr, cols)[0]
+    for weights, eb in ((None, 4), (w, 8)):
+        g = og.Graph.from_csr(ptr, cols, weights)
+        for split in (0, 8) if weights is not None and pack else (0,):
+            g.prepare(approach, edge_budget_bytes=len(cols) * eb // 2, advisek=0.5, flags=flags, split_weight=split)
+            for _ in range(2):
+                assert np.array_equal(g.cc()[0], cc)
+                assert np.array_equal(g.bfs(src)[0], bfs)
+                assert np.array_equal(g.msbfs(np.array([src, 0], np.uint32))[0][0], bfs)
+                if weights is not None:
+                    for delta in (0, 16):
+                        g.set_tuning(delta=delta)
+                        assert np.array_equal(g.sssp(src)[0], sssp)
+        g.close()

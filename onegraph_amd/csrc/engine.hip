@@ -1174,13 +1174,15 @@ __device__ __forceinline__ uint64_t d_mix64(uint64_t z) {
 // values and four degrees per 16-byte load.  Few, large workgroups
 // (stats_grid): each ends with three device-scope atomics on one line, which
 // queue at about 12 ns each (1024 workgroups of 256: 41 us at 1 M vertices).
+// ctl, when given: nothing is summed while the traversal has a frontier.
 constexpr int kStatsBlock = 1024;
 __global__ __launch_bounds__(kStatsBlock) void k_reach_stats(const uint32_t *__restrict__ val,
-                                                        const uint64_t *__restrict__ ptr,
-                                                        const uint32_t *__restrict__ deg,
-                                                        const uint32_t *__restrict__ hdeg, uint64_t V,
-                                                        unsigned long long *counters, unsigned long long *spread,
-                                                             RoundClock *clk) {
+                                                             const uint64_t *__restrict__ ptr,
+                                                             const uint32_t *__restrict__ deg,
+                                                             const uint32_t *__restrict__ hdeg, uint64_t V,
+                                                             unsigned long long *counters, unsigned long long *spread,
+                                                             RoundClock *clk, const RoundCtl *ctl = nullptr) {
+    if (ctl && ctl->live) return;
     __shared__ unsigned long long s_sum[3];
     if (threadIdx.x < 3) s_sum[threadIdx.x] = 0;
     clock_stamp(clk, kClkFront, kClkOther);
@@ -1233,6 +1235,233 @@ __global__ __launch_bounds__(kStatsBlock) void k_reach_stats(const uint32_t *__r
     __syncthreads();
     if (threadIdx.x < 3 && s_sum[threadIdx.x]) atomicAdd(counters + 2 + threadIdx.x, s_sum[threadIdx.x]);
     if (blockIdx.x == 0) fold_spread(spread, counters);
+}
+
+// ----------------------------------------------------------- small graphs
+//
+// A whole traversal in one launch of one workgroup, for graphs whose values fit
+// its LDS.  Values, the frontier bitmaps and the round's queue live in LDS, so a
+// round costs two barriers instead of two launches, and nothing but rows is
+// read from memory; the end writes the result, the digest and the statistics,
+// to pinned host memory too, so that the host waits for one flag.  What bounds
+// it: the latency of row bounds and edges on a few hundred rows in flight, and one
+// compute unit's load rate, hence the limits.  Measured through the binding
+// (R-MAT, one launch / rounds): BFS 1000 vertices 12 K edges 45 / 152 us, 8000 /
+// 108 K 104 / 167, 16384 / 228 K 170 / 166; SSSP 4000 / 52 K 117 / 353, 16384 /
+// 228 K 380 / 414, 330 K 548 / 464; CC, whose first rounds relax every vertex,
+// 8000 / 168 K 118 / 170 but 16384 / 58 K 289 / 272.
+constexpr uint32_t kSmallV = 1u << 14;
+constexpr uint32_t kSmallVcc = 1u << 13;
+constexpr uint64_t kSmallE = 3u << 16;
+constexpr int kSmallBlock = 1024;
+constexpr uint32_t kSmallMid = 32, kSmallLong = 512;  // rows: 8 lanes, a wave, the workgroup
+
+struct SmallArgs {
+    const uint64_t *ptr;
+    const void *edges;
+    uint32_t wbits, V, src;
+    uint32_t *val;             // V values out
+    uint32_t *host;            // and here (pinned host memory) unless null
+    RunBlock *blk, *h_blk;     // statistics (h_blk: pinned, or null)
+    unsigned long long *done;  // pinned flag raised to 1 at the end, or null
+    bool check;                // offsets that do not run from 0 to E: no run, they are left in counters[14..15]
+    uint64_t E;
+};
+
+constexpr size_t small_lds(uint64_t V) { return 4 * V + 8 * ((V + 31) / 32) + 2 * ((V + 1) / 2 * 2); }
+
+template <int ALGO, bool W, bool PK>
+__global__ __launch_bounds__(kSmallBlock) void k_small(SmallArgs a) {
+    extern __shared__ uint32_t s_mem[];
+    __shared__ uint32_t s_n[4];                       // rows of the round: short, wave, workgroup, without edges
+    __shared__ unsigned long long s_tot[6];           // updates, edges, vertices; reached, traversed, digest
+    __shared__ uint16_t s_long[kSmallE / kSmallLong];
+    const unsigned long long t0 = wall_clock64();
+    if (a.check) {
+        const uint64_t p0 = a.ptr[0], p1 = a.ptr[a.V];
+        if (threadIdx.x == 0) {
+            a.blk->counters[14] = p0;
+            a.blk->counters[15] = p1;
+        }
+        if (p0 != 0 || p1 != a.E) return;
+    }
+    const uint32_t V = a.V, nw = (V + 31) / 32, tid = threadIdx.x, lane = tid & (kWave - 1);
+    uint32_t *val = s_mem, *cur = val + V, *nxt = cur + nw;
+    uint16_t *q = (uint16_t *)(nxt + nw);  // short rows from the front, wave rows from the back
+    for (uint32_t v = tid; v < V; v += kSmallBlock) val[v] = ALGO == ALGO_CC ? v : v == a.src ? 1u : OG_UNREACHED;
+    for (uint32_t i = tid; i < nw; i += kSmallBlock) {
+        if (ALGO == ALGO_CC) cur[i] = i + 1 < nw || V % 32 == 0 ? 0xFFFFFFFFu : (1u << (V % 32)) - 1u;
+        else cur[i] = i == a.src / 32 ? 1u << (a.src % 32) : 0u;
+        nxt[i] = 0;
+    }
+    if (tid < 6) s_tot[tid] = 0;
+    uint32_t upd = 0, rounds = 0, nodes = 0, empty = 0;
+    uint64_t work = 0;
+    // offers N edges of a lane
+    auto relax = [&](auto &to, auto &wt, uint32_t ok, uint32_t du) {
+        constexpr int N = sizeof(to) / sizeof(uint32_t);
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const uint32_t nd = offer<ALGO>(du, wt[k]);
+            if (!((ok >> k) & 1) || nd >= val[to[k]]) continue;
+            if (nd < atomicMin(&val[to[k]], nd)) {
+                atomicOr(&nxt[to[k] / 32], 1u << (to[k] % 32));
+                ++upd;
+            }
+        }
+    };
+    auto row = [&](uint32_t u, uint32_t sub, uint32_t L) {
+        const uint64_t b = a.ptr[u], e = a.ptr[u + 1];
+        const uint32_t du = val[u];
+        for (uint64_t i = b + sub; i < e; i += (uint64_t)kRelaxBatch * L) {
+            uint32_t to[kRelaxBatch], wt[kRelaxBatch], ok = 0;
+#pragma unroll
+            for (int k = 0; k < kRelaxBatch; ++k) {
+                to[k] = wt[k] = 0;
+                if (i + (uint64_t)k * L < e) {
+                    load_edge<W, PK>(a.edges, i + (uint64_t)k * L, a.wbits, to[k], wt[k]);
+                    ok |= 1u << k;
+                }
+            }
+            relax(to, wt, ok, du);
+        }
+    };
+    for (;;) {
+        if (tid < 4) s_n[tid] = 0;
+        __syncthreads();
+        // the round's queues, four vertices of a lane in flight
+        for (uint32_t v0 = 0; v0 < V; v0 += 4 * kSmallBlock) {
+            uint64_t b[4], e[4];
+            bool on[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t v = v0 + k * kSmallBlock + tid;
+                on[k] = v < V && (cur[v / 32] >> (v % 32)) & 1;
+                b[k] = on[k] ? a.ptr[v] : 0;
+                e[k] = on[k] ? a.ptr[v + 1] : 0;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (!__ballot(on[k])) continue;
+                const uint64_t d = e[k] - b[k];
+                work += d;
+                const int c = !on[k] ? 4 : d == 0 ? 3 : d <= kSmallMid ? 0 : d <= kSmallLong ? 1 : 2;
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const uint64_t m = __ballot(c == x);
+                    if (!m) continue;
+                    uint32_t at = 0;
+                    if (lane == 0) at = atomicAdd(&s_n[x], (uint32_t)__popcll(m));
+                    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+                    at += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+                    if (c != x || x == 3) continue;
+                    const uint16_t v = (uint16_t)(v0 + k * kSmallBlock + tid);
+                    if (x == 0) q[at] = v;
+                    else if (x == 1) q[V - 1 - at] = v;
+                    else if (at < kSmallE / kSmallLong) s_long[at] = v;  // (always, but for offsets that fall)
+                }
+            }
+        }
+        __syncthreads();
+        const uint32_t n0 = s_n[0], n1 = s_n[1], n2 = min(s_n[2], (uint32_t)(kSmallE / kSmallLong)), nz = s_n[3];
+        if (!(n0 | n1 | n2 | nz)) break;
+        ++rounds;
+        nodes += n0 + n1 + n2 + nz;
+        empty += nz;
+        for (uint32_t i = tid; i < nw; i += kSmallBlock) cur[i] = 0;
+        for (uint32_t i = 0; i < n2; ++i) row(s_long[i], tid, kSmallBlock);
+        for (uint32_t i = tid / kWave; i < n1; i += kSmallBlock / kWave) row(q[V - 1 - i], lane, kWave);
+        // short rows, two per group of lanes in flight
+        constexpr uint32_t L = 8, G = kSmallBlock / L;
+        for (uint32_t i = tid / L; i < n0; i += 2 * G) {
+            uint32_t to[2][kSmallMid / L], wt[2][kSmallMid / L], ok[2] = {0, 0}, u[2] = {0, 0};
+            uint64_t b[2], e[2];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const bool in = i + r * G < n0;
+                u[r] = in ? q[i + r * G] : 0;
+                b[r] = in ? a.ptr[u[r]] : 0;
+                e[r] = in ? a.ptr[u[r] + 1] : 0;
+            }
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int k = 0; k < (int)(kSmallMid / L); ++k) {
+                    const uint64_t x = b[r] + tid % L + (uint64_t)k * L;
+                    to[r][k] = wt[r][k] = 0;
+                    if (x < e[r]) {
+                        load_edge<W, PK>(a.edges, x, a.wbits, to[r][k], wt[r][k]);
+                        ok[r] |= 1u << k;
+                    }
+                }
+#pragma unroll
+            for (int r = 0; r < 2; ++r) relax(to[r], wt[r], ok[r], val[u[r]]);
+        }
+        __syncthreads();
+        uint32_t *t = cur;
+        cur = nxt;
+        nxt = t;
+    }
+    // the result and its sums
+    uint64_t reached = 0, trav = 0, dig = 0;
+    for (uint32_t v = tid; v < V; v += kSmallBlock) {
+        const uint32_t x = val[v];
+        a.val[v] = x;
+        if (a.host) a.host[v] = x;
+        if (x != OG_UNREACHED) {
+            ++reached;
+            trav += a.ptr[v + 1] - a.ptr[v];
+            dig += d_mix64(((uint64_t)v << 32) | x);
+        }
+    }
+    const uint64_t sums[5] = {wave_scan_u64(upd), wave_scan_u64(work), wave_scan_u64(reached), wave_scan_u64(trav),
+                              wave_scan_u64(dig)};
+    if (lane == kWave - 1)
+#pragma unroll
+        for (int i = 0; i < 5; ++i) atomicAdd(&s_tot[i], (unsigned long long)sums[i]);
+    if (a.done) __threadfence_system();
+    __syncthreads();
+    if (tid != 0) return;
+    auto fill = [&](RunBlock *o) {
+        RoundCtl c{};
+        c.rounds = rounds;
+        c.compactions = rounds + 1;
+        c.halt = 1;
+        c.nverts = V;
+        c.node_sum = nodes;
+        c.static_node_sum = nodes - empty;
+        c.work_edges = c.static_work_edges = s_tot[1];
+        o->ctl = c;
+        o->clk.acc[kClkRelax] = wall_clock64() - t0;
+        o->clk.acc[kClkFront] = o->clk.acc[kClkOther] = 0;
+        for (int i = 0; i < 14; ++i) o->counters[i] = 0;
+        o->counters[kUpdStatic] = s_tot[0];
+        o->counters[2] = s_tot[2];
+        o->counters[3] = s_tot[3];
+        o->counters[4] = s_tot[4];
+    };
+    if (a.h_blk) fill(a.h_blk);
+    else fill(a.blk);
+    if (a.done) {
+        __threadfence_system();
+        __hip_atomic_store(a.done, 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// Launches k_small on s; its dynamic LDS exceeds what a kernel gets unasked.
+template <int ALGO, bool W, bool PK>
+static void launch_small(const SmallArgs &a, hipStream_t s) {
+    static std::atomic<uint64_t> asked{0};  // devices, by bit
+    int dev = 0;
+    OG_HIP(hipGetDevice(&dev));
+    const uint64_t bit = dev < 64 ? 1ull << dev : 0;
+    if (!(asked.load(std::memory_order_acquire) & bit)) {
+        OG_HIP(hipFuncSetAttribute((const void *)k_small<ALGO, W, PK>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)small_lds(kSmallV)));
+        asked.fetch_or(bit, std::memory_order_release);
+    }
+    hipLaunchKernelGGL((k_small<ALGO, W, PK>), dim3(1), dim3(kSmallBlock), small_lds(a.V), s, a);
+    OG_HIP(hipGetLastError());
 }
 
 // ------------------------------------------------------- multi-source BFS
@@ -2942,6 +3171,33 @@ static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats 
     OG_HIP(hipStreamSynchronize(d->s_static));
     OG_HIP(hipStreamSynchronize(s));
     Stopwatch total;
+    // A small graph wholly in HBM: one launch (the A/B flags keep the rounds)
+    if (!d->managed && d->plan.vsplit >= V && V <= (ALGO == ALGO_CC ? kSmallVcc : kSmallV) && d->E <= kSmallE &&
+        !(d->flags & (OG_PLAN_NO_FUSE | OG_PLAN_NO_OVERLAP))) {
+        if (out && (!d->out || d->out->bytes < V * 4)) d->out = out_stage(V * 4);
+        std::unique_lock<std::mutex> use;
+        if (out) use = std::unique_lock<std::mutex>(d->out->use, std::try_to_lock);
+        const bool direct = use.owns_lock() && d->out->bytes >= V * 4;
+        __atomic_store_n(d->fr.h_progress, 0ull, __ATOMIC_RELEASE);
+        const SmallArgs a{d->d_ptr, d->d_static, d->wbits, (uint32_t)V, src, d->d_val,
+                          direct ? (uint32_t *)d->out->buf : nullptr, d->fr.blk, d->fr.h_blk, d->fr.h_progress, false, 0};
+        if (W && d->packed) launch_small<ALGO, W, true>(a, s);
+        else launch_small<ALGO, W, false>(a, s);
+        wait_progress(d->fr.h_progress, 1, s);
+        if (!__atomic_load_n(d->fr.h_progress, __ATOMIC_ACQUIRE)) OG_HIP(hipStreamSynchronize(s));
+        st.total_ms = total.ms();
+        if (direct) std::memcpy(out, d->out->buf, V * 4);
+        else if (out) copy_to_host(d, out, d->d_val, V * 4, s);
+        tm.stat.launches = 1;
+        tm.clocked = kClsStat;
+        collect_loop<ALGO, W>(d, st);
+        st.reached = d->fr.h_blk->counters[2];
+        st.traversed_edges = d->fr.h_blk->counters[3];
+        st.checksum = d->fr.h_blk->counters[4];
+        finish_stats(st, tm, gather_ms, overload_wall, d, 8);
+        if (stats) *stats = st;
+        return;
+    }
     auto begin = [&](const RoundCtl &c) {
         hipLaunchKernelGGL((k_run_init<ALGO == ALGO_CC>), dim3(fill_grid(d->Vpad / 4)), dim3(kBlock), 0, s, d->d_val,
                            d->fr.flag, V, d->Vpad, src, d->fr.blk, d->fr.spread, c);

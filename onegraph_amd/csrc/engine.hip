@@ -47,11 +47,6 @@ __global__ void k_fill_u8(uint8_t *a, uint64_t n, uint8_t v) {
         a[i] = v;
 }
 
-__global__ void k_set_source(uint32_t *val, uint8_t *flag, uint32_t src) {
-    val[src] = 1;
-    flag[src] = 1;
-}
-
 __device__ __forceinline__ void clock_stamp(RoundClock *clk, int prev, int kind) {
     if (clk && blockIdx.x == 0 && threadIdx.x == 0) {
         const unsigned long long t = wall_clock64();
@@ -550,8 +545,6 @@ static RoundCtl ctl_begin(uint64_t V, uint32_t delta, uint32_t defer, uint64_t d
     c.halt = 1;
     return c;
 }
-
-__global__ void k_ctl_set(RoundCtl *ctl, RoundCtl c) { *ctl = c; }
 
 // ---------------------------------------------------------------- relax
 
@@ -3831,9 +3824,8 @@ constexpr uint64_t kNaHub = kNaList + na_up(4 * kNoAllocMaxV);
 constexpr uint64_t kNaDoff = kNaHub + na_up(8 * kNoAllocHubCap);
 constexpr uint64_t kNaTot = kNaDoff + na_up(8 * 16);
 constexpr uint64_t kNaInfo = kNaTot + na_up(8 * totals_words(kNoAllocMaxBlk));
-constexpr uint64_t kNaCtl = kNaInfo + na_up(sizeof(FrontierInfo));
-constexpr uint64_t kNaCounters = kNaCtl + na_up(sizeof(RoundCtl));
-constexpr uint64_t kNaSpread = kNaCounters + na_up(16 * 8);
+constexpr uint64_t kNaBlk = kNaInfo + na_up(sizeof(FrontierInfo));
+constexpr uint64_t kNaSpread = kNaBlk + na_up(sizeof(RunBlock));
 constexpr uint64_t kNoAllocScratchBytes = kNaSpread + na_up(8 * kSpreadWords);
 
 // The scratch memory of og_bfs_device_noalloc.  In host code `scratch` is a
@@ -3862,93 +3854,118 @@ static uint8_t *noalloc_scratch(int dev) {
     return (uint8_t *)g_na_ptr[dev];
 }
 
+// Start of an allocation-free run, one launch: levels, flags, totals, counters
+// and traversal state.  Row offsets that do not run from 0 to E end the run
+// before it begins and leave the levels alone; counters[14..15] keep them.
+__global__ __launch_bounds__(kBlock) void k_noalloc_init(const uint64_t *__restrict__ ptr, uint64_t V, uint64_t E,
+                                                         uint32_t src, uint32_t *__restrict__ levels,
+                                                         uint8_t *__restrict__ flag, uint64_t Vpad,
+                                                         unsigned long long *__restrict__ tot, uint64_t ntot,
+                                                         unsigned long long *__restrict__ spread, RunBlock *blk,
+                                                         FrontierInfo *info, RoundCtl c) {
+    const uint64_t tid = (uint64_t)blockIdx.x * kBlock + threadIdx.x, nth = (uint64_t)gridDim.x * kBlock;
+    const uint64_t p0 = ptr[0], p1 = ptr[V];
+    const bool good = p0 == 0 && p1 == E;
+    if (tid == 0) {
+        c.live = good ? 1u : 0u;
+        blk->ctl = c;
+        for (int i = 0; i < 16; ++i) blk->counters[i] = i == 14 ? p0 : i == 15 ? p1 : 0;
+        *info = FrontierInfo{};
+    }
+    for (uint64_t i = tid; i < ntot; i += nth) tot[i] = i >= kTotSlot && i < kTotArrive && i % kTotLine == 3 ? ~0ull : 0ull;
+    for (uint64_t i = tid; i < kSpreadWords; i += nth) spread[i] = 0;
+    if (!good) return;
+    for (uint64_t v = tid; v < V; v += nth) levels[v] = v == src ? 1u : OG_UNREACHED;
+    for (uint64_t v = tid; v < Vpad; v += nth) flag[v] = v == src ? 1 : 0;
+}
+
 static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t V, uint64_t E, uint32_t src,
                         uint32_t *d_levels, hipStream_t s, og_run_stats *stats) {
     int dev = 0;
     OG_HIP(hipGetDevice(&dev));
     uint8_t *base = noalloc_scratch(dev);
-    uint64_t ends[2] = {1, 1};
-    OG_HIP(hipMemcpyAsync(&ends[0], d_ptr, 8, hipMemcpyDeviceToHost, s));
-    OG_HIP(hipMemcpyAsync(&ends[1], d_ptr + V, 8, hipMemcpyDeviceToHost, s));
-    OG_HIP(hipStreamSynchronize(s));
-    if (ends[0] != 0 || ends[1] != E)
-        raise(OG_EINVAL, "row offsets must run from 0 to E=%llu over V+1 entries (got %llu .. %llu)",
-              (unsigned long long)E, (unsigned long long)ends[0], (unsigned long long)ends[1]);
-    const uint64_t Vpad = (V + 15) / 16 * 16;
-    const uint32_t nblk = (uint32_t)((Vpad + verts_per_block(1) - 1) / verts_per_block(1));
-    uint8_t *flag = base + kNaFlag;
-    uint32_t *list = (uint32_t *)(base + kNaList);
-    uint64_t *hub = (uint64_t *)(base + kNaHub);
-    uint64_t *doff = (uint64_t *)(base + kNaDoff);
-    const CompactTotals ct{(unsigned long long *)(base + kNaTot), nblk, 1};  // (no dynamic list)
-    FrontierInfo *info = (FrontierInfo *)(base + kNaInfo);
-    RoundCtl *ctl = (RoundCtl *)(base + kNaCtl);
-    unsigned long long *ctr = (unsigned long long *)(base + kNaCounters);
-    unsigned long long *spread = (unsigned long long *)(base + kNaSpread);
-    const Tuning tn;  // default bins: the hub bound above assumes its t2 and tile
-    static_assert(Tuning{}.t2 == 4096 && Tuning{}.tile == 2048, "hub capacity bound follows the default tuning");
-    Stopwatch total;
-    // clear what must start at zero: fill kernels (no memset nodes)
-    hipLaunchKernelGGL(k_fill_u8, dim3(fill_grid(Vpad)), dim3(256), 0, s, flag, Vpad, (uint8_t)0);
-    static_assert(kNaSpread == kNaCounters + 16 * 8 + 128, "cleared together");
-    hipLaunchKernelGGL(k_fill_u32, dim3(16), dim3(256), 0, s, (uint32_t *)ctr, (uint64_t)(kNoAllocScratchBytes - kNaCounters) / 4, 0u);
-    hipLaunchKernelGGL(k_fill_u32, dim3(fill_grid(V)), dim3(256), 0, s, d_levels, V, OG_UNREACHED);
-    hipLaunchKernelGGL(k_set_source, dim3(1), dim3(1), 0, s, d_levels, flag, src);
-    hipLaunchKernelGGL(k_ctl_set, dim3(1), dim3(1), 0, s, ctl, ctl_begin(V, 0, 0, 0, false));
-    hipLaunchKernelGGL(k_totals_init, dim3(fill_grid(totals_words(nblk))), dim3(256), 0, s, ct.t, totals_words(nblk));
-    auto compact = [&] {
-        hipLaunchKernelGGL(k_frontier_compact<1>, dim3(nblk), dim3(kCompactBlock), 0, s, flag, (uint8_t *)nullptr, Vpad, V,
-                           d_ptr, (const uint64_t *)nullptr, (const uint32_t *)nullptr, (const uint32_t *)nullptr, tn,
-                           (const uint32_t *)nullptr, ctl, ct, info, list, hub, kNoAllocHubCap, doff,
-                           (uint32_t *)nullptr, (uint64_t)0, (RoundClock *)nullptr, (int)kClkOther, (unsigned long long *)nullptr);
+    RunBlock *blk = (RunBlock *)(base + kNaBlk);
+    RunBlock h{};
+    auto check_ends = [&] {
+        if (h.counters[14] != 0 || h.counters[15] != E)
+            raise(OG_EINVAL, "row offsets must run from 0 to E=%llu over V+1 entries (got %llu .. %llu)",
+                  (unsigned long long)E, h.counters[14], h.counters[15]);
     };
-    RoundRelax r{};
-    r.list = list;
-    r.info = info;
-    r.ptr = d_ptr;
-    r.sedges = d_cols;
-    r.hub = hub;
-    r.hub_cap = kNoAllocHubCap;
-    r.tile = tn.tile;
-    r.cd = 0;  // the whole graph is static: three bins in one launch
-    r.vsplit = V;
-    r.spread = spread;
-    const RelaxArgs a{d_levels, flag, nullptr, nullptr, 0, nullptr, nullptr};
-    static_assert(Tuning{}.lpv0 == 8, "the relax below is instantiated for 8 lanes per bin-0 vertex");
-    compact();
-    OG_HIP(hipGetLastError());
-    RoundCtl h{};
-    for (;;) {
-        for (int k = 0; k < kRoundBatch; ++k) {
-            hipLaunchKernelGGL((k_relax_round<ALGO_BFS, false, false, 8>), dim3(kFuseStatic * kHubGridCap),
-                               dim3(kBlock), (size_t)tn.tile * 4, s, r, a);
-            compact();
-        }
+    auto fetch = [&] {
         OG_HIP(hipGetLastError());
-        OG_HIP(hipMemcpyAsync(&h, ctl, sizeof h, hipMemcpyDeviceToHost, s));
+        OG_HIP(hipMemcpyAsync(&h, blk, sizeof h, hipMemcpyDeviceToHost, s));
         OG_HIP(hipStreamSynchronize(s));
-        if (!h.live) break;
+    };
+    Stopwatch total;
+    if (V <= kSmallV && E <= kSmallE) {
+        launch_small<ALGO_BFS, false, false>(
+            SmallArgs{d_ptr, d_cols, 0, (uint32_t)V, src, d_levels, nullptr, blk, nullptr, nullptr, true, E}, s);
+        fetch();
+        check_ends();
+    } else {
+        const uint64_t Vpad = (V + 15) / 16 * 16;
+        const uint32_t nblk = (uint32_t)((Vpad + verts_per_block(1) - 1) / verts_per_block(1));
+        uint8_t *flag = base + kNaFlag;
+        uint32_t *list = (uint32_t *)(base + kNaList);
+        uint64_t *hub = (uint64_t *)(base + kNaHub);
+        uint64_t *doff = (uint64_t *)(base + kNaDoff);
+        const CompactTotals ct{(unsigned long long *)(base + kNaTot), nblk, 1};  // (no dynamic list)
+        FrontierInfo *info = (FrontierInfo *)(base + kNaInfo);
+        unsigned long long *spread = (unsigned long long *)(base + kNaSpread);
+        const Tuning tn;  // default bins: the hub bound above assumes its t2 and tile
+        static_assert(Tuning{}.t2 == 4096 && Tuning{}.tile == 2048, "hub capacity bound follows the default tuning");
+        hipLaunchKernelGGL(k_noalloc_init, dim3(fill_grid(V)), dim3(kBlock), 0, s, d_ptr, V, E, src, d_levels, flag, Vpad,
+                           ct.t, totals_words(nblk), spread, blk, info, ctl_begin(V, 0, 0, 0, false));
+        auto compact = [&] {
+            hipLaunchKernelGGL(k_frontier_compact<1>, dim3(nblk), dim3(kCompactBlock), 0, s, flag, (uint8_t *)nullptr,
+                               Vpad, V, d_ptr, (const uint64_t *)nullptr, (const uint32_t *)nullptr,
+                               (const uint32_t *)nullptr, tn, (const uint32_t *)nullptr, &blk->ctl, ct, info, list, hub,
+                               kNoAllocHubCap, doff, (uint32_t *)nullptr, (uint64_t)0, (RoundClock *)nullptr,
+                               (int)kClkOther, (unsigned long long *)nullptr);
+        };
+        RoundRelax r{};
+        r.list = list;
+        r.info = info;
+        r.ptr = d_ptr;
+        r.sedges = d_cols;
+        r.hub = hub;
+        r.hub_cap = kNoAllocHubCap;
+        r.tile = tn.tile;
+        r.cd = 0;  // the whole graph is static: three bins in one launch
+        r.vsplit = V;
+        r.spread = spread;
+        const RelaxArgs a{d_levels, flag, nullptr, nullptr, 0, nullptr, nullptr};
+        static_assert(Tuning{}.lpv0 == 8, "the relax below is instantiated for 8 lanes per bin-0 vertex");
+        compact();
+        // the first batch covers most traversals of skewed graphs: an empty
+        // round costs about 8 us, a host round trip 25
+        for (int rounds = 2 * kRoundBatch;; rounds = kRoundBatch) {
+            for (int k = 0; k < rounds; ++k) {
+                hipLaunchKernelGGL((k_relax_round<ALGO_BFS, false, false, 8>), dim3(kFuseStatic * kHubGridCap),
+                                   dim3(kBlock), (size_t)tn.tile * 4, s, r, a);
+                compact();
+            }
+            hipLaunchKernelGGL(k_reach_stats, dim3(stats_grid(V)), dim3(kStatsBlock), 0, s, d_levels, d_ptr,
+                               (const uint32_t *)nullptr, (const uint32_t *)nullptr, V, blk->counters, spread,
+                               (RoundClock *)nullptr, (const RoundCtl *)&blk->ctl);
+            fetch();
+            check_ends();
+            if (!h.ctl.live) break;
+        }
     }
-    const double ms = total.ms();
-    hipLaunchKernelGGL(k_reach_stats, dim3(stats_grid(V)), dim3(kStatsBlock), 0, s, d_levels, d_ptr,
-                       (const uint32_t *)nullptr, (const uint32_t *)nullptr, V, ctr, spread, (RoundClock *)nullptr);
-    OG_HIP(hipGetLastError());
-    unsigned long long hc[16];
-    OG_HIP(hipMemcpyAsync(hc, ctr, sizeof hc, hipMemcpyDeviceToHost, s));
-    OG_HIP(hipStreamSynchronize(s));
     if (stats) {
         og_run_stats st{};
         st.approach = OG_ASCETIC;
-        st.iterations = h.rounds;
-        st.node_sum = h.node_sum;
-        st.static_node_sum = h.static_node_sum;
-        st.work_edges = h.work_edges;
-        st.static_work_edges = h.static_work_edges;
-        st.updates = hc[0];
-        st.reached = hc[2];
-        st.traversed_edges = hc[3];
-        st.checksum = hc[4];
-        st.total_ms = ms;
+        st.iterations = h.ctl.rounds;
+        st.node_sum = h.ctl.node_sum;
+        st.static_node_sum = h.ctl.static_node_sum;
+        st.work_edges = h.ctl.work_edges;
+        st.static_work_edges = h.ctl.static_work_edges;
+        st.updates = h.counters[0];
+        st.reached = h.counters[2];
+        st.traversed_edges = h.counters[3];
+        st.checksum = h.counters[4];
+        st.total_ms = total.ms();
         *stats = st;
     }
 }

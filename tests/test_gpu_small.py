@@ -8,6 +8,7 @@ import pytest
 
 import onegraph_amd as og
 import oracle
+from test_zz_no_alloc import _Hip
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +54,31 @@ def test_small_edges(V, E):
         if flags == og.PLAN_NO_FUSE:  # the general rounds count the same
             assert stats[0] == small
     g.close()
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("V,E", [(1, 1), (33, 200), (4097, 30000), (16384, LIMIT), (16385, LIMIT), (16384, LIMIT + 1)])
+def test_small_device_arrays(gpu, V, E, shift):
+    """The entry over device arrays, with levels at any word of an allocation;
+    wrong offsets are refused with the levels untouched."""
+    ptr, cols, _, src = _graph(V, E, V + 3 * E)
+    hip = _Hip()
+    try:
+        full = np.append(ptr, np.uint64(E)).astype(np.uint64)
+        off = full.copy()
+        off[0] = 1
+        d_ptr, d_off, d_cols = hip.upload(full), hip.upload(off), hip.upload(cols)
+        lv = hip.upload(np.full(V + 2 + shift, 77, np.uint32))
+        at = lv + 4 * shift
+        with pytest.raises(og.OgError):
+            og.bfs_device_noalloc(d_off, d_cols, V, E, src, at)
+        assert (hip.download(lv, np.uint32, V + 2 + shift) == 77).all()
+        want = oracle.bfs(ptr, cols, src)[0]
+        for _ in range(2):
+            st = og.bfs_device_noalloc(d_ptr, d_cols, V, E, src, at)
+            got = hip.download(lv, np.uint32, V + 2 + shift)
+            assert np.array_equal(got[shift:shift + V], want)
+            assert (got[shift + V:] == 77).all() and (got[:shift] == 77).all()
+            assert st["reached"] == int((want != og.UNREACHED).sum())
+    finally:
+        hip.free()

@@ -332,8 +332,9 @@ og_status og_autotune(og_graph *g, uint32_t algo, uint32_t source, uint32_t runs
 
 /* Multi-source BFS (no reference counterpart; the reference runs one source
  * per bfs_opt iteration, BFS/oneGraph_BFS/CalculateOpt.h:55-209).  Sources
- * go in batches of 64, each batch one frontier traversal carrying a u64
- * mask per vertex, on the approach given to og_prepare.  Outputs (each may
+ * go in batches of 64, each a u64 mask per vertex, two batches to a frontier
+ * traversal while more than 64 sources are left, on the approach given to
+ * og_prepare (iterations and work_edges count traversals).  Outputs (each may
  * be NULL): levels[i*V + v] in the og_bfs convention, checksums[i] =
  * og_levels_checksum of source i's levels, reached[i] = vertices reached. */
 og_status og_msbfs(og_graph *g, const uint32_t *sources, uint32_t num_sources,

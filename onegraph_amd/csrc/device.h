@@ -43,9 +43,12 @@ constexpr int64_t kNotResident = INT64_MIN;
 constexpr uint32_t kLinkLine = 128;
 constexpr uint64_t kSlotTargetBytes = 256ull << 20;  // preferred slot (chunk) size
 
-enum Algo { ALGO_BFS = 0, ALGO_SSSP = 1, ALGO_CC = 2, ALGO_MSBFS = 3 };
+enum Algo { ALGO_BFS = 0, ALGO_SSSP = 1, ALGO_CC = 2, ALGO_MSBFS = 3, ALGO_MSBFS2 = 4 };
 
-constexpr int kMsWidth = 64;            // sources per multi-source batch (bits of a u64 mask)
+constexpr int kMsWidth = 64;            // sources per mask of the multi-source BFS (bits of a u64)
+// Masks of a multi-source traversal (ALGO_MSBFS2: two batches of 64 sources
+// that walk the graph together); 0: one value per vertex instead.
+constexpr int ms_masks(int algo) { return algo == ALGO_MSBFS ? 1 : algo == ALGO_MSBFS2 ? 2 : 0; }
 
 // Per-vertex state the relax kernels touch.
 struct RelaxArgs {
@@ -425,12 +428,15 @@ struct DeviceState {
     std::unique_ptr<WorkerPool> pool;
 
     // multi-source BFS state (allocated on first use)
-    ulonglong2 *d_vn = nullptr;      // V: sources that reached v, sources offered to v this round
-    uint64_t *d_front = nullptr;     // V: sources whose frontier holds v
-    uint8_t *d_mlvl = nullptr;       // V x 64 levels, vertex-major (0 = unreached); only when levels are asked for
-    unsigned long long *d_mpart = nullptr;  // per commit workgroup: digest, reached, traversed of the 64 sources
-    uint32_t *d_msrc = nullptr;      // 64 sources of the batch
-    unsigned long long *d_msum = nullptr;  // 2 x 64: checksum, reached per source
+    // Multi-source BFS with one mask per vertex (d_ms[0]) and two (d_ms[1])
+    struct MsState {
+        ulonglong2 *vn = nullptr;            // masks x V: sources that reached v, sources offered to v this round
+        uint64_t *front = nullptr;           // masks x V: sources whose frontier holds v
+        unsigned long long *part = nullptr;  // per commit workgroup: digest, reached, traversed of the sources
+        uint32_t *src = nullptr;             // the batch's sources
+        unsigned long long *sum = nullptr;   // per mask 3 x 64: digest, reached, traversed per source
+        uint8_t *lvl = nullptr;              // masks x V x 64 levels, vertex-major (0 = unreached); only when levels are asked for
+    } d_ms[2];
     uint32_t *d_extract = nullptr;   // u32 levels of extract_cap sources on their way to the host
     uint32_t extract_cap = 0;
     // direction-optimising BFS: in-edge CSR (OG_PLAN_DIRECTION_OPT)

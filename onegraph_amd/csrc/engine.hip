@@ -562,12 +562,42 @@ __device__ __forceinline__ uint32_t offer(uint32_t du, uint32_t wt) {
 
 // What a frontier vertex carries to its out-edges: its value, or for the
 // multi-source BFS the mask of sources whose frontier holds it.
+template <int H>
+struct MaskOf {
+    uint64_t m[H];
+    MaskOf() = default;
+    __device__ __forceinline__ MaskOf(int) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) m[h] = 0;
+    }
+    __device__ __forceinline__ bool any() const {
+        uint64_t x = 0;
+#pragma unroll
+        for (int h = 0; h < H; ++h) x |= m[h];
+        return x != 0;
+    }
+};
 template <int ALGO> struct SrcOf { using T = uint32_t; };
-template <> struct SrcOf<ALGO_MSBFS> { using T = uint64_t; };
+template <> struct SrcOf<ALGO_MSBFS> { using T = MaskOf<1>; };
+template <> struct SrcOf<ALGO_MSBFS2> { using T = MaskOf<2>; };
+
+// Whether a frontier vertex has anything to offer in this round.
+template <int ALGO>
+__device__ __forceinline__ bool offers(const typename SrcOf<ALGO>::T &s) {
+    if constexpr (ms_masks(ALGO) != 0) return s.any();
+    else return true;
+}
 
 template <int ALGO>
 __device__ __forceinline__ typename SrcOf<ALGO>::T load_src(const RelaxArgs &a, uint32_t u) {
-    if constexpr (ALGO == ALGO_MSBFS) return a.pull ? a.front[u] & ~*a.pull : a.front[u];
+    if constexpr (ms_masks(ALGO) != 0) {
+        constexpr int H = ms_masks(ALGO);
+        MaskOf<H> s;
+#pragma unroll
+        for (int h = 0; h < H; ++h) s.m[h] = a.front[(uint64_t)u * H + h];
+        if (H == 1 && a.pull) s.m[0] &= ~*a.pull;
+        return s;
+    }
     else return a.val[u];
 }
 
@@ -578,9 +608,15 @@ __device__ __forceinline__ typename SrcOf<ALGO>::T load_src(const RelaxArgs &a, 
 // atomic that finds nothing to do but never loses an update.
 template <int ALGO>
 __device__ __forceinline__ typename SrcOf<ALGO>::T peek(const RelaxArgs &a, uint32_t to) {
-    if constexpr (ALGO == ALGO_MSBFS) {
-        const ulonglong2 x = a.vn[to];
-        return x.x | x.y;
+    if constexpr (ms_masks(ALGO) != 0) {
+        constexpr int H = ms_masks(ALGO);
+        MaskOf<H> s;
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            const ulonglong2 x = a.vn[(uint64_t)to * H + h];
+            s.m[h] = x.x | x.y;
+        }
+        return s;
     }
     else return a.val[to];
 }
@@ -603,17 +639,26 @@ __device__ __forceinline__ typename SrcOf<ALGO>::T peek(const RelaxArgs &a, uint
 // searches).  The two masks share a 16-byte load: with the offers unseen, every
 // edge of a dense round into a well-connected vertex repeated its atomic (R-MAT
 // 4 M vertices, 64 sources, the three dense rounds: 3.75, 2.43, 1.69 -> 1.86,
-// 1.84, 1.70 ms, the last ones the link's).
+// 1.84, 1.70 ms, the last ones the link's; 128 sources 1.87, 1.82, 1.75).
 template <int ALGO, int N, bool AGAIN = false, class Src>
 __device__ __forceinline__ uint32_t commit(const RelaxArgs &a, Src src, const uint32_t (&to)[N], const uint32_t (&wt)[N],
                                            const typename SrcOf<ALGO>::T (&seen)[N], uint32_t ok) {
     uint32_t c = 0;
-    if constexpr (ALGO == ALGO_MSBFS) {
+    if constexpr (ms_masks(ALGO) != 0) {
+        constexpr int H = ms_masks(ALGO);
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-            const uint64_t m = (ok >> k) & 1 ? src(k) & ~seen[k] : 0;
-            if (!m) continue;
-            atomicOr(&a.vn[to[k]].y, (unsigned long long)m);
+            if (!((ok >> k) & 1)) continue;
+            const MaskOf<H> s = src(k);
+            bool any = false;
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                const uint64_t m = s.m[h] & ~seen[k].m[h];
+                if (!m) continue;
+                atomicOr(&a.vn[(uint64_t)to[k] * H + h].y, (unsigned long long)m);
+                any = true;
+            }
+            if (!any) continue;
             a.flag[to[k]] = 1;
             ++c;
         }
@@ -684,7 +729,7 @@ __device__ __forceinline__ uint32_t relax_group_body(const uint32_t *__restrict_
         uint64_t b, e;
         row_range(ptr, a.pmid, heavy, u, b, e);
         const auto s = load_src<ALGO>(a, u);
-        if (ALGO == ALGO_MSBFS && !s) continue;  // all of u's sources go bottom-up this round
+        if (!offers<ALGO>(s)) continue;  // all of u's sources go bottom-up this round
         for (uint64_t i = b + sub; i < e; i += (uint64_t)kRelaxBatch * LPV) {
             uint32_t to[kRelaxBatch], wt[kRelaxBatch];
             typename SrcOf<ALGO>::T seen[kRelaxBatch];
@@ -736,7 +781,7 @@ __device__ __forceinline__ uint32_t relax_hub_body(const uint64_t *__restrict__ 
         const uint64_t e = min(re, b + tile);
         const uint32_t cnt = (uint32_t)(e - b);
         const auto s = load_src<ALGO>(a, u);
-        if (ALGO == ALGO_MSBFS && !s) continue;  // block-uniform: u is the same for every thread
+        if (!offers<ALGO>(s)) continue;  // block-uniform: u is the same for every thread
         for (uint32_t k = threadIdx.x; k < cnt; k += kBlock) {
             if (WIDE)
                 ((uint2 *)s_edges)[k] = ((const uint2 *)edges)[b + k];
@@ -1469,13 +1514,14 @@ constexpr int kMsSums = 3 * kMsWidth;  // digest, reached, traversed per source
 
 // Start of a batch, one launch: masks, flags and partial sums cleared, the
 // traversal state set (levels, when kept, are cleared apart).
+template <int H>
 __global__ __launch_bounds__(kBlock) void k_ms_clear(ulonglong2 *__restrict__ vn, uint64_t *__restrict__ front,
                                                      uint8_t *__restrict__ flag, uint64_t V, uint64_t Vpad,
                                                      unsigned long long *__restrict__ part, uint64_t nparts,
                                                      RoundCtl *ctl, RoundCtl c) {
     const uint64_t tid = (uint64_t)blockIdx.x * kBlock + threadIdx.x, nth = (uint64_t)gridDim.x * kBlock;
     if (tid == 0) *ctl = c;
-    for (uint64_t v = tid; v < V; v += nth) {
+    for (uint64_t v = tid; v < H * V; v += nth) {
         vn[v] = make_ulonglong2(0, 0);
         front[v] = 0;
     }
@@ -1483,17 +1529,20 @@ __global__ __launch_bounds__(kBlock) void k_ms_clear(ulonglong2 *__restrict__ vn
     for (uint64_t i = tid; i < nparts; i += nth) part[i] = 0;
 }
 
-// Seeds up to 64 sources: bit j of the masks of source j, level 1, and its
-// terms in the sums of the first workgroup.
+// Seeds up to 64 H sources: bit j % 64 of mask j / 64 of source j, level 1,
+// and its terms in the sums of the first workgroup.
+template <int H>
 __global__ void k_ms_init(const uint32_t *__restrict__ src, uint32_t n, ulonglong2 *vn, uint64_t *front, uint8_t *flag,
-                          uint8_t *lvl, const uint64_t *__restrict__ ptr, unsigned long long *part) {
-    const uint32_t j = threadIdx.x;
-    if (j < n) {
-        const uint32_t s = src[j];
-        atomicOr(&vn[s].x, 1ull << j);
-        atomicOr((unsigned long long *)(front + s), 1ull << j);
+                          uint8_t *lvl, uint64_t V, const uint64_t *__restrict__ ptr, unsigned long long *part) {
+    const uint32_t j = threadIdx.x % kMsWidth, h = threadIdx.x / kMsWidth;
+    if (threadIdx.x < n) {
+        const uint32_t s = src[threadIdx.x];
+        const uint64_t at = (uint64_t)s * H + h;
+        atomicOr(&vn[at].x, 1ull << j);
+        atomicOr((unsigned long long *)(front + at), 1ull << j);
         flag[s] = 1;
-        if (lvl) lvl[(uint64_t)s * kMsWidth + j] = 1;
+        if (lvl) lvl[((uint64_t)h * V + s) * kMsWidth + j] = 1;
+        part += h * kMsSums;
         part[j] = d_mix64(((uint64_t)s << 32) | 1u);
         part[kMsWidth + j] = 1;
         part[2 * kMsWidth + j] = ptr[s + 1] - ptr[s];
@@ -1514,72 +1563,88 @@ __global__ void k_ms_init(const uint32_t *__restrict__ src, uint32_t n, ulonglon
 // with the terms per source, 172 now; one lane per vertex with a loop over
 // its sources and byte stores took 640, and a digest pass at the end 757).  The sums of a
 // workgroup go to its own slots of `part`.
-template <bool LEVELS>
+template <bool LEVELS, int H>
 __global__ __launch_bounds__(kBlock) void k_ms_commit(uint8_t *__restrict__ flag, uint64_t V, ulonglong2 *__restrict__ vn,
                                                       uint64_t *__restrict__ front, uint8_t *__restrict__ lvl,
                                                       const uint64_t *__restrict__ ptr,
                                                       const uint32_t *__restrict__ deg,
                                                       const uint32_t *__restrict__ hdeg, RoundCtl *ctl,
                                                       unsigned long long *__restrict__ part, RoundClock *clk) {
-    __shared__ unsigned long long s_sum[kMsSums];
+    constexpr int G = kMsGroups / H;
+    __shared__ unsigned long long s_sum[H * kMsSums];
     clock_stamp(clk, kClkRelax, kClkOther);
-    for (int i = threadIdx.x; i < kMsSums; i += kBlock) s_sum[i] = 0;
+    for (int i = threadIdx.x; i < H * kMsSums; i += kBlock) s_sum[i] = 0;
     const uint32_t lv32 = ctl->rounds + 1;
     const uint32_t level = min(lv32, 255u);
     const int lane = threadIdx.x & (kWave - 1);
     const uint64_t nwaves = (uint64_t)gridDim.x * (kBlock / kWave);
-    uint64_t h = 0, fc = 0;  // digest; reached << kMsFcShift | traversed
+    uint64_t sum[H], fc[H];  // digest; reached << kMsFcShift | traversed
+#pragma unroll
+    for (int h = 0; h < H; ++h) sum[h] = fc[h] = 0;
     __syncthreads();
     for (uint64_t g0 = (uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; g0 * kWave < V;
-         g0 += kMsGroups * nwaves) {
-        bool on[kMsGroups];
-        uint64_t nw[kMsGroups], dv[kMsGroups], mix[kMsGroups];
+         g0 += G * nwaves) {
+        bool on[G];
+        uint64_t nw[G][H], dv[G], mix[G];
 #pragma unroll
-        for (int k = 0; k < kMsGroups; ++k) {
+        for (int k = 0; k < G; ++k) {
             const uint64_t v = (g0 + k * nwaves) * kWave + lane;
             on[k] = v < V && flag[v];
         }
-        ulonglong2 x[kMsGroups];
+        ulonglong2 x[G][H];
 #pragma unroll
-        for (int k = 0; k < kMsGroups; ++k) {
+        for (int k = 0; k < G; ++k) {
             const uint64_t v = (g0 + k * nwaves) * kWave + lane;
-            x[k] = on[k] ? vn[v] : make_ulonglong2(0, 0);
+#pragma unroll
+            for (int h = 0; h < H; ++h) x[k][h] = on[k] ? vn[v * H + h] : make_ulonglong2(0, 0);
             dv[k] = on[k] ? round_deg(deg, hdeg, ptr, nullptr, false, v) : 0;
         }
 #pragma unroll
-        for (int k = 0; k < kMsGroups; ++k) {
+        for (int k = 0; k < G; ++k) {
             const uint64_t v = (g0 + k * nwaves) * kWave + lane;
-            nw[k] = x[k].y & ~x[k].x;
+            uint64_t any = 0;
+#pragma unroll
+            for (int h = 0; h < H; ++h) any |= nw[k][h] = x[k][h].y & ~x[k][h].x;
             mix[k] = d_mix64((v << 32) | level);
             dv[k] |= 1ull << kMsFcShift;
             if (!on[k]) continue;
-            vn[v] = make_ulonglong2(x[k].x | nw[k], 0);
-            front[v] = nw[k];
-            if (!nw[k]) flag[v] = 0;
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                vn[v * H + h] = make_ulonglong2(x[k][h].x | nw[k][h], 0);
+                front[v * H + h] = nw[k][h];
+            }
+            if (!any) flag[v] = 0;
         }
 #pragma unroll
-        for (int k = 0; k < kMsGroups; ++k) {
-            uint64_t todo = __ballot(nw[k] != 0);
-            if (todo && lv32 > 255) ctl->overflow = 1;
-            while (todo) {
-                const int l = __builtin_ctzll(todo);
-                todo &= todo - 1;
-                const uint64_t m = wave_read_u64(nw[k], l), d = wave_read_u64(dv[k], l), z = wave_read_u64(mix[k], l);
-                if (__builtin_amdgcn_inverse_ballot_w64(m)) {
-                    h += z;
-                    fc += d;
-                    if (LEVELS) lvl[((g0 + k * nwaves) * kWave + l) * kMsWidth + lane] = (uint8_t)level;
+        for (int k = 0; k < G; ++k)
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                uint64_t todo = __ballot(nw[k][h] != 0);
+                if (todo && lv32 > 255) ctl->overflow = 1;
+                while (todo) {
+                    const int l = __builtin_ctzll(todo);
+                    todo &= todo - 1;
+                    const uint64_t m = wave_read_u64(nw[k][h], l), d = wave_read_u64(dv[k], l), z = wave_read_u64(mix[k], l);
+                    if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+                        sum[h] += z;
+                        fc[h] += d;
+                        if (LEVELS)
+                            lvl[((uint64_t)h * V + (g0 + k * nwaves) * kWave + l) * kMsWidth + lane] = (uint8_t)level;
+                    }
                 }
             }
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+        if (__ballot(fc[h] != 0)) {
+            unsigned long long *const o = s_sum + h * kMsSums;
+            atomicAdd(&o[lane], (unsigned long long)sum[h]);
+            atomicAdd(&o[kMsWidth + lane], (unsigned long long)(fc[h] >> kMsFcShift));
+            atomicAdd(&o[2 * kMsWidth + lane], (unsigned long long)(fc[h] & ((1ull << kMsFcShift) - 1)));
         }
-    }
-    if (__ballot(fc != 0)) {
-        atomicAdd(&s_sum[lane], (unsigned long long)h);
-        atomicAdd(&s_sum[kMsWidth + lane], (unsigned long long)(fc >> kMsFcShift));
-        atomicAdd(&s_sum[2 * kMsWidth + lane], (unsigned long long)(fc & ((1ull << kMsFcShift) - 1)));
-    }
     __syncthreads();
-    if (threadIdx.x < kMsSums && s_sum[threadIdx.x]) part[(uint64_t)blockIdx.x * kMsSums + threadIdx.x] += s_sum[threadIdx.x];
+    for (int i = threadIdx.x; i < H * kMsSums; i += kBlock)
+        if (s_sum[i]) part[(uint64_t)blockIdx.x * H * kMsSums + i] += s_sum[i];
 }
 
 // The sources' sums over the commit's workgroups; folds the batch's work
@@ -1592,7 +1657,8 @@ __global__ __launch_bounds__(1024) void k_ms_sum(const unsigned long long *__res
     const uint32_t col = blockIdx.x * kMsWidth + threadIdx.x % kMsWidth;
     if (blockIdx.x == 0) fold_spread(spread, counters);
     uint64_t x = 0;
-    for (uint32_t b = threadIdx.x / kMsWidth; b < n; b += 1024 / kMsWidth) x += part[(uint64_t)b * kMsSums + col];
+    const uint64_t row = (uint64_t)gridDim.x * kMsWidth;  // a workgroup of this kernel per 64 sums
+    for (uint32_t b = threadIdx.x / kMsWidth; b < n; b += 1024 / kMsWidth) x += part[b * row + col];
     s[threadIdx.x] = x;
     __syncthreads();
     if (threadIdx.x < kMsWidth) {
@@ -2574,8 +2640,10 @@ static void gather(DeviceState *d, const og_graph *g, uint32_t ndyn, uint64_t c0
     else d->pool->run(part);
 }
 
+template <int ALGO>
 static RelaxArgs relax_args(DeviceState *d) {
-    return RelaxArgs{d->d_val, d->fr.flag, d->d_vn, d->d_front, d->wbits, nullptr, d->run_pmid};
+    const DeviceState::MsState &m = d->d_ms[ms_masks(ALGO) == 2];
+    return RelaxArgs{d->d_val, d->fr.flag, m.vn, m.front, d->wbits, nullptr, d->run_pmid};
 }
 
 // Grids of device-count launches: the kernels stride over whatever count
@@ -2641,12 +2709,12 @@ static bool launch_static(DeviceState *d, const FrontierInfo *hfi, const Span &s
     if (hfi && !(hfi->n[0] | hfi->n[1] | hfi->n[2])) return false;
     if ((d->flags & OG_PLAN_NO_OVERLAP) || d->plan.vsplit >= d->V) {  // nothing to overlap with
         span(kClsStat, d->s_compute,
-             [&] { launch_static_relax<ALGO, W>(d, d->fr, hfi, relax_args(d), d->s_compute); });
+             [&] { launch_static_relax<ALGO, W>(d, d->fr, hfi, relax_args<ALGO>(d), d->s_compute); });
         return false;
     }
     OG_HIP(hipEventRecord(d->ev_fork, d->s_compute));
     OG_HIP(hipStreamWaitEvent(d->s_static, d->ev_fork, 0));
-    span(kClsStat, d->s_static, [&] { launch_static_relax<ALGO, W>(d, d->fr, hfi, relax_args(d), d->s_static); });
+    span(kClsStat, d->s_static, [&] { launch_static_relax<ALGO, W>(d, d->fr, hfi, relax_args<ALGO>(d), d->s_static); });
     OG_HIP(hipEventRecord(d->ev_static, d->s_static));
     return true;
 }
@@ -2655,7 +2723,7 @@ template <int ALGO, bool W, bool PACKED, bool DIRECT>
 static void launch_dyn(DeviceState *d, unsigned grid, const void *src, uint64_t c0, uint64_t c1) {
     hipLaunchKernelGGL((k_relax_dyn<ALGO, W, PACKED, DIRECT>), dim3(grid), dim3(kBlock), 0, d->s_compute, d->fr.list,
                        d->fr.info, d->fr.doff, src, c0, c1, d->d_ptr, d->dyn_base, (const void *)d->d_staging,
-                       DIRECT ? (const int64_t *)d->d_rdelta : nullptr, d->wbits, relax_args(d),
+                       DIRECT ? (const int64_t *)d->d_rdelta : nullptr, d->wbits, relax_args<ALGO>(d),
                        DIRECT ? (const uint64_t *)d->d_lpos : nullptr, d->split_nl, d->plan.vsplit,
                        DIRECT && c0 == 0 ? (const uint32_t *)d->fr.dchunk : nullptr, DIRECT ? d->lbits : 0u, d->fr.spread);
 }
@@ -2667,7 +2735,7 @@ static void launch_dyn(DeviceState *d, unsigned grid, const void *src, uint64_t 
 template <int ALGO, bool W, bool PK, int LPV>
 static void launch_round_lpv(DeviceState *d, const RoundRelax &r, unsigned grid, size_t lds) {
     hipLaunchKernelGGL((k_relax_round<ALGO, W, PK, LPV>), dim3(grid), dim3(kBlock), lds, d->s_compute, r,
-                       relax_args(d));
+                       relax_args<ALGO>(d));
 }
 
 template <int ALGO, bool W, bool PK>
@@ -2834,7 +2902,7 @@ static bool run_ring(DeviceState *d, const og_graph *g, const FrontierInfo &fi, 
         auto relax = [&](auto kernel) {
             if (grid)
                 hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), 0, s, e0, e1, d->d_ring_tab + ch.tab, d->fr.info,
-                                   d->d_ptr, stage, lr->lbits, ch.first, d->d_mark, relax_args(d), d->fr.spread);
+                                   d->d_ptr, stage, lr->lbits, ch.first, d->d_mark, relax_args<ALGO>(d), d->fr.spread);
         };
         if (W && d->packed) relax(k_relax_range<ALGO, W, true>);
         else relax(k_relax_range<ALGO, W, false>);
@@ -2895,7 +2963,7 @@ static void run_dynamic(DeviceState *d, const og_graph *g, const FrontierInfo &f
 // Algorithmic bytes per relaxed edge: column (+ weight) and the target state.
 template <int ALGO, bool W>
 constexpr uint64_t edge_bytes_alg() {
-    return ALGO == ALGO_MSBFS ? 12ull : (ALGO == ALGO_SSSP ? 12ull : 8ull);
+    return ms_masks(ALGO) ? 4ull + 8ull * ms_masks(ALGO) : (ALGO == ALGO_SSSP ? 12ull : 8ull);
 }
 
 constexpr int kRoundBatch = 4;     // device-driven rounds enqueued per host check
@@ -2981,7 +3049,7 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
                     span(kClsDyn, s, [&] { launch_dyn_any<ALGO, W>(d, d->lbits ? d->hd_link : d->hd_dyn, 0, ~0ull, 0, true); });
                     OG_HIP(hipStreamWaitEvent(d->s_static, d->ev_fork, 0));
                     span(kClsStat, d->s_static,
-                         [&] { launch_static_relax<ALGO, W>(d, d->fr, nullptr, relax_args(d), d->s_static); });
+                         [&] { launch_static_relax<ALGO, W>(d, d->fr, nullptr, relax_args<ALGO>(d), d->s_static); });
                     OG_HIP(hipEventRecord(d->ev_static, d->s_static));
                     joined = true;
                 } else {
@@ -3213,91 +3281,129 @@ static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats 
     if (stats) *stats = st;
 }
 
-// Multi-source BFS: sources in batches of 64; per vertex, u64 masks of the
-// sources that reached it, that were offered to it this round (side by side)
-// and whose frontier holds it; levels as u8 per (vertex, source) when the
+// Multi-source BFS: sources in batches of 64, two batches walking the graph
+// together while more than 64 sources are left; per vertex and batch, u64 masks
+// of the sources that reached it, that were offered to it this round (side by
+// side) and whose frontier holds it; levels as u8 per (vertex, source) when the
 // caller wants them.
 constexpr uint64_t kExtractBytes = 256ull << 20;  // device buffer of levels on their way to the host, at most
+
+// One traversal from nb <= 64 H sources.
+template <int H, bool W>
+static void ms_batch(og_graph *g, DeviceState *d, const uint32_t *sources, uint32_t nb, uint32_t *levels,
+                     uint64_t *checksums, uint64_t *reached, og_run_stats &st, RunTimers &tm, double &gather_ms,
+                     double &overload_wall, const Stopwatch &total, double &device_ms) {
+    constexpr int ALGO = H == 1 ? ALGO_MSBFS : ALGO_MSBFS2;
+    const uint64_t V = d->V;
+    hipStream_t s = d->s_compute;
+    DeviceState::MsState &m = d->d_ms[H - 1];
+    const unsigned cgrid =
+        (unsigned)std::min<uint64_t>(kMsCommitGrid, std::max<uint64_t>(1, (V + kBlock - 1) / kBlock));
+    if (!m.sum) {
+        if (!m.vn) m.vn = (ulonglong2 *)d->dalloc(H * V * 16);
+        if (!m.front) m.front = (uint64_t *)d->dalloc(H * V * 8);
+        if (!m.src) m.src = (uint32_t *)d->dalloc(H * kMsWidth * 4);
+        if (!m.part) m.part = (unsigned long long *)d->dalloc((uint64_t)cgrid * H * kMsSums * 8);
+        m.sum = (unsigned long long *)d->dalloc(H * kMsSums * 8);
+    }
+    if (levels && !m.lvl) m.lvl = (uint8_t *)d->dalloc(H * V * kMsWidth);
+    if (levels && !d->d_extract) {
+        d->extract_cap = (uint32_t)std::min<uint64_t>(kMsWidth, std::max<uint64_t>(1, kExtractBytes / (V * 4)));
+        d->d_extract = (uint32_t *)d->dalloc((uint64_t)d->extract_cap * V * 4);
+    }
+    uint8_t *const lvl = levels ? m.lvl : nullptr;
+    std::vector<unsigned long long> hsum(H * kMsSums);
+    if (lvl) OG_HIP(hipMemsetAsync(lvl, 0, H * V * kMsWidth, s));
+    OG_HIP(hipMemcpyAsync(m.src, sources, nb * 4, hipMemcpyHostToDevice, s));
+    auto begin = [&](const RoundCtl &c) {
+        hipLaunchKernelGGL(k_ms_clear<H>, dim3(fill_grid(V)), dim3(kBlock), 0, s, m.vn, m.front, d->fr.flag, V, d->Vpad,
+                           m.part, (uint64_t)cgrid * H * kMsSums, d->fr.ctl, c);
+        hipLaunchKernelGGL(k_ms_init<H>, dim3(1), dim3(H * kMsWidth), 0, s, m.src, nb, m.vn, m.front, d->fr.flag, lvl, V,
+                           d->d_ptr, m.part);
+        OG_HIP(hipGetLastError());
+    };
+    auto commit = [&](RoundClock *clk) {
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(cgrid), dim3(kBlock), 0, s, d->fr.flag, V, m.vn, m.front, lvl, d->d_ptr,
+                               d->d_deg, d->deg_heavy(), d->fr.ctl, m.part, clk);
+        };
+        if (lvl) launch(k_ms_commit<true, H>);
+        else launch(k_ms_commit<false, H>);
+        OG_HIP(hipGetLastError());
+    };
+    frontier_loop<ALGO, W>(g, d, st, tm, gather_ms, overload_wall, begin, commit, false, lvl != nullptr);
+    hipLaunchKernelGGL(k_ms_sum, dim3(3 * H), dim3(1024), 0, s, m.part, cgrid, m.sum, d->fr.counters, d->fr.spread,
+                       tm.clocked >= 0 ? d->fr.clk : nullptr);
+    OG_HIP(hipGetLastError());
+    OG_HIP(hipMemcpyAsync(d->fr.h_blk, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
+    OG_HIP(hipMemcpyAsync(hsum.data(), m.sum, H * kMsSums * 8, hipMemcpyDeviceToHost, s));
+    OG_HIP(hipStreamSynchronize(s));
+    device_ms = total.ms();
+    collect_loop<ALGO, W>(d, st);
+    for (uint32_t j = 0; j < nb; ++j) {
+        const unsigned long long *const x = hsum.data() + j / kMsWidth * kMsSums + j % kMsWidth;
+        if (checksums) checksums[j] = x[0];
+        if (reached) reached[j] = x[kMsWidth];
+        st.reached += x[kMsWidth];
+        st.traversed_edges += x[2 * kMsWidth];
+        st.checksum += x[0];
+    }
+    if (!levels) return;
+    for (uint32_t j = 0; j < nb;) {  // groups of sources of one mask
+        const uint32_t h = j / kMsWidth, j0 = j % kMsWidth;
+        const uint32_t nj = std::min({d->extract_cap, nb - j, (uint32_t)kMsWidth - j0});
+        hipLaunchKernelGGL(k_ms_extract, dim3((unsigned)std::min<uint64_t>(8192, (V + kWave - 1) / kWave)), dim3(kBlock),
+                           0, s, lvl + (uint64_t)h * V * kMsWidth, V, j0, nj, d->d_extract);
+        OG_HIP(hipGetLastError());
+        copy_to_host(d, levels + (uint64_t)j * V, d->d_extract, (uint64_t)nj * V * 4, s);
+        j += nj;
+    }
+}
+
+// Whether two batches of sources walk the graph together.  A dense round costs
+// the reading of the edges (over the link, or random reads of the targets'
+// masks, whose line two batches share), so a walk with two masks per vertex
+// takes little more than one with one: R-MAT 4 M vertices 67 M edges, 128
+// sources, 0.4 of the edges in HBM: 12.0 -> 6.8 ms, in HBM 6.1 -> 4.4; 4096
+// vertices 0.48 -> 0.26; 72 sources 11.0 -> 6.4, 5.4 -> 4.0, 0.46 -> 0.25.  It was faster at
+// every size and for as few as 8 sources in the second batch; the line is the
+// memory that the wider masks (and levels) take, an eighth of what is free.
+static bool ms_wide(const DeviceState *d, uint32_t left, bool levels) {
+    if (left <= kMsWidth) return false;
+    const DeviceState::MsState &m = d->d_ms[1];
+    const uint64_t more = (m.sum ? 0 : 48 * d->V) + (levels && !m.lvl ? 2 * kMsWidth * d->V : 0);
+    if (!more) return true;
+    size_t free = 0, all = 0;
+    OG_HIP(hipMemGetInfo(&free, &all));
+    return more <= free / 8;
+}
 
 template <bool W>
 static void run_msbfs(og_graph *g, const uint32_t *sources, uint32_t n, uint32_t *levels, uint64_t *checksums,
                       uint64_t *reached, og_run_stats *stats) {
     DeviceState *d = g->dev;
-    const uint64_t V = d->V;
     hipStream_t s = d->s_compute;
-    const unsigned cgrid =
-        (unsigned)std::min<uint64_t>(kMsCommitGrid, std::max<uint64_t>(1, (V + kBlock - 1) / kBlock));
-    if (!d->d_vn) {
-        d->d_vn = (ulonglong2 *)d->dalloc(V * 16);
-        d->d_front = (uint64_t *)d->dalloc(V * 8);
-        d->d_msrc = (uint32_t *)d->dalloc(kMsWidth * 4);
-        d->d_msum = (unsigned long long *)d->dalloc(kMsSums * 8);
-        d->d_mpart = (unsigned long long *)d->dalloc((uint64_t)cgrid * kMsSums * 8);
-    }
-    if (levels && !d->d_mlvl) {
-        d->d_mlvl = (uint8_t *)d->dalloc(V * kMsWidth);
-        d->extract_cap = (uint32_t)std::min<uint64_t>(kMsWidth, std::max<uint64_t>(1, kExtractBytes / (V * 4)));
-        d->d_extract = (uint32_t *)d->dalloc((uint64_t)d->extract_cap * V * 4);
-    }
-    uint8_t *const lvl = levels ? d->d_mlvl : nullptr;
-    std::vector<unsigned long long> hsum(kMsSums);
     og_run_stats st{};
     st.approach = (uint32_t)d->approach;
     RunTimers tm;
     d->events.reset();
-    double gather_ms = 0, overload_wall = 0;
+    double gather_ms = 0, overload_wall = 0, device_ms = 0;
     OG_HIP(hipStreamSynchronize(d->s_copy));
     OG_HIP(hipStreamSynchronize(d->s_static));
     OG_HIP(hipStreamSynchronize(s));
     Stopwatch total;
     OG_HIP(hipMemsetAsync(d->fr.blk, 0, sizeof(RunBlock), s));
     OG_HIP(hipMemsetAsync(d->fr.spread, 0, kSpreadWords * 8, s));
-    double device_ms = 0;
-    for (uint32_t b0 = 0; b0 < n; b0 += kMsWidth) {
-        const uint32_t nb = std::min<uint32_t>(kMsWidth, n - b0);
-        if (lvl) OG_HIP(hipMemsetAsync(lvl, 0, V * kMsWidth, s));
-        OG_HIP(hipMemcpyAsync(d->d_msrc, sources + b0, nb * 4, hipMemcpyHostToDevice, s));
-        auto begin = [&](const RoundCtl &c) {
-            hipLaunchKernelGGL(k_ms_clear, dim3(fill_grid(V)), dim3(kBlock), 0, s, d->d_vn, d->d_front, d->fr.flag, V,
-                               d->Vpad, d->d_mpart, (uint64_t)cgrid * kMsSums, d->fr.ctl, c);
-            hipLaunchKernelGGL(k_ms_init, dim3(1), dim3(kMsWidth), 0, s, d->d_msrc, nb, d->d_vn, d->d_front,
-                               d->fr.flag, lvl, d->d_ptr, d->d_mpart);
-            OG_HIP(hipGetLastError());
+    for (uint32_t b0 = 0, nb = 0; b0 < n; b0 += nb) {
+        const bool wide = ms_wide(d, n - b0, levels != nullptr);
+        nb = std::min<uint32_t>(wide ? 2 * kMsWidth : kMsWidth, n - b0);
+        auto run = [&](auto batch) {
+            batch(g, d, sources + b0, nb, levels ? levels + (uint64_t)b0 * d->V : nullptr,
+                  checksums ? checksums + b0 : nullptr, reached ? reached + b0 : nullptr, st, tm, gather_ms,
+                  overload_wall, total, device_ms);
         };
-        auto commit = [&](RoundClock *clk) {
-            if (lvl)
-                hipLaunchKernelGGL(k_ms_commit<true>, dim3(cgrid), dim3(kBlock), 0, s, d->fr.flag, V, d->d_vn,
-                                   d->d_front, lvl, d->d_ptr, d->d_deg, d->deg_heavy(), d->fr.ctl, d->d_mpart, clk);
-            else
-                hipLaunchKernelGGL(k_ms_commit<false>, dim3(cgrid), dim3(kBlock), 0, s, d->fr.flag, V, d->d_vn,
-                                   d->d_front, lvl, d->d_ptr, d->d_deg, d->deg_heavy(), d->fr.ctl, d->d_mpart, clk);
-            OG_HIP(hipGetLastError());
-        };
-        frontier_loop<ALGO_MSBFS, W>(g, d, st, tm, gather_ms, overload_wall, begin, commit, false, lvl != nullptr);
-        hipLaunchKernelGGL(k_ms_sum, dim3(3), dim3(1024), 0, s, d->d_mpart, cgrid, d->d_msum,
-                           d->fr.counters, d->fr.spread, tm.clocked >= 0 ? d->fr.clk : nullptr);
-        OG_HIP(hipGetLastError());
-        OG_HIP(hipMemcpyAsync(d->fr.h_blk, d->fr.blk, sizeof(RunBlock), hipMemcpyDeviceToHost, s));
-        OG_HIP(hipMemcpyAsync(hsum.data(), d->d_msum, kMsSums * 8, hipMemcpyDeviceToHost, s));
-        OG_HIP(hipStreamSynchronize(s));
-        device_ms = total.ms();
-        collect_loop<ALGO_MSBFS, W>(d, st);
-        for (uint32_t j = 0; j < nb; ++j) {
-            if (checksums) checksums[b0 + j] = hsum[j];
-            if (reached) reached[b0 + j] = hsum[kMsWidth + j];
-            st.reached += hsum[kMsWidth + j];
-            st.traversed_edges += hsum[2 * kMsWidth + j];
-            st.checksum += hsum[j];
-        }
-        if (levels)
-            for (uint32_t j = 0; j < nb; j += d->extract_cap) {
-                const uint32_t nj = std::min(d->extract_cap, nb - j);
-                hipLaunchKernelGGL(k_ms_extract,
-                                   dim3((unsigned)std::min<uint64_t>(8192, (V + kWave - 1) / kWave)), dim3(kBlock), 0, s,
-                                   lvl, V, j, nj, d->d_extract);
-                OG_HIP(hipGetLastError());
-                copy_to_host(d, levels + (uint64_t)(b0 + j) * V, d->d_extract, (uint64_t)nj * V * 4, s);
-            }
+        if (wide) run(ms_batch<2, W>);
+        else run(ms_batch<1, W>);
     }
     st.total_ms = device_ms;
     if (!n) *d->fr.h_blk = RunBlock{};

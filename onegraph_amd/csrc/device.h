@@ -300,14 +300,12 @@ struct MemPool {
 
 // The dynamic region as chunks of whole rows that cross the link in vertex
 // order, straight from the host copy (no gather), through a ring of `ring`
-// slots of `slot` words in the staging share: PageRank's iterations, and rounds
-// of the copy loader that relax much of the region.
+// slots of `slot` words in the staging share (PageRank's iterations).
 struct LinkRing {
     struct Chunk {
         uint32_t va, vb;       // vertices
         uint64_t word, words;  // of the host source
         uint32_t first;        // bits before the first edge
-        uint64_t tab = 0;      // its entries in DeviceState::d_ring_tab
     };
     std::vector<Chunk> chunks;
     uint32_t ring = 0;
@@ -379,6 +377,7 @@ struct DeviceState {
     bool packed = false;
     uint32_t wbits = 0;
     uint32_t deb = 4;                // bytes per dynamic-region edge on the link (= eb)
+    bool in_place = false;           // traversals read the dynamic region in pinned host memory
     uint64_t dyn_base = 0;           // first edge of the dynamic region (= ptr[vsplit])
     const void *h_dyn = nullptr;     // host source of dynamic edges (packed copy or the CSR)
     const void *hd_dyn = nullptr;    // the same, as a device address (zero-copy mode)
@@ -398,8 +397,6 @@ struct DeviceState {
     const uint32_t *h_link = nullptr;   // pinned
     const void *hd_link = nullptr;      // the same, as a device address
     std::shared_ptr<LinkRing> link_ring;  // built on first use
-    uint8_t *d_mark = nullptr;       // V: vertices a ring round relaxes (zero between rounds)
-    uint32_t *d_ring_tab = nullptr;  // rows of the ring chunks' workgroups (k_relax_range)
     uint64_t dyn_resident = 0;       // zero-copy: dynamic edges held in d_staging (whole chunks)
     int64_t *d_rdelta = nullptr;     // zero-copy: per chunk of kResChunk vertices (index v >> kResChunkShift),
                                      // d_staging index - host-array position, or kNotResident; two per

@@ -983,72 +983,6 @@ __global__ __launch_bounds__(kBlock) void k_relax_dyn(const uint32_t *__restrict
     if (DIRECT) wave_count(spread, kHbmEdges, h);
 }
 
-// Marks the dynamic list's vertices for k_relax_range (or unmarks them).
-__global__ void k_mark(const uint32_t *__restrict__ dlist, uint32_t n, uint8_t *__restrict__ mark, uint8_t x) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) mark[dlist[i]] = x;
-}
-
-// Ring chunk of a dynamic round: relaxes the edges [e0, e1) whose source is
-// marked.  The chunk's whole rows sit in `stage` (whole edges, or with lbits a
-// stream of lbits-bit words from bit `first` on).  Edge-parallel like
-// relax_dyn_body: a workgroup takes kDynEdgesPerBlock consecutive edges, whose
-// rows `tab` (the vertex of each workgroup's first edge, and of the chunk's
-// last) bounds, and finds an edge's row by binary search, in LDS unless empty
-// rows make the slice too long.  A chunk holds some 10^5 edges, so what bounds
-// it is the longest chain of dependent reads (rows by groups of lanes, long rows
-// by workgroups: 40-160 us per chunk of 660 K edges, this way 17-35).
-struct RangeLds {
-    uint64_t off[kDynEdgesPerBlock + 2];
-};
-template <int ALGO, bool W, bool PK>
-__global__ __launch_bounds__(kBlock) void k_relax_range(uint64_t e0, uint64_t e1, const uint32_t *__restrict__ tab,
-                                                        const FrontierInfo *__restrict__ info,
-                                                        const uint64_t *__restrict__ ptr,
-                                                        const uint32_t *__restrict__ stage, uint32_t lbits,
-                                                        uint32_t first, const uint8_t *__restrict__ mark, RelaxArgs a,
-                                                        unsigned long long *spread) {
-    __shared__ RangeLds L;
-    const bool heavy = info->heavy != 0;
-    const uint64_t x0 = e0 + (uint64_t)blockIdx.x * kDynEdgesPerBlock, x1 = min(x0 + kDynEdgesPerBlock, e1);
-    const uint32_t u0 = tab[blockIdx.x], nv = tab[blockIdx.x + 1] - u0 + 1;
-    const bool local = nv <= kDynEdgesPerBlock + 1;
-    if (local)
-        for (uint32_t k = threadIdx.x; k <= nv; k += kBlock) L.off[k] = ptr[(uint64_t)u0 + k];
-    __syncthreads();
-    uint32_t to[kDynEdgesPerThread], wt[kDynEdgesPerThread], ok = 0;
-    typename SrcOf<ALGO>::T sv[kDynEdgesPerThread], seen[kDynEdgesPerThread];
-#pragma unroll
-    for (int j = 0; j < kDynEdgesPerThread; ++j) {
-        const uint64_t x = x0 + threadIdx.x + (uint64_t)j * kBlock;
-        to[j] = 0;
-        wt[j] = 0;
-        sv[j] = 0;
-        seen[j] = 0;
-        if (x >= x1) continue;
-        uint32_t lo = 0, hi = nv;  // largest row that starts at or before x
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if ((local ? L.off[mid] : ptr[(uint64_t)u0 + mid]) <= x) lo = mid; else hi = mid;
-        }
-        const uint32_t u = u0 + lo;
-        if (!mark[u] || (a.pmid && (x >= a.pmid[u]) != heavy)) continue;
-        sv[j] = load_src<ALGO>(a, u);
-        ok |= 1u << j;
-        if (lbits) {
-            const uint32_t w = link_word(stage, x - e0, lbits, first);
-            to[j] = W ? w >> a.wbits : w;
-            wt[j] = W ? w & ((1u << a.wbits) - 1u) : 1u;
-        } else {
-            load_edge<W, PK>(stage, x - e0, a.wbits, to[j], wt[j]);
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < kDynEdgesPerThread; ++j)
-        if ((ok >> j) & 1) seen[j] = peek<ALGO>(a, to[j]);
-    const uint32_t c = commit<ALGO, kDynEdgesPerThread>(a, [&](int j) { return sv[j]; }, to, wt, seen, ok);
-    wave_count(spread, kUpdDynamic, c);
-}
-
 // One round's relax in a single launch: static bins 0 and 1, hub tiles and
 // the zero-copy dynamic region side by side, so a device-driven round needs
 // no second stream (the fork and join of which cost tens of microseconds per
@@ -2383,7 +2317,20 @@ static void prepare_impl(og_graph *g, og_approach approach, const og_plan_params
         if (pl.vsplit < V) {
             // PageRank streams its dynamic region through the slots (vertex-
             // aligned chunks), so a pull-layout graph always gets them
-            const bool zc = (p.flags & OG_PLAN_ZERO_COPY) != 0 && g->kind != OG_KIND_PULL;
+            //
+            // Traversals read the dynamic rows where they are, in pinned host
+            // memory, also when the copy loader was asked for: an active row
+            // crosses the link once at the link's speed and no round waits
+            // for the host, where gathering took the host's threads (16 GB/s)
+            // and two round trips per round (BFS R-MAT 1 M, a quarter of the
+            // edges on the device: gathered and copied 5.0 ms, rows moved
+            // whole through a ring of slots 2.9, in place 1.1).  Gathered
+            // chunks stay for graphs in pageable memory and for the A/B flags.
+            const bool zc = g->kind != OG_KIND_PULL &&
+                            ((p.flags & OG_PLAN_ZERO_COPY) ||
+                             (!(p.flags & (OG_PLAN_NO_OVERLAP | OG_PLAN_NO_FUSE)) &&
+                              (d->packed || (eb == 8 ? g->pinned_wedges : g->pinned_cols))));
+            d->in_place = zc;
             // Staging slots: gather, copy and relax of consecutive chunks
             // overlap.  Chunks of ~kSlotTargetBytes: smaller ones cost more
             // in per-chunk gather dispatch and launches than they save in
@@ -2396,10 +2343,10 @@ static void prepare_impl(og_graph *g, og_approach approach, const og_plan_params
             while (ns > 2 && pl.staging_edges / ns < maxdyn) --ns;
             d->nslots = ns;
             d->slot_edges = pl.staging_edges / ns;
+            if (d->slot_edges == 0 && (!zc || !(p.flags & OG_PLAN_ZERO_COPY)))
+                raise(OG_EBUDGET, "edge budget leaves %llu staging edges for %llu dynamic-region edges",
+                      (unsigned long long)pl.staging_edges, (unsigned long long)(E - g->ptr[pl.vsplit]));
             if (!zc) {
-                if (d->slot_edges == 0)
-                    raise(OG_EBUDGET, "edge budget leaves %llu staging edges for %llu dynamic-region edges",
-                          (unsigned long long)pl.staging_edges, (unsigned long long)(E - g->ptr[pl.vsplit]));
                 d->d_staging = d->dalloc((uint64_t)ns * d->slot_edges * eb);
                 d->h_stage.resize(ns);
                 d->ev_h2d.assign(ns, nullptr);
@@ -2835,86 +2782,6 @@ static void launch_dyn_any(DeviceState *d, const void *src, uint64_t c0, uint64_
     OG_HIP(hipGetLastError());
 }
 
-// A dynamic round of the copy loader that relaxes much of the region: its rows
-// cross the link whole, in vertex order, through the chunk ring, and the relax
-// picks the active ones.  Against the gather, which the host's threads build at
-// about 16 GB/s and a list and prefix copied back first, it moves the rest of the
-// region too, at the link's speed and in the link format: it pays from about
-// kRingShare of the region's edges on.  (BFS R-MAT 1 M, a quarter of the edges on
-// the device: 4.4 -> 3.0 ms.)  False: not such a round, or a row is too long.
-constexpr double kRingShare = 0.125;
-
-template <int ALGO, bool W>
-static bool run_ring(DeviceState *d, const og_graph *g, const FrontierInfo &fi, RunTimers &tm, og_run_stats &st) {
-    if ((d->flags & OG_PLAN_NO_OVERLAP) || (double)fi.dyn_deg < kRingShare * (double)(g->E - d->dyn_base)) return false;
-    LinkRing *lr = link_ring(d, g);
-    if (!lr) return false;
-    hipStream_t s = d->s_compute;
-    if (!d->d_mark) {
-        d->d_mark = (uint8_t *)d->dalloc(d->V);
-        hipLaunchKernelGGL(k_fill_u8, dim3(fill_grid(d->V)), dim3(256), 0, s, d->d_mark, d->V, (uint8_t)0);
-        // per chunk, the row of every kDynEdgesPerBlock-th edge and of the last
-        std::vector<uint32_t> tab;
-        for (LinkRing::Chunk &ch : lr->chunks) {
-            ch.tab = tab.size();
-            const uint64_t a0 = g->ptr[ch.va], a1 = g->ptr[ch.vb];
-            uint64_t v = ch.va;
-            for (uint64_t x = a0; x < a1; x += kDynEdgesPerBlock) {
-                while (g->ptr[v + 1] <= x) ++v;
-                tab.push_back((uint32_t)v);
-            }
-            if (a1 > a0) {
-                while (g->ptr[v + 1] < a1) ++v;
-                tab.push_back((uint32_t)v);
-            }
-        }
-        d->d_ring_tab = (uint32_t *)d->dalloc(std::max<size_t>(tab.size(), 1) * 4);
-        OG_HIP(hipMemcpy(d->d_ring_tab, tab.data(), tab.size() * 4, hipMemcpyHostToDevice));
-    }
-    const uint32_t *dlist = d->fr.list + d->plan.vsplit;
-    hipLaunchKernelGGL(k_mark, dim3(fill_grid(fi.n[3])), dim3(256), 0, s, dlist, fi.n[3], d->d_mark, (uint8_t)1);
-    OG_HIP(hipGetLastError());
-    const uint64_t nc = lr->chunks.size();
-    auto copy = [&](uint64_t k) {  // consecutive copies on two streams: one's hand-over hides behind the other
-        const LinkRing::Chunk &ch = lr->chunks[k];
-        const uint32_t slot = (uint32_t)(k % lr->ring);
-        const hipStream_t on = k & 1 ? d->s_static : d->s_copy;
-        if (k >= lr->ring) OG_HIP(hipStreamWaitEvent(on, lr->ev_use[slot], 0));
-        if (ch.words)
-            OG_HIP(hipMemcpyAsync((uint32_t *)d->d_staging + slot * lr->slot, lr->src + ch.word, ch.words * 4,
-                                  hipMemcpyHostToDevice, on));
-        OG_HIP(hipEventRecord(lr->ev_h2d[slot], on));
-        st.h2d_bytes += ch.words * 4;
-        st.chunks++;
-    };
-    // one pair of events per round: a pair per chunk stalls the stream as long
-    // as the chunk's copy takes
-    EventSpan copies(d, &tm.copy, d->s_copy), relaxes(d, &tm.dyn, s);
-    uint64_t copied = 0;
-    while (copied < std::min<uint64_t>(lr->ring, nc)) copy(copied++);
-    for (uint64_t k = 0; k < nc; ++k) {
-        const LinkRing::Chunk &ch = lr->chunks[k];
-        const uint32_t slot = (uint32_t)(k % lr->ring);
-        const uint32_t *stage = (const uint32_t *)d->d_staging + slot * lr->slot;
-        const uint64_t e0 = g->ptr[ch.va], e1 = g->ptr[ch.vb];
-        const unsigned grid = (unsigned)((e1 - e0 + kDynEdgesPerBlock - 1) / kDynEdgesPerBlock);
-        OG_HIP(hipStreamWaitEvent(s, lr->ev_h2d[slot], 0));
-        auto relax = [&](auto kernel) {
-            if (grid)
-                hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), 0, s, e0, e1, d->d_ring_tab + ch.tab, d->fr.info,
-                                   d->d_ptr, stage, lr->lbits, ch.first, d->d_mark, relax_args<ALGO>(d), d->fr.spread);
-        };
-        if (W && d->packed) relax(k_relax_range<ALGO, W, true>);
-        else relax(k_relax_range<ALGO, W, false>);
-        OG_HIP(hipGetLastError());
-        OG_HIP(hipEventRecord(lr->ev_use[slot], s));
-        if (copied < nc) copy(copied++);
-    }
-    hipLaunchKernelGGL(k_mark, dim3(fill_grid(fi.n[3])), dim3(256), 0, s, dlist, fi.n[3], d->d_mark, (uint8_t)0);
-    OG_HIP(hipGetLastError());
-    return true;
-}
-
 // Staged dynamic region of a round whose summary the host holds: the host
 // gathers the active edges into pinned slots and the copy stream moves them
 // while the other slot is relaxed.
@@ -2924,7 +2791,6 @@ static void run_dynamic(DeviceState *d, const og_graph *g, const FrontierInfo &f
     const uint32_t ndyn = fi.n[3];
     const uint64_t D = fi.dyn_deg;
     if (!ndyn || !D) return;
-    if (run_ring<ALGO, W>(d, g, fi, tm, st)) return;
     const uint32_t *d_dlist = d->fr.list + d->plan.vsplit;
     const uint64_t eb = d->deb;
     OG_HIP(hipMemcpyAsync(d->h_dlist, d_dlist, (size_t)ndyn * 4, hipMemcpyDeviceToHost, d->s_copy));
@@ -2996,9 +2862,8 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
     // round; when none is left it moves to (smallest held-back value + delta).
     const uint32_t delta = ALGO == ALGO_SSSP ? d->tune.delta : 0;
     const uint32_t *nf_val = delta ? d->d_val : nullptr;
-    const bool zero_copy = (d->flags & OG_PLAN_ZERO_COPY) != 0;
     const bool has_dyn = d->plan.vsplit < d->V;
-    const bool staged = has_dyn && !zero_copy;
+    const bool staged = has_dyn && !d->in_place;
     // deferring dynamic vertices reorders relaxations across levels, which
     // only the atomicMin relaxes (SSSP, CC) tolerate.  CC starts with every
     // vertex active: unless a tuning says otherwise its dynamic vertices wait
@@ -3166,7 +3031,6 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
 template <int ALGO, bool W>
 static void collect_loop(DeviceState *d, og_run_stats &st) {
     const RoundCtl c = d->fr.h_blk->ctl;
-    const bool zero_copy = (d->flags & OG_PLAN_ZERO_COPY) != 0;
     const bool has_dyn = d->plan.vsplit < d->V;
     if (c.overflow) raise(OG_EUNSUPPORTED, "multi-source BFS deeper than 254 levels");
     st.iterations += c.rounds;
@@ -3180,7 +3044,7 @@ static void collect_loop(DeviceState *d, og_run_stats &st) {
     st.relax_static_bytes += 24ull * c.static_node_sum + per_edge * c.static_work_edges;
     st.relax_dynamic_bytes += 24ull * c.dyn_node_sum + per_edge * dyn_edges;
     st.frontier_bytes += 2ull * d->Vpad * c.compactions + 4ull * c.node_sum;
-    if (has_dyn && zero_copy) {  // every active dynamic edge read in place (HBM-resident ones taken off later)
+    if (has_dyn && d->in_place) {  // every active dynamic edge read in place (HBM-resident ones taken off later)
         st.h2d_bytes += dyn_edges;
         st.chunks += c.dyn_rounds;
     }
@@ -3197,7 +3061,7 @@ static void finish_stats(og_run_stats &st, RunTimers &tm, double gather_ms, doub
     st.updates = ctr[0] + ctr[1];
     // zero-copy: h2d_bytes counts edges so far; those served from the
     // HBM-resident blocks did not cross the link
-    if (d->flags & OG_PLAN_ZERO_COPY) {
+    if (d->in_place) {
         const uint64_t crossed = st.h2d_bytes - std::min<uint64_t>(st.h2d_bytes, ctr[5]);
         st.h2d_bytes = d->lbits ? (crossed * d->lbits + 7) / 8 : crossed * d->deb;
     }

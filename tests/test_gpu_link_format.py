@@ -69,11 +69,11 @@ def test_pagerank_chunk_ring(V, frac, fp64):
 
 @pytest.mark.parametrize("pack", [True, False])
 @pytest.mark.parametrize("approach", ["ascetic", "subway"])
-def test_copy_loader_ring(approach, pack):
-    """Rounds of the copy loader that relax much of the dynamic region (whole
-    rows through the chunk ring), on rows that a workgroup's slice cannot hold
-    in LDS (5000 empty rows in a stretch), that span several workgroups (9000
-    edges) and that end at chunk ends."""
+def test_copy_loader(approach, pack):
+    """The copy loader, which reads pinned rows in place, and with NO_OVERLAP
+    gathers and copies them: rounds that relax a few rows and most of the dynamic
+    region, 5000 empty rows in a stretch, a row that spans several workgroups
+    (9000 edges).  Both against the oracle, and the same rounds and edges."""
     V = 30001
     rng = np.random.default_rng(5)
     deg = rng.integers(0, 9, V)
@@ -84,19 +84,26 @@ def test_copy_loader_ring(approach, pack):
     cols = rng.integers(0, V, int(ptr[-1])).astype(np.uint32)
     w = rng.integers(1, 64, len(cols)).astype(np.uint32)
     ptr = ptr[:-1].copy()
-    flags = 0 if pack else og.PLAN_NO_PACK
+    base = 0 if pack else og.PLAN_NO_PACK
     src = 21000
     bfs, sssp, cc = oracle.bfs(ptr, cols, src)[0], oracle.sssp(ptr, cols, w, src), oracle.cc(ptr, cols)[0]
     for weights, eb in ((None, 4), (w, 8)):
         g = og.Graph.from_csr(ptr, cols, weights)
         for split in (0, 8) if weights is not None and pack else (0,):
-            g.prepare(approach, edge_budget_bytes=len(cols) * eb // 2, advisek=0.5, flags=flags, split_weight=split)
-            for _ in range(2):
-                assert np.array_equal(g.cc()[0], cc)
-                assert np.array_equal(g.bfs(src)[0], bfs)
-                assert np.array_equal(g.msbfs(np.array([src, 0], np.uint32))[0][0], bfs)
-                if weights is not None:
-                    for delta in (0, 16):
-                        g.set_tuning(delta=delta)
-                        assert np.array_equal(g.sssp(src)[0], sssp)
+            counts = []
+            for flags in (base, base | og.PLAN_NO_OVERLAP, base | og.PLAN_NO_GRAPH):
+                g.prepare(approach, edge_budget_bytes=len(cols) * eb // 2, advisek=0.5, flags=flags, split_weight=split)
+                for _ in range(2):
+                    g.set_tuning(delta=0)
+                    assert np.array_equal(g.cc()[0], cc)
+                    lv, st = g.bfs(src)
+                    assert np.array_equal(lv, bfs)
+                    counts.append([st[k] for k in ("iterations", "node_sum", "work_edges", "reached", "checksum")])
+                    assert st["chunks"] > 0 and st["h2d_bytes"] > 0
+                    assert np.array_equal(g.msbfs(np.array([src, 0], np.uint32))[0][0], bfs)
+                    if weights is not None:
+                        for delta in (0, 16):
+                            g.set_tuning(delta=delta)
+                            assert np.array_equal(g.sssp(src)[0], sssp)
+            assert all(c == counts[0] for c in counts)
         g.close()

@@ -416,12 +416,14 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
         // One launch per iteration, enqueued a few ahead of the device:
         // iterations past the last one return at once.
         constexpr uint32_t kAhead = 4;
-        EventSpan span(d, &tc_static, s);
-        for (uint32_t k = 0; k < prm.max_iterations; ++k) {
-            if (k >= kAhead) wait_progress(d->h_progress, (unsigned long long)(k - kAhead + 1) << 1, s);
-            if (__atomic_load_n(d->h_progress, __ATOMIC_ACQUIRE) & 1) break;
-            turn(k);
-            pull_static(s, d->h_progress);
+        {
+            EventSpan span(d, &tc_static, s);
+            for (uint32_t k = 0; k < prm.max_iterations; ++k) {
+                if (k >= kAhead) wait_progress(d->h_progress, (unsigned long long)(k - kAhead + 1) << 1, s);
+                if (__atomic_load_n(d->h_progress, __ATOMIC_ACQUIRE) & 1) break;
+                turn(k);
+                pull_static(s, d->h_progress);
+            }
         }
         OG_HIP(hipMemcpyAsync(d->h_prstate, d->d_prstate, sizeof(PrState), hipMemcpyDeviceToHost, s));
         OG_HIP(hipStreamSynchronize(s));

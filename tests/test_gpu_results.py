@@ -48,6 +48,21 @@ def test_fp64_ranks(V):
     g.close()
 
 
+@pytest.mark.parametrize("share", [1.0, 0.5])
+@pytest.mark.parametrize("fp64", [False, True])
+def test_ranks_not_wanted(fp64, share):
+    """Statistics alone: nothing after the iterations waits for the stream."""
+    V = 40000
+    ptr = 8 * np.arange(V, dtype=np.uint64)
+    cols = ((np.arange(8 * V) * 7) % V).astype(np.uint32)
+    g = og.Graph.from_csr(ptr, cols, out_degree=np.bincount(cols, minlength=V).astype(np.uint32))
+    g.prepare("ascetic", edge_budget_bytes=int(32 * V * share), advisek=1.0 if share == 1 else 0.5)
+    for _ in range(5):
+        r, st = g.pagerank(fp64=fp64, want_values=False)
+        assert r is None and st["iterations"] == g.pagerank(fp64=fp64)[1]["iterations"]
+    g.close()
+
+
 def test_results_leave_at_once():
     sizes = [1 << 20, 65537, 300001, (1 << 21) + 1]
     graphs = [_ring(V) for V in sizes]

@@ -128,7 +128,7 @@ def base_record(metric_value, unit, steps, warmup, ms, dtype, config, higher=Tru
 
 
 KERNEL_NAMES = {"relax_static": "k_relax_group / k_relax_hub (static region)",
-                "relax_dynamic": "k_relax_dyn (dynamic region)", "frontier": "k_frontier_count/scan/write",
+                "relax_dynamic": "k_relax_dyn (dynamic region)", "frontier": "k_frontier_compact",
                 "relax_round": "k_relax_round (static bins + zero-copy dynamic region, one launch)"}
 
 

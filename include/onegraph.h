@@ -191,7 +191,11 @@ typedef struct og_plan_params {
                                    (for A/B timing)                              */
 #define OG_PLAN_ZERO_COPY 2u    /* dynamic region: the relax reads active edges
                                    straight from pinned host memory over the link
-                                   (no staging copies, no host gather); the
+                                   (no staging copies, no host gather; refused
+                                   for pageable memory).  Without the flag
+                                   traversals do the same wherever the device can
+                                   map the rows, and gather and copy chunks
+                                   elsewhere and with NO_OVERLAP or NO_FUSE.  The
                                    staging share of the budget keeps the chunks
                                    of 32 vertices whose rows cost the most link
                                    lines per edge resident in HBM instead      */
@@ -253,14 +257,17 @@ typedef struct og_run_stats {
     uint64_t static_node_sum;     /* reference staticnodeSum                      */
     uint64_t static_work_edges;   /* edges relaxed out of the static region       */
     uint64_t h2d_bytes;           /* dynamic-region payload copied host->device   */
-    uint64_t chunks;              /* dynamic-region copies issued                 */
+    uint64_t chunks;              /* dynamic-region copies issued, or rounds that
+                                     read dynamic rows in place                   */
     double total_ms;              /* reference totalProcess                       */
     double pre_ms;                /* reference preProcess (classify/compact/scan) */
     double static_ms;             /* reference staticProcess                      */
     double overload_ms;           /* reference overloadProcess                    */
     double overload_move_ms;      /* reference overloadMoveProcess (copy stream)  */
-    double gather_ms;             /* host gather of active dynamic edges          */
-    /* Kernel timing from HIP events on the launching stream. */
+    double gather_ms;             /* host gather of active dynamic edges (0 when
+                                     they are read in place)                      */
+    /* Kernel timing: the device's clock, stamped by the rounds' kernels, where a
+     * round is one relax launch, HIP events on the launching stream elsewhere. */
     double relax_static_kernel_ms;  uint64_t relax_static_launches;  uint64_t relax_static_bytes;
     double relax_dynamic_kernel_ms; uint64_t relax_dynamic_launches; uint64_t relax_dynamic_bytes;
     double frontier_kernel_ms;      uint64_t frontier_launches;      uint64_t frontier_bytes;
@@ -357,7 +364,7 @@ og_status og_probe_host_link(uint64_t bytes, double *contig_gbs, double *scatter
  * and levels (V, written in the og_bfs convention) are device pointers;
  * stream is a hipStream_t (NULL: the null stream).  The call allocates
  * nothing: its flags, bin lists, hub tiles and counters live in one static
- * device array of about 10.4 MiB per GPU, held until the process ends,
+ * device array of about 10.5 MiB per GPU, held until the process ends,
  * which limits it to V <= 2^21 and E <= 2^26 (OG_EINVAL beyond).  Calls
  * that overlap on one GPU share that array and race; it synchronises the
  * stream once per 4 rounds.  stats may be NULL (kernel timings stay 0). */

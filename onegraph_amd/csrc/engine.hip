@@ -1,7 +1,7 @@
 // Frontier engine for BFS, SSSP and CC on gfx950: wave64 ballot/scan frontier
 // compaction, degree-binned relax kernels over the HBM-resident static region,
-// and the dynamic-region loader that streams active edges from pinned host
-// memory through a double-buffered staging area on a copy stream.
+// and the dynamic-region loaders: the relax reads active rows where they are, in
+// pinned host memory, or the host streams them through staging slots.
 //
 // One iteration (reference loop: BFS/oneGraph_BFS/CalculateOpt.h:75-188):
 //   1. k_frontier_compact: one pass over the next-frontier flags builds the
@@ -15,10 +15,10 @@
 //      bfs_kernelStatic (gpu_kernels.h:211-241), sssp_kernel
 //      (SSSP/oneGraph/gpu_kernels.h:177-203), cc_kernelStaticSwap
 //      (CC/onegraph/gpu_kernels.h:133-157).
-//   3. dynamic region: the host gathers the active edges of the sorted dynamic
-//      list into a pinned slot (H5, GraphMeta.h:470-506), hipMemcpyAsync moves
-//      the slot on the copy stream while the other slot is being gathered, and
-//      an edge-parallel relax consumes it (K8/K10/K12).
+//   3. dynamic region: an edge-parallel relax reads the active rows over the
+//      link (K8/K10/K12); in pageable memory the host gathers the active edges of
+//      the sorted dynamic list into a pinned slot (H5, GraphMeta.h:470-506) and
+//      hipMemcpyAsync moves the slot while the other one is being gathered.
 #include <algorithm>
 #include <atomic>
 #include <vector>

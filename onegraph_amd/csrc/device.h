@@ -51,6 +51,7 @@ constexpr int kMsWidth = 64;            // sources per mask of the multi-source 
 constexpr int ms_masks(int algo) { return algo == ALGO_MSBFS ? 1 : algo == ALGO_MSBFS2 ? 2 : 0; }
 
 // Per-vertex state the relax kernels touch.
+struct RoundCtl;
 struct RelaxArgs {
     uint32_t *val;        // BFS level / SSSP distance / CC label
     uint8_t *flag;        // next-frontier flags
@@ -60,6 +61,9 @@ struct RelaxArgs {
     const uint64_t *pull; // multi-source, optional: sources relaxed bottom-up this round
                           // (left out of the top-down relax)
     const uint64_t *pmid; // light/heavy split, optional: end of each row's light edges
+    RoundCtl *ctl;        // with the split: notes that the round put a value below its threshold
+    // of a lane, filled and noted by the kernels (relax_begin, relax_end)
+    mutable uint32_t thresh = 0, near = 0;
 };
 
 // Edge range of u in a round: the whole row, or with the light/heavy split
@@ -153,6 +157,7 @@ struct RoundCtl {
     uint32_t halt;               // 1 (device-driven runs): once a compaction finds nothing live, the
                                  // compactions of rounds enqueued past the end skip their sweep
     uint32_t hold;               // defer 1: the next compaction holds the dynamic vertices back
+    uint32_t near;               // split: the round's relax put a value below thresh (set by the relax kernels)
 };
 
 // Time of a device-driven run by kind of work, from the device's constant

@@ -134,7 +134,7 @@ __global__ void k_totals_init(unsigned long long *t, uint64_t n) {
 // far << 1 | traversal ended.
 __device__ __forceinline__ void compact_finish(const CompactTotals &ct, FrontierInfo *__restrict__ info,
                                                uint64_t *__restrict__ doff, RoundCtl *__restrict__ ctl,
-                                               unsigned long long *progress) {
+                                               unsigned long long *progress, bool was_heavy) {
     const uint32_t lane = threadIdx.x;
     RoundCtl c = *ctl;
     uint64_t zf = 0, sd = 0, lh = 0, mf = ~0ull, a01 = 0, ath = 0, dyn = 0, wn = 0, wd = 0;
@@ -179,7 +179,6 @@ __device__ __forceinline__ void compact_finish(const CompactTotals &ct, Frontier
     const uint32_t lagging = (uint32_t)lh, hd = (uint32_t)(lh >> 32);
     fi.dyn_held = hd ? 1u : 0u;
     const uint64_t snodes = (uint64_t)fi.n[0] + fi.n[1] + fi.nhub;
-    const bool was_heavy = c.mode != 0;
     const uint64_t active = snodes + fi.n[3] + fi.nzero;
     // light/heavy split: light rounds count the vertices they relax (they
     // turn heavy-pending); once a bucket's light rounds find nothing near,
@@ -202,7 +201,7 @@ __device__ __forceinline__ void compact_finish(const CompactTotals &ct, Frontier
     // edges exceed 1/14 of the unexplored ones, back to top-down when
     // the frontier falls below V / 24.
     fi.pull = 0;
-    fi.heavy = c.mode;
+    fi.heavy = was_heavy ? 1u : 0u;
     if (c.dir_opt && active) {
         const uint64_t mf2 = fi.static_deg + fi.dyn_deg;
         if (!c.pull && mf2 > c.unexplored / 14) c.pull = 1;
@@ -241,6 +240,7 @@ __device__ __forceinline__ void compact_finish(const CompactTotals &ct, Frontier
     if (c.defer == kDeferOnce) c.hold = c.hold && active ? 1u : 0u;
     else c.hold = c.defer == 1 && !was_heavy && active ? 1u : 0u;
     c.mode = heavy_next ? 1u : 0u;
+    c.near = 0;
     *ctl = c;
     if (progress)
         __hip_atomic_store(progress, (unsigned long long)c.compactions << 1 | (fi.live ? 0u : 1u), __ATOMIC_RELAXED,
@@ -290,8 +290,13 @@ __global__ __launch_bounds__(kCompactBlock) void k_frontier_compact(
     // the summary and the traversal state stand
     if (ctl->halt && !ctl->live) return;
     // light/heavy split: a heavy compaction collects the heavy-pending
-    // vertices (no near-far test) and sizes them by their heavy edges
-    const bool heavy = pmid && ctl->mode;
+    // vertices (no near-far test) and sizes them by their heavy edges.  It does so at
+    // once when the light round before it put nothing below the threshold: its
+    // sweep would find nothing near, and the next one would collect them (six of
+    // the 28 rounds of an in-memory SSSP, about 13 us each: 757 -> 700 us, out of
+    // memory 16.5 -> 16.3 ms).  A deferred order keeps near vertices flagged, so
+    // there only the sweep can tell.
+    const bool heavy = pmid && (ctl->mode || (ctl->hpend && !ctl->near && !ctl->defer));
     const bool mark = pmid && !heavy;  // light round: relaxed vertices turn heavy-pending
     uint8_t *flag = heavy ? hflag : flag_a;
     const uint32_t *val = heavy ? nullptr : val_a;
@@ -307,7 +312,7 @@ __global__ __launch_bounds__(kCompactBlock) void k_frontier_compact(
     if (!__syncthreads_or(any != 0)) {  // no flags here (most blocks in a small round)
         if (threadIdx.x < kWave) {
             const bool last = threadIdx.x == 0 && arrive_last(ct);
-            if (__ballot(last)) compact_finish(ct, info, doff, ctl, progress);
+            if (__ballot(last)) compact_finish(ct, info, doff, ctl, progress, heavy);
         }
         return;
     }
@@ -520,7 +525,7 @@ __global__ __launch_bounds__(kCompactBlock) void k_frontier_compact(
         // (the word belongs to this thread alone)
         if (mark && hw) *(uint32_t *)(hflag + v0 + q * kWin) |= hw;
     }
-    if (wid == 0 && __ballot(last)) compact_finish(ct, info, doff, ctl, progress);
+    if (wid == 0 && __ballot(last)) compact_finish(ct, info, doff, ctl, progress, heavy);
 }
 
 // Traversal state at the start: near-far width `delta` with the first
@@ -621,6 +626,21 @@ __device__ __forceinline__ typename SrcOf<ALGO>::T peek(const RelaxArgs &a, uint
     else return a.val[to];
 }
 
+// A relax kernel's start and end: the threshold that an improvement is compared
+// with, and whether any of the wave's fell below it (every writer stores the
+// same).  Once per wave: read and noted beside each atomic they cost the dense
+// rounds of an in-memory SSSP a tenth.
+template <int ALGO>
+__device__ __forceinline__ void relax_begin(const RelaxArgs &a) {
+    a.near = 0;
+    a.thresh = ALGO == ALGO_SSSP && a.ctl ? a.ctl->thresh : 0u;
+}
+
+template <int ALGO>
+__device__ __forceinline__ void relax_end(const RelaxArgs &a) {
+    if (ALGO == ALGO_SSSP && __ballot(a.near != 0) && threadIdx.x % kWave == 0) a.ctl->near = 1;
+}
+
 // Applies N offers of a lane (edge k valid when bit k of `ok` is set, its
 // source's state src(k)) and returns how many improved their target (which is
 // then flagged for the next frontier).
@@ -699,6 +719,7 @@ __device__ __forceinline__ uint32_t commit(const RelaxArgs &a, Src src, const ui
             if (((ok >> k) & 1) && nd[k] < x[k]) {
                 a.flag[to[k]] = 1;
                 ++c;
+                a.near |= nd[k] < a.thresh ? 1u : 0u;
             }
     }
     return c;
@@ -760,7 +781,9 @@ __global__ __launch_bounds__(kBlock) void k_relax_group(const uint32_t *__restri
                                                         const uint64_t *__restrict__ ptr,
                                                         const void *__restrict__ edges, RelaxArgs a,
                                                         unsigned long long *spread) {
+    relax_begin<ALGO>(a);
     wave_count(spread, kUpdStatic, relax_group_body<ALGO, W, PK, LPV>(list, vsplit, bin, info, ptr, edges, a, blockIdx.x, gridDim.x));
+    relax_end<ALGO>(a);
 }
 
 template <int ALGO, bool W, bool PK>
@@ -824,7 +847,9 @@ __global__ __launch_bounds__(kBlock) void k_relax_hub(const uint64_t *__restrict
                                                       const void *__restrict__ edges, RelaxArgs a,
                                                       unsigned long long *spread) {
     extern __shared__ uint32_t s_edges[];
+    relax_begin<ALGO>(a);
     wave_count(spread, kUpdStatic, relax_hub_body<ALGO, W, PK>(hub, hub_cap, info, tile, ptr, edges, a, s_edges, blockIdx.x, gridDim.x));
+    relax_end<ALGO>(a);
 }
 
 // Dynamic region, edges [c0, min(c1, D)) of the concatenated active dynamic
@@ -976,9 +1001,11 @@ __global__ __launch_bounds__(kBlock) void k_relax_dyn(const uint32_t *__restrict
                                                       uint32_t lbits, unsigned long long *spread) {
     __shared__ DynLds L;
     uint32_t h = 0;
+    relax_begin<ALGO>(a);
     const uint32_t c = relax_dyn_body<ALGO, W, PACKED, DIRECT>(list, info, doff, stage, c0, c1max, ptr, dbase, resident,
                                                                rdelta, wbits, a, lpos, nl, vsplit, dchunk, lbits, L,
                                                                blockIdx.x, gridDim.x, h);
+    relax_end<ALGO>(a);
     wave_count(spread, kUpdDynamic, c);
     if (DIRECT) wave_count(spread, kHbmEdges, h);
 }
@@ -1020,6 +1047,7 @@ template <int ALGO, bool W, bool PK, int LPV>
 __global__ __launch_bounds__(kBlock) void k_relax_round(RoundRelax r, RelaxArgs a) {
     extern __shared__ uint64_t s_fuse[];
     clock_stamp(r.clk, kClkFront, kClkRelax);
+    relax_begin<ALGO>(a);
     const uint32_t P = kFuseStatic + r.cd;
     const uint32_t K = gridDim.x / P;
     const uint32_t k = blockIdx.x / P, j = blockIdx.x - k * P;
@@ -1041,6 +1069,7 @@ __global__ __launch_bounds__(kBlock) void k_relax_round(RoundRelax r, RelaxArgs 
         wave_count(r.spread, kUpdDynamic, c);
         wave_count(r.spread, kHbmEdges, h);
     }
+    relax_end<ALGO>(a);
 }
 
 // Served BFS (the query server's 64-slot engines): bottom-up scan for the
@@ -2590,7 +2619,8 @@ static void gather(DeviceState *d, const og_graph *g, uint32_t ndyn, uint64_t c0
 template <int ALGO>
 static RelaxArgs relax_args(DeviceState *d) {
     const DeviceState::MsState &m = d->d_ms[ms_masks(ALGO) == 2];
-    return RelaxArgs{d->d_val, d->fr.flag, m.vn, m.front, d->wbits, nullptr, d->run_pmid};
+    return RelaxArgs{d->d_val, d->fr.flag, m.vn, m.front, d->wbits, nullptr, d->run_pmid,
+                     d->run_pmid ? d->fr.ctl : nullptr};
 }
 
 // Grids of device-count launches: the kernels stride over whatever count
@@ -3904,7 +3934,7 @@ static void noalloc_bfs(const uint64_t *d_ptr, const uint32_t *d_cols, uint64_t 
         r.cd = 0;  // the whole graph is static: three bins in one launch
         r.vsplit = V;
         r.spread = spread;
-        const RelaxArgs a{d_levels, flag, nullptr, nullptr, 0, nullptr, nullptr};
+        const RelaxArgs a{d_levels, flag, nullptr, nullptr, 0, nullptr, nullptr, nullptr};
         static_assert(Tuning{}.lpv0 == 8, "the relax below is instantiated for 8 lanes per bin-0 vertex");
         compact();
         // the first batch covers most traversals of skewed graphs: an empty

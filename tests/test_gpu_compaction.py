@@ -47,3 +47,35 @@ def test_compaction_window_edges(V, plan):
             g.set_tuning(defer=defer)
             assert np.array_equal(g.cc()[0], oracle.cc(ptr, cols)[0]), (split, defer)
     g.close()
+
+
+@pytest.mark.parametrize("flags", [0, og.PLAN_NO_GRAPH, og.PLAN_NO_FUSE, og.PLAN_NO_OVERLAP, og.PLAN_ZERO_COPY])
+@pytest.mark.parametrize("weights", ["light", "heavy", "at the split", "mixed"])
+def test_heavy_rounds_follow_at_once(weights, flags):
+    """Light/heavy split: a light round that puts nothing below the threshold is
+    followed by the heavy round.  Paths (every round has one vertex) beside a
+    random graph, edges of one kind only and of both, buckets below, at and above
+    the split, deferred orders (which keep the empty sweep)."""
+    V, split = 20011, 8
+    rng = np.random.default_rng(3)
+    deg = rng.integers(0, 5, V)
+    deg[:300] = 1  # a path of 300
+    ptr = np.zeros(V + 1, np.uint64)
+    ptr[1:] = np.cumsum(deg)
+    E = int(ptr[-1])
+    cols = rng.integers(0, V, E).astype(np.uint32)
+    cols[:300] = np.arange(1, 301)
+    lo, hi = {"light": (1, split), "heavy": (split, 64), "at the split": (split - 1, split + 1), "mixed": (1, 64)}[weights]
+    w = rng.integers(lo, hi, E).astype(np.uint32)
+    w[-1] = 63
+    ptr = ptr[:-1].copy()
+    ref = oracle.sssp(ptr, cols, w, 0)
+    g = og.Graph.from_csr(ptr, cols, w)
+    for share in (1.0, 0.3):
+        g.prepare("ascetic", edge_budget_bytes=int(8 * E * share), advisek=1.0 if share == 1 else 0.5,
+                  flags=flags if share < 1 else flags & ~og.PLAN_ZERO_COPY, split_weight=split)
+        for delta in (1, 8, 256):
+            for defer in (0, 1, 2):
+                g.set_tuning(delta=delta, defer=defer)
+                assert np.array_equal(g.sssp(0)[0], ref), (share, delta, defer)
+    g.close()

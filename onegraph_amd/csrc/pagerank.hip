@@ -377,7 +377,8 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
     if (cap > d->pr_partial_cap) {
         d->d_partial = (double *)d->dalloc(cap * 2 * sizeof(double));
         d->d_prtot = (unsigned long long *)d->dalloc(totals_words(cap) * 8);
-        OG_HIP(hipMemset(d->d_prtot, 0, totals_words(cap) * 8));
+        // (on the stream whose kernels count in them: it does not wait for the null stream)
+        OG_HIP(hipMemsetAsync(d->d_prtot, 0, totals_words(cap) * 8, s));
         d->pr_partial_cap = cap;
     }
     T *contrib[2] = {(T *)d->d_contrib[0], (T *)d->d_contrib[1]};

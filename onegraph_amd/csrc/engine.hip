@@ -1774,10 +1774,10 @@ static std::shared_ptr<OutStage> out_stage(size_t n) {
 }
 
 static void copy_chunks_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStream_t s) {
-    if (!d->h_chunk[0]) {
-        for (auto &p : d->h_chunk) p = d->palloc(kOutChunk);
-        for (auto &e : d->ev_chunk) OG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
+    for (auto &p : d->h_chunk)
+        if (!p) p = d->palloc(kOutChunk);
+    for (auto &e : d->ev_chunk)
+        if (!e) OG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     if (!d->pool) d->pool.reset(new WorkerPool(d->host_threads));
     const size_t nch = (n + kOutChunk - 1) / kOutChunk;
     auto issue = [&](size_t k) {

@@ -364,15 +364,18 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
     hipStream_t s = d->s_compute;
     const unsigned igrid = (unsigned)std::min<uint64_t>(1024, grid_of(V));
     const uint64_t cap = std::max<uint64_t>(pp.blocks, igrid);
+    // (each by itself: a call that ran out of memory leaves the rest to the next)
+    if (!d->d_prstate) d->d_prstate = (PrState *)d->dalloc(sizeof(PrState));
+    if (!d->h_prstate) d->h_prstate = (PrState *)d->palloc(sizeof(PrState));
+    if (!d->h_progress) d->h_progress = (unsigned long long *)d->palloc(sizeof(unsigned long long));
+    // sized for double so either precision fits
+    if (!d->d_rank) d->d_rank = d->dalloc(V * 8);
+    for (auto &c : d->d_contrib)
+        if (!c) c = d->dalloc(V * 8);
     if (!d->d_outdeg) {
-        d->d_outdeg = (uint32_t *)d->dalloc(V * 4);
-        OG_HIP(hipMemcpy(d->d_outdeg, g->out_degree, V * 4, hipMemcpyHostToDevice));
-        d->d_prstate = (PrState *)d->dalloc(sizeof(PrState));
-        d->h_prstate = (PrState *)d->palloc(sizeof(PrState));
-        d->h_progress = (unsigned long long *)d->palloc(sizeof(unsigned long long));
-        // sized for double so either precision fits
-        d->d_rank = d->dalloc(V * 8);
-        for (auto &c : d->d_contrib) c = d->dalloc(V * 8);
+        uint32_t *od = (uint32_t *)d->dalloc(V * 4);
+        OG_HIP(hipMemcpy(od, g->out_degree, V * 4, hipMemcpyHostToDevice));
+        d->d_outdeg = od;
     }
     if (cap > d->pr_partial_cap) {
         d->d_partial = (double *)d->dalloc(cap * 2 * sizeof(double));

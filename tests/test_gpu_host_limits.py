@@ -40,3 +40,34 @@ def test_pagerank_clears_on_its_own_stream(gpu, tmp_path):
             if not t:
                 assert shim.shim_fills_stream() > mine
     """)
+
+
+def test_runs_after_a_refused_allocation(gpu, tmp_path):
+    """A first call that runs out of memory part of the way fails with that
+    status, and the next one, with memory, is whole: PageRank's state and the two
+    chunks of results above 8 MB."""
+    hip_shim.run(tmp_path, PULL + """
+    V = (1 << 21) + 5
+    ptr, cols, od = pull(V)
+    ref = oracle.pagerank(od, ptr, cols)[0]
+    g = og.Graph.from_csr(ptr, cols, out_degree=od)
+    g.prepare("ascetic", edge_budget_bytes=4 * len(cols), advisek=1.0)
+
+    def refused(deny, lo, hi, name, call):
+        before = shim.shim_denied()
+        deny(lo, hi)
+        try:
+            call()
+            raise SystemExit("not refused")
+        except og.OgError as e:
+            assert e.name == name, e
+        finally:
+            deny(1, 0)
+        assert shim.shim_denied() > before
+
+    refused(shim.shim_deny_device, 8 * V, 8 * V, "OG_ENOMEM_DEVICE", g.pagerank)   # ranks, contributions
+    refused(shim.shim_deny_device, 4 * V, 4 * V, "OG_ENOMEM_DEVICE", g.pagerank)   # out-degrees
+    refused(shim.shim_deny_pinned, 8 << 20, 8 << 20, "OG_ENOMEM_HOST", lambda: g.pagerank(fp64=True))
+    for fp64 in (True, False):
+        assert np.abs(g.pagerank(fp64=fp64)[0] - ref).max() < 1e-6
+    """)

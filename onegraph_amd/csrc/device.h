@@ -285,13 +285,19 @@ struct MemPool {
         device_bytes += bytes;
         return p;
     }
-    void *palloc(size_t bytes) {
+    // null when there is no memory
+    void *try_palloc(size_t bytes) {
         void *p = nullptr;
         if (hipHostMalloc(&p, bytes ? bytes : 8, hipHostMallocDefault) != hipSuccess || !p) {
             (void)hipGetLastError();
-            raise(OG_ENOMEM_HOST, "pinned host allocation of %zu bytes failed", bytes);
+            return nullptr;
         }
         pin.push_back(p);
+        return p;
+    }
+    void *palloc(size_t bytes) {
+        void *p = try_palloc(bytes);
+        if (!p) raise(OG_ENOMEM_HOST, "pinned host allocation of %zu bytes failed", bytes);
         return p;
     }
     void release() {
@@ -384,7 +390,8 @@ struct DeviceState {
     uint32_t deb = 4;                // bytes per dynamic-region edge on the link (= eb)
     bool in_place = false;           // traversals read the dynamic region in pinned host memory
     uint64_t dyn_base = 0;           // first edge of the dynamic region (= ptr[vsplit])
-    const void *h_dyn = nullptr;     // host source of dynamic edges (packed copy or the CSR)
+    const void *h_dyn = nullptr;     // host source of dynamic edges (packed copy, null once the link format has
+                                     // taken its place, or the CSR)
     const void *hd_dyn = nullptr;    // the same, as a device address (zero-copy mode)
     uint64_t slot_dyn = 0;           // dynamic edges per staging slot in the transfer format
     // zero-copy with the light/heavy split: the host copy of the dynamic

@@ -2161,17 +2161,27 @@ LinkRing *link_ring(DeviceState *d, const og_graph *g) {
     return r.get();
 }
 
-// Link format of the dynamic region (DeviceState::lbits): packs the host
-// layout's words `src` into a pinned stream of lbits-bit words, when they are
-// narrow enough.  Edge targets need the bits of V - 1, weighted words wbits
-// more; with V of a few million a quarter to a third of the bytes go (ER 3 M
-// x 32, 22 bits: PageRank 66 -> 46 ms, CC 7.9 -> 6.6 ms; preparing the
-// packed copy takes 12 ms more).
-static void pack_link(DeviceState *d, const og_graph *g, const uint32_t *src, uint64_t n) {
+// Bits per edge of the link format (DeviceState::lbits): those of V - 1, for
+// packed weighted words the weight's more; 0 where they are too many, or
+// where nothing would read it: traversals that gather chunks take whole edges, and a
+// weighted graph that is not packed keeps its 8-byte ones.
+static uint32_t link_bits(const DeviceState *d, const og_graph *g) {
+    if (!d->in_place && g->kind != OG_KIND_PULL) return 0;
+    if (g->kind == OG_KIND_WEIGHTED && !d->packed) return 0;
     const uint32_t bits = std::max(bits_of(g->V - 1), 1u) + (d->packed ? d->wbits : 0);
-    if (bits > kLinkBitsMax || !n) return;
+    return bits <= kLinkBitsMax ? bits : 0;
+}
+
+// Packs the host layout's words `src` into a pinned stream of `bits`-bit words.
+// With V of a few million a quarter to a third of the bytes go (ER 3 M
+// x 32, 22 bits: PageRank 66 -> 46 ms, CC 7.9 -> 6.6 ms; preparing the
+// packed copy takes 12 ms more).  Without pinned memory for it the edges stay
+// as they are.
+static void pack_link(DeviceState *d, uint32_t bits, const uint32_t *src, uint64_t n) {
+    if (!bits || !n) return;
     const uint64_t words = (n * bits + 31) / 32 + 2;
-    uint32_t *dst = (uint32_t *)d->palloc(words * 4);
+    uint32_t *dst = (uint32_t *)d->mem.try_palloc(words * 4);
+    if (!dst) return;
     dst[words - 1] = dst[words - 2] = 0;
     // groups of 32 edges fill `bits` whole words
     parallel_for((n + 31) / 32, 1 << 15, 0, [&](uint64_t b, uint64_t e, unsigned) {
@@ -2410,8 +2420,18 @@ static void prepare_impl(og_graph *g, og_approach approach, const og_plan_params
                                       d->s_compute));
                 OG_HIP(hipStreamSynchronize(d->s_compute));
             }
+            // With the link format in place of it, the packed copy is only a
+            // step on the way and need not be pinned.
+            const uint32_t bits = link_bits(d.get(), g);
+            std::unique_ptr<uint32_t[]> step;
             if (d->packed) {
-                uint32_t *pk = (uint32_t *)d->palloc(std::max<uint64_t>(nd, 1) * 4);
+                uint32_t *pk;
+                if (zc && bits && nd) {
+                    step.reset(new uint32_t[nd]);
+                    pk = step.get();
+                } else {
+                    pk = (uint32_t *)d->palloc(std::max<uint64_t>(nd, 1) * 4);
+                }
                 if (!lpos.empty()) pack_split_rows(g, pl.vsplit, d->wbits, d->split_weight, lpos.data(), pk);
                 else pack_rows(g, pl.vsplit, V, d->wbits, d->split_weight, pk);
                 d->h_dyn = pk;
@@ -2422,19 +2442,26 @@ static void prepare_impl(og_graph *g, og_approach approach, const og_plan_params
             if (zc) {
                 if (!d->packed && !(eb == 8 ? g->pinned_wedges : g->pinned_cols))
                     raise(OG_EUNSUPPORTED, "zero-copy loading needs the graph in pinned host memory");
-                // map the allocation's base, then offset to the dynamic region
-                const void *hbase = d->packed ? d->h_dyn : g->edge_data();
-                void *hd = nullptr;
-                OG_HIP(hipHostGetDevicePointer(&hd, (void *)hbase, 0));
-                d->hd_dyn = (const uint8_t *)hd + ((const uint8_t *)d->h_dyn - (const uint8_t *)hbase);
                 // Reading in place needs no transit slots, so the staging
                 // share of the budget keeps part of the dynamic region
                 // resident in HBM instead.
                 stage_resident(d.get(), g, pl.vsplit, pl.staging_edges, lpos);
             }
-            // (a weighted graph that is not packed keeps its 8-byte edges)
-            if (g->kind != OG_KIND_WEIGHTED || d->packed)
-                pack_link(d.get(), g, (const uint32_t *)d->h_dyn, nd);
+            pack_link(d.get(), bits, (const uint32_t *)d->h_dyn, nd);
+            if (step) {
+                if (d->lbits) {
+                    d->h_dyn = nullptr;
+                } else {  // no link format after all
+                    d->h_dyn = std::memcpy(d->palloc(nd * 4), step.get(), nd * 4);
+                }
+            }
+            if (zc && d->h_dyn) {
+                // map the allocation's base, then offset to the dynamic region
+                const void *hbase = d->packed ? d->h_dyn : g->edge_data();
+                void *hd = nullptr;
+                OG_HIP(hipHostGetDevicePointer(&hd, (void *)hbase, 0));
+                d->hd_dyn = (const uint8_t *)hd + ((const uint8_t *)d->h_dyn - (const uint8_t *)hbase);
+            }
         }
     }
 

@@ -65,6 +65,13 @@ int hipMemsetAsync(void *p, int v, size_t n, void *s) {
     atomic_fetch_add(s ? &fills_stream : &fills_null, 1);
     return ((int (*)(void *, int, size_t, void *))real("hipMemsetAsync"))(p, v, n, s);
 }
+int shim_pinned_has(size_t n) {
+    int has = 0;
+    pthread_mutex_lock(&mu);
+    for (int i = 0; i < 1 << 14; ++i) has |= rec[i].p && rec[i].pin && rec[i].n == n;
+    pthread_mutex_unlock(&mu);
+    return has;
+}
 void shim_deny_pinned(size_t lo, size_t hi) { deny_pin.lo = lo; deny_pin.hi = hi; }
 void shim_deny_device(size_t lo, size_t hi) { deny_dev.lo = lo; deny_dev.hi = hi; }
 long shim_denied(void) { return atomic_load(&denied); }
@@ -80,6 +87,7 @@ shim = C.CDLL({so!r}, mode=C.RTLD_GLOBAL)   # before the library is loaded: its 
 shim.shim_deny_pinned.argtypes = shim.shim_deny_device.argtypes = [C.c_size_t, C.c_size_t]
 for name in ("denied", "fills_null", "fills_stream", "live_pinned", "live_device"):
     getattr(shim, "shim_" + name).restype = C.c_long
+shim.shim_pinned_has.argtypes = [C.c_size_t]
 sys.path.insert(0, {root!r})
 import numpy as np
 import onegraph_amd as og

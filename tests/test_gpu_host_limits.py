@@ -71,3 +71,79 @@ def test_runs_after_a_refused_allocation(gpu, tmp_path):
     for fp64 in (True, False):
         assert np.abs(g.pagerank(fp64=fp64)[0] - ref).max() < 1e-6
     """)
+
+
+LINK = """
+def graph(V, weighted, seed=3):
+    rng = np.random.default_rng(seed)
+    deg = rng.integers(0, 9, V)
+    deg[0] = 5
+    ptr = np.zeros(V + 1, np.uint64)
+    ptr[1:] = np.cumsum(deg)
+    E = int(ptr[-1])
+    cols, w = rng.integers(0, V, E).astype(np.uint32), rng.integers(1, 64, E).astype(np.uint32)
+    return og.Graph.from_csr(ptr[:-1].copy(), cols, w if weighted else None), ptr, cols, w
+
+def link_bytes(ptr, plan, bits):   # of the narrow words of the dynamic region
+    n = int(ptr[-1] - ptr[plan["vsplit"]])
+    return ((n * bits + 31) // 32 + 2) * 4, 4 * n
+"""
+
+
+def test_link_format_only_where_it_is_read(gpu, tmp_path):
+    """The narrow copy of the dynamic region is built for rounds that read it, in
+    place of the packed words; loaders that gather chunks hold whole edges only."""
+    hip_shim.run(tmp_path, LINK + """
+    V = 70001
+    for weighted, bits in ((False, 17), (True, 23)):
+        g, ptr, cols, w = graph(V, weighted)
+        E = len(cols)
+        for flags, split in ((0, 0), (og.PLAN_ZERO_COPY, 0), (og.PLAN_ZERO_COPY | og.PLAN_NO_OVERLAP, 0),
+                             (og.PLAN_NO_OVERLAP, 0), (og.PLAN_NO_FUSE, 0)) + (((0, 8),) if weighted else ()):
+            plan = g.prepare("ascetic", edge_budget_bytes=2 * E, advisek=0.5, flags=flags, split_weight=split)
+            narrow, whole = link_bytes(ptr, plan, bits)
+            in_place = flags & og.PLAN_ZERO_COPY or not flags
+            assert shim.shim_pinned_has(narrow) == bool(in_place), (weighted, flags)
+            if weighted:
+                assert shim.shim_pinned_has(whole) == (not in_place), flags
+            assert np.array_equal(g.bfs(0)[0], oracle.bfs(ptr[:-1], cols, 0)[0]), (weighted, flags)
+            if weighted:
+                assert np.array_equal(g.sssp(0)[0], oracle.sssp(ptr[:-1], cols, w, 0)), flags
+        g.close()
+    """)
+
+
+def test_no_memory_for_the_link_format(gpu, tmp_path):
+    """Without pinned memory for the narrow words the edges cross as they are."""
+    hip_shim.run(tmp_path, LINK + PULL + """
+    V = 70001
+    for weighted, bits in ((False, 17), (True, 23)):
+        g, ptr, cols, w = graph(V, weighted)
+        for flags, split in ((0, 0), (og.PLAN_ZERO_COPY, 0)) + (((0, 8),) if weighted else ()):
+            plan = g.prepare("ascetic", edge_budget_bytes=2 * len(cols), advisek=0.5, flags=flags, split_weight=split)
+            narrow, whole = link_bytes(ptr, plan, bits)
+            before = shim.shim_denied()
+            shim.shim_deny_pinned(narrow, narrow)
+            g.prepare("ascetic", edge_budget_bytes=2 * len(cols), advisek=0.5, flags=flags, split_weight=split)
+            shim.shim_deny_pinned(1, 0)
+            assert shim.shim_denied() == before + 1
+            for _ in range(2):
+                lv, st = g.bfs(0)
+                assert np.array_equal(lv, oracle.bfs(ptr[:-1], cols, 0)[0])
+                assert st["h2d_bytes"] % 4 == 0 and st["h2d_bytes"] > 0
+                assert np.array_equal(g.cc()[0], oracle.cc(ptr[:-1], cols)[0])
+                if weighted:
+                    g.set_tuning(delta=16)
+                    assert np.array_equal(g.sssp(0)[0], oracle.sssp(ptr[:-1], cols, w, 0))
+        g.close()
+    ptr, cols, od = pull(V)
+    g = og.Graph.from_csr(ptr, cols, out_degree=od)
+    plan = g.prepare("ascetic", edge_budget_bytes=2 * len(cols), advisek=0.5)
+    narrow, whole = link_bytes(np.append(ptr, np.uint64(len(cols))), plan, 17)
+    before = shim.shim_denied()
+    shim.shim_deny_pinned(narrow, narrow)
+    g.prepare("ascetic", edge_budget_bytes=2 * len(cols), advisek=0.5)
+    shim.shim_deny_pinned(1, 0)
+    assert shim.shim_denied() == before + 1
+    assert np.abs(g.pagerank()[0] - oracle.pagerank(od, ptr, cols)[0]).max() < 1e-6
+    """)

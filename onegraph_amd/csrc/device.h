@@ -339,12 +339,15 @@ struct LinkRing {
 // 0.75 ms).  One copy uses it at a time; another that finds it taken goes
 // through the runtime.
 struct OutStage {
-    std::mutex use;
+    std::mutex use;        // held by the copy that uses the rest
     char *buf = nullptr;
     size_t bytes = 0;
     unsigned long long *flag = nullptr;
     unsigned long long seq = 0;
     std::unique_ptr<WorkerPool> pool;
+    // Makes ready for a result of n bytes (`use` held); false when that is too
+    // large or there is no memory for it.
+    bool reserve(size_t n);
     ~OutStage();
 };
 

@@ -1736,41 +1736,49 @@ OutStage::~OutStage() {
     if (flag) (void)hipHostFree(flag);
 }
 
-// The staging, ready for results of n bytes (at most kOutMax) unless it is in
-// use (then it stays as it is).
-static std::shared_ptr<OutStage> out_stage(size_t n) {
+bool OutStage::reserve(size_t n) {
+    if (n > kOutMax) return false;
+    const size_t want = n <= kOutAlone ? kOutAlone : kOutMax;
+    auto pinned = [](size_t b) -> void * {
+        void *p = nullptr;
+        if (hipHostMalloc(&p, b, hipHostMallocDefault) == hipSuccess) return p;
+        (void)hipGetLastError();
+        return nullptr;
+    };
+    if (want > bytes) {
+        char *p = (char *)pinned(want);
+        if (!p) return false;
+        if (buf) (void)hipHostFree(buf);
+        buf = p;
+        bytes = want;
+    }
+    if (!flag) {
+        const size_t fb = kOutMax / kOutSlab * sizeof(unsigned long long);
+        flag = (unsigned long long *)pinned(fb);
+        if (!flag) return false;
+        std::memset(flag, 0, fb);
+    }
+    if (n > kOutAlone && !pool) pool.reset(new WorkerPool(std::min(4u, default_threads())));
+    return true;
+}
+
+// The process's staging.
+static std::shared_ptr<OutStage> out_stage() {
     static std::mutex mu;
     static std::weak_ptr<OutStage> shared;
-    std::shared_ptr<OutStage> o;
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        o = shared.lock();
-        if (!o) shared = o = std::make_shared<OutStage>();
-    }
-    std::unique_lock<std::mutex> use(o->use, std::try_to_lock);
-    if (!use.owns_lock()) return o;
-    const size_t want = n <= kOutAlone ? kOutAlone : kOutMax;
-    if (want > o->bytes) {
-        char *p = nullptr;
-        if (hipHostMalloc((void **)&p, want, hipHostMallocDefault) != hipSuccess || !p) {
-            (void)hipGetLastError();
-            raise(OG_ENOMEM_HOST, "pinned host allocation of %zu bytes failed", want);
-        }
-        if (o->buf) (void)hipHostFree(o->buf);
-        o->buf = p;
-        o->bytes = want;
-    }
-    if (!o->flag) {
-        const size_t fb = kOutMax / kOutSlab * sizeof(unsigned long long);
-        if (hipHostMalloc((void **)&o->flag, fb, hipHostMallocDefault) != hipSuccess || !o->flag) {
-            (void)hipGetLastError();
-            o->flag = nullptr;
-            raise(OG_ENOMEM_HOST, "pinned host allocation of %zu bytes failed", fb);
-        }
-        std::memset(o->flag, 0, fb);
-    }
-    if (n > kOutAlone && !o->pool) o->pool.reset(new WorkerPool(std::min(4u, default_threads())));
+    std::lock_guard<std::mutex> lk(mu);
+    std::shared_ptr<OutStage> o = shared.lock();
+    if (!o) shared = o = std::make_shared<OutStage>();
     return o;
+}
+
+// The staging with room for a result of n bytes, taken; or not (no lock): in
+// use, or no memory.
+static std::unique_lock<std::mutex> take_stage(DeviceState *d, size_t n) {
+    if (!d->out) d->out = out_stage();
+    std::unique_lock<std::mutex> use(d->out->use, std::try_to_lock);
+    if (use.owns_lock() && !d->out->reserve(n)) use.unlock();
+    return use;
 }
 
 static void copy_chunks_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStream_t s) {
@@ -1805,14 +1813,13 @@ static void copy_chunks_to_host(DeviceState *d, void *dst, const void *src, size
 void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStream_t s) {
     if (!n) return;
     if (n > kOutMax) return copy_chunks_to_host(d, dst, src, n, s);
-    if (!d->out || d->out->bytes < n) d->out = out_stage(n);
-    OutStage &o = *d->out;
-    std::unique_lock<std::mutex> use(o.use, std::try_to_lock);
-    if (!use.owns_lock() || o.bytes < n) {
+    const std::unique_lock<std::mutex> use = take_stage(d, n);
+    if (!use.owns_lock()) {
         OG_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, s));
         OG_HIP(hipStreamSynchronize(s));
         return;
     }
+    OutStage &o = *d->out;
     const size_t slabs = (n + kOutSlab - 1) / kOutSlab;
     const unsigned long long seq = ++o.seq;
     hipLaunchKernelGGL(k_export, dim3((unsigned)slabs), dim3(kBlock), 0, s, (const uint32_t *)src, (uint64_t)(n / 4),
@@ -2501,7 +2508,7 @@ static void prepare_impl(og_graph *g, og_approach approach, const og_plan_params
     d->d_val = (uint32_t *)d->dalloc(d->Vpad * sizeof(uint32_t));
     OG_HIP(hipStreamSynchronize(d->s_compute));
     frontier_alloc(d.get(), g, d->fr, d->mem);
-    if (V * sizeof(uint32_t) <= kOutMax) d->out = out_stage(V * sizeof(uint32_t));
+    (void)take_stage(d.get(), V * sizeof(uint32_t));
     pl.device_bytes = d->device_bytes();
     if (info) *info = pl;
     g->dev = d.release();
@@ -3156,10 +3163,9 @@ static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats 
     // A small graph wholly in HBM: one launch (the A/B flags keep the rounds)
     if (!d->managed && d->plan.vsplit >= V && V <= (ALGO == ALGO_CC ? kSmallVcc : kSmallV) && d->E <= kSmallE &&
         !(d->flags & (OG_PLAN_NO_FUSE | OG_PLAN_NO_OVERLAP))) {
-        if (out && (!d->out || d->out->bytes < V * 4)) d->out = out_stage(V * 4);
         std::unique_lock<std::mutex> use;
-        if (out) use = std::unique_lock<std::mutex>(d->out->use, std::try_to_lock);
-        const bool direct = use.owns_lock() && d->out->bytes >= V * 4;
+        if (out) use = take_stage(d, V * 4);
+        const bool direct = use.owns_lock();
         __atomic_store_n(d->fr.h_progress, 0ull, __ATOMIC_RELEASE);
         const SmallArgs a{d->d_ptr, d->d_static, d->wbits, (uint32_t)V, src, d->d_val,
                           direct ? (uint32_t *)d->out->buf : nullptr, d->fr.blk, d->fr.h_blk, d->fr.h_progress, false, 0};

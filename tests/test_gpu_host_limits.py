@@ -147,3 +147,27 @@ def test_no_memory_for_the_link_format(gpu, tmp_path):
     assert shim.shim_denied() == before + 1
     assert np.abs(g.pagerank()[0] - oracle.pagerank(od, ptr, cols)[0]).max() < 1e-6
     """)
+
+
+def test_no_memory_for_the_result_staging(gpu, tmp_path):
+    """Results up to 8 MB leave through pinned staging of 256 KiB or 8 MiB and
+    flags of 2 KiB; without any one of them they leave through the runtime, from
+    the one-launch traversal too.  Preparing and running do not fail, and
+    staging is used again once there is memory."""
+    hip_shim.run(tmp_path, LINK + """
+    for size in (256 << 10, 8 << 20, 2048):
+        for V in (3000, 70001, 300001):
+            g, ptr, cols, w = graph(V, True)
+            ref = oracle.bfs(ptr[:-1], cols, 0)[0], oracle.sssp(ptr[:-1], cols, w, 0)
+            before = shim.shim_denied()
+            shim.shim_deny_pinned(size, size)
+            g.prepare("ascetic", edge_budget_bytes=8 * len(cols), advisek=1.0)
+            for _ in range(2):
+                assert np.array_equal(g.bfs(0)[0], ref[0])
+                assert np.array_equal(g.sssp(0)[0], ref[1])
+            if size == 2048 or (size == 256 << 10) == (4 * V <= 256 << 10):
+                assert shim.shim_denied() > before, (size, V)
+            shim.shim_deny_pinned(1, 0)
+            assert np.array_equal(g.bfs(0)[0], ref[0])
+            g.close()       # (the process's staging goes with the last preparation)
+    """)

@@ -1826,7 +1826,7 @@ void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStrea
                        (uint32_t *)o.buf, o.flag, seq);
     OG_HIP(hipGetLastError());
     std::atomic<size_t> next{0}, copied{0};
-    std::atomic<bool> failed{false};
+    std::atomic<int> failed{hipSuccess};
     // thread 0 asks the stream now and then: a device error ends every wait
     auto pause = [&](unsigned t, uint64_t spins) {
         if (spins % 2048) {
@@ -1835,7 +1835,7 @@ void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStrea
         }
         if (t == 0) {
             const hipError_t e = hipStreamQuery(s);
-            if (e != hipSuccess && e != hipErrorNotReady) failed.store(true);
+            if (e != hipSuccess && e != hipErrorNotReady) failed.store(e);
         }
         std::this_thread::yield();
     };
@@ -1854,7 +1854,10 @@ void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStrea
     };
     if (n > kOutAlone && o.pool) o.pool->run(work);
     else work(0);
-    if (failed.load()) OG_HIP(hipStreamSynchronize(s));
+    if (failed.load()) {  // slabs are missing, also if the stream recovers
+        (void)hipStreamSynchronize(s);
+        OG_HIP((hipError_t)failed.load());
+    }
 }
 
 // Largest number of hub tiles any frontier can produce for the current tuning.

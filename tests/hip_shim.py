@@ -1,7 +1,8 @@
 """A library that stands between libonegraph and the HIP runtime in a child
-process: it can refuse pinned or device allocations by size, and it counts what
-the calls did.  Nothing it does reaches the GPU: refused calls return an error
-from the host, all others go to the runtime as they are."""
+process: it can refuse pinned or device allocations by size, leave a launch out
+and report an error for a stream's state, and it counts what the calls did.
+Nothing it does reaches the GPU: such calls end on the host, all others go to
+the runtime as they are."""
 import os
 import subprocess
 import sys
@@ -72,6 +73,19 @@ int shim_pinned_has(size_t n) {
     pthread_mutex_unlock(&mu);
     return has;
 }
+typedef struct { unsigned x, y, z; } Dim;
+static atomic_int query_error;
+static unsigned skip_grid, skip_block;
+int hipStreamQuery(void *s) {
+    if (atomic_load(&query_error)) return 999;
+    return ((int (*)(void *))real("hipStreamQuery"))(s);
+}
+int hipLaunchKernel(const void *f, Dim g, Dim b, void **a, size_t lds, void *s) {
+    if (skip_grid && g.x == skip_grid && b.x == skip_block) return 0;
+    return ((int (*)(const void *, Dim, Dim, void **, size_t, void *))real("hipLaunchKernel"))(f, g, b, a, lds, s);
+}
+void shim_query_error(int on) { atomic_store(&query_error, on); }
+void shim_skip_launch(unsigned grid, unsigned block) { skip_grid = grid; skip_block = block; }
 void shim_deny_pinned(size_t lo, size_t hi) { deny_pin.lo = lo; deny_pin.hi = hi; }
 void shim_deny_device(size_t lo, size_t hi) { deny_dev.lo = lo; deny_dev.hi = hi; }
 long shim_denied(void) { return atomic_load(&denied); }
@@ -96,14 +110,13 @@ assert og.device_count() > 0
 """
 
 
-def run(tmp_path, code, timeout=100):
-    """Runs `code` in a child whose library calls go through the shim; returns
-    what it printed.  Its asserts fail the test."""
+def run(tmp_path, *code, timeout=100):
+    """Runs the pieces of code (each with an indent of its own) in a child whose
+    library calls go through the shim.  Its asserts fail the test."""
     src, so = str(tmp_path / "shim.c"), str(tmp_path / "shim.so")
     with open(src, "w") as f:
         f.write(SOURCE)
     subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", so, src, "-ldl", "-lpthread"], check=True)
-    r = subprocess.run([sys.executable, "-u", "-c", HEAD.format(so=so, root=ROOT) + textwrap.dedent(code)],
-                       capture_output=True, text=True, timeout=timeout, cwd=ROOT)
-    assert r.returncode == 0, r.stdout + r.stderr
-    return r.stdout
+    text = "\n".join([HEAD.format(so=so, root=ROOT)] + [textwrap.dedent(c) for c in code] + ["print('done')"])
+    r = subprocess.run([sys.executable, "-u", "-c", text], capture_output=True, text=True, timeout=timeout, cwd=ROOT)
+    assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout + r.stderr

@@ -24,7 +24,7 @@ def test_pagerank_clears_on_its_own_stream(gpu, tmp_path):
     """The arrival counters are cleared on the stream that counts in them (the
     others do not wait for the null stream), at the first run and after a tuning
     that takes more workgroups."""
-    hip_shim.run(tmp_path, PULL + """
+    hip_shim.run(tmp_path, PULL, """
     ptr, cols, od = pull(40000)
     ref = oracle.pagerank(od, ptr, cols)[0]
     g = og.Graph.from_csr(ptr, cols, out_degree=od)
@@ -46,7 +46,7 @@ def test_runs_after_a_refused_allocation(gpu, tmp_path):
     """A first call that runs out of memory part of the way fails with that
     status, and the next one, with memory, is whole: PageRank's state and the two
     chunks of results above 8 MB."""
-    hip_shim.run(tmp_path, PULL + """
+    hip_shim.run(tmp_path, PULL, """
     V = (1 << 21) + 5
     ptr, cols, od = pull(V)
     ref = oracle.pagerank(od, ptr, cols)[0]
@@ -93,7 +93,7 @@ def link_bytes(ptr, plan, bits):   # of the narrow words of the dynamic region
 def test_link_format_only_where_it_is_read(gpu, tmp_path):
     """The narrow copy of the dynamic region is built for rounds that read it, in
     place of the packed words; loaders that gather chunks hold whole edges only."""
-    hip_shim.run(tmp_path, LINK + """
+    hip_shim.run(tmp_path, LINK, """
     V = 70001
     for weighted, bits in ((False, 17), (True, 23)):
         g, ptr, cols, w = graph(V, weighted)
@@ -115,7 +115,7 @@ def test_link_format_only_where_it_is_read(gpu, tmp_path):
 
 def test_no_memory_for_the_link_format(gpu, tmp_path):
     """Without pinned memory for the narrow words the edges cross as they are."""
-    hip_shim.run(tmp_path, LINK + PULL + """
+    hip_shim.run(tmp_path, LINK, PULL, """
     V = 70001
     for weighted, bits in ((False, 17), (True, 23)):
         g, ptr, cols, w = graph(V, weighted)
@@ -154,7 +154,7 @@ def test_no_memory_for_the_result_staging(gpu, tmp_path):
     flags of 2 KiB; without any one of them they leave through the runtime, from
     the one-launch traversal too.  Preparing and running do not fail, and
     staging is used again once there is memory."""
-    hip_shim.run(tmp_path, LINK + """
+    hip_shim.run(tmp_path, LINK, """
     for size in (256 << 10, 8 << 20, 2048):
         for V in (3000, 70001, 300001):
             g, ptr, cols, w = graph(V, True)
@@ -170,4 +170,28 @@ def test_no_memory_for_the_result_staging(gpu, tmp_path):
             shim.shim_deny_pinned(1, 0)
             assert np.array_equal(g.bfs(0)[0], ref[0])
             g.close()       # (the process's staging goes with the last preparation)
+    """)
+
+
+def test_missing_slabs_are_an_error(gpu, tmp_path):
+    """A result whose slabs do not come (the export is left out, the stream
+    reports an error once and synchronises without) is an error, not an array
+    with holes."""
+    hip_shim.run(tmp_path, LINK, """
+    V = 300001
+    g, ptr, cols, w = graph(V, False)
+    g.prepare("ascetic", edge_budget_bytes=4 * len(cols), advisek=1.0)
+    ref = oracle.bfs(ptr[:-1], cols, 0)[0]
+    assert np.array_equal(g.bfs(0)[0], ref)
+    shim.shim_skip_launch((4 * V + 32767) // 32768, 256)
+    shim.shim_query_error(1)
+    try:
+        g.bfs(0)
+        raise SystemExit("no error")
+    except og.OgError as e:
+        assert e.name == "OG_EHIP", e
+    shim.shim_skip_launch(0, 0)
+    shim.shim_query_error(0)
+    for _ in range(3):
+        assert np.array_equal(g.bfs(0)[0], ref)
     """)

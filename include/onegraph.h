@@ -171,7 +171,8 @@ typedef struct og_plan_params {
                                    the reference auto rule (GraphMeta.h:311-324) */
     uint32_t param_size;        /* reference paramSize (17 BFS/SSSP/CC, 19 PR);
                                    only used when edge_budget_bytes == 0      */
-    uint32_t host_threads;      /* gather threads; 0 = hardware concurrency   */
+    uint32_t host_threads;      /* gather and result-copy threads; 0 =
+                                   hardware concurrency                        */
     uint32_t flags;             /* OG_PLAN_* bits                             */
     uint32_t split_weight;      /* SSSP light/heavy split (delta-stepping,
                                    Meyer & Sanders): > 0 stores each row of

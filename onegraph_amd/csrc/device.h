@@ -345,9 +345,9 @@ struct OutStage {
     unsigned long long *flag = nullptr;
     unsigned long long seq = 0;
     std::unique_ptr<WorkerPool> pool;
-    // Makes ready for a result of n bytes (`use` held); false when that is too
-    // large or there is no memory for it.
-    bool reserve(size_t n);
+    // Makes ready for a result of n bytes that up to `threads` threads copy out
+    // (`use` held); false when that is too large or there is no memory for it.
+    bool reserve(size_t n, unsigned threads);
     ~OutStage();
 };
 

@@ -1736,7 +1736,7 @@ OutStage::~OutStage() {
     if (flag) (void)hipHostFree(flag);
 }
 
-bool OutStage::reserve(size_t n) {
+bool OutStage::reserve(size_t n, unsigned threads) {
     if (n > kOutMax) return false;
     const size_t want = n <= kOutAlone ? kOutAlone : kOutMax;
     auto pinned = [](size_t b) -> void * {
@@ -1758,7 +1758,7 @@ bool OutStage::reserve(size_t n) {
         if (!flag) return false;
         std::memset(flag, 0, fb);
     }
-    if (n > kOutAlone && !pool) pool.reset(new WorkerPool(std::min(4u, default_threads())));
+    if (n > kOutAlone && threads > 1 && !pool) pool.reset(new WorkerPool(std::min(4u, default_threads())));
     return true;
 }
 
@@ -1777,7 +1777,7 @@ static std::shared_ptr<OutStage> out_stage() {
 static std::unique_lock<std::mutex> take_stage(DeviceState *d, size_t n) {
     if (!d->out) d->out = out_stage();
     std::unique_lock<std::mutex> use(d->out->use, std::try_to_lock);
-    if (use.owns_lock() && !d->out->reserve(n)) use.unlock();
+    if (use.owns_lock() && !d->out->reserve(n, d->host_threads)) use.unlock();
     return use;
 }
 
@@ -1839,7 +1839,10 @@ void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStrea
         }
         std::this_thread::yield();
     };
+    // (the pool is the process's: of its threads as many as this preparation may use)
+    const unsigned threads = n > kOutAlone && o.pool ? std::min(o.pool->size(), d->host_threads) : 1;
     auto work = [&](unsigned t) {
+        if (t >= threads) return;
         for (size_t i = next.fetch_add(1); i < slabs; i = next.fetch_add(1)) {
             for (uint64_t spins = 1; __atomic_load_n(o.flag + i, __ATOMIC_ACQUIRE) != seq; ++spins) {
                 if (failed.load(std::memory_order_relaxed)) return;
@@ -1852,7 +1855,7 @@ void copy_to_host(DeviceState *d, void *dst, const void *src, size_t n, hipStrea
         if (t == 0)
             for (uint64_t spins = 1; copied.load() < slabs && !failed.load(); ++spins) pause(t, spins);
     };
-    if (n > kOutAlone && o.pool) o.pool->run(work);
+    if (threads > 1) o.pool->run(work);
     else work(0);
     if (failed.load()) {  // slabs are missing, also if the stream recovers
         (void)hipStreamSynchronize(s);

@@ -195,3 +195,26 @@ def test_missing_slabs_are_an_error(gpu, tmp_path):
     for _ in range(3):
         assert np.array_equal(g.bfs(0)[0], ref)
     """)
+
+
+def test_host_threads_bound_result_copies(gpu, tmp_path):
+    """Results of 1.2 MB: with host_threads = 1 no threads are kept for them, with
+    4 three helpers beside the caller."""
+    hip_shim.run(tmp_path, LINK, """
+    import os
+    V = 300001
+    g, ptr, cols, w = graph(V, False)
+    ref = oracle.bfs(ptr[:-1], cols, 0)[0]
+
+    def threads_with(n):
+        g.prepare("ascetic", edge_budget_bytes=4 * len(cols), advisek=1.0, host_threads=n)
+        for _ in range(3):
+            assert np.array_equal(g.bfs(0)[0], ref)
+        return len(os.listdir("/proc/self/task"))
+
+    threads_with(1)     # (the runtime's own threads are there now)
+    one = threads_with(1)
+    assert threads_with(4) == one + 3
+    assert threads_with(2) == one + 3   # (one pool for the process)
+    assert threads_with(1) == one
+    """)

@@ -267,7 +267,12 @@ class EventPool {
 
 // Owner of device and pinned host allocations; frees them all at once.
 struct MemPool {
-    std::vector<void *> dev, pin;
+    struct Block {
+        void *p;
+        size_t bytes;
+    };
+    std::vector<Block> dev;
+    std::vector<void *> pin;
     uint64_t device_bytes = 0;
     MemPool() = default;
     MemPool(const MemPool &) = delete;
@@ -281,9 +286,21 @@ struct MemPool {
             (void)hipGetLastError();
             raise(OG_ENOMEM_DEVICE, "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
         }
-        dev.push_back(p);
+        dev.push_back({p, bytes});
         device_bytes += bytes;
         return p;
+    }
+    // Gives one device allocation back before the others (null: nothing).
+    template <class T>
+    void dfree(T *&p) {
+        for (size_t i = 0; p && i < dev.size(); ++i)
+            if (dev[i].p == p) {
+                device_bytes -= dev[i].bytes;
+                dev.erase(dev.begin() + i);
+                (void)hipFree(p);
+                break;
+            }
+        p = nullptr;
     }
     // null when there is no memory
     void *try_palloc(size_t bytes) {
@@ -301,7 +318,7 @@ struct MemPool {
         return p;
     }
     void release() {
-        for (void *p : dev) (void)hipFree(p);
+        for (const Block &b : dev) (void)hipFree(b.p);
         for (void *p : pin) (void)hipHostFree(p);
         dev.clear();
         pin.clear();
@@ -439,16 +456,17 @@ struct DeviceState {
     EventPool events;
     std::unique_ptr<WorkerPool> pool;
 
-    // multi-source BFS state (allocated on first use)
-    // Multi-source BFS with one mask per vertex (d_ms[0]) and two (d_ms[1])
+    // Multi-source BFS state, allocated on first use (ms_state) for walks of
+    // `masks` masks per vertex; what is there for two serves walks of one.
     struct MsState {
         ulonglong2 *vn = nullptr;            // masks x V: sources that reached v, sources offered to v this round
         uint64_t *front = nullptr;           // masks x V: sources whose frontier holds v
         unsigned long long *part = nullptr;  // per commit workgroup: digest, reached, traversed of the sources
         uint32_t *src = nullptr;             // the batch's sources
         unsigned long long *sum = nullptr;   // per mask 3 x 64: digest, reached, traversed per source
-        uint8_t *lvl = nullptr;              // masks x V x 64 levels, vertex-major (0 = unreached); only when levels are asked for
-    } d_ms[2];
+        uint8_t *lvl = nullptr;              // lvl_masks x V x 64 levels, vertex-major (0 = unreached); only when levels are asked for
+        uint32_t masks = 0, lvl_masks = 0;
+    } d_ms;
     uint32_t *d_extract = nullptr;   // u32 levels of extract_cap sources on their way to the host
     uint32_t extract_cap = 0;
     // direction-optimising BFS: in-edge CSR (OG_PLAN_DIRECTION_OPT)

@@ -2658,7 +2658,7 @@ static void gather(DeviceState *d, const og_graph *g, uint32_t ndyn, uint64_t c0
 
 template <int ALGO>
 static RelaxArgs relax_args(DeviceState *d) {
-    const DeviceState::MsState &m = d->d_ms[ms_masks(ALGO) == 2];
+    const DeviceState::MsState &m = d->d_ms;
     return RelaxArgs{d->d_val, d->fr.flag, m.vn, m.front, d->wbits, nullptr, d->run_pmid,
                      d->run_pmid ? d->fr.ctl : nullptr};
 }
@@ -3221,6 +3221,41 @@ static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats 
 // caller wants them.
 constexpr uint64_t kExtractBytes = 256ull << 20;  // device buffer of levels on their way to the host, at most
 
+// Workgroups of the commit sweep.
+static unsigned ms_commit_grid(uint64_t V) {
+    return (unsigned)std::min<uint64_t>(kMsCommitGrid, std::max<uint64_t>(1, (V + kBlock - 1) / kBlock));
+}
+
+// The state for a walk of H masks per vertex.  Narrower arrays leave before
+// wider ones take their place, with the captured rounds that hold their addresses.
+static DeviceState::MsState &ms_state(DeviceState *d, uint32_t H, bool levels) {
+    DeviceState::MsState &m = d->d_ms;
+    const uint64_t V = d->V;
+    if (m.masks < H) {
+        if (m.vn) d->round_graph.reset();
+        m.masks = 0;
+        d->mem.dfree(m.vn);
+        d->mem.dfree(m.front);
+        d->mem.dfree(m.src);
+        d->mem.dfree(m.part);
+        d->mem.dfree(m.sum);
+        m.vn = (ulonglong2 *)d->dalloc(H * V * 16);
+        m.front = (uint64_t *)d->dalloc(H * V * 8);
+        m.src = (uint32_t *)d->dalloc(H * kMsWidth * 4);
+        m.part = (unsigned long long *)d->dalloc((uint64_t)ms_commit_grid(V) * H * kMsSums * 8);
+        m.sum = (unsigned long long *)d->dalloc(H * kMsSums * 8);
+        m.masks = H;
+    }
+    if (levels && m.lvl_masks < H) {
+        if (m.lvl) d->round_graph.reset();
+        m.lvl_masks = 0;
+        d->mem.dfree(m.lvl);
+        m.lvl = (uint8_t *)d->dalloc(H * V * kMsWidth);
+        m.lvl_masks = H;
+    }
+    return m;
+}
+
 // One traversal from nb <= 64 H sources.
 template <int H, bool W>
 static void ms_batch(og_graph *g, DeviceState *d, const uint32_t *sources, uint32_t nb, uint32_t *levels,
@@ -3229,17 +3264,8 @@ static void ms_batch(og_graph *g, DeviceState *d, const uint32_t *sources, uint3
     constexpr int ALGO = H == 1 ? ALGO_MSBFS : ALGO_MSBFS2;
     const uint64_t V = d->V;
     hipStream_t s = d->s_compute;
-    DeviceState::MsState &m = d->d_ms[H - 1];
-    const unsigned cgrid =
-        (unsigned)std::min<uint64_t>(kMsCommitGrid, std::max<uint64_t>(1, (V + kBlock - 1) / kBlock));
-    if (!m.sum) {
-        if (!m.vn) m.vn = (ulonglong2 *)d->dalloc(H * V * 16);
-        if (!m.front) m.front = (uint64_t *)d->dalloc(H * V * 8);
-        if (!m.src) m.src = (uint32_t *)d->dalloc(H * kMsWidth * 4);
-        if (!m.part) m.part = (unsigned long long *)d->dalloc((uint64_t)cgrid * H * kMsSums * 8);
-        m.sum = (unsigned long long *)d->dalloc(H * kMsSums * 8);
-    }
-    if (levels && !m.lvl) m.lvl = (uint8_t *)d->dalloc(H * V * kMsWidth);
+    DeviceState::MsState &m = ms_state(d, H, levels != nullptr);
+    const unsigned cgrid = ms_commit_grid(V);
     if (levels && !d->d_extract) {
         d->extract_cap = (uint32_t)std::min<uint64_t>(kMsWidth, std::max<uint64_t>(1, kExtractBytes / (V * 4)));
         d->d_extract = (uint32_t *)d->dalloc((uint64_t)d->extract_cap * V * 4);
@@ -3303,8 +3329,8 @@ static void ms_batch(og_graph *g, DeviceState *d, const uint32_t *sources, uint3
 // memory that the wider masks (and levels) take, an eighth of what is free.
 static bool ms_wide(const DeviceState *d, uint32_t left, bool levels) {
     if (left <= kMsWidth) return false;
-    const DeviceState::MsState &m = d->d_ms[1];
-    const uint64_t more = (m.sum ? 0 : 48 * d->V) + (levels && !m.lvl ? 2 * kMsWidth * d->V : 0);
+    const DeviceState::MsState &m = d->d_ms;
+    const uint64_t more = (24 * (2 - m.masks) + (levels ? kMsWidth * (2 - m.lvl_masks) : 0)) * d->V;
     if (!more) return true;
     size_t free = 0, all = 0;
     OG_HIP(hipMemGetInfo(&free, &all));

@@ -218,3 +218,34 @@ def test_host_threads_bound_result_copies(gpu, tmp_path):
     assert threads_with(2) == one + 3   # (one pool for the process)
     assert threads_with(1) == one
     """)
+
+
+def test_multi_source_state_of_one_width(gpu, tmp_path):
+    """A preparation that has served short and long batches holds the state of the
+    widest, not of both: 48 bytes a vertex, with levels 128 more, beside what is
+    independent of the graph (2048 workgroups' sums, the turned levels).  Replayed
+    rounds follow the state when it moves."""
+    hip_shim.run(tmp_path, LINK, """
+    V = 300001
+    g, ptr, cols, w = graph(V, False)
+    rng = np.random.default_rng(5)
+    src = rng.choice(np.flatnonzero(np.diff(ptr.astype(np.int64)) > 0), 100).astype(np.uint32)
+    ref = np.array([oracle.bfs(ptr[:-1], cols, int(s))[0] for s in src])
+    sums = np.array([og.levels_checksum(r) for r in ref], np.uint64)
+    fixed = 2 * 2048 * 3 * 64 * 8 + (1 << 16)
+    for budget, k, flags in ((4 * len(cols), 1.0, 0), (2 * len(cols), 0.5, og.PLAN_ZERO_COPY)):
+        for order in ((30, 100, 64, 65, 30), (100, 1, 100)):
+            g.prepare("ascetic", edge_budget_bytes=budget, advisek=k, flags=flags)
+            assert np.array_equal(g.msbfs(src[:0], want_levels=False)[1], sums[:0])
+            base = shim.shim_live_device()
+            for n in order:
+                for _ in range(2):
+                    assert np.array_equal(g.msbfs(src[:n], want_levels=False)[1], sums[:n]), n
+            assert shim.shim_live_device() - base <= 48 * V + fixed, (shim.shim_live_device() - base) / V
+            for n in order:
+                for _ in range(2):
+                    lv, cs, _, _ = g.msbfs(src[:n])
+                    assert np.array_equal(lv, ref[:n]) and np.array_equal(cs, sums[:n]), n
+                    assert np.array_equal(g.msbfs(src[:n], want_levels=False)[1], sums[:n]), n
+            assert shim.shim_live_device() - base <= (48 + 128 + 4 * 64) * V + fixed
+    """)

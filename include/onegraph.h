@@ -296,7 +296,11 @@ og_status og_cc(og_graph *g, uint32_t *labels, og_run_stats *stats);
 
 /* Shapes of the static-region relax and the SSSP round order.  The reference
  * has one shape: one work-item per vertex, grid 1024*108
- * (BFS/oneGraph_BFS/globals.h:16-17). */
+ * (BFS/oneGraph_BFS/globals.h:16-17).  og_bfs, og_sssp and og_cc on a graph
+ * wholly in HBM of up to 16384 vertices (og_cc: 8192) and 196608 edges run in
+ * one launch that has none of these shapes, and every improved vertex relaxes
+ * in the next round (OG_PLAN_NO_FUSE or NO_OVERLAP keep the rounds); the
+ * tuning then governs og_msbfs and a server's BFS alone. */
 typedef struct og_tuning {
     uint32_t t1;     /* bin 0: 1 <= degree <= t1, lpv0 lanes per vertex          */
     uint32_t lpv0;   /* 1, 2, 4, 8, 16, 32 or 64                                  */
@@ -332,7 +336,9 @@ og_status og_set_tuning(og_graph *g, const og_tuning *t);
  * candidate tunings (coordinate descent: defer for SSSP / CC with a dynamic
  * region, delta for SSSP, then t1 with lpv0, t2, tile, and dyn_grid with a
  * dynamic region; the median of `runs` timed runs each), installs the fastest and
- * returns it with its time.  Results do not depend on the tuning.  The
+ * returns it with its time.  Results do not depend on the tuning.  Where
+ * `algo` runs in one launch (og_tuning) nothing is tried: the tuning stays and is
+ * returned with its time.  The
  * workgroup size stays 256 (four 64-lane waves); the grid shapes tuned are
  * the lanes per vertex of bin 0 and the dynamic relax's workgroups. */
 og_status og_autotune(og_graph *g, uint32_t algo, uint32_t source, uint32_t runs,

@@ -3151,6 +3151,14 @@ static void finish_stats(og_run_stats &st, RunTimers &tm, double gather_ms, doub
     st.gather_ms = gather_ms;
 }
 
+// Whether a run is one launch of k_small: a small graph wholly in HBM (the A/B
+// flags keep the rounds).
+template <int ALGO>
+static bool one_launch(const DeviceState *d) {
+    return !d->managed && d->plan.vsplit >= d->V && d->V <= (ALGO == ALGO_CC ? kSmallVcc : kSmallV) &&
+           d->E <= kSmallE && !(d->flags & (OG_PLAN_NO_FUSE | OG_PLAN_NO_OVERLAP));
+}
+
 template <int ALGO, bool W>
 static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats *stats, DeviceState *dv = nullptr) {
     DeviceState *d = dv ? dv : g->dev;
@@ -3166,9 +3174,7 @@ static void run_frontier(og_graph *g, uint32_t src, uint32_t *out, og_run_stats 
     OG_HIP(hipStreamSynchronize(d->s_static));
     OG_HIP(hipStreamSynchronize(s));
     Stopwatch total;
-    // A small graph wholly in HBM: one launch (the A/B flags keep the rounds)
-    if (!d->managed && d->plan.vsplit >= V && V <= (ALGO == ALGO_CC ? kSmallVcc : kSmallV) && d->E <= kSmallE &&
-        !(d->flags & (OG_PLAN_NO_FUSE | OG_PLAN_NO_OVERLAP))) {
+    if (one_launch<ALGO>(d)) {
         std::unique_lock<std::mutex> use;
         if (out) use = take_stage(d, V * 4);
         const bool direct = use.owns_lock();
@@ -3810,7 +3816,13 @@ extern "C" og_status og_autotune(og_graph *g, uint32_t algo, uint32_t source, ui
             apply_tuning(g, &cur);
         };
         const bool has_dyn = g->dev->plan.vsplit < g->V;
-        for (int pass = 0; pass < 2; ++pass) {
+        // a run in one launch has no shape to tune: the candidates would differ
+        // by noise, and other calls on the preparation would get the choice
+        const bool fixed = algo == OG_TUNE_BFS    ? one_launch<ALGO_BFS>(g->dev)
+                           : algo == OG_TUNE_SSSP ? one_launch<ALGO_SSSP>(g->dev)
+                           : algo == OG_TUNE_CC   ? one_launch<ALGO_CC>(g->dev)
+                                                  : false;
+        for (int pass = 0; pass < 2 && !fixed; ++pass) {
             if ((algo == OG_TUNE_SSSP || algo == OG_TUNE_CC) && has_dyn)
                 for (uint32_t df : {0u, 1u, 2u}) {
                     if (df == 2 && algo != OG_TUNE_SSSP) continue;

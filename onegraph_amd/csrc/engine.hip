@@ -2132,9 +2132,11 @@ static void stage_resident(DeviceState *d, const og_graph *g, uint64_t vsplit, u
     OG_HIP(hipStreamSynchronize(d->s_compute));
 }
 
-// Slots of the chunk ring: small enough that a few are on their way while
-// others are used, large enough that a copy takes longer than its hand-over
-// (4 MiB: 73 us on the link).
+// Slots of the chunk ring: two to kRing of them, as many as have kRingSlotBytes,
+// which take the staging share between them.  At least that large, a copy takes
+// longer than its hand-over (4 MiB: 73 us on the link); a share above 32 MiB
+// makes them larger, since what the ring holds is what crosses the link
+// while the static rows are summed.
 constexpr uint64_t kRingSlotBytes = 4ull << 20;
 constexpr uint32_t kRing = 8;
 

@@ -437,11 +437,14 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
         // The copies run ahead of the pulls by the ring, into the next
         // iteration too (its edges are the same whatever the ranks are), so
         // the link does not wait for the end of an iteration nor, while the
-        // ring fills, for the static pull.  Consecutive copies alternate
+        // ring fills, for the static pull; an iteration that turns out to be the
+        // last has up to a ring of copies enqueued for nothing, which are not
+        // counted.  Consecutive copies alternate
         // between two streams: the hand-over from a copy to the next one's
         // wait costs about 30 us, hidden behind the other stream's copy.
         LinkRing &lr = *pp.link;
         const uint64_t nc = lr.chunks.size();
+        const uint64_t limit = prm.max_iterations * nc;
         uint64_t copied = 0, pulled = 0;
         auto copy_next = [&] {
             const LinkRing::Chunk &ch = lr.chunks[copied % nc];
@@ -452,8 +455,6 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
             if (ch.words)
                 OG_HIP(hipMemcpyAsync(dslot, lr.src + ch.word, ch.words * 4, hipMemcpyHostToDevice, on));
             OG_HIP(hipEventRecord(lr.ev_h2d[slot], on));
-            st.run.h2d_bytes += ch.words * 4;
-            st.run.chunks++;
             ++copied;
         };
         {
@@ -461,7 +462,7 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
             while (it < prm.max_iterations) {
                 turn(it);
                 // the copies first: what the ring holds crosses the link beside the static pull
-                while (copied < pulled + std::min<uint64_t>(lr.ring, nc)) copy_next();
+                while (copied < std::min(pulled + std::min<uint64_t>(lr.ring, nc), limit)) copy_next();
                 if (sgrid) {
                     EventSpan span(d, &tc_static, s);
                     pull_static(s, nullptr);
@@ -480,9 +481,11 @@ static void run_pr(og_graph *g, const og_pr_params &prm, T *out, og_pr_stats *st
                     }
                     poff += gr;
                     OG_HIP(hipEventRecord(lr.ev_use[slot], s));
-                    // the slots that are free, the one this chunk leaves among them
-                    const bool last = it + 1 == prm.max_iterations;
-                    while (copied < pulled + 1 + lr.ring && !(last && copied % nc == 0 && copied > pulled)) copy_next();
+                    st.run.h2d_bytes += ch.words * 4;
+                    st.run.chunks++;
+                    // the slots that are free, the one this chunk leaves among them,
+                    // up to the next iteration's last chunk
+                    while (copied < std::min({pulled + 1 + lr.ring, (it + 2) * nc, limit})) copy_next();
                 }
                 hipLaunchKernelGGL(k_pr_finish, dim3(1), dim3(1024), 0, s, d->d_partial, (uint32_t)poff, d->d_prstate,
                                    d->h_progress);

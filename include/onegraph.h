@@ -311,12 +311,16 @@ typedef struct og_tuning {
                         improved vertex every round (the reference's order)     */
     uint32_t defer;  /* SSSP / CC: 1 = a round with static-region work holds the
                         dynamic-region vertices back, so the link rows are read
-                        once the in-HBM part has settled, in denser rounds; 0 =
-                        both regions every round (the reference's order);
-                        SSSP with delta > 0: 2 = lagged, a dynamic-region
+                        once the in-HBM part has settled, in denser rounds.
+                        SSSP: 0 = both regions every round (the reference's
+                        order); with delta > 0, 2 = lagged, a dynamic-region
                         vertex relaxes only after the static vertices of its
                         near-far bucket have settled, so its link row is
-                        read about once                                          */
+                        read about once.
+                        CC, which starts with every vertex active: 0 = the
+                        dynamic vertices wait until the static region has settled
+                        once, then both regions every round; 2 = both regions
+                        every round from the start (the reference's order)      */
     uint32_t dyn_grid; /* workgroups of the dynamic-region relax, 0 = 8192; fewer
                         leave CUs to the static relax it overlaps with           */
 } og_tuning;

@@ -2938,13 +2938,16 @@ static void frontier_loop(og_graph *g, DeviceState *d, og_run_stats &st, RunTime
     const bool staged = has_dyn && !d->in_place;
     // deferring dynamic vertices reorders relaxations across levels, which
     // only the atomicMin relaxes (SSSP, CC) tolerate.  CC starts with every
-    // vertex active: unless a tuning says otherwise its dynamic vertices wait
-    // until the static region has settled once, so that most of them carry
-    // their final label when their rows cross the link (ER 3 M x 32, a
-    // quarter of the edges on the device: the rows are read once instead of
-    // about twice, 10.5 -> 7.9 ms).
+    // vertex active: at 0 its dynamic vertices wait until the static region has
+    // settled once, so that most of them carry their final label when their rows
+    // cross the link (ER 3 M x 32, a quarter of the edges on the device: the
+    // rows are read once instead of about twice, 10.5 -> 7.9 ms); 2 is both
+    // regions every round.
     uint32_t defer = (ALGO == ALGO_SSSP || ALGO == ALGO_CC) && has_dyn ? d->tune.defer : 0;
-    if (ALGO == ALGO_CC && has_dyn && d->plan.vsplit && !defer) defer = kDeferOnce;
+    if (ALGO == ALGO_CC) {
+        if (defer == 2) defer = 0;
+        else if (defer == 0 && has_dyn && d->plan.vsplit) defer = kDeferOnce;
+    }
     const bool dir_opt = ALGO == ALGO_BFS && d->d_in_ptr != nullptr;
     // light/heavy split: near-far SSSP on a graph prepared with it
     const bool split = ALGO == ALGO_SSSP && delta && d->d_pmid;
@@ -3827,7 +3830,6 @@ extern "C" og_status og_autotune(og_graph *g, uint32_t algo, uint32_t source, ui
         for (int pass = 0; pass < 2 && !fixed; ++pass) {
             if ((algo == OG_TUNE_SSSP || algo == OG_TUNE_CC) && has_dyn)
                 for (uint32_t df : {0u, 1u, 2u}) {
-                    if (df == 2 && algo != OG_TUNE_SSSP) continue;
                     og_tuning c = cur;
                     c.defer = df;
                     trial(c);

@@ -214,6 +214,10 @@ typedef struct og_plan_params {
                                    parent, stopping at the first); needs the
                                    in-edge CSR on the device (E * 4 + V * 8
                                    bytes beyond the edge budget)               */
+#define OG_PLAN_TEST_WIDE_LISTS 0x80000000u /* testing: the compaction counts the
+                                   dynamic list's vertices and edges in two words,
+                                   as it does where they do not fit 64 bits
+                                   together                                      */
 
 typedef struct og_plan_info {
     uint64_t total_budget_edges;  /* reference total_gpu_size               */

@@ -23,6 +23,7 @@ PLAN_NO_PACK = 4
 PLAN_NO_GRAPH = 8
 PLAN_DIRECTION_OPT = 16
 PLAN_NO_FUSE = 32
+PLAN_TEST_WIDE_LISTS = 0x80000000  # testing: the compaction's two-word counts (onegraph.h OG_PLAN_TEST_WIDE_LISTS)
 EDGES_SYMMETRIZE, EDGES_KEEP_SELF_LOOPS, EDGES_ONE_BASED, EDGES_WEIGHTED = 1, 2, 4, 8
 
 STATUS = {

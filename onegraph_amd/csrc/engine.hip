@@ -1893,7 +1893,7 @@ void frontier_alloc(DeviceState *d, const og_graph *g, Frontier &f, MemPool &m) 
     f.tot = (unsigned long long *)m.dalloc(totals_words(f.nblk) * 8);
     // dynamic list: its count and its edges in one word when they fit
     const uint32_t nb = bits_of(V - d->plan.vsplit), eb = bits_of(dyn_edges);
-    f.dsh = nb + eb <= 64 && nb < 64 ? std::max(nb, 1u) : 0;
+    f.dsh = nb + eb <= 64 && nb < 64 && !(d->flags & OG_PLAN_TEST_WIDE_LISTS) ? std::max(nb, 1u) : 0;
     hipLaunchKernelGGL(k_totals_init, dim3(fill_grid(totals_words(f.nblk))), dim3(256), 0, d->s_compute, f.tot,
                        totals_words(f.nblk));
     OG_HIP(hipGetLastError());

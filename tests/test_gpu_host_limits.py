@@ -249,3 +249,46 @@ def test_multi_source_state_of_one_width(gpu, tmp_path):
                     assert np.array_equal(g.msbfs(src[:n], want_levels=False)[1], sums[:n]), n
             assert shim.shim_live_device() - base <= (48 + 128 + 4 * 64) * V + fixed
     """)
+
+
+def test_graph_in_pageable_memory(gpu, tmp_path):
+    """A graph that could not be pinned: traversals gather chunks and need the
+    slots alone pinned, PageRank copies from where the edges are; zero-copy is
+    refused."""
+    hip_shim.run(tmp_path, LINK, PULL, """
+    V = 70001
+    E = graph(V, False)[1][-1]
+    shim.shim_deny_pinned(int(4 * E), int(4 * E))
+    g, ptr, cols, w = graph(V, False)
+    shim.shim_deny_pinned(1, 0)
+    try:
+        g.prepare("ascetic", edge_budget_bytes=2 * len(cols), advisek=0.5, flags=og.PLAN_ZERO_COPY)
+        raise SystemExit("not refused")
+    except og.OgError as e:
+        assert e.name == "OG_EUNSUPPORTED", e
+    plan = g.prepare("ascetic", edge_budget_bytes=2 * len(cols), advisek=0.5)
+    narrow, whole = link_bytes(ptr, plan, 17)
+    before = shim.shim_denied()
+    shim.shim_deny_pinned(narrow, narrow)
+    g.prepare("ascetic", edge_budget_bytes=2 * len(cols), advisek=0.5)
+    assert shim.shim_denied() == before
+    shim.shim_deny_pinned(1, 0)
+    for _ in range(2):
+        lv, st = g.bfs(0)
+        assert np.array_equal(lv, oracle.bfs(ptr[:-1], cols, 0)[0]) and st["gather_ms"] > 0
+        assert np.array_equal(g.cc()[0], oracle.cc(ptr[:-1], cols)[0])
+    ptr, cols, od = pull(V)
+    shim.shim_deny_pinned(4 * len(cols), 4 * len(cols))
+    g = og.Graph.from_csr(ptr, cols, out_degree=od)
+    shim.shim_deny_pinned(1, 0)
+    ref = oracle.pagerank(od, ptr, cols)[0]
+    for deny in (0, 1):
+        plan = g.prepare("ascetic", edge_budget_bytes=2 * len(cols), advisek=0.5)
+        if deny:
+            narrow, whole = link_bytes(np.append(ptr, np.uint64(len(cols))), plan, 17)
+            shim.shim_deny_pinned(narrow, narrow)
+            g.prepare("ascetic", edge_budget_bytes=2 * len(cols), advisek=0.5)
+            shim.shim_deny_pinned(1, 0)
+        for _ in range(2):
+            assert np.abs(g.pagerank()[0] - ref).max() < 1e-6
+    """)

@@ -47,7 +47,7 @@ def pick_source(ptr, E, seed):
 
 
 def kernel_table(st):
-    """Per-class algorithmic GB/s from the engine's HIP-event timings.  A
+    """Per-class algorithmic GB/s from the engine's kernel timings.  A
     zero-copy round that relaxes both regions in one launch (k_relax_round)
     is timed as the dynamic class; its row then carries the static bytes too."""
     rows = {}
@@ -133,7 +133,7 @@ KERNEL_NAMES = {"relax_static": "k_relax_group / k_relax_hub (static region)",
 
 
 def roofline_of(stats_list, zero_copy=False, traffic=None):
-    """Roofline of the dominant kernel class (most HIP-event time).
+    """Roofline of the dominant kernel class (most kernel time).
 
     In HBM (static relax, frontier, a staged dynamic relax reading its slot)
     the bound is HBM: achieved = algorithmic bytes / kernel time against
@@ -182,13 +182,15 @@ def roofline_of(stats_list, zero_copy=False, traffic=None):
 
 def plan_flags(args, approach, loader=None):
     """og_plan_params.flags for a workload: the dynamic-region loader and
-    the link format (USM reads the CSR in place and takes neither)."""
+    the link format (USM reads the CSR in place and takes neither).  "copy" is
+    the host gather with copies, which pinned graphs take with NO_FUSE (without
+    a flag their rows are read in place)."""
     import onegraph_amd as og
 
     if approach == "usm":
         return 0
     loader = loader or args.loader
-    return ((og.PLAN_ZERO_COPY if loader == "zerocopy" else 0) | (og.PLAN_NO_PACK if args.no_pack else 0) |
+    return ((og.PLAN_ZERO_COPY if loader == "zerocopy" else og.PLAN_NO_FUSE) | (og.PLAN_NO_PACK if args.no_pack else 0) |
             (og.PLAN_NO_OVERLAP if args.no_overlap else 0) | (og.PLAN_NO_FUSE if args.no_fuse else 0))
 
 
@@ -955,7 +957,7 @@ def main():
             ms2 = 1e3 * w2 / len(s2)
             cmp[ap_name] = {"ms_per_step": round(ms2, 3), "gteps": round(trav / (ms2 * 1e-3) / 1e9, 4),
                             "h2d_bytes": s2[-1]["h2d_bytes"], "iterations": s2[-1]["iterations"],
-                            "loader": "copy" if ap_name == "subway" else "mapped host memory"}
+                            "loader": "gather and copy" if ap_name == "subway" else "mapped host memory"}
         out["compare"] = cmp
 
     # correctness of the measured path + CPU baseline (oracle, single thread)

@@ -36,7 +36,8 @@ static void usage(FILE *f) {
             "                 [--weight-seed S]] [--check FILE [--check-tol T]]\n"
             "                [--loader copy|zerocopy] [--delta W] [--split-weight W] [--direction-opt]\n"
             "                [--autotune]\n"
-            "  --loader zerocopy: the dynamic region is read in place over the host link;\n"
+            "  --loader zerocopy: the dynamic region is read in place over the host link,\n"
+            "  which copy (the default) does too where the memory is pinned;\n"
             "  --delta W: SSSP near-far bucket width; --split-weight W: SSSP rows store\n"
             "  edges lighter than W first (delta-stepping light/heavy); --direction-opt:\n"
             "  bottom-up BFS rounds (whole graph in HBM); --autotune: tune bins, delta and\n"

@@ -278,16 +278,24 @@ struct MemPool {
     MemPool(const MemPool &) = delete;
     MemPool &operator=(const MemPool &) = delete;
     ~MemPool() { release(); }
-    void *dalloc(size_t bytes) {
+    // null when there is no memory (the error in *err)
+    void *try_dalloc(size_t bytes, hipError_t *err = nullptr) {
         void *p = nullptr;
         if (bytes == 0) bytes = 256;
-        hipError_t e = hipMalloc(&p, bytes);
+        const hipError_t e = hipMalloc(&p, bytes);
+        if (err) *err = e;
         if (e != hipSuccess) {
             (void)hipGetLastError();
-            raise(OG_ENOMEM_DEVICE, "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
+            return nullptr;
         }
         dev.push_back({p, bytes});
         device_bytes += bytes;
+        return p;
+    }
+    void *dalloc(size_t bytes) {
+        hipError_t e = hipSuccess;
+        void *p = try_dalloc(bytes, &e);
+        if (!p) raise(OG_ENOMEM_DEVICE, "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
         return p;
     }
     // Gives one device allocation back before the others (null: nothing).

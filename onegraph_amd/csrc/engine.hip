@@ -3277,9 +3277,12 @@ static void ms_batch(og_graph *g, DeviceState *d, const uint32_t *sources, uint3
     hipStream_t s = d->s_compute;
     DeviceState::MsState &m = ms_state(d, H, levels != nullptr);
     const unsigned cgrid = ms_commit_grid(V);
-    if (levels && !d->d_extract) {
-        d->extract_cap = (uint32_t)std::min<uint64_t>(kMsWidth, std::max<uint64_t>(1, kExtractBytes / (V * 4)));
-        d->d_extract = (uint32_t *)d->dalloc((uint64_t)d->extract_cap * V * 4);
+    if (levels && !d->d_extract) {  // fewer sources at a time where memory is short
+        uint32_t cap = (uint32_t)std::min<uint64_t>(kMsWidth, std::max<uint64_t>(1, kExtractBytes / (V * 4)));
+        void *p = nullptr;
+        while (cap > 1 && !(p = d->mem.try_dalloc((uint64_t)cap * V * 4))) cap /= 2;
+        d->d_extract = (uint32_t *)(p ? p : d->dalloc((uint64_t)cap * V * 4));
+        d->extract_cap = cap;
     }
     uint8_t *const lvl = levels ? m.lvl : nullptr;
     std::vector<unsigned long long> hsum(H * kMsSums);

@@ -292,3 +292,23 @@ def test_graph_in_pageable_memory(gpu, tmp_path):
         for _ in range(2):
             assert np.abs(g.pagerank()[0] - ref).max() < 1e-6
     """)
+
+
+def test_levels_with_little_memory(gpu, tmp_path):
+    """Level arrays leave the device for up to 64 sources at a time, for fewer
+    where there is no memory for that."""
+    hip_shim.run(tmp_path, LINK, """
+    V = 70001
+    g, ptr, cols, w = graph(V, False)
+    src = np.arange(70, dtype=np.uint32)
+    ref = np.array([oracle.bfs(ptr[:-1], cols, int(s))[0] for s in src])
+    for n, room in ((64, 64), (70, 128)):   # the levels take 64 or 128 bytes a vertex, 64 turned ones 256
+        g.prepare("ascetic", edge_budget_bytes=4 * len(cols), advisek=1.0)
+        g.msbfs(src[:n], want_levels=False)
+        before = shim.shim_denied()
+        shim.shim_deny_device(room * V + 1, 1 << 40)
+        for _ in range(2):
+            assert np.array_equal(g.msbfs(src[:n])[0], ref[:n])
+        shim.shim_deny_device(1, 0)
+        assert shim.shim_denied() > before
+    """)

@@ -580,30 +580,6 @@ __device__ __forceinline__ uint64_t wave_read_u64(uint64_t x, int l) {
     return ((uint64_t)hi << 32) | lo;
 }
 
-// Exclusive scan over the block of x (u64); *total receives the block sum.
-// `lds` must hold blockDim.x / 64 entries.  Contains __syncthreads.
-__device__ __forceinline__ uint64_t block_exclusive_scan(uint64_t x, uint64_t *total, uint64_t *lds) {
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-    const int nw = blockDim.x / kWave;
-    uint64_t inc = x;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        uint64_t y = shfl_up_u64(inc, o);
-        if (lane >= o) inc += y;
-    }
-    if (lane == kWave - 1) lds[wid] = inc;
-    __syncthreads();
-    uint64_t before = 0, tot = 0;
-    for (int w = 0; w < nw; ++w) {
-        uint64_t s = lds[w];
-        before += (w < wid) ? s : 0;
-        tot += s;
-    }
-    __syncthreads();
-    *total = tot;
-    return before + inc - x;
-}
-
 // N independent exclusive scans over the block in one pass (one LDS round):
 // ex[i] = sum of x[i] over lower threads, tot[i] = block sum.  `lds` must
 // hold N * blockDim.x / 64 entries.  Contains __syncthreads.
@@ -639,13 +615,6 @@ __device__ __forceinline__ void block_scan_n(const uint64_t (&x)[N], uint64_t (&
         tot[i] = t;
     }
     __syncthreads();
-}
-
-// Sum over the block; result valid in every thread.  Contains __syncthreads.
-__device__ __forceinline__ uint64_t block_sum(uint64_t x, uint64_t *lds) {
-    uint64_t t;
-    (void)block_exclusive_scan(x, &t, lds);
-    return t;
 }
 
 // Work counters of a run's relax kernels, spread over kSpread lines of 16

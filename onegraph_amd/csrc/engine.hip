@@ -17,7 +17,7 @@
 //      (CC/onegraph/gpu_kernels.h:133-157).
 //   3. dynamic region: an edge-parallel relax reads the active rows over the
 //      link (K8/K10/K12); in pageable memory the host gathers the active edges of
-//      the sorted dynamic list into a pinned slot (H5, GraphMeta.h:470-506) and
+//      the dynamic list into a pinned slot (H5, GraphMeta.h:470-506) and
 //      hipMemcpyAsync moves the slot while the other one is being gathered.
 #include <algorithm>
 #include <atomic>
@@ -32,19 +32,9 @@ namespace og {
 
 // ================================================================= kernels
 
-__global__ void k_fill_u32(uint32_t *a, uint64_t n, uint32_t v) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        a[i] = v;
-}
-
 __global__ void k_iota(uint32_t *a, uint64_t n) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
         a[i] = (uint32_t)i;
-}
-
-__global__ void k_fill_u8(uint8_t *a, uint64_t n, uint8_t v) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        a[i] = v;
 }
 
 __device__ __forceinline__ void clock_stamp(RoundClock *clk, int prev, int kind) {
@@ -1251,6 +1241,12 @@ __global__ __launch_bounds__(kStatsBlock) void k_reach_stats(const uint32_t *__r
 // 108 K 104 / 167, 16384 / 228 K 170 / 166; SSSP 4000 / 52 K 117 / 353, 16384 /
 // 228 K 380 / 414, 330 K 548 / 464; CC, whose first rounds relax every vertex,
 // 8000 / 168 K 118 / 170 but 16384 / 58 K 289 / 272.
+// SSSP relaxes every improved vertex in the next round here, whatever the
+// bucket width.  On deep graphs that is mostly the faster way too (one launch /
+// near-far rounds at delta 256, ms: a path of 16384 53 / 235, a grid of
+// 128 x 128 1.8 / 4.9, 16000 x 12 random near neighbours on a ring 3.6 / 5.3),
+// but not where shorter hops keep improving every long one (v to v + j at weight
+// j * j: 4000 vertices x 40 160 / 57, 1000 x 196 21 / 15, 500 x 390 5.7 / 7.6).
 constexpr uint32_t kSmallV = 1u << 14;
 constexpr uint32_t kSmallVcc = 1u << 13;
 constexpr uint64_t kSmallE = 3u << 16;
@@ -3882,11 +3878,12 @@ extern "C" og_status og_autotune(og_graph *g, uint32_t algo, uint32_t source, ui
 // og_bfs_device_noalloc: og_bfs over a CSR that already sits in device
 // memory, for callers that cannot allocate (hipMalloc / hipFree / an
 // allocating library call) at run time.  Every buffer beyond the caller's
-// inputs and output -- next-frontier flags, bin lists, hub tiles, per-block
-// counts, the round's summary and control block, counters -- lives in the
+// inputs and output -- next-frontier flags, bin lists, hub tiles, compaction
+// totals, the round's summary and control block, counters -- lives in the
 // file-scope device array `scratch` below, sized for V <= kNoAllocMaxV and
 // E <= kNoAllocMaxE.  Rounds are enqueued directly (no captured hipGraph, no
-// events) and cleared with fill kernels, so the call allocates nothing.
+// events) after one kernel that sets everything up, so the call allocates
+// nothing; graphs of k_small's size take its one launch.
 // Each GPU holds its own copy of `scratch` until the process ends; calls
 // that overlap on one GPU share it and race.
 

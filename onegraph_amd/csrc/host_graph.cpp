@@ -138,7 +138,10 @@ void parallel_for(uint64_t n, uint64_t grain, unsigned threads,
     };
     std::vector<std::thread> ts;
     ts.reserve(threads - 1);
-    for (unsigned t = 1; t < threads; ++t) ts.emplace_back(body, t);
+    try {
+        for (unsigned t = 1; t < threads; ++t) ts.emplace_back(body, t);
+    } catch (const std::system_error &) {  // no more threads: the chunks go to those there are
+    }
     body(0);
     for (auto &t : ts) t.join();
     if (err) std::rethrow_exception(err);
@@ -146,7 +149,11 @@ void parallel_for(uint64_t n, uint64_t grain, unsigned threads,
 
 WorkerPool::WorkerPool(unsigned n) {
     if (n == 0) n = default_threads();
-    for (unsigned i = 1; i < n; ++i) workers_.push_back(new std::thread(&WorkerPool::loop, this, i));
+    workers_.reserve(n);
+    try {
+        for (unsigned i = 1; i < n; ++i) workers_.push_back(new std::thread(&WorkerPool::loop, this, i));
+    } catch (const std::system_error &) {  // no more threads: the pool has those there are
+    }
 }
 
 WorkerPool::~WorkerPool() {
